@@ -314,7 +314,7 @@ __device__ __forceinline__ void wave_ranks_for(int E, const int (&id)[kTopK], in
 __global__ __launch_bounds__(kDispThreads) void dispatch_scatter_kernel(
     const int *__restrict__ topk_i, const int *__restrict__ pos, int T, int E,
     const int *__restrict__ blk_counts, int n_blk, int *__restrict__ perm, int *__restrict__ rowmap,
-    int *__restrict__ inv, int n_ct_gate_up, int n_ct_down, PlanOut plan) {
+    int *__restrict__ inv, int *__restrict__ blk_expert, int n_ct_gate_up, int n_ct_down, PlanOut plan) {
   __shared__ int wave_cnt[kDispThreads / 64][256];
   __shared__ int sh_base[256], sh_off[256], sh_row0[256];
   __shared__ ExpertInfo sh_info[256];
@@ -379,6 +379,7 @@ __global__ __launch_bounds__(kDispThreads) void dispatch_scatter_kernel(
     const int prow = sh_row0[e] + r;
     perm[sh_off[e] + r] = a;
     rowmap[prow] = a;
+    if (blk_expert && prow % kRowBlock == 0) blk_expert[prow / kRowBlock] = e;
     out_inv[k] = prow;
   }
   *reinterpret_cast<int4 *>(inv + (size_t)t * kTopK) =
@@ -394,7 +395,7 @@ constexpr int kSmallRounds = 1;
 __global__ __launch_bounds__(kDispThreads) void dispatch_small_kernel(
     const int *__restrict__ topk_i, const int *__restrict__ pos, int T, int E, int n_ct_gate_up,
     int n_ct_down, PlanOut out, int *__restrict__ perm, int *__restrict__ rowmap,
-    int *__restrict__ inv) {
+    int *__restrict__ inv, int *__restrict__ blk_expert) {
   __shared__ int hist[kSmallRounds][256];  // per round and expert: count, then exclusive base
   __shared__ int sh_off[256], sh_row0[256];
   __shared__ int wave_cnt[kDispThreads / 64][256];
@@ -466,6 +467,7 @@ __global__ __launch_bounds__(kDispThreads) void dispatch_small_kernel(
         const int prow = sh_row0[e] + rk;
         perm[sh_off[e] + rk] = t * kTopK + k;
         rowmap[prow] = t * kTopK + k;
+        if (blk_expert && prow % kRowBlock == 0) blk_expert[prow / kRowBlock] = e;
         out_inv[k] = prow;
       }
       *reinterpret_cast<int4 *>(inv + (size_t)t * kTopK) =
@@ -488,16 +490,12 @@ __global__ __launch_bounds__(kDispThreads) void dispatch_small_kernel(
 // DIRECT: there was no dispatch pass (see DirectIds).  The row of assignment
 // (t, k) is its expert's slot plus the number of lower assignments of the batch
 // with the same expert, which the workgroup's 256 threads count with a ballot.
-// SPLIT: the down GEMM summed its reduction in two parts (down_k_split); the
-// second part's rows lie part_stride floats behind the first's and are added to
-// them before the weighting.
-template <bool RESID, bool DIRECT, bool SPLIT>
+template <bool RESID, bool DIRECT>
 __global__ __launch_bounds__(256) void combine_kernel(const float *__restrict__ y,
                                                      const int *__restrict__ inv,
                                                      const float *__restrict__ topk_v,
                                                      const int *__restrict__ pos, void *outp, int H,
-                                                     int ldy, int accumulate, DirectIds ids,
-                                                     size_t part_stride) {
+                                                     int ldy, int accumulate, DirectIds ids) {
   const int t = blockIdx.x;
   const bool active = !(pos && pos[t] < 0);
   if (!active && (accumulate || RESID)) return;
@@ -537,11 +535,7 @@ __global__ __launch_bounds__(256) void combine_kernel(const float *__restrict__ 
 #pragma unroll
     for (int k = 0; k < kTopK; k++) {
       if (p[k] >= 0) {
-        float4 v = reinterpret_cast<const float4 *>(y + (size_t)p[k] * ldy)[c];
-        if (SPLIT) {
-          const float4 v2 = reinterpret_cast<const float4 *>(y + part_stride + (size_t)p[k] * ldy)[c];
-          v.x += v2.x; v.y += v2.y; v.z += v2.z; v.w += v2.w;
-        }
+        const float4 v = reinterpret_cast<const float4 *>(y + (size_t)p[k] * ldy)[c];
         s.x += w[k] * v.x; s.y += w[k] * v.y; s.z += w[k] * v.z; s.w += w[k] * v.w;
       }
     }
@@ -576,46 +570,35 @@ hipError_t launch_dispatch(const int *topk_i, const int *pos, int T, int E, int 
   if (n_blk <= kSmallRounds) {
     // small batches: one workgroup does both passes, one launch fewer
     dispatch_small_kernel<<<1, kDispThreads, 0, s>>>(topk_i, pos, T, E, n_ct_gate_up, n_ct_down, plan,
-                                                     d.perm, d.rowmap, d.inv);
+                                                     d.perm, d.rowmap, d.inv, d.blk_expert);
     return hipGetLastError();
   }
   dispatch_count_kernel<<<n_blk, kDispThreads, 0, s>>>(topk_i, pos, T, E, d.blk_counts, d.rowmap,
                                                        fill_rows, d.perm);
   dispatch_scatter_kernel<<<n_blk, kDispThreads, 0, s>>>(topk_i, pos, T, E, d.blk_counts, n_blk, d.perm,
-                                                         d.rowmap, d.inv, n_ct_gate_up, n_ct_down, plan);
+                                                         d.rowmap, d.inv, d.blk_expert, n_ct_gate_up, n_ct_down, plan);
   return hipGetLastError();
 }
 
 template <bool RESID>
-static hipError_t launch_combine_any(const float *y, int ldy, int y_parts, size_t part_stride, const int *inv,
-                                     const float *topk_v, const int *pos, void *out, int T, int H,
-                                     int accumulate, const DirectIds &direct, hipStream_t s) {
-  static_assert(kSmallBatchKSplit == 2, "the combine adds two parts");
-  if (y_parts != 1 && y_parts != kSmallBatchKSplit) return hipErrorInvalidValue;
-  const bool split = y_parts == 2;
-#define MOE_COMBINE(DIRECT, SPLIT)                                                                             \
-  combine_kernel<RESID, DIRECT, SPLIT><<<T, 256, 0, s>>>(y, inv, topk_v, pos, out, H, ldy, accumulate, direct, \
-                                                         part_stride)
-  if (direct.topk_i) {
-    if (split) MOE_COMBINE(true, true); else MOE_COMBINE(true, false);
-  } else {
-    if (split) MOE_COMBINE(false, true); else MOE_COMBINE(false, false);
-  }
-#undef MOE_COMBINE
+static hipError_t launch_combine_any(const float *y, int ldy, const int *inv, const float *topk_v, const int *pos,
+                                     void *out, int T, int H, int accumulate, const DirectIds &direct,
+                                     hipStream_t s) {
+  if (direct.topk_i)
+    combine_kernel<RESID, true><<<T, 256, 0, s>>>(y, inv, topk_v, pos, out, H, ldy, accumulate, direct);
+  else
+    combine_kernel<RESID, false><<<T, 256, 0, s>>>(y, inv, topk_v, pos, out, H, ldy, accumulate, direct);
   return hipGetLastError();
 }
 
-hipError_t launch_combine(const float *y, int ldy, int y_parts, size_t part_stride, const int *inv,
-                          const float *topk_v, const int *pos, float *out, int T, int H, int accumulate,
-                          const DirectIds &direct, hipStream_t s) {
-  return launch_combine_any<false>(y, ldy, y_parts, part_stride, inv, topk_v, pos, out, T, H, accumulate, direct,
-                                   s);
+hipError_t launch_combine(const float *y, int ldy, const int *inv, const float *topk_v, const int *pos, float *out,
+                          int T, int H, int accumulate, const DirectIds &direct, hipStream_t s) {
+  return launch_combine_any<false>(y, ldy, inv, topk_v, pos, out, T, H, accumulate, direct, s);
 }
 
-hipError_t launch_combine_residual(const float *y, int ldy, int y_parts, size_t part_stride, const int *inv,
-                                   const float *topk_v, const int *pos, uint16_t *x, int T, int H,
-                                   const DirectIds &direct, hipStream_t s) {
-  return launch_combine_any<true>(y, ldy, y_parts, part_stride, inv, topk_v, pos, x, T, H, 0, direct, s);
+hipError_t launch_combine_residual(const float *y, int ldy, const int *inv, const float *topk_v, const int *pos,
+                                   uint16_t *x, int T, int H, const DirectIds &direct, hipStream_t s) {
+  return launch_combine_any<true>(y, ldy, inv, topk_v, pos, x, T, H, 0, direct, s);
 }
 
 }  // namespace moe

@@ -9,8 +9,9 @@
 // gate_up epilogue), ordered [row block of 32][k block of 16]: every global load
 // is a contiguous 16 bytes per lane and is already in register order.  The row
 // operand of gate_up is the token rows themselves, bf16 row-major, found through
-// the dispatch's row map: there is no gathered copy (gemm_tile_gl for the large
-// batches, the GATHER form of gemm_tile for the small ones).
+// the dispatch's row map: there is no gathered copy (gemm_tile_gl).
+//
+// Batches with few rows per expert run the kernels of stream.hip instead.
 //
 // Tiling.  A workgroup of NW waves owns a tile of (RBT*32) rows x
 // (NW*NBW*32) columns of one expert.  The waves split the columns only: each
@@ -25,28 +26,26 @@
 //     ring by DMA (global_load_lds_dwordx4), R-1 steps ahead of the MFMAs;
 //   * the column operand is private to a wave in this layout, so it never
 //     touches LDS: it is loaded into an R-slot ring of VGPRs, R-1 steps ahead.
-// The full-height configuration runs R = 4 (3 steps x 32 KB = 96 KB in flight
+// R is 4 (3 steps x 32 KB = 96 KB in flight
 // per CU: measured against 3, 5, 6 and 7, a deeper ring gains nothing in the
 // main loop and costs the time its longer fill takes at the start of every
 // tile, 0.7 % of the layer per stage at 4096 tokens; with 3 the main loop
-// starves); the small-batch configuration, a stream of weights through two or
-// three workgroups per CU, runs R = 7.  These loads
+// starves).  These loads
 // complete in the order they were issued, so waiting for "all but the newest n"
 // (s_waitcnt vmcnt(n)) picks out exactly the step that is needed next and
-// leaves the later ones in flight (the GATHER variant of gemm_tile counts
-// differently, see there).
+// leaves the later ones in flight.
 //
 // Tile order.  Workgroup ids are dealt round-robin to the 8 XCDs, each with
 // its own L2.  Logical tile ids are laid out (expert, group of up to four row
 // tiles, column tile, row tile) with the row tile fastest, and XCD x takes a
 // contiguous range of them (see build_plan and write_expert_tiles: about an
 // eighth by estimated cost): the tiles an XCD runs at one time share a few row
-// tiles of the expert and a few column slabs of its weights.  (Batches of at most 64 tokens
-// have no tile table at all: see DIRECT at the kernel.)
+// tiles of the expert and a few column slabs of its weights.
 #include <type_traits>
 #include <utility>
 
 #include "moe_internal.h"
+#include "swiglu.h"
 
 namespace moe {
 
@@ -66,26 +65,9 @@ __device__ __forceinline__ void static_for(F &&f) {
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
-// run.cpp:709-726: gate clamped from above, up clamped on both sides, then
-// gate * sigmoid(alpha * gate) * (up + 1).  u1 is up + 1 already (the 1 rides
-// in the accumulator's start value together with the bias).
-__device__ __forceinline__ float swiglu_shifted(float g, float u1, float limit) {
-  constexpr float kNegAlphaLog2e = -kAlpha * 1.4426950408889634f;
-  g = fminf(g, limit);
-  u1 = __builtin_amdgcn_fmed3f(u1, 1.0f - limit, 1.0f + limit);
-  const float s = __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(kNegAlphaLog2e * g));
-  return g * s * u1;
-}
-
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-
-// two floats -> packed bf16, round to nearest even (v_cvt_pk_bf16_f32); a in the low half
-__device__ __forceinline__ uint32_t pack_bf16(float a, float b) {
-  f32x2 v = {a, b};
-  return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2));
-}
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
@@ -187,15 +169,12 @@ struct StageRing {
 
 // NW waves side by side over the columns, NBW column blocks per wave, R ring
 // slots (LDS stages for the row operand, register slots for the column operand).
-// RBM = row blocks per tile at most: it sizes the LDS stages, and with them how
-// many workgroups share a CU; WAVES = waves per SIMD the registers are held to.
-template <int NW_, int NBW_, int R_, int RBM_ = kTileRows / kRowBlock, int WAVES_ = 1>
+template <int NW_, int NBW_, int R_>
 struct GemmCfg {
   static constexpr int NW = NW_, NBW = NBW_, R = R_, KPS = 2;
   static constexpr int THREADS = NW * 64;
-  static constexpr int WAVES = WAVES_;
   static constexpr int TILE_NB = NW * NBW;              // column blocks per tile
-  static constexpr int RBT_MAX = RBM_;                   // row blocks per tile, at most
+  static constexpr int RBT_MAX = kTileRows / kRowBlock;  // row blocks per tile, at most
   static constexpr int STAGE = RBT_MAX * KPS * 64;       // uint4 per LDS stage (16 KB)
   static constexpr int EPI_LD = NBW * 32 + 8;            // floats per buffered output row
   static constexpr int EPI_WAVE = 32 * EPI_LD / 4;       // uint4 per wave of epilogue buffer
@@ -217,34 +196,21 @@ struct GemmCfg {
 // wave, RBT * RS are staged per step (blocks past the tile's rbt repeat its
 // last one and are not stored).
 //
-// GATHER (gate_up of the small-batch configuration): the row operand's DMA reads
-// the token rows themselves, every lane at the address of its own row (rowmap)
-// -- 32 bytes per row and instruction instead of 1 KB in one piece.  While the
-// GEMM is a stream of weights that is free; on tiles 4 to 8 row blocks high the
-// address work of 32 cache lines per instruction costs the main loop a quarter,
-// which is why the large batches fetch whole lines (gemm_tile_gl).  Here the
-// waits count DMA only (see WAIT_DMA_*).
-template <int RBT, int RS, typename C, bool GATE_UP, bool FP4, bool GATHER>
-__device__ __forceinline__ void gemm_tile(const uint4 *__restrict__ a_frag,  // [rb][KB][64]; GATHER: token rows [T][KB*2]
+// gemm_tile is the down GEMM; gate_up, whose row operand is scattered, is
+// gemm_tile_gl below.
+template <int RBT, int RS, typename C, bool FP4>
+__device__ __forceinline__ void gemm_tile(const uint4 *__restrict__ a_frag,  // [rb][KB][64]
                                           const uint4 *__restrict__ b_frag,  // expert: [nb][KB][64], FP4: [nb/2][KB/2][64]
                                           const uint16_t *__restrict__ b_scale,  // FP4: expert's [nb/2][KB/2][32] byte pairs
                                           int KB, int rb0, int rbt, int nb0, int nb_valid,
-                                          // the part of the reduction this workgroup sums: steps (of 32 k)
-                                          // [ks_begin, ks_begin + ks_count); the bias goes in with the first
-                                          int ks_begin, int ks_count,
-                                          const int *__restrict__ rowmap,    // GATHER: padded row -> assignment
-                                          int map_rb0,                       // row block that rowmap[0] belongs to
-                                          const float *__restrict__ bias_a,  // gate / down bias (expert)
-                                          const float *__restrict__ bias_b,  // up bias (expert)
-                                          void *__restrict__ outp, int out_ld, float limit,
+                                          const float *__restrict__ bias,  // expert's
+                                          float *__restrict__ y, int out_ld,
                                           // One __restrict__ pointer per LDS stage: after
                                           // inlining the compiler can tell a read of one stage
                                           // from the DMA that fills another and waits only for
                                           // the fill of the stage it reads.
                                           uint4 *__restrict__ s0, uint4 *__restrict__ s1,
                                           uint4 *__restrict__ s2, uint4 *__restrict__ s3,
-                                          uint4 *__restrict__ s4, uint4 *__restrict__ s5,
-                                          uint4 *__restrict__ s6,
                                           // The epilogue buffers are not carved out of the
                                           // ring: the compiler would make every read of them
                                           // wait for all outstanding vector memory operations,
@@ -252,7 +218,7 @@ __device__ __forceinline__ void gemm_tile(const uint4 *__restrict__ a_frag,  // 
                                           uint4 *__restrict__ epi) {
   StageRing<C::R> ring;
   {
-    uint4 *const all[7] = {s0, s1, s2, s3, s4, s5, s6};
+    uint4 *const all[4] = {s0, s1, s2, s3};
 #pragma unroll
     for (int i = 0; i < C::R; i++) ring.p[i] = all[i];
   }
@@ -275,78 +241,35 @@ __device__ __forceinline__ void gemm_tile(const uint4 *__restrict__ a_frag,  // 
   const int cw = RS == 1 ? w : w % (NW / RS);  // the wave's place among the columns
   const int rg = RS == 1 ? 0 : w / (NW / RS);  // ... and among the row groups
 
-  // The accumulators start from the bias (the up half of gate_up from bias + 1,
-  // see swiglu_shifted).  gate_up computes the transposed product (weights as
-  // the MFMA's first operand): register q of lane l is then weight row
-  // 8*(q/4) + 4*(l/32) + q%4 of its block and token l % 32.  down computes the
-  // product as it is: register q is token 8*(q/4) + 4*(l/32) + q%4, lane l
-  // column l % 32.  The bias loads go out first and are consumed after the
-  // pipeline's loads have been issued.
-  static_assert(!GATE_UP || NBW % 2 == 0, "gate and up blocks of a pair must sit in one wave");
-  float4 bias_g[NBW / 2 + 1][4], bias_u[NBW / 2 + 1][4];
+  // The accumulators start from the bias.  Register q of lane l is token
+  // 8*(q/4) + 4*(l/32) + q%4 of its row block, lane l column l % 32.  The bias
+  // loads go out first and are consumed after the pipeline's loads have been issued.
   float bias_d[NBW];
-  if (GATE_UP) {
-    // a wave past the matrix's last column (last column tile only) reads the
-    // last valid pair's bias: the expert's bias vector ends there
-    const int P_last = ((nb0 + nb_valid) >> 1) - 1;
-    const int P0 = (nb0 + cw * NBW) >> 1;
 #pragma unroll
-    for (int p = 0; p < NBW / 2; p++) {
-      const int P = min(P0 + p, P_last);
-#pragma unroll
-      for (int g = 0; g < 4; g++) {
-        const int j = kRowBlock * P + 8 * g + 4 * (lane >> 5);
-        bias_g[p][g] = *reinterpret_cast<const float4 *>(bias_a + j);
-        bias_u[p][g] = *reinterpret_cast<const float4 *>(bias_b + j);
-      }
-    }
-  } else {
-#pragma unroll
-    for (int j = 0; j < NBW; j++)
-      bias_d[j] = ks_begin == 0 ? bias_a[kRowBlock * (nb0 + min(cw * NBW + j, nb_valid - 1)) + (lane & 31)] : 0.f;
-  }
+  for (int j = 0; j < NBW; j++) bias_d[j] = bias[kRowBlock * (nb0 + min(cw * NBW + j, nb_valid - 1)) + (lane & 31)];
   f32x16 acc[RBT][NBW];
 
-  const int steps_total = KB / KPS;
-  const int n_steps = ks_count;
-  const uint4 *a_src = a_frag + ((size_t)rb0 * KB + ks_begin * KPS) * 64 + lane;
-  // GATHER: per DMA of a step, this lane's place in its token's row (16-byte
-  // units: a row is KB * 2 of them, a k block 2, the lane's half of it 1).
-  // Padding rows read token 0; their products are never used.
-  uint32_t lane_off[LA];
-  if (GATHER) {
-#pragma unroll
-    for (int m = 0; m < LA; m++) {
-      const int c = min(m * NW + w, A_CH - 1);
-      const int blk = RS == 1 ? c / KPS : min(c / KPS, rbt - 1);
-      const int a = rowmap[(rb0 - map_rb0 + blk) * kRowBlock + (lane & 31)];
-      const int tok = a >= 0 ? a / kTopK : 0;
-      lane_off[m] = (uint32_t)tok * (uint32_t)(KB * 2) + (ks_begin * KPS + c % KPS) * 2 + (lane >> 5);
-    }
-  }
+  const int n_steps = KB / KPS;
+  const uint4 *a_src = a_frag + (size_t)rb0 * KB * 64 + lane;
   // Column blocks past the end of the matrix (last column tile only) re-load
   // the last valid block; their products are never stored.
   const uint4 *b_src[NBW];
   const uint16_t *s_src = nullptr;
   if (FP4) {
     const size_t pair = (size_t)((nb0 + min(cw * NBW, nb_valid - NBW)) >> 1);
-    b_src[0] = b_frag + (pair * steps_total + ks_begin) * 64 + lane;
-    s_src = b_scale + (pair * steps_total + ks_begin) * 32 + (lane & 31);
+    b_src[0] = b_frag + pair * n_steps * 64 + lane;
+    s_src = b_scale + pair * n_steps * 32 + (lane & 31);
   } else {
 #pragma unroll
     for (int j = 0; j < NBW; j++)
-      b_src[j] = b_frag + ((size_t)(nb0 + min(cw * NBW + j, nb_valid - 1)) * KB + ks_begin * KPS) * 64 + lane;
+      b_src[j] = b_frag + (size_t)(nb0 + min(cw * NBW + j, nb_valid - 1)) * KB * 64 + lane;
   }
 
   // Row operand: chunk c of a step (c = pass*NW + wave) is row block c / KPS, k block c % KPS.
   auto issue_a = [&](uint4 *st, int ks, int m) {
     const int c = min(m * NW + w, A_CH - 1);
     const int blk = RS == 1 ? c / KPS : min(c / KPS, rbt - 1);
-    if (GATHER) {
-      dma_to_lds_16(a_frag + lane_off[m] + ks * (KPS * 2), st + c * 64);
-    } else {
-      dma_to_lds_16(a_src + ((size_t)blk * KB + ks * KPS + c % KPS) * 64, st + c * 64);
-    }
+    dma_to_lds_16(a_src + ((size_t)blk * KB + ks * KPS + c % KPS) * 64, st + c * 64);
   };
   // Column operand: register m of a slot is column block m / KPS, k block m % KPS.
   // FP4: load 0 of a slot is the chunk of nibbles, load 1 the two scale bytes.
@@ -383,8 +306,7 @@ __device__ __forceinline__ void gemm_tile(const uint4 *__restrict__ a_frag,  // 
     fa[buf][i] = __builtin_bit_cast(bf16x8, st[((i * RS + rg) * KPS + kk) * 64 + lane]);
   };
   auto mma = [](bf16x8 rows, bf16x8 colv, f32x16 c) {
-    return GATE_UP ? __builtin_amdgcn_mfma_f32_32x32x16_bf16(colv, rows, c, 0, 0, 0)
-                   : __builtin_amdgcn_mfma_f32_32x32x16_bf16(rows, colv, c, 0, 0, 0);
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(rows, colv, c, 0, 0, 0);
   };
   // column operand of (slot, column block j, k block kk)
   auto cols_of = [&](int slot, int j, int kk) {
@@ -394,19 +316,13 @@ __device__ __forceinline__ void gemm_tile(const uint4 *__restrict__ a_frag,  // 
       return __builtin_bit_cast(bf16x8, bq[slot][j * KPS + kk]);
     }
   };
-  static_assert(R >= 3 && R <= 7, "up to seven stage arrays are passed in");
+  static_assert(R >= 3 && R <= 4, "up to four stage arrays are passed in");
   // "Step s of the row operand has landed" as a bound on the vector-memory
   // counter.  The loads are issued in the order A(0) B(0) A(1) B(1) ... and
   // complete in that order, so all but the newest n outstanding means step s has
-  // landed with n = everything issued behind it.  With the scattered DMA of the
-  // GATHER form and the mixed count, wrong token rows were once seen in this
-  // configuration (several workgroups per CU, ring of 7), different from run to
-  // run; the cause was never established (the same scattered DMA with the mixed
-  // count gives the same bits in every run on the large batches).  Here the
-  // bound counts the DMAs behind step s only, which holds whatever the register
-  // loads do and costs nothing while the tile is a stream of weights.
-  constexpr int WAIT_DMA_FILL = GATHER ? LA * (R - 1) : LPS * (R - 2) + LA;  // A(0), A(0..R-1) issued
-  constexpr int WAIT_DMA_STEP = GATHER ? LA * (R - 2) : LPS * (R - 2);       // A(ks+1) at step ks
+  // landed with n = everything issued behind it.
+  constexpr int WAIT_DMA_FILL = LPS * (R - 2) + LA;  // A(0), A(0..R-1) issued
+  constexpr int WAIT_DMA_STEP = LPS * (R - 2);       // A(ks+1) at step ks
 
   // Issue order per wave: A(0) B(0) A(1) B(1) ... ; at the top of step ks the row
   // operand is issued through step ks+R-1 and the column operand through ks+R-2
@@ -420,27 +336,12 @@ __device__ __forceinline__ void gemm_tile(const uint4 *__restrict__ a_frag,  // 
     for (int m = 0; m < LB; m++) issue_b(s, min(s, last), m);
     __builtin_amdgcn_sched_barrier(0);  // the counted waits rely on this issue order
   }
-  if (GATE_UP) {
 #pragma unroll
-    for (int p = 0; p < NBW / 2; p++)
+  for (int j = 0; j < NBW; j++)
 #pragma unroll
-      for (int g = 0; g < 4; g++)
+    for (int i = 0; i < RBT; i++)
 #pragma unroll
-        for (int i = 0; i < RBT; i++) {
-          const float4 bg = bias_g[p][g], bu = bias_u[p][g];
-          acc[i][2 * p][4 * g + 0] = bg.x; acc[i][2 * p][4 * g + 1] = bg.y;
-          acc[i][2 * p][4 * g + 2] = bg.z; acc[i][2 * p][4 * g + 3] = bg.w;
-          acc[i][2 * p + 1][4 * g + 0] = bu.x + 1.0f; acc[i][2 * p + 1][4 * g + 1] = bu.y + 1.0f;
-          acc[i][2 * p + 1][4 * g + 2] = bu.z + 1.0f; acc[i][2 * p + 1][4 * g + 3] = bu.w + 1.0f;
-        }
-  } else {
-#pragma unroll
-    for (int j = 0; j < NBW; j++)
-#pragma unroll
-      for (int i = 0; i < RBT; i++)
-#pragma unroll
-        for (int q = 0; q < 16; q++) acc[i][j][q] = bias_d[j];
-  }
+      for (int q = 0; q < 16; q++) acc[i][j][q] = bias_d[j];
 #pragma unroll
   for (int m = 0; m < LA; m++) issue_a(ring.p[R - 1], min(R - 1, last), m);
   WAIT_VMCNT(WAIT_DMA_FILL);
@@ -512,57 +413,31 @@ __device__ __forceinline__ void gemm_tile(const uint4 *__restrict__ a_frag,  // 
 
   // Epilogue.
   if (cw * NBW >= nb_valid) return;  // a wave without columns (last column tile only)
-  if (GATE_UP) {
-    gate_up_epilogue<RBT, RS, C>(acc, outp, out_ld, limit, rb0, rbt, nb0, nb_valid, cw, rg, lane);
-  } else if constexpr (C::RBT_MAX == 2) {
-    // Small-batch configuration: the rows go out straight from the accumulators
-    // (register q of lane l is token 8*(q/4) + 4*(l/32) + q%4, column l % 32: a
-    // store writes two rows of 128 contiguous bytes).  No LDS buffer, so that a
-    // third workgroup fits a CU; at full tile height the two forms take the same
-    // time.
-    static_assert(RS == 1, "the small-batch configuration has no row split");
-    float *y = reinterpret_cast<float *>(outp);
-    const int n = lane & 31;
-    const int rsub = 4 * (lane >> 5);
+  constexpr int LD = C::EPI_LD;  // +8 floats keep the two lane halves on different banks
+  float *ef = reinterpret_cast<float *>(epi + w * C::EPI_WAVE);
+  const int n = lane & 31;
+  const int rsub = 4 * (lane >> 5);
+  const int col0 = kRowBlock * (nb0 + cw * NBW);
 #pragma unroll
-    for (int i = 0; i < RBT; i++) {
-      const size_t row0 = (size_t)(rb0 + i) * kRowBlock;
+  for (int i = 0; i < RBT; i++) {
+    const int blk = i * RS + rg;
+    if (RS > 1 && blk >= rbt) break;
 #pragma unroll
-      for (int j = 0; j < NBW; j++) {
-        if (cw * NBW + j >= nb_valid) continue;
-        float *dst = y + row0 * out_ld + kRowBlock * (nb0 + cw * NBW + j) + n;
+    for (int j = 0; j < NBW; j++)
 #pragma unroll
-        for (int q = 0; q < 16; q++) dst[(size_t)(8 * (q >> 2) + rsub + (q & 3)) * out_ld] = acc[i][j][q];
+      for (int q = 0; q < 16; q++) {
+        const int r = 8 * (q >> 2) + rsub + (q & 3);
+        ef[r * LD + 32 * j + n] = acc[i][j][q];
       }
-    }
-  } else {
-    constexpr int LD = C::EPI_LD;  // +8 floats keep the two lane halves on different banks
-    float *y = reinterpret_cast<float *>(outp);
-    float *ef = reinterpret_cast<float *>(epi + w * C::EPI_WAVE);
-    const int n = lane & 31;
-    const int rsub = 4 * (lane >> 5);
-    const int col0 = kRowBlock * (nb0 + cw * NBW);
+    const size_t row0 = (size_t)(rb0 + blk) * kRowBlock;
 #pragma unroll
-    for (int i = 0; i < RBT; i++) {
-      const int blk = i * RS + rg;
-      if (RS > 1 && blk >= rbt) break;
-#pragma unroll
-      for (int j = 0; j < NBW; j++)
-#pragma unroll
-        for (int q = 0; q < 16; q++) {
-          const int r = 8 * (q >> 2) + rsub + (q & 3);
-          ef[r * LD + 32 * j + n] = acc[i][j][q];
-        }
-      const size_t row0 = (size_t)(rb0 + blk) * kRowBlock;
-#pragma unroll
-      for (int t = 0; t < NBW * 4; t++) {
-        const int idx = t * 64 + lane;
-        const int r = idx / (NBW * 8);
-        const int c4 = idx % (NBW * 8);
-        const float4 v = *reinterpret_cast<const float4 *>(ef + r * LD + 4 * c4);
-        if (cw * NBW + c4 / 8 < nb_valid)
-          *reinterpret_cast<float4 *>(y + (row0 + r) * out_ld + col0 + 4 * c4) = v;
-      }
+    for (int t = 0; t < NBW * 4; t++) {
+      const int idx = t * 64 + lane;
+      const int r = idx / (NBW * 8);
+      const int c4 = idx % (NBW * 8);
+      const float4 v = *reinterpret_cast<const float4 *>(ef + r * LD + 4 * c4);
+      if (cw * NBW + c4 / 8 < nb_valid)
+        *reinterpret_cast<float4 *>(y + (row0 + r) * out_ld + col0 + 4 * c4) = v;
     }
   }
 }
@@ -573,7 +448,7 @@ constexpr int kLineStages = 4;
 // gate_up of the large batches without a gathered copy of the routed rows: the
 // row operand's DMA reads the token rows themselves, WHOLE CACHE LINES at a time.
 // One instruction fetches 8 rows x 128 bytes (64 k); a scattered DMA that takes
-// 32 bytes of 32 rows per instruction (the small-batch form in gemm_tile) costs
+// 32 bytes of 32 rows per instruction costs
 // the main loop a quarter more, and 64 bytes of 16 rows an eighth.
 //
 // So the row operand is staged in double steps: a double stage holds 64 k of
@@ -837,77 +712,22 @@ __device__ __forceinline__ void gemm_tile_gl(const uint4 *__restrict__ x_rows,  
   gate_up_epilogue<RBT, RS, C>(acc, outp, out_ld, limit, rb0, rbt, nb0, nb_valid, cw, rg, lane);
 }
 
-// DIRECT (small-batch configuration only): there is no plan.  A workgroup is
-// one column tile of one expert (see the mapping below); its 256 threads look at one
-// assignment of the batch each and find the expert's rows with a ballot (see
-// DirectIds).  An expert without rows ends its workgroups here.
-template <typename C, bool GATE_UP, bool FP4, bool GATHER, bool DIRECT = false>
-__global__ __launch_bounds__(C::THREADS, C::WAVES) void grouped_gemm_kernel(
+template <typename C, bool GATE_UP, bool FP4>
+__global__ __launch_bounds__(C::THREADS, 1) void grouped_gemm_kernel(
     const uint4 *__restrict__ a_frag, const uint4 *__restrict__ w_frag,
     const uint16_t *__restrict__ w_scale,
     const float *__restrict__ bias_a, const float *__restrict__ bias_b,
     const TileDesc *__restrict__ tiles, const int *__restrict__ totals,
-    const int *__restrict__ rowmap, void *__restrict__ outp, int K, int N, float limit,
-    DirectIds ids, size_t split_stride) {
-  static_assert(!GATHER || GATE_UP, "only the first GEMM reads token rows");
-  static_assert(!DIRECT || (C::RBT_MAX * kRowBlock == kDirectSlotRows && C::THREADS == kDirectTokens * kTopK),
-                "a direct batch: one thread per assignment, an expert's slot is one tile high");
-  constexpr int R = C::R;
-  static_assert(R <= 7, "seven stage arrays are declared below");
-  __shared__ uint4 st0[C::STAGE], st1[C::STAGE], st2[C::STAGE], st3[C::STAGE], st4[C::STAGE],
-      st5[C::STAGE], st6[C::STAGE], st7[C::STAGE];  // those a variant does not use take no room
-  __shared__ uint4 epi[C::RBT_MAX == 2 ? 1 : C::NW * C::EPI_WAVE];  // the small-batch configuration stores directly
+    const int *__restrict__ rowmap, void *__restrict__ outp, int K, int N, float limit) {
+  static_assert(C::R <= 4 && C::RBT_MAX == 8, "stage arrays and tile heights below");
+  __shared__ uint4 st0[C::STAGE], st1[C::STAGE], st2[C::STAGE], st3[C::STAGE];
+  __shared__ uint4 st4[GATE_UP ? C::STAGE : 1], st5[GATE_UP ? C::STAGE : 1], st6[GATE_UP ? C::STAGE : 1],
+      st7[GATE_UP ? C::STAGE : 1];
+  __shared__ uint4 epi[GATE_UP ? 1 : C::NW * C::EPI_WAVE];
   const int KB = K / kFragK;
   const int nb_total = (GATE_UP ? 2 * N : N) / kRowBlock;  // weight row blocks per expert
-  const int n_ct = (nb_total + C::TILE_NB - 1) / C::TILE_NB;
   TileDesc tc;
-  __shared__ int direct_rows[kDirectSlotRows];  // slot row -> assignment, -1 = padding
-  __shared__ int direct_cnt[C::NW];
-  const int *map = rowmap;
-  if constexpr (DIRECT) {
-    const int tid = threadIdx.x;
-    // Workgroup ids are dealt round-robin to the 8 XCDs: XCD x takes the experts
-    // x, x + 8, ..., all column tiles of an expert, so that the expert's rows
-    // (which every one of its column tiles reads) are fetched into one L2
-    // instead of eight.
-    const int xcd = blockIdx.x & (kXcds - 1), idx = blockIdx.x >> 3;
-    const int e = (idx / n_ct) * kXcds + xcd;
-    if (e >= ids.E) return;  // surplus workgroups of the grid (experts not a multiple of 8)
-    const bool mine = direct_expert_of(ids, tid) == e;
-    const unsigned long long bal = __ballot(mine);
-    if ((tid & 63) == 0) direct_cnt[tid >> 6] = __popcll(bal);
-    if (tid < kDirectSlotRows) direct_rows[tid] = -1;
-    __syncthreads();
-    int before = 0, count = 0;
-#pragma unroll
-    for (int ww = 0; ww < C::NW; ww++) {
-      const int c = direct_cnt[ww];
-      if (ww < (tid >> 6)) before += c;
-      count += c;
-    }
-    if (count == 0) return;
-    if (GATHER) {
-      const int r = before + __popcll(bal & ((1ull << (tid & 63)) - 1ull));
-      if (mine && r < kDirectSlotRows) direct_rows[r] = tid;
-      __syncthreads();
-      map = direct_rows;
-    }
-    tc.e = e;
-    tc.nt = idx % n_ct;
-    tc.rb0 = e * (kDirectSlotRows / kRowBlock);
-    tc.rbt = (min(count, kDirectSlotRows) + kRowBlock - 1) / kRowBlock;
-  } else {
-    if (!locate_tile(tiles, totals + (GATE_UP ? kTotBoundsGateUp : kTotBoundsDown), tc)) return;
-  }
-  const int map_rb0 = DIRECT ? tc.rb0 : 0;
-  // The down GEMM of the small-batch configuration splits the reduction over
-  // gridDim.y workgroups; part p writes its sums to its own copy of the output,
-  // split_stride bytes behind the one before (the combine adds the parts up).
-  const int steps_total = K / (kFragK * C::KPS);
-  const int ks_per = (steps_total + (int)gridDim.y - 1) / (int)gridDim.y;
-  const int ks_begin = GATE_UP ? 0 : (int)blockIdx.y * ks_per;
-  const int ks_count = GATE_UP ? steps_total : min(ks_per, steps_total - ks_begin);
-  if (!GATE_UP) outp = static_cast<char *>(outp) + (size_t)blockIdx.y * split_stride;
+  if (!locate_tile(tiles, totals + (GATE_UP ? kTotBoundsGateUp : kTotBoundsDown), tc)) return;
   const int nb0 = tc.nt * C::TILE_NB;
   const int nb_valid = min(C::TILE_NB, nb_total - nb0);
   // per expert: bf16 nb_total * KB fragments of 1 KB; MXFP4 (nb_total/2) * (KB/2) chunks of 1 KB
@@ -915,49 +735,42 @@ __global__ __launch_bounds__(C::THREADS, C::WAVES) void grouped_gemm_kernel(
   const uint16_t *b_scale = FP4 ? w_scale + (size_t)tc.e * nb_total * KB * 8 : nullptr;
   const float *ba = bias_a + (size_t)tc.e * N;
   const float *bb = GATE_UP ? bias_b + (size_t)tc.e * N : nullptr;
-  // large batches of gate_up read the token rows by whole cache lines (gemm_tile_gl)
-  constexpr bool LINES = GATHER && C::RBT_MAX == 8;
 #define MOE_TILE_RS(n, rs)                                                                                    \
   do {                                                                                                        \
-    if constexpr (LINES && rs <= 2) {                                                                         \
-      gemm_tile_gl<n, rs, C, FP4>(a_frag, b_frag, b_scale, KB, tc.rb0, tc.rbt, nb0, nb_valid, rowmap, ba, bb, \
-                                  outp, N, limit, st0, st1, st2, st3, st4, st5, st6, st7);                    \
+    if constexpr (GATE_UP) {                                                                                  \
+      if constexpr (rs <= 2)                                                                                  \
+        gemm_tile_gl<n, rs, C, FP4>(a_frag, b_frag, b_scale, KB, tc.rb0, tc.rbt, nb0, nb_valid, rowmap, ba,   \
+                                    bb, outp, N, limit, st0, st1, st2, st3, st4, st5, st6, st7);              \
     } else {                                                                                                  \
-      gemm_tile<n, rs, C, GATE_UP, FP4, GATHER>(a_frag, b_frag, b_scale, KB, tc.rb0, tc.rbt, nb0, nb_valid,   \
-                                                ks_begin, ks_count, map, map_rb0, ba, bb, outp, N, limit,     \
-                                                st0, st1, st2, st3, st4, st5, st6, epi);                      \
+      gemm_tile<n, rs, C, FP4>(a_frag, b_frag, b_scale, KB, tc.rb0, tc.rbt, nb0, nb_valid, ba,                \
+                               static_cast<float *>(outp), N, st0, st1, st2, st3, epi);                       \
     }                                                                                                         \
   } while (0)
 #define MOE_TILE(n) MOE_TILE_RS(n, 1)
-  if constexpr (C::RBT_MAX == 8) {
-    // the last column tile, when only a quarter or half of the waves have columns in it
-    const int rs = row_split_of(nb_valid, C::NW, C::NBW);
-    if (!GATE_UP && rs == 4) {  // gate_up comes in (gate, up) pairs of pairs: never a quarter
-      if (tc.rbt <= 4) MOE_TILE_RS(1, 4); else MOE_TILE_RS(2, 4);
-      return;
+  // the last column tile, when only a quarter or half of the waves have columns in it
+  const int rs = row_split_of(nb_valid, C::NW, C::NBW);
+  if (!GATE_UP && rs == 4) {  // gate_up comes in (gate, up) pairs of pairs: never a quarter
+    if (tc.rbt <= 4) MOE_TILE_RS(1, 4); else MOE_TILE_RS(2, 4);
+    return;
+  }
+  if (rs == 2) {
+    switch ((tc.rbt + 1) >> 1) {
+      case 1: MOE_TILE_RS(1, 2); break;
+      case 2: MOE_TILE_RS(2, 2); break;
+      case 3: MOE_TILE_RS(3, 2); break;
+      default: MOE_TILE_RS(4, 2); break;
     }
-    if (rs == 2) {
-      switch ((tc.rbt + 1) >> 1) {
-        case 1: MOE_TILE_RS(1, 2); break;
-        case 2: MOE_TILE_RS(2, 2); break;
-        case 3: MOE_TILE_RS(3, 2); break;
-        default: MOE_TILE_RS(4, 2); break;
-      }
-      return;
-    }
-    switch (tc.rbt) {
-      case 1: MOE_TILE(1); break;
-      case 2: MOE_TILE(2); break;
-      case 3: MOE_TILE(3); break;
-      case 4: MOE_TILE(4); break;
-      case 5: MOE_TILE(5); break;
-      case 6: MOE_TILE(6); break;
-      case 7: MOE_TILE(7); break;
-      default: MOE_TILE(8); break;
-    }
-  } else {
-    static_assert(C::RBT_MAX == 2, "tile heights of the small-batch configuration");
-    if (tc.rbt == 1) MOE_TILE(1); else MOE_TILE(2);
+    return;
+  }
+  switch (tc.rbt) {
+    case 1: MOE_TILE(1); break;
+    case 2: MOE_TILE(2); break;
+    case 3: MOE_TILE(3); break;
+    case 4: MOE_TILE(4); break;
+    case 5: MOE_TILE(5); break;
+    case 6: MOE_TILE(6); break;
+    case 7: MOE_TILE(7); break;
+    default: MOE_TILE(8); break;
   }
 #undef MOE_TILE
 #undef MOE_TILE_RS
@@ -968,76 +781,38 @@ __global__ __launch_bounds__(C::THREADS, C::WAVES) void grouped_gemm_kernel(
 using CfgGemm = GemmCfg<4, 2, 4>;
 static_assert(CfgGemm::RBT_MAX * kRowBlock == kTileRows && CfgGemm::TILE_NB == kGemmTileNb,
               "tile plan of build_plan");
-// Batches of at most 64 tokens: no expert has more than 64 rows, every tile is
-// one or two row blocks high and the GEMMs are a stream of weights.  What
-// limits that stream is the bytes one CU keeps in flight, so the same kernel is
-// built with LDS stages for two row blocks and registers for two waves per
-// SIMD, and several workgroups share a CU.
-using CfgGemmSmall = GemmCfg<4, 2, 7, 2, 2>;
-using CfgGemmSmallFp4 = GemmCfg<4, 2, 7, 2, 3>;
-constexpr int kSmallBatchTokens = CfgGemmSmall::RBT_MAX * kRowBlock;
 
 // w_scale == nullptr: w holds bf16 fragments; otherwise w holds MXFP4 chunks and
 // w_scale their scale bytes (pack_fp4_kernel).
-// CF: the configuration of the MXFP4 instance (its column operand's ring takes a
-// third of the registers, so the small-batch down GEMM, which has no LDS buffer
-// for its output, can be held to three waves per SIMD; holding gate_up to the
-// same bound changes nothing in its register count and cost it 3 us per call).
-template <typename C, bool GATE_UP, bool GATHER = false, bool DIRECT = false, typename CF = C>
-static hipError_t launch_gemm(const uint4 *a, const uint4 *w, const uint16_t *w_scale, const float *ba,
+template <bool GATE_UP>
+static hipError_t launch_gemm(const void *a, const void *w, const uint16_t *w_scale, const float *ba,
                               const float *bb, const DispatchBuffers &d, void *out, int K, int N,
-                              float limit, int mt_cap, const DirectIds &direct, int k_split,
-                              size_t split_stride, hipStream_t s) {
+                              float limit, int mt_cap, hipStream_t s) {
+  using C = CfgGemm;
   const int nb_total = (GATE_UP ? 2 * N : N) / kRowBlock;
   const int n_ct = (nb_total + C::TILE_NB - 1) / C::TILE_NB;
-  const dim3 grid(DIRECT ? kXcds * ((direct.E + kXcds - 1) / kXcds) * n_ct : kXcds * xcd_tile_cap(mt_cap * n_ct),
-                  GATE_UP ? 1 : k_split);
+  const int grid = kXcds * xcd_tile_cap(mt_cap * n_ct);
   const TileDesc *tiles = GATE_UP ? d.tiles_gate_up : d.tiles_down;
+  const uint4 *af = static_cast<const uint4 *>(a), *wf = static_cast<const uint4 *>(w);
   if (w_scale) {
-    grouped_gemm_kernel<CF, GATE_UP, true, GATHER, DIRECT><<<grid, CF::THREADS, 0, s>>>(
-        a, w, w_scale, ba, bb, tiles, d.totals, d.rowmap, out, K, N, limit, direct, split_stride);
+    grouped_gemm_kernel<C, GATE_UP, true><<<grid, C::THREADS, 0, s>>>(af, wf, w_scale, ba, bb, tiles, d.totals,
+                                                                      d.rowmap, out, K, N, limit);
   } else {
-    grouped_gemm_kernel<C, GATE_UP, false, GATHER, DIRECT><<<grid, C::THREADS, 0, s>>>(
-        a, w, nullptr, ba, bb, tiles, d.totals, d.rowmap, out, K, N, limit, direct, split_stride);
+    grouped_gemm_kernel<C, GATE_UP, false><<<grid, C::THREADS, 0, s>>>(af, wf, nullptr, ba, bb, tiles, d.totals,
+                                                                       d.rowmap, out, K, N, limit);
   }
   return hipGetLastError();
 }
 
 hipError_t launch_gate_up(const uint16_t *x, const void *w1, const uint16_t *w1_scale, const float *b1g,
                           const float *b1u, const DispatchBuffers &d, uint16_t *act, int H, int IM,
-                          float limit, int mt_cap, int max_rows, const DirectIds &direct, hipStream_t s) {
-  static_assert(kSmallBatchTokens == kSmallBatchRows, "small_batch() and the small-batch configuration");
-  const uint4 *w = reinterpret_cast<const uint4 *>(w1);
-  const uint4 *rows = reinterpret_cast<const uint4 *>(x);
-  if (direct.topk_i)
-    return launch_gemm<CfgGemmSmall, true, true, true>(rows, w, w1_scale, b1g, b1u, d, act, H, IM, limit,
-                                                       mt_cap, direct, 1, 0, s);
-  // either way the row operand is read from the token rows: 32 bytes of 32 rows per
-  // instruction in the small-batch configuration, whole lines of 8 rows otherwise
-  if (small_batch(max_rows))
-    return launch_gemm<CfgGemmSmall, true, true>(rows, w, w1_scale, b1g, b1u, d, act, H, IM, limit, mt_cap,
-                                                 direct, 1, 0, s);
-  return launch_gemm<CfgGemm, true, true>(rows, w, w1_scale, b1g, b1u, d, act, H, IM, limit, mt_cap, direct, 1, 0,
-                                          s);
+                          float limit, int mt_cap, hipStream_t s) {
+  return launch_gemm<true>(x, w1, w1_scale, b1g, b1u, d, act, H, IM, limit, mt_cap, s);
 }
 
 hipError_t launch_down(const uint16_t *act, const void *w2, const uint16_t *w2_scale, const float *b2,
-                       const DispatchBuffers &d, float *y, int H, int IM, int mt_cap, int max_rows,
-                       const DirectIds &direct, int k_split, size_t split_stride, hipStream_t s) {
-  const uint4 *a = reinterpret_cast<const uint4 *>(act);
-  const uint4 *w = reinterpret_cast<const uint4 *>(w2);
-  // The smallest batches: a workgroup is one stream of weights, and the few
-  // experts such a batch reaches leave most CUs without one.  Two workgroups
-  // per tile then sum half of the reduction each into their own copy of the
-  // rows (down_k_split; the combine adds the two parts).
-  const int ks = small_batch(max_rows) ? k_split : 1;
-  if (direct.topk_i)
-    return launch_gemm<CfgGemmSmall, false, false, true, CfgGemmSmallFp4>(a, w, w2_scale, b2, nullptr, d, y, IM, H,
-                                                                          0.f, mt_cap, direct, ks, split_stride, s);
-  if (small_batch(max_rows))
-    return launch_gemm<CfgGemmSmall, false, false, false, CfgGemmSmallFp4>(a, w, w2_scale, b2, nullptr, d, y, IM, H,
-                                                                           0.f, mt_cap, direct, ks, split_stride, s);
-  return launch_gemm<CfgGemm, false>(a, w, w2_scale, b2, nullptr, d, y, IM, H, 0.f, mt_cap, direct, 1, 0, s);
+                       const DispatchBuffers &d, float *y, int H, int IM, int mt_cap, hipStream_t s) {
+  return launch_gemm<false>(act, w2, w2_scale, b2, nullptr, d, y, IM, H, 0.f, mt_cap, s);
 }
 
 }  // namespace moe

@@ -72,9 +72,8 @@ struct moe_handle {
   // moe_get_dispatch that asks for the plan afterwards.  topk_i == nullptr: none.
   DirectIds unplanned{nullptr, nullptr, 0, 0};
   // expert pipeline
-  uint16_t *act = nullptr;  // SwiGLU output, bf16 fragments
-  float *y = nullptr;       // down output [a_pad_cap, Hp], then the second part of a split reduction
-  int y_parts = 1;          // copies of y the last down GEMM wrote (down_k_split)
+  uint16_t *act = nullptr;  // SwiGLU output, bf16: fragments or rows (stream_batch)
+  float *y = nullptr;       // down output [a_pad_cap, Hp]
   uint16_t *t_norm = nullptr;  // normalised rows of moe_block_forward [max_tokens, H], allocated on first use
   uint16_t *x_pad = nullptr;   // the batch's rows widened to Hp columns [max_tokens, Hp]; only where Hp != H
 
@@ -144,26 +143,29 @@ inline int down_col_tiles(const moe_handle *h) {
 // Stages 3-4 on the plan of the last dispatch: gate_up GEMM with the SwiGLU (it
 // reads the routed token rows itself, there is no gathered copy), down GEMM.
 // Leaves the per-assignment rows in h->y.
-// max_rows: no expert is given more rows than this (T when the ids of a token are distinct).
-int run_gemms(moe_handle *h, int layer, const uint16_t *x, int T, int max_rows, const DirectIds &direct,
-              hipStream_t s, StageTimer &tm) {
+int run_gemms(moe_handle *h, int layer, const uint16_t *x, int T, const DirectIds &direct, hipStream_t s,
+              StageTimer &tm) {
   const moe_config &c = h->cfg;
   const LayerWeights &lw = h->layers[layer];
-  const int A = T * kTopK;
-  const int mt_cap = A / kTileRows + c.experts;
+  const void *w1 = lw.w1q ? static_cast<const void *>(lw.w1q) : lw.w1;
+  const void *w2 = lw.w2q ? static_cast<const void *>(lw.w2q) : lw.w2;
   HIP_TRY(tm.mark(MOE_STAGE_GATE_UP));
   if (h->Hp != c.hidden) {  // a hidden size that is not a multiple of 64: rows widened with zeros
     HIP_TRY(launch_pad_rows(x, h->x_pad, T, c.hidden, h->Hp, s));
     x = h->x_pad;
   }
-  HIP_TRY(launch_gate_up(x, lw.w1q ? static_cast<const void *>(lw.w1q) : lw.w1, lw.w1s, lw.b1g, lw.b1u,
-                         h->disp, h->act, h->Hp, h->IMp, c.swiglu_limit, mt_cap, max_rows, direct, s));
+  if (stream_batch(T, c.experts)) {
+    const int tiles = stream_tile_cap(T, c.experts);
+    HIP_TRY(launch_stream_gate_up(x, w1, lw.w1s, lw.b1g, lw.b1u, h->disp, h->act, h->Hp, h->IMp, c.swiglu_limit,
+                                  tiles, direct, s));
+    HIP_TRY(tm.mark(MOE_STAGE_DOWN));
+    HIP_TRY(launch_stream_down(h->act, w2, lw.w2s, lw.b2, h->disp, h->y, h->Hp, h->IMp, tiles, direct, s));
+    return MOE_OK;
+  }
+  const int mt_cap = gemm_tile_cap(T, c.experts);
+  HIP_TRY(launch_gate_up(x, w1, lw.w1s, lw.b1g, lw.b1u, h->disp, h->act, h->Hp, h->IMp, c.swiglu_limit, mt_cap, s));
   HIP_TRY(tm.mark(MOE_STAGE_DOWN));
-  HIP_TRY(launch_down(h->act, lw.w2q ? static_cast<const void *>(lw.w2q) : lw.w2, lw.w2s, lw.b2,
-                      h->disp, h->y, h->Hp, h->IMp, mt_cap, max_rows, direct,
-                      down_k_split(max_rows, h->IMp, h->Hp, c.experts, T),
-                      (size_t)h->a_pad_cap * h->Hp * sizeof(float), s));
-  h->y_parts = down_k_split(max_rows, h->IMp, h->Hp, c.experts, T);
+  HIP_TRY(launch_down(h->act, w2, lw.w2s, lw.b2, h->disp, h->y, h->Hp, h->IMp, mt_cap, s));
   return MOE_OK;
 }
 
@@ -173,11 +175,9 @@ int run_combine(moe_handle *h, const float *topk_v, const int *pos, int T, float
                 uint16_t *resid, const DirectIds &direct, hipStream_t s, StageTimer &tm) {
   HIP_TRY(tm.mark(MOE_STAGE_COMBINE));
   if (out) {
-    HIP_TRY(launch_combine(h->y, h->Hp, h->y_parts, (size_t)h->a_pad_cap * h->Hp, h->disp.inv, topk_v, pos, out, T,
-                           h->cfg.hidden, accumulate, direct, s));
+    HIP_TRY(launch_combine(h->y, h->Hp, h->disp.inv, topk_v, pos, out, T, h->cfg.hidden, accumulate, direct, s));
   } else {
-    HIP_TRY(launch_combine_residual(h->y, h->Hp, h->y_parts, (size_t)h->a_pad_cap * h->Hp, h->disp.inv, topk_v, pos,
-                                    resid, T, h->cfg.hidden, direct, s));
+    HIP_TRY(launch_combine_residual(h->y, h->Hp, h->disp.inv, topk_v, pos, resid, T, h->cfg.hidden, direct, s));
   }
   HIP_TRY(tm.mark(MOE_NUM_STAGES));
   return MOE_OK;
@@ -198,7 +198,7 @@ int run_experts(moe_handle *h, int layer, const uint16_t *x, const int *pos, con
   h->unplanned = direct;
   h->disp_tokens = -1;  // the plan now belongs to this call, not to a moe_dispatch
   h->gemms_done = false;
-  int rc = run_gemms(h, layer, x, T, max_rows, direct, s, tm);
+  int rc = run_gemms(h, layer, x, T, direct, s, tm);
   if (rc != MOE_OK) return rc;
   return run_combine(h, topk_v, pos, T, out, accumulate, resid, direct, s, tm);
 }
@@ -256,18 +256,18 @@ int moe_create(const moe_config *cfg, moe_handle **out) {
   ALLOC(h->disp.perm, (size_t)h->a_cap);
   ALLOC(h->disp.rowmap, (size_t)h->a_pad_cap);
   ALLOC(h->disp.inv, (size_t)h->a_cap);
+  ALLOC(h->disp.blk_expert, (size_t)h->a_pad_cap / kRowBlock);
   ALLOC(h->disp.info, (size_t)E);
   ALLOC(h->disp.totals, (size_t)kTotInts);
   {
-    const int mt_cap = h->a_cap / kTileRows + E;  // row tiles at max_tokens, at most
+    const int mt_cap = gemm_tile_cap(T, E);  // row tiles at max_tokens, at most
     h->disp.tile_cap_gate_up = mt_cap * gate_up_col_tiles(h);
     h->disp.tile_cap_down = mt_cap * down_col_tiles(h);
   }
   ALLOC(h->disp.tiles_gate_up, (size_t)h->disp.tile_cap_gate_up);
   ALLOC(h->disp.tiles_down, (size_t)h->disp.tile_cap_down);
   ALLOC(h->act, (size_t)h->a_pad_cap * h->IMp);
-  // behind the rows of y: the second part of a split reduction (small batches, see down_k_split)
-  ALLOC(h->y, ((size_t)h->a_pad_cap + (kSmallBatchKSplit - 1) * small_batch_pad_rows(E)) * h->Hp);
+  ALLOC(h->y, (size_t)h->a_pad_cap * h->Hp);
   if (h->Hp != H) ALLOC(h->x_pad, (size_t)T * h->Hp);
 #undef ALLOC
   h->disp.a_pad_cap = h->a_pad_cap;
@@ -291,7 +291,7 @@ int moe_destroy(moe_handle *h) {
   }
   (void)hipFree(h->topk_i); (void)hipFree(h->topk_v);
   (void)hipFree(h->disp.blk_counts); (void)hipFree(h->disp.offsets); (void)hipFree(h->disp.perm);
-  (void)hipFree(h->disp.rowmap); (void)hipFree(h->disp.inv); (void)hipFree(h->disp.info); (void)hipFree(h->disp.totals);
+  (void)hipFree(h->disp.rowmap); (void)hipFree(h->disp.inv); (void)hipFree(h->disp.info); (void)hipFree(h->disp.blk_expert); (void)hipFree(h->disp.totals);
   (void)hipFree(h->disp.tiles_gate_up); (void)hipFree(h->disp.tiles_down);
   (void)hipFree(h->act); (void)hipFree(h->y); (void)hipFree(h->t_norm); (void)hipFree(h->x_pad);
   for (hipEvent_t ev : h->events) (void)hipEventDestroy(ev);
@@ -522,9 +522,7 @@ int moe_expert_gemms(moe_handle *h, int layer, const uint16_t *x, int n_tokens, 
   hipStream_t s = static_cast<hipStream_t>(stream);
   StageTimer tm(h, nullptr);  // stage-level calls are not timed
   tm.ev = nullptr;
-  // the ids of a moe_dispatch come from outside and may name an expert in several slots of a token
-  const int max_rows = h->distinct_ids ? n_tokens : n_tokens * kTopK;
-  rc = run_gemms(h, layer, x, n_tokens, max_rows, DirectIds{nullptr, nullptr, 0, 0}, s, tm);
+  rc = run_gemms(h, layer, x, n_tokens, DirectIds{nullptr, nullptr, 0, 0}, s, tm);
   if (rc == MOE_OK) h->gemms_done = true;
   return rc;
 }

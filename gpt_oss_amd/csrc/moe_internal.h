@@ -133,6 +133,7 @@ struct DispatchBuffers {
   int *perm;          // [A]     position -> assignment id
   int *rowmap;        // [A_pad] padded position -> assignment id, -1 = padding
   int *inv;           // [A]     assignment id -> padded position, -1 = inactive
+  int *blk_expert;    // [A_pad / 32] row block of the padded rows -> expert (nullptr: not wanted)
   ExpertInfo *info;   // [E]
   int *totals;        // [kTotInts]: total row tiles, padded rows, assignments; XCD bounds of both GEMMs
   int a_pad_cap;      // capacity of rowmap in rows
@@ -169,50 +170,45 @@ __device__ __forceinline__ int direct_expert_of(const DirectIds &d, int a) {
 inline bool direct_plan_fits(int T, int max_rows, int E, int a_pad_cap) {
   return T <= kDirectTokens && max_rows <= kDirectSlotRows && kDirectSlotRows * E <= a_pad_cap;
 }
-// gate_up reads the routed token rows of x itself, through rowmap; there is no
-// gathered copy.  Batches in which no expert has more than kSmallBatchRows rows
-// run the small-batch configuration of both GEMMs.
-constexpr int kSmallBatchRows = 64;
-inline bool small_batch(int max_rows) { return max_rows <= kSmallBatchRows; }
-// Parts the down GEMM's reduction is split into (each part writes its own copy
-// of the output rows, which the combine adds up): two in the small-batch
-// configuration while the experts a batch of T tokens can reach have at most
-// one tile per CU between them -- a tile is one stream of weights there, and a
-// CU takes in two to three such streams at once --, else one.  Measured with
-// MXFP4 weights at 32 experts: a layer call at 1 token 54.8 -> 47.9 us, at 4
-// tokens 65 -> 62; from 8 tokens on the split gains nothing (the first GEMM's
-// workgroups already fill the CUs when the second starts).
-constexpr int kSmallBatchKSplit = 2;
-constexpr int kCus = 256;
-inline int down_k_split(int max_rows, int inter_padded, int hidden_padded, int E, int T) {
-  if (!small_batch(max_rows) || inter_padded < 64) return 1;
-  const int n_ct = (hidden_padded / kRowBlock + kGemmTileNb - 1) / kGemmTileNb;
-  const long long reach = (long long)T * kTopK < E ? (long long)T * kTopK : E;
-  return reach * n_ct <= kCus ? kSmallBatchKSplit : 1;
+// Batches in which the weights are a stream run the kernels of stream.hip: up to
+// kDirectTokens tokens, and up to kStreamMeanRows rows per active expert on
+// average when every expert is active.  Those kernels take 32 rows per tile, and
+// an expert with more streams its weights again: measured on either side of the
+// line, us per layer call with the kernels of stream.hip and of gemm.hip:
+//   32 experts, MXFP4:  128 tokens 125 / 157, 192: 146 / 158, 256: 186 / 179
+//   32 experts, bf16:   128 tokens 297 / 319, 192: 325 / 319, 256: 471 / 332
+//   128 experts, MXFP4: 400 tokens 383 / 518, 800: 502 / 538, 1200: 698 / 562
+//   128 experts, bf16:  400 tokens 1057 / 1170, 800: 1354 / 1205
+// The rule knows nothing of the weights' format: both formats give the same bits.
+constexpr int kStreamMeanRows = 20;
+inline bool stream_batch(int T, int E) { return T <= kDirectTokens || T * kTopK <= kStreamMeanRows * E; }
+// row tiles of the grouped GEMMs in all, at most: row blocks of 32 (stream.hip) or tiles of 256 rows (gemm.hip)
+inline int stream_tile_cap(int T, int E) {
+  const int A = T * kTopK;
+  return A < E ? A : (A / kRowBlock + E < A ? A / kRowBlock + E : A);
 }
-// The rows a small batch can reach in the padded row space: every expert's
-// rows rounded up to 32, or its fixed slot of 64 rows without a dispatch pass.
-inline int small_batch_pad_rows(int E) {
-  const int planned = kSmallBatchRows * kTopK + kTileGran * E, slots = kDirectSlotRows * E;
-  return planned > slots ? planned : slots;
-}
+inline int gemm_tile_cap(int T, int E) { return T * kTopK / kTileRows + E; }
+// The first GEMM reads the routed token rows of x itself, through rowmap; there is
+// no gathered copy.  act holds the activation in the order the second GEMM of the
+// same file reads it: MFMA fragments (gemm.hip) or rows (stream.hip).
 hipError_t launch_gate_up(const uint16_t *x, const void *w1, const uint16_t *w1_scale, const float *b1g,
                           const float *b1u, const DispatchBuffers &d, uint16_t *act, int H, int IM,
-                          float limit, int mt_cap, int max_rows, const DirectIds &direct, hipStream_t s);
-// k_split: parts of the reduction (down_k_split); split_stride: bytes between the copies of y they write
+                          float limit, int mt_cap, hipStream_t s);
 hipError_t launch_down(const uint16_t *act, const void *w2, const uint16_t *w2_scale, const float *b2,
-                       const DispatchBuffers &d, float *y, int H, int IM, int mt_cap, int max_rows,
-                       const DirectIds &direct, int k_split, size_t split_stride, hipStream_t s);
+                       const DispatchBuffers &d, float *y, int H, int IM, int mt_cap, hipStream_t s);
+// tiles: experts that can have rows (ids.topk_i given) or row blocks of the plan, at most
+hipError_t launch_stream_gate_up(const uint16_t *x, const void *w1, const uint16_t *w1_scale, const float *b1g,
+                                 const float *b1u, const DispatchBuffers &d, uint16_t *act, int H, int IM,
+                                 float limit, int tiles, const DirectIds &ids, hipStream_t s);
+hipError_t launch_stream_down(const uint16_t *act, const void *w2, const uint16_t *w2_scale, const float *b2,
+                              const DispatchBuffers &d, float *y, int H, int IM, int tiles, const DirectIds &ids,
+                              hipStream_t s);
 // direct.topk_i != nullptr: the rows of y are found from the ids (inv is not read)
-// ldy: floats per row of y (the padded hidden size).  y_parts copies of y lie
-// part_stride floats apart (the parts of a split reduction, see down_k_split);
-// a row of the down projection is their sum, added in that order.
-hipError_t launch_combine(const float *y, int ldy, int y_parts, size_t part_stride, const int *inv,
-                          const float *topk_v, const int *pos, float *out, int T, int H, int accumulate,
-                          const DirectIds &direct, hipStream_t s);
-hipError_t launch_combine_residual(const float *y, int ldy, int y_parts, size_t part_stride, const int *inv,
-                                   const float *topk_v, const int *pos, uint16_t *x, int T, int H,
-                                   const DirectIds &direct, hipStream_t s);
+// ldy: floats per row of y (the padded hidden size)
+hipError_t launch_combine(const float *y, int ldy, const int *inv, const float *topk_v, const int *pos, float *out,
+                          int T, int H, int accumulate, const DirectIds &direct, hipStream_t s);
+hipError_t launch_combine_residual(const float *y, int ldy, const int *inv, const float *topk_v, const int *pos,
+                                   uint16_t *x, int T, int H, const DirectIds &direct, hipStream_t s);
 hipError_t launch_rmsnorm(const uint16_t *x, const float *weight, const int *pos, uint16_t *t_out,
                           int T, int H, hipStream_t s);
 

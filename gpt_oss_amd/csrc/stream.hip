@@ -1,0 +1,393 @@
+// Grouped expert GEMMs of the batches in which the weights are a stream: few rows
+// per expert, so the time is that of reading the weights once.  Same contract as
+// the kernels of gemm.hip (matmul/matmul.cpp:1023-1914, SwiGLU of run.cpp:709-726).
+//
+// A wave owns a pair of column blocks (64 columns) of one expert and a slice of
+// the reduction, and shares nothing with other waves until its slice is done: the
+// weights and the token rows go straight into registers, D steps of 32 k ahead,
+// there is no LDS stage, no barrier and no DMA in the loop.  The KW waves of a
+// workgroup take the KW slices of the same columns and add their sums through
+// LDS at the end, in a fixed order.  Compared with one workgroup per 256 columns
+// whose waves walk the whole reduction in lock step (gemm_tile), a wave's chain
+// of dependent steps is KW times shorter, there are KW times as many streams,
+// and a late load holds up one wave instead of four.
+//
+// The products are v_mfma_f32_16x16x32_bf16: 16 token rows at a time, which is
+// what an expert has in such a batch.  The weights are the first operand, so a
+// lane ends with four consecutive weight rows of one token.  Lane l = 16 q + r of
+// either operand holds row r and the 8 k of piece (q >> 1) + 2 (q & 1) of the
+// step's four: that is the order in which one v_permlane16_swap turns a pair of
+// 32-row weight fragments (pack.hip) into two 16-row ones.
+//
+// Bound by HBM with bf16 weights; with MXFP4 weights the conversions, the rows'
+// loads through L1 and the few microseconds in which a launch fills and drains
+// show as well.  Measured at 2880 x 2880 and 32 experts, against the kernels this
+// replaces (us, gate_up + down): 24 tokens bf16 157 + 81 (6.8 and 6.6 TB/s; were
+// 199 + 105), 64 tokens MXFP4 50 + 29 (were 60 + 40), 1 token MXFP4 10 + 6 (27 +
+// 16).  What that rests on, by leaving it out: the weights' non-temporal loads
+// (bf16 174 + 90 with plain ones), two pairs of columns per wave that share the
+// rows they load (MXFP4 55 + 32 with one; where that would leave fewer than
+// kStreamTwoPairs workgroups of work, one), no refill loads past the slice's end
+// (MXFP4 57 + 32 with them).  The number of slices (1, 2 or 4) matters to the
+// small launches only.
+//
+// Every path a batch can take at its size (whole layer, caller's routing, stage
+// by stage; bf16 and MXFP4 weights) runs these kernels with the same slices, so
+// they all give the same bits.
+#include <type_traits>
+
+#include "moe_internal.h"
+#include "swiglu.h"
+
+#ifndef PIN
+#define PIN
+#endif
+#ifndef OCC
+#define OCC 4
+#endif
+#ifndef D1
+#define D1 8
+#endif
+#ifndef D1B
+#define D1B 4
+#endif
+#ifndef D2
+#define D2 4
+#endif
+#ifndef D2B
+#define D2B 3
+#endif
+#ifndef NPV
+#define NPV 1
+#endif
+namespace moe {
+
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+constexpr int kStreamKw = 4;     // waves of a workgroup = slices of the reduction
+constexpr int kStreamCols = 64;  // columns of a pair of column blocks
+constexpr int kStreamRows = 32;  // rows of a tile, at most
+// MXFP4: with this many column tiles of one pair or more, a wave takes two pairs
+constexpr int kStreamTwoPairs = 1024;
+
+// Orders LDS traffic only: the loads in flight stay in flight.
+__device__ __forceinline__ void stream_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+// One wave's share of a tile: RG groups of 16 rows times NP pairs of column
+// blocks over the steps [ks0, ks0 + n) of 32 k.  a_rows: rows of lda 16-byte
+// pieces; row[g]: the row this lane feeds in group g.  np_valid: pairs inside
+// the matrix; one past it repeats the first, and its sums are not used.
+template <int NP, int RG, int D, bool FP4>
+__device__ __forceinline__ void stream_slice(const uint4 *__restrict__ a_rows, int lda, const int (&row)[RG],
+                                             const uint4 *__restrict__ w, const uint16_t *__restrict__ ws, int KB,
+                                             int np_valid, int ks0, int n, int lane, f32x4 (&acc)[NP][4][RG]) {
+  constexpr int WR = FP4 ? 1 : 4;  // 16-byte registers of weights per pair and step
+  const int r = lane & 15, q = lane >> 4;
+  const int piece = (q >> 1) + 2 * (q & 1);
+  // addresses: a base that is the same for the whole wave and moves with the step,
+  // plus a 32-bit offset per lane that does not
+  uint32_t a_off[RG];
+#pragma unroll
+  for (int g = 0; g < RG; g++) a_off[g] = ((uint32_t)row[g] * (uint32_t)lda + piece) * 16u;
+  // bf16: fragment (block b, k block kb) is 64 pieces; this lane's piece of half hh is
+  // kb = q & 1, (q >> 1) * 32 + 16 hh + r.  FP4: one chunk of 64 pieces per step.
+  const uint32_t w_off = FP4 ? lane * 16u : ((q & 1) * 64 + (q >> 1) * 32 + r) * 16u;
+  // scale bytes of a step: 16 bits per row; loaded as the 32 bits of two rows, of which the lane shifts its own down
+  const uint32_t s_off = (lane & 30) * 2u, s_shift = (lane & 1) * 16u;
+  u32x4 wq[D][NP][WR], xa[D][RG];
+  uint32_t sc[D][NP];
+  auto load = [&](int d, int s) {
+    const size_t k = ks0 + s;
+#pragma unroll
+    for (int p = 0; p < NP; p++) {
+      const size_t pair = p < np_valid ? p : 0;
+      // the weights are read once: they go past the caches (measured, see above)
+      if (FP4) {
+        const char *wb = reinterpret_cast<const char *>(w) + pair * KB * 512 + k * 1024;
+        const char *sb = reinterpret_cast<const char *>(ws) + pair * KB * 32 + k * 64;
+        wq[d][p][0] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(wb + w_off));
+        sc[d][p] = *reinterpret_cast<const uint32_t *>(sb + s_off);
+      } else {
+        const char *wb = reinterpret_cast<const char *>(w) + pair * KB * 2048 + k * 2048;
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+          wq[d][p][i] = __builtin_nontemporal_load(
+              reinterpret_cast<const u32x4 *>(wb + (size_t)(i >> 1) * KB * 1024 + (i & 1) * 256 + w_off));
+      }
+    }
+    const char *ab = reinterpret_cast<const char *>(a_rows) + k * 64;
+#pragma unroll
+    for (int g = 0; g < RG; g++) xa[d][g] = *reinterpret_cast<const u32x4 *>(ab + a_off[g]);
+  };
+#pragma unroll
+  for (int p = 0; p < NP; p++)
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+#pragma unroll
+      for (int g = 0; g < RG; g++) acc[p][i][g] = f32x4{0.f, 0.f, 0.f, 0.f};
+  auto compute = [&](int d) {
+#pragma unroll
+    for (int p = 0; p < NP; p++) {
+      bf16x8 wf[4];  // 16 weight rows each: [2 * block + half]
+      if constexpr (FP4) {
+        const uint32_t own = sc[d][p] >> s_shift;
+        const u32x2 ss = __builtin_amdgcn_permlane16_swap(own, own, false, false);
+#pragma unroll
+        for (int b = 0; b < 2; b++) {
+          const u32x2 nn = __builtin_amdgcn_permlane16_swap(wq[d][p][0][2 * b], wq[d][p][0][2 * b + 1], false, false);
+#pragma unroll
+          for (int hh = 0; hh < 2; hh++) {
+            const float scale = __uint_as_float(((ss[hh] >> (8 * b)) & 0xffu) << 23);  // 2^(s - 127)
+            const uint32_t nib = nn[hh];
+            const bf16x2 p0 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(nib, scale, 0);
+            const bf16x2 p1 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(nib, scale, 1);
+            const bf16x2 p2 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(nib, scale, 2);
+            const bf16x2 p3 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(nib, scale, 3);
+            wf[2 * b + hh] = bf16x8{p0[0], p0[1], p1[0], p1[1], p2[0], p2[1], p3[0], p3[1]};
+          }
+        }
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; i++) wf[i] = __builtin_bit_cast(bf16x8, wq[d][p][i]);
+      }
+#pragma unroll
+      for (int i = 0; i < 4; i++)
+#pragma unroll
+        for (int g = 0; g < RG; g++)
+          acc[p][i][g] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[i], __builtin_bit_cast(bf16x8, xa[d][g]),
+                                                                 acc[p][i][g], 0, 0, 0);
+    }
+  };
+  if (n <= 0) return;  // a short reduction has fewer steps than slices
+  // Rounds of D steps.  The refill of a round is the next round's loads, so the
+  // last one has none; the steps that pad it load the slice's last step again (at
+  // most D - 1 of them, real traffic: the loads go past the caches) and are not
+  // multiplied.
+#pragma unroll
+  for (int d = 0; d < D; d++) load(d, min(d, n - 1));
+  int s = 0;
+  for (; s + D < n; s += D) {
+#pragma unroll
+    for (int d = 0; d < D; d++) {
+      compute(d);
+      load(d, min(s + d + D, n - 1));
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+#pragma unroll
+  for (int d = 0; d < D; d++)
+    if (s + d < n) compute(d);
+}
+
+// Sum of the slices in their order, bias, SwiGLU and the rows out.  A unit is 16
+// columns (gate_up: 16 of gate and the same 16 of up) of one group of rows, in
+// which a lane holds four consecutive columns of one row; the waves share them.
+template <int RG, bool GATE_UP>
+__device__ __forceinline__ void stream_finish(const f32x4 *part, const float *__restrict__ bias_a,
+                                              const float *__restrict__ bias_b, int P, int row0, int rows,
+                                              void *__restrict__ outp, int ldo, float limit, int w, int lane) {
+  const int r = lane & 15, q = lane >> 4;
+  auto sum = [&](int i, int g) {
+    f32x4 v = part[(i * RG + g) * 64 + lane];
+#pragma unroll
+    for (int k = 1; k < kStreamKw; k++) v += part[((k * 4 + i) * RG + g) * 64 + lane];
+    return v;
+  };
+  constexpr int UNITS = (GATE_UP ? 2 : 4) * RG;
+  for (int u = w; u < UNITS; u += kStreamKw) {
+    const int i = u / RG, g = u % RG;
+    const int row = 16 * g + r;
+    if (GATE_UP) {
+      const int j = kRowBlock * P + 16 * i + 4 * q;
+      const f32x4 bg = *reinterpret_cast<const f32x4 *>(bias_a + j), bu = *reinterpret_cast<const f32x4 *>(bias_b + j);
+      const f32x4 ga = sum(i, g) + bg, up = sum(2 + i, g) + (bu + 1.0f);
+      const uint32_t lo = pack_bf16(swiglu_shifted(ga[0], up[0], limit), swiglu_shifted(ga[1], up[1], limit));
+      const uint32_t hi = pack_bf16(swiglu_shifted(ga[2], up[2], limit), swiglu_shifted(ga[3], up[3], limit));
+      if (row < rows)
+        *reinterpret_cast<uint2 *>(static_cast<uint16_t *>(outp) + (size_t)(row0 + row) * ldo + j) = make_uint2(lo, hi);
+    } else {
+      const int j = kStreamCols * P + 16 * i + 4 * q;
+      const f32x4 v = sum(i, g) + *reinterpret_cast<const f32x4 *>(bias_a + j);
+      if (row < rows) *reinterpret_cast<f32x4 *>(static_cast<float *>(outp) + (size_t)(row0 + row) * ldo + j) = v;
+    }
+  }
+}
+
+// DIRECT: there is no plan.  The workgroup reads the batch's ids (one per
+// thread), lists the experts that have rows in a bit mask and finds the rows of
+// its own by ballot; workgroup i * wgs + c is column tile c of the i-th expert
+// with rows, so that the column tiles of the few experts a small batch reaches
+// spread over all XCDs.  Otherwise a tile is a row block of the plan's padded rows.
+template <int NP, bool GATE_UP, bool FP4, bool DIRECT>
+__global__ __launch_bounds__(kStreamKw * 64, NP == 1 ? 4 : 3) void stream_gemm_kernel(
+    const uint4 *__restrict__ a_rows, const uint4 *__restrict__ w_frag, const uint16_t *__restrict__ w_scale,
+    const float *__restrict__ bias_a, const float *__restrict__ bias_b, const int *__restrict__ rowmap,
+    const int *__restrict__ blk_expert, const int *__restrict__ totals, void *__restrict__ outp, int K, int N,
+    float limit, DirectIds ids) {
+  constexpr int RG = kStreamRows / 16;
+  __shared__ f32x4 part[kStreamKw * 4 * RG * 64];
+  __shared__ int rows_sh[DIRECT ? kDirectSlotRows : kStreamRows];  // row of the tile -> token
+  const int tid = threadIdx.x;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int n_cols = GATE_UP ? 2 * N : N;
+  const int pairs = n_cols / kStreamCols;
+  const int wgs = (pairs + NP - 1) / NP;
+  const int ti = blockIdx.x / wgs, P = (blockIdx.x - ti * wgs) * NP;
+  const int np_valid = min(NP, pairs - P);
+  const int KB = K / kFragK, steps = K / 32;
+  const int per = (steps + kStreamKw - 1) / kStreamKw;
+  const int ks0 = min(w * per, steps), n = min(per, steps - ks0);
+  int e, row0, count;
+  if constexpr (DIRECT) {
+    static_assert(kStreamKw * 64 == kDirectTokens * kTopK, "one thread per assignment");
+    __shared__ uint32_t mask[8];
+    __shared__ int cnt[kStreamKw];
+    const int lane = tid & 63;
+    const int mine = direct_expert_of(ids, tid);
+    if (tid < 8) mask[tid] = 0;
+    stream_barrier();
+    if (mine >= 0) atomicOr(&mask[mine >> 5], 1u << (mine & 31));
+    stream_barrier();
+    e = -1;
+    int left = ti;
+    for (int ww = 0; ww < (ids.E + 31) / 32; ww++) {
+      uint32_t m = __builtin_amdgcn_readfirstlane(mask[ww]);
+      const int c = __builtin_popcount(m);
+      if (left < c) {
+        for (int i = 0; i < left; i++) m &= m - 1;
+        e = ww * 32 + __builtin_ctz(m);
+        break;
+      }
+      left -= c;
+    }
+    e = __builtin_amdgcn_readfirstlane(e);
+    if (e < 0) return;  // fewer experts than the grid provides for
+    const unsigned long long bal = __ballot(mine == e);
+    if (lane == 0) cnt[w] = __popcll(bal);
+    stream_barrier();
+    int before = 0;
+    count = 0;
+#pragma unroll
+    for (int ww = 0; ww < kStreamKw; ww++) {
+      const int c = cnt[ww];
+      if (ww < w) before += c;
+      count += c;
+    }
+    count = __builtin_amdgcn_readfirstlane(min(count, kDirectSlotRows));
+    row0 = e * kDirectSlotRows;
+    if (GATE_UP) {
+      const int at = before + __popcll(bal & ((1ull << lane) - 1ull));
+      if (mine == e && at < kDirectSlotRows) rows_sh[at] = tid / kTopK;
+      stream_barrier();
+    }
+  } else {
+    if (ti >= totals[kTotRows] / kRowBlock) return;  // surplus workgroups of the upper-bound grid
+    const int lane = tid & 63;
+    e = __builtin_amdgcn_readfirstlane(blk_expert[ti]);
+    row0 = ti * kRowBlock;
+    const int a = lane < kStreamRows ? rowmap[row0 + lane] : -1;
+    count = __popcll(__ballot(a >= 0));  // the valid rows of a block come first
+    if (GATE_UP) {
+      if (w == 0 && lane < count) rows_sh[lane] = a / kTopK;
+      stream_barrier();
+    }
+  }
+  const size_t blk0 = (size_t)e * (n_cols / kRowBlock) + 2 * P;
+  const uint4 *wp = w_frag + blk0 * (size_t)(KB * (FP4 ? 16 : 64));
+  const uint16_t *sp = FP4 ? w_scale + blk0 * KB * 8 : nullptr;
+  const float *ba = bias_a + (size_t)e * N;
+  const float *bb = GATE_UP ? bias_b + (size_t)e * N : nullptr;
+  // (gridDim.y: workgroups that share an expert's tiles of 32 rows)
+  for (int r0 = blockIdx.y * kStreamRows; r0 < count; r0 += gridDim.y * kStreamRows) {
+    const int rows = min(count - r0, kStreamRows);
+    // (a second round is rare: keeps what depends on the lane from being computed
+    // ahead of the loop and held, or spilled, through it)
+    int lane = tid & 63;
+    asm volatile("" : "+v"(lane));
+    // lanes past the last row repeat it; their sums are not stored
+    int row[RG];
+#pragma unroll
+    for (int g = 0; g < RG; g++) {
+      const int rr = r0 + min(16 * g + (lane & 15), rows - 1);
+      row[g] = GATE_UP ? rows_sh[rr] : row0 + rr;
+    }
+    auto tile = [&](auto g_c, auto d_c, const auto &tile_row) {
+      constexpr int G = decltype(g_c)::value;
+      f32x4 acc[NP][4][G];
+      stream_slice<NP, G, decltype(d_c)::value, FP4>(a_rows, K / 8, tile_row, wp, sp, KB, np_valid, ks0, n, lane, acc);
+#pragma unroll
+      for (int p = 0; p < NP; p++) {
+        if (p >= np_valid) break;
+        if (p || r0 != (int)blockIdx.y * kStreamRows) stream_barrier();  // the sums before have been read
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+#pragma unroll
+          for (int g = 0; g < G; g++) part[((w * 4 + i) * G + g) * 64 + lane] = acc[p][i][g];
+        stream_barrier();
+        stream_finish<G, GATE_UP>(part, ba, bb, P + p, row0 + r0, rows, outp, N, limit, w, lane);
+      }
+    };
+    // steps ahead: as many as the registers of three or four waves per SIMD hold
+    // (more gain nothing: at 64 tokens and MXFP4 weights the same time with 4, 6 and 8)
+    using One = std::integral_constant<int, 1>;
+    using Two = std::integral_constant<int, 2>;
+    if (rows <= 16) {
+      const int one[1] = {row[0]};
+      tile(One{}, std::integral_constant<int, FP4 ? (NP == 1 ? 6 : 4) : 4>{}, one);
+    } else {
+      tile(Two{}, std::integral_constant<int, FP4 ? (NP == 1 ? 4 : 2) : 3>{}, row);
+    }
+  }
+}
+
+template <int NP, bool GATE_UP>
+static hipError_t launch_stream_np(const uint4 *a, const uint4 *w, const uint16_t *w_scale, const float *ba,
+                                   const float *bb, const DispatchBuffers &d, void *out, int K, int N, float limit,
+                                   int tiles, const DirectIds &ids, hipStream_t s) {
+  const int pairs = (GATE_UP ? 2 * N : N) / kStreamCols;
+  // Without a plan an expert may have two tiles: one workgroup takes both, one
+  // after the other, unless most experts are likely to have two.
+  const bool two_tiles = ids.topk_i && ids.T > kStreamRows && ids.T * kTopK > kStreamRows / 2 * ids.E;
+  const dim3 grid(tiles * ((pairs + NP - 1) / NP), two_tiles ? 2 : 1);
+#define MOE_STREAM(FP4, DIRECT)                                                 \
+  stream_gemm_kernel<NP, GATE_UP, FP4, DIRECT><<<grid, kStreamKw * 64, 0, s>>>( \
+      a, w, w_scale, ba, bb, d.rowmap, d.blk_expert, d.totals, out, K, N, limit, ids)
+  if constexpr (NP == 1) {
+    if (!w_scale) {
+      if (ids.topk_i) MOE_STREAM(false, true); else MOE_STREAM(false, false);
+      return hipGetLastError();
+    }
+  }
+  if (ids.topk_i) MOE_STREAM(true, true); else MOE_STREAM(true, false);
+#undef MOE_STREAM
+  return hipGetLastError();
+}
+
+template <bool GATE_UP>
+static hipError_t launch_stream(const void *a, const void *w, const uint16_t *w_scale, const float *ba,
+                                const float *bb, const DispatchBuffers &d, void *out, int K, int N, float limit,
+                                int tiles, const DirectIds &ids, hipStream_t s) {
+  const uint4 *af = static_cast<const uint4 *>(a), *wf = static_cast<const uint4 *>(w);
+  const int pairs = (GATE_UP ? 2 * N : N) / kStreamCols;
+  if (w_scale && tiles * pairs >= kStreamTwoPairs)
+    return launch_stream_np<2, GATE_UP>(af, wf, w_scale, ba, bb, d, out, K, N, limit, tiles, ids, s);
+  return launch_stream_np<1, GATE_UP>(af, wf, w_scale, ba, bb, d, out, K, N, limit, tiles, ids, s);
+}
+
+hipError_t launch_stream_gate_up(const uint16_t *x, const void *w1, const uint16_t *w1_scale, const float *b1g,
+                                 const float *b1u, const DispatchBuffers &d, uint16_t *act, int H, int IM,
+                                 float limit, int tiles, const DirectIds &ids, hipStream_t s) {
+  return launch_stream<true>(x, w1, w1_scale, b1g, b1u, d, act, H, IM, limit, tiles, ids, s);
+}
+
+hipError_t launch_stream_down(const uint16_t *act, const void *w2, const uint16_t *w2_scale, const float *b2,
+                              const DispatchBuffers &d, float *y, int H, int IM, int tiles, const DirectIds &ids,
+                              hipStream_t s) {
+  return launch_stream<false>(act, w2, w2_scale, b2, nullptr, d, y, IM, H, 0.f, tiles, ids, s);
+}
+
+}  // namespace moe

@@ -1,0 +1,75 @@
+"""The kernels of the batches in which the weights are a stream (stream.hip) at
+the sizes where they can go wrong: one row, a group of 16 rows and one more, a
+tile of 32 and one more, an expert with several tiles, with and without a plan;
+reductions with fewer steps than slices and with slices of unequal length; an odd
+number of column pairs where a wave takes two.
+
+Bars as in test_gpu_parity.py: max-abs 2e-2 and rel-L2 1e-3 of the oracle on the
+same bf16 inputs; the two weight formats bit for bit."""
+import numpy as np
+import pytest
+
+from gpt_oss_amd import abi, synth
+from oracle import binding as ob
+
+pytestmark = pytest.mark.gpu
+
+W = ("w_router", "b_router", "w_mlp1", "b_mlp1", "w_mlp2", "b_mlp2")
+
+
+@pytest.mark.parametrize("rows", [1, 16, 17, 32, 33, 64, 65, 150])
+@pytest.mark.parametrize("H,IM", [(64, 64), (192, 320), (704, 64)])
+def test_rows_of_an_expert(rows, H, IM):
+    """Every token names the experts 2, 30, 31 and 0: each has all the rows."""
+    E = 32
+    sh = synth.LayerShape("rows", rows, H, IM, E)
+    L = {k: (synth.round_bf16(v) if v.dtype == np.float32 else v) for k, v in synth.make_layer(sh, seed=rows).items()}
+    m = abi.Moe(H, IM, E, max_tokens=rows, swiglu_limit=sh.limit)
+    m.upload_layer(0, *[L[k] for k in W])
+    ids = [2, 30, 31, 0]
+    ti = np.tile(np.array(ids, np.int32), (rows, 1))
+    tv = np.random.default_rng(rows).random((rows, 4)).astype(np.float32)
+    want = np.zeros((rows, H), np.float32)
+    for t in range(rows):
+        for k, e in enumerate(ids):
+            want[t] += tv[t, k] * ob.expert_token(L["x"][t], L["w_mlp1"][e], L["b_mlp1"][e], L["w_mlp2"][e],
+                                                  L["b_mlp2"][e], sh.limit, mode=ob.ROUND_ACT_BF16)
+    dx = abi.DevBuf.from_numpy(synth.to_bf16_bits(L["x"]))
+    dti, dtv, dout = abi.DevBuf.from_numpy(ti), abi.DevBuf.from_numpy(tv), abi.DevBuf(rows * H * 4)
+    first = None
+    for distinct in (True, False):  # up to 64 tokens: without a plan, and with one
+        m.set_distinct_ids(distinct)
+        dout.memset(0xFF)
+        m.experts(0, dx, None, dti, dtv, rows, dout)
+        abi.sync()
+        got = dout.download((rows, H), np.float32)
+        assert np.abs(got - want).max() <= 2e-2 and np.linalg.norm(got - want) <= 1e-3 * np.linalg.norm(want)
+        first = got if first is None else first
+        assert np.array_equal(got, first)
+    m.close()
+
+
+@pytest.mark.parametrize("T", [2, 40, 65])
+def test_two_pairs_of_columns_per_wave(T):
+    """128 experts and nine pairs of columns: MXFP4 waves take two pairs each from
+    40 tokens on (the last of a row has one), one pair at 2 tokens."""
+    sh = synth.LayerShape("pairs", T, 576, 576, 128)
+    x = synth.round_bf16(synth.make_activations(sh))
+    wr, br = (synth.round_bf16(a) for a in synth.make_router(sh))
+    b1k, s1, b1, b2k, s2, b2 = synth.make_experts_mxfp4(sh)
+    b1, b2 = synth.round_bf16(b1), synth.round_bf16(b2)
+    w1, w2 = ob.mxfp4_dequant(b1k, s1), ob.mxfp4_dequant(b2k, s2)
+    m4 = abi.Moe(sh.hidden, sh.inter, sh.experts, max_tokens=T, swiglu_limit=sh.limit)
+    m4.upload_layer_mxfp4(0, wr, br, b1k, s1, b1, b2k, s2, b2)
+    m16 = abi.Moe(sh.hidden, sh.inter, sh.experts, max_tokens=T, swiglu_limit=sh.limit)
+    m16.upload_layer(0, wr, br, w1, b1, w2, b2)
+    a, b = abi.run_layer(m4, 0, x, None), abi.run_layer(m16, 0, x, None)
+    assert np.array_equal(a["topk_i"], b["topk_i"]) and np.array_equal(a["out"], b["out"])
+    rows = np.arange(min(T, 16))
+    want = ob.moe_layer(np.ascontiguousarray(x[rows]), None, wr, br, w1, b1, w2, b2, 4, sh.limit,
+                        mode=ob.ROUND_ACT_BF16 | ob.PAR_TOKENS)
+    got = a["out"][rows]
+    assert np.linalg.norm(got - want) <= 1e-3 * np.linalg.norm(want)
+    assert np.abs(got - want).max() <= 2e-2 * max(1.0, float(np.abs(want).max()))
+    m4.close()
+    m16.close()
