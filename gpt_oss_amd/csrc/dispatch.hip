@@ -487,42 +487,20 @@ __global__ __launch_bounds__(kDispThreads) void dispatch_small_kernel(
 // utility/utility.cpp:158-173; call getp_run.cpp:846-852); inactive rows are
 // left alone.
 //
-// DIRECT: there was no dispatch pass (see DirectIds).  The row of assignment
-// (t, k) is its expert's slot plus the number of lower assignments of the batch
-// with the same expert, which the workgroup's 256 threads count with a ballot.
-template <bool RESID, bool DIRECT>
+// One workgroup per token; for few tokens gridDim.y workgroups share its columns
+// (a single token: 5.4 -> 2.7 us with that and inv in place of a ballot over the ids).
+template <bool RESID>
 __global__ __launch_bounds__(256) void combine_kernel(const float *__restrict__ y,
                                                      const int *__restrict__ inv,
                                                      const float *__restrict__ topk_v,
                                                      const int *__restrict__ pos, void *outp, int H,
-                                                     int ldy, int accumulate, DirectIds ids) {
+                                                     int ldy, int accumulate) {
   const int t = blockIdx.x;
   const bool active = !(pos && pos[t] < 0);
   if (!active && (accumulate || RESID)) return;
   int p[kTopK] = {-1, -1, -1, -1};
   float w[kTopK] = {0.f, 0.f, 0.f, 0.f};
-  if (DIRECT) {
-    __shared__ int lower[256 / 64][kTopK];
-    const int tid = threadIdx.x;
-    const int mine = direct_expert_of(ids, tid);
-    int e[kTopK];
-#pragma unroll
-    for (int k = 0; k < kTopK; k++) {
-      e[k] = direct_expert_of(ids, t * kTopK + k);
-      const unsigned long long bal = __ballot(e[k] >= 0 && mine == e[k] && tid < t * kTopK + k);
-      if ((tid & 63) == 0) lower[tid >> 6][k] = __popcll(bal);
-    }
-    __syncthreads();
-#pragma unroll
-    for (int k = 0; k < kTopK; k++) {
-      const int r = lower[0][k] + lower[1][k] + lower[2][k] + lower[3][k];
-      if (e[k] >= 0 && r < kDirectSlotRows) p[k] = e[k] * kDirectSlotRows + r;
-    }
-    if (active) {
-      const float4 wv = *reinterpret_cast<const float4 *>(topk_v + (size_t)t * kTopK);
-      w[0] = wv.x; w[1] = wv.y; w[2] = wv.z; w[3] = wv.w;
-    }
-  } else if (active) {
+  if (active) {
     const int4 pi = *reinterpret_cast<const int4 *>(inv + (size_t)t * kTopK);
     const float4 wv = *reinterpret_cast<const float4 *>(topk_v + (size_t)t * kTopK);
     p[0] = pi.x; p[1] = pi.y; p[2] = pi.z; p[3] = pi.w;
@@ -530,7 +508,7 @@ __global__ __launch_bounds__(256) void combine_kernel(const float *__restrict__ 
   }
   float4 *o = reinterpret_cast<float4 *>(reinterpret_cast<float *>(outp) + (size_t)t * H);
   uint2 *xr = reinterpret_cast<uint2 *>(reinterpret_cast<uint16_t *>(outp) + (size_t)t * H);
-  for (int c = threadIdx.x; c < H / 4; c += 256) {
+  for (int c = blockIdx.y * 256 + threadIdx.x; c < H / 4; c += gridDim.y * 256) {
     float4 s = (!RESID && accumulate) ? o[c] : make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
     for (int k = 0; k < kTopK; k++) {
@@ -582,23 +560,21 @@ hipError_t launch_dispatch(const int *topk_i, const int *pos, int T, int E, int 
 
 template <bool RESID>
 static hipError_t launch_combine_any(const float *y, int ldy, const int *inv, const float *topk_v, const int *pos,
-                                     void *out, int T, int H, int accumulate, const DirectIds &direct,
-                                     hipStream_t s) {
-  if (direct.topk_i)
-    combine_kernel<RESID, true><<<T, 256, 0, s>>>(y, inv, topk_v, pos, out, H, ldy, accumulate, direct);
-  else
-    combine_kernel<RESID, false><<<T, 256, 0, s>>>(y, inv, topk_v, pos, out, H, ldy, accumulate, direct);
+                                     void *out, int T, int H, int accumulate, hipStream_t s) {
+  // workgroups of one token each fill the GPU from about four per CU on
+  const dim3 grid(T, T < 4 * kCus ? (H / 4 + 255) / 256 : 1);
+  combine_kernel<RESID><<<grid, 256, 0, s>>>(y, inv, topk_v, pos, out, H, ldy, accumulate);
   return hipGetLastError();
 }
 
 hipError_t launch_combine(const float *y, int ldy, const int *inv, const float *topk_v, const int *pos, float *out,
-                          int T, int H, int accumulate, const DirectIds &direct, hipStream_t s) {
-  return launch_combine_any<false>(y, ldy, inv, topk_v, pos, out, T, H, accumulate, direct, s);
+                          int T, int H, int accumulate, hipStream_t s) {
+  return launch_combine_any<false>(y, ldy, inv, topk_v, pos, out, T, H, accumulate, s);
 }
 
 hipError_t launch_combine_residual(const float *y, int ldy, const int *inv, const float *topk_v, const int *pos,
-                                   uint16_t *x, int T, int H, const DirectIds &direct, hipStream_t s) {
-  return launch_combine_any<true>(y, ldy, inv, topk_v, pos, x, T, H, 0, direct, s);
+                                   uint16_t *x, int T, int H, hipStream_t s) {
+  return launch_combine_any<true>(y, ldy, inv, topk_v, pos, x, T, H, 0, s);
 }
 
 }  // namespace moe

@@ -172,12 +172,12 @@ int run_gemms(moe_handle *h, int layer, const uint16_t *x, int T, const DirectId
 // Stage 6: out != nullptr: out (+)= sum_k w[t,k] * y[row of (t,k)], fp32.
 // Otherwise resid (bf16, in place) += that sum.
 int run_combine(moe_handle *h, const float *topk_v, const int *pos, int T, float *out, int accumulate,
-                uint16_t *resid, const DirectIds &direct, hipStream_t s, StageTimer &tm) {
+                uint16_t *resid, hipStream_t s, StageTimer &tm) {
   HIP_TRY(tm.mark(MOE_STAGE_COMBINE));
   if (out) {
-    HIP_TRY(launch_combine(h->y, h->Hp, h->disp.inv, topk_v, pos, out, T, h->cfg.hidden, accumulate, direct, s));
+    HIP_TRY(launch_combine(h->y, h->Hp, h->disp.inv, topk_v, pos, out, T, h->cfg.hidden, accumulate, s));
   } else {
-    HIP_TRY(launch_combine_residual(h->y, h->Hp, h->disp.inv, topk_v, pos, resid, T, h->cfg.hidden, direct, s));
+    HIP_TRY(launch_combine_residual(h->y, h->Hp, h->disp.inv, topk_v, pos, resid, T, h->cfg.hidden, s));
   }
   HIP_TRY(tm.mark(MOE_NUM_STAGES));
   return MOE_OK;
@@ -200,7 +200,7 @@ int run_experts(moe_handle *h, int layer, const uint16_t *x, const int *pos, con
   h->gemms_done = false;
   int rc = run_gemms(h, layer, x, T, direct, s, tm);
   if (rc != MOE_OK) return rc;
-  return run_combine(h, topk_v, pos, T, out, accumulate, resid, direct, s, tm);
+  return run_combine(h, topk_v, pos, T, out, accumulate, resid, s, tm);
 }
 
 }  // namespace
@@ -540,7 +540,7 @@ int moe_combine(moe_handle *h, const float *topk_v, const int *pos, int n_tokens
   if (!topk_v || !out) return fail(MOE_ERR_BAD_ARG, "null device pointer");
   StageTimer tm(h, nullptr);
   tm.ev = nullptr;
-  return run_combine(h, topk_v, pos, n_tokens, out, accumulate, nullptr, DirectIds{nullptr, nullptr, 0, 0},
+  return run_combine(h, topk_v, pos, n_tokens, out, accumulate, nullptr,
                      static_cast<hipStream_t>(stream), tm);
 }
 

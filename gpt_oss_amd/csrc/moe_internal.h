@@ -146,8 +146,8 @@ hipError_t launch_dispatch(const int *topk_i, const int *pos, int T, int E, int 
 
 // Batches of at most kDirectTokens tokens run without a dispatch pass: the 256
 // threads of a workgroup hold one assignment each, so every workgroup of the
-// GEMMs and of the combine reads the batch's expert ids itself and finds its
-// rows with a ballot.  Expert e owns the padded rows [e * kDirectSlotRows,
+// GEMMs reads the batch's expert ids itself and finds its rows with a ballot; the
+// first GEMM leaves inv for the combine.  Expert e owns the padded rows [e * kDirectSlotRows,
 // (e + 1) * kDirectSlotRows); inside them its assignments stand in ascending
 // order, as the dispatch kernels place them.  Requires that no expert is given
 // more than kDirectSlotRows assignments.  topk_i == nullptr: not in use, the
@@ -180,6 +180,7 @@ inline bool direct_plan_fits(int T, int max_rows, int E, int a_pad_cap) {
 //   128 experts, MXFP4: 400 tokens 383 / 518, 800: 502 / 538, 1200: 698 / 562
 //   128 experts, bf16:  400 tokens 1057 / 1170, 800: 1354 / 1205
 // The rule knows nothing of the weights' format: both formats give the same bits.
+constexpr int kCus = 256;
 constexpr int kStreamMeanRows = 20;
 inline bool stream_batch(int T, int E) { return T <= kDirectTokens || T * kTopK <= kStreamMeanRows * E; }
 // row tiles of the grouped GEMMs in all, at most: row blocks of 32 (stream.hip) or tiles of 256 rows (gemm.hip)
@@ -203,12 +204,11 @@ hipError_t launch_stream_gate_up(const uint16_t *x, const void *w1, const uint16
 hipError_t launch_stream_down(const uint16_t *act, const void *w2, const uint16_t *w2_scale, const float *b2,
                               const DispatchBuffers &d, float *y, int H, int IM, int tiles, const DirectIds &ids,
                               hipStream_t s);
-// direct.topk_i != nullptr: the rows of y are found from the ids (inv is not read)
 // ldy: floats per row of y (the padded hidden size)
 hipError_t launch_combine(const float *y, int ldy, const int *inv, const float *topk_v, const int *pos, float *out,
-                          int T, int H, int accumulate, const DirectIds &direct, hipStream_t s);
+                          int T, int H, int accumulate, hipStream_t s);
 hipError_t launch_combine_residual(const float *y, int ldy, const int *inv, const float *topk_v, const int *pos,
-                                   uint16_t *x, int T, int H, const DirectIds &direct, hipStream_t s);
+                                   uint16_t *x, int T, int H, hipStream_t s);
 hipError_t launch_rmsnorm(const uint16_t *x, const float *weight, const int *pos, uint16_t *t_out,
                           int T, int H, hipStream_t s);
 

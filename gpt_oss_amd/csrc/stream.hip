@@ -226,8 +226,8 @@ template <int NP, bool GATE_UP, bool FP4, bool DIRECT>
 __global__ __launch_bounds__(kStreamKw * 64, NP == 1 ? 4 : 3) void stream_gemm_kernel(
     const uint4 *__restrict__ a_rows, const uint4 *__restrict__ w_frag, const uint16_t *__restrict__ w_scale,
     const float *__restrict__ bias_a, const float *__restrict__ bias_b, const int *__restrict__ rowmap,
-    const int *__restrict__ blk_expert, const int *__restrict__ totals, void *__restrict__ outp, int K, int N,
-    float limit, DirectIds ids) {
+    const int *__restrict__ blk_expert, const int *__restrict__ totals, int *__restrict__ inv,
+    void *__restrict__ outp, int K, int N, float limit, DirectIds ids) {
   constexpr int RG = kStreamRows / 16;
   __shared__ f32x4 part[kStreamKw * 4 * RG * 64];
   __shared__ int rows_sh[DIRECT ? kDirectSlotRows : kStreamRows];  // row of the tile -> token
@@ -248,6 +248,9 @@ __global__ __launch_bounds__(kStreamKw * 64, NP == 1 ? 4 : 3) void stream_gemm_k
     __shared__ int cnt[kStreamKw];
     const int lane = tid & 63;
     const int mine = direct_expert_of(ids, tid);
+    // the first column tile's workgroups also write where each assignment's row is, for the combine
+    const bool writes_inv = GATE_UP && P == 0 && blockIdx.y == 0;
+    if (writes_inv && ti == 0 && mine < 0 && tid < ids.T * kTopK) inv[tid] = -1;
     if (tid < 8) mask[tid] = 0;
     stream_barrier();
     if (mine >= 0) atomicOr(&mask[mine >> 5], 1u << (mine & 31));
@@ -282,6 +285,7 @@ __global__ __launch_bounds__(kStreamKw * 64, NP == 1 ? 4 : 3) void stream_gemm_k
     if (GATE_UP) {
       const int at = before + __popcll(bal & ((1ull << lane) - 1ull));
       if (mine == e && at < kDirectSlotRows) rows_sh[at] = tid / kTopK;
+      if (mine == e && writes_inv) inv[tid] = at < kDirectSlotRows ? row0 + at : -1;
       stream_barrier();
     }
   } else {
@@ -355,7 +359,7 @@ static hipError_t launch_stream_np(const uint4 *a, const uint4 *w, const uint16_
   const dim3 grid(tiles * ((pairs + NP - 1) / NP), two_tiles ? 2 : 1);
 #define MOE_STREAM(FP4, DIRECT)                                                 \
   stream_gemm_kernel<NP, GATE_UP, FP4, DIRECT><<<grid, kStreamKw * 64, 0, s>>>( \
-      a, w, w_scale, ba, bb, d.rowmap, d.blk_expert, d.totals, out, K, N, limit, ids)
+      a, w, w_scale, ba, bb, d.rowmap, d.blk_expert, d.totals, d.inv, out, K, N, limit, ids)
   if constexpr (NP == 1) {
     if (!w_scale) {
       if (ids.topk_i) MOE_STREAM(false, true); else MOE_STREAM(false, false);
