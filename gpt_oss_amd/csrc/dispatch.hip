@@ -47,6 +47,7 @@ struct PlanOut {
   int *totals;
   TileDesc *tiles_gate_up, *tiles_down;
   int tile_cap_gate_up, tile_cap_down;
+  int tile_rb;  // row blocks of the tallest tile
 };
 
 // The tiles of expert ee in the tile sequences of both GEMMs.  An expert's row
@@ -113,8 +114,7 @@ __device__ __forceinline__ int build_plan(int count, int E, int n_ct_gate_up, in
   ExpertInfo *info = out.info;
   int *totals = out.totals;
   const int n_rb = (count + kRowBlock - 1) / kRowBlock;
-  constexpr int kTileRb = kTileRows / kRowBlock;
-  const int n_mt = (n_rb + kTileRb - 1) / kTileRb;
+  const int n_mt = (n_rb + out.tile_rb - 1) / out.tile_rb;
   const int rb = n_mt ? n_rb / n_mt : 0;
   const int extra = n_mt ? n_rb - rb * n_mt : 0;
   // cost of one column tile's worth of the expert's row tiles
@@ -250,7 +250,7 @@ __device__ __forceinline__ int build_plan(int count, int E, int n_ct_gate_up, in
 }
 
 // The row-tile plan (see build_plan): an expert with M rows has ceil(M / 32) row
-// blocks, cut into n_mt = ceil(row blocks / 8) tiles as evenly as they go: the
+// blocks, cut into n_mt = ceil(row blocks / tile_rb) tiles as evenly as they go: the
 // first `extra` tiles are rb + 1 row blocks high, the others rb.  Its segment in
 // the padded row space is its row blocks and no more, so an expert pads to at
 // most 31 rows.  The tile sequence of either GEMM (n_ct column tiles per row
@@ -530,7 +530,7 @@ __global__ __launch_bounds__(256) void combine_kernel(const float *__restrict__ 
 }
 
 hipError_t launch_dispatch(const int *topk_i, const int *pos, int T, int E, int n_ct_gate_up,
-                           int n_ct_down, const DispatchBuffers &d, hipStream_t s) {
+                           int n_ct_down, int tile_rows, const DispatchBuffers &d, hipStream_t s) {
   const int n_blk = (T + kDispThreads - 1) / kDispThreads;
   // Rows of the padded space this batch can reach: every expert rounds its
   // rows up to a multiple of 32.
@@ -545,6 +545,7 @@ hipError_t launch_dispatch(const int *topk_i, const int *pos, int T, int E, int 
   plan.tiles_down = d.tiles_down;
   plan.tile_cap_gate_up = d.tile_cap_gate_up;
   plan.tile_cap_down = d.tile_cap_down;
+  plan.tile_rb = tile_rows / kRowBlock;
   if (n_blk <= kSmallRounds) {
     // small batches: one workgroup does both passes, one launch fewer
     dispatch_small_kernel<<<1, kDispThreads, 0, s>>>(topk_i, pos, T, E, n_ct_gate_up, n_ct_down, plan,
@@ -659,7 +660,7 @@ extern "C" int moe_dispatch_static(const int *topk_i, const int *pos, int n_toke
   // no GEMM follows: with no column tiles the plan kernel writes no tile tables
   d.tiles_gate_up = d.tiles_down = nullptr;
   d.tile_cap_gate_up = d.tile_cap_down = 0;
-  const hipError_t el = launch_dispatch(topk_i, pos, n_tokens, n_experts, 0, 0, d, static_cast<hipStream_t>(stream));
+  const hipError_t el = launch_dispatch(topk_i, pos, n_tokens, n_experts, 0, 0, kTileRows, d, static_cast<hipStream_t>(stream));
   if (el != hipSuccess)
     return set_error(MOE_ERR_HIP, "dispatch launch failed: %s", hipGetErrorString(el));
   return MOE_OK;

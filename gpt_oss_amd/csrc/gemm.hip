@@ -99,6 +99,14 @@ __device__ __forceinline__ void dma_to_lds_16(const uint4 *g, uint4 *lds_wave_ba
   __builtin_amdgcn_global_load_lds(g, lds_wave_base, 16, 0, 0);
 }
 
+// 16 bytes of the column operand.  STREAM: past the caches (see gemm_streams_weights).
+template <bool STREAM>
+__device__ __forceinline__ u32x4 load_cols(const uint4 *g) {
+  const u32x4 *v = reinterpret_cast<const u32x4 *>(g);
+  if constexpr (STREAM) return __builtin_nontemporal_load(v);
+  return *v;
+}
+
 // s_waitcnt with only the vector-memory counter constrained (gfx9 encoding).
 // Loads return in order, so "at most n outstanding" means "all but the newest n
 // have landed".  The compiler places its own waits before the first use of
@@ -168,14 +176,14 @@ struct StageRing {
 };
 
 // NW waves side by side over the columns, NBW column blocks per wave, R ring
-// slots (LDS stages for the row operand, register slots for the column operand).
-template <int NW_, int NBW_, int R_>
+// slots (LDS stages for the row operand, register slots for the column operand),
+// tiles of up to RBT_MAX row blocks, WGS workgroups per CU.
+template <int NW_, int NBW_, int R_, int RBT_MAX_, int WGS_>
 struct GemmCfg {
-  static constexpr int NW = NW_, NBW = NBW_, R = R_, KPS = 2;
+  static constexpr int NW = NW_, NBW = NBW_, R = R_, RBT_MAX = RBT_MAX_, WGS = WGS_, KPS = 2;
   static constexpr int THREADS = NW * 64;
   static constexpr int TILE_NB = NW * NBW;              // column blocks per tile
-  static constexpr int RBT_MAX = kTileRows / kRowBlock;  // row blocks per tile, at most
-  static constexpr int STAGE = RBT_MAX * KPS * 64;       // uint4 per LDS stage (16 KB)
+  static constexpr int STAGE = RBT_MAX * KPS * 64;      // uint4 per LDS stage (16 KB at 8 row blocks)
   static constexpr int EPI_LD = NBW * 32 + 8;            // floats per buffered output row
   static constexpr int EPI_WAVE = 32 * EPI_LD / 4;       // uint4 per wave of epilogue buffer
 };
@@ -198,7 +206,7 @@ struct GemmCfg {
 //
 // gemm_tile is the down GEMM; gate_up, whose row operand is scattered, is
 // gemm_tile_gl below.
-template <int RBT, int RS, typename C, bool FP4>
+template <int RBT, int RS, typename C, bool FP4, bool STREAM>
 __device__ __forceinline__ void gemm_tile(const uint4 *__restrict__ a_frag,  // [rb][KB][64]
                                           const uint4 *__restrict__ b_frag,  // expert: [nb][KB][64], FP4: [nb/2][KB/2][64]
                                           const uint16_t *__restrict__ b_scale,  // FP4: expert's [nb/2][KB/2][32] byte pairs
@@ -278,12 +286,12 @@ __device__ __forceinline__ void gemm_tile(const uint4 *__restrict__ a_frag,  // 
   auto issue_b = [&](int slot, int ks, int m) {
     if (FP4) {
       if (m == 0) {
-        bq[slot][0] = *reinterpret_cast<const u32x4 *>(b_src[0] + (size_t)ks * 64);
+        bq[slot][0] = load_cols<STREAM>(b_src[0] + (size_t)ks * 64);
       } else {
         bsc[slot] = s_src[(size_t)ks * 32];
       }
     } else {
-      bq[slot][m] = *reinterpret_cast<const u32x4 *>(b_src[m / KPS] + (size_t)(ks * KPS + m % KPS) * 64);
+      bq[slot][m] = load_cols<STREAM>(b_src[m / KPS] + (size_t)(ks * KPS + m % KPS) * 64);
     }
   };
   // FP4: the decoded operands of the step at hand, [column block][k block].
@@ -470,7 +478,7 @@ constexpr int kLineStages = 4;
 // an odd step 2d+1 needs, and B(ks+1), which every step's successor needs.  Even
 // steps need no barrier: they read a double stage that landed before the
 // previous odd step's barrier and refill nothing.
-template <int RBT, int RS, typename C, bool FP4>
+template <int RBT, int RS, typename C, bool FP4, bool STREAM>
 __device__ __forceinline__ void gemm_tile_gl(const uint4 *__restrict__ x_rows,  // token rows [T][KB * 2] of 16 bytes
                                              const uint4 *__restrict__ b_frag,
                                              const uint16_t *__restrict__ b_scale, int KB, int rb0, int rbt,
@@ -483,7 +491,7 @@ __device__ __forceinline__ void gemm_tile_gl(const uint4 *__restrict__ x_rows,  
                                              uint4 *__restrict__ s5, uint4 *__restrict__ s6,
                                              uint4 *__restrict__ s7) {
   constexpr int NBW = C::NBW, KPS = C::KPS, RB = C::R, NW = C::NW, R2 = kLineStages;
-  static_assert(KPS == 2 && NW == 4 && RB == 4 && C::RBT_MAX == 8 && (RS == 1 || RS == 2), "shape of the line gather");
+  static_assert(KPS == 2 && NW == 4 && RB == 4 && C::RBT_MAX <= 8 && (RS == 1 || RS == 2), "shape of the line gather");
   constexpr int NB = RBT * RS;                // row blocks staged per step
   constexpr int LA2 = NB;                     // DMA loads per wave and double step: one per row block
   constexpr int LB = FP4 ? 2 : NBW * KPS;     // register loads per wave and step
@@ -567,12 +575,12 @@ __device__ __forceinline__ void gemm_tile_gl(const uint4 *__restrict__ x_rows,  
   auto issue_b = [&](int slot, int ks, int m) {
     if (FP4) {
       if (m == 0) {
-        bq[slot][0] = *reinterpret_cast<const u32x4 *>(b_src[0] + (size_t)ks * 64);
+        bq[slot][0] = load_cols<STREAM>(b_src[0] + (size_t)ks * 64);
       } else {
         bsc[slot] = s_src[(size_t)ks * 32];
       }
     } else {
-      bq[slot][m] = *reinterpret_cast<const u32x4 *>(b_src[m / KPS] + (size_t)(ks * KPS + m % KPS) * 64);
+      bq[slot][m] = load_cols<STREAM>(b_src[m / KPS] + (size_t)(ks * KPS + m % KPS) * 64);
     }
   };
   bf16x8 bdec[NBW][KPS];
@@ -712,17 +720,21 @@ __device__ __forceinline__ void gemm_tile_gl(const uint4 *__restrict__ x_rows,  
   gate_up_epilogue<RBT, RS, C>(acc, outp, out_ld, limit, rb0, rbt, nb0, nb_valid, cw, rg, lane);
 }
 
-template <typename C, bool GATE_UP, bool FP4>
-__global__ __launch_bounds__(C::THREADS, 1) void grouped_gemm_kernel(
+template <typename C, bool GATE_UP, bool FP4, bool STREAM>
+__global__ __launch_bounds__(C::THREADS, C::WGS) void grouped_gemm_kernel(
     const uint4 *__restrict__ a_frag, const uint4 *__restrict__ w_frag,
     const uint16_t *__restrict__ w_scale,
     const float *__restrict__ bias_a, const float *__restrict__ bias_b,
     const TileDesc *__restrict__ tiles, const int *__restrict__ totals,
     const int *__restrict__ rowmap, void *__restrict__ outp, int K, int N, float limit) {
-  static_assert(C::R <= 4 && C::RBT_MAX == 8, "stage arrays and tile heights below");
-  __shared__ uint4 st0[C::STAGE], st1[C::STAGE], st2[C::STAGE], st3[C::STAGE];
-  __shared__ uint4 st4[GATE_UP ? C::STAGE : 1], st5[GATE_UP ? C::STAGE : 1], st6[GATE_UP ? C::STAGE : 1],
-      st7[GATE_UP ? C::STAGE : 1];
+  static_assert(C::R <= 4 && (C::RBT_MAX == 4 || C::RBT_MAX == 8), "stage arrays and tile heights below");
+  // gate_up: 4 KB per row block and double stage, four row blocks to an array;
+  // down: one array per stage
+  constexpr int ST_EVEN = GATE_UP ? 4 * 256 : C::STAGE;
+  constexpr int ST_ODD = GATE_UP ? (C::RBT_MAX == 8 ? 4 * 256 : 1) : C::STAGE;
+  __shared__ uint4 st0[ST_EVEN], st1[ST_ODD], st2[ST_EVEN], st3[ST_ODD];
+  __shared__ uint4 st4[GATE_UP ? ST_EVEN : 1], st5[GATE_UP ? ST_ODD : 1], st6[GATE_UP ? ST_EVEN : 1],
+      st7[GATE_UP ? ST_ODD : 1];
   __shared__ uint4 epi[GATE_UP ? 1 : C::NW * C::EPI_WAVE];
   const int KB = K / kFragK;
   const int nb_total = (GATE_UP ? 2 * N : N) / kRowBlock;  // weight row blocks per expert
@@ -735,84 +747,117 @@ __global__ __launch_bounds__(C::THREADS, 1) void grouped_gemm_kernel(
   const uint16_t *b_scale = FP4 ? w_scale + (size_t)tc.e * nb_total * KB * 8 : nullptr;
   const float *ba = bias_a + (size_t)tc.e * N;
   const float *bb = GATE_UP ? bias_b + (size_t)tc.e * N : nullptr;
-#define MOE_TILE_RS(n, rs)                                                                                    \
-  do {                                                                                                        \
-    if constexpr (GATE_UP) {                                                                                  \
-      if constexpr (rs <= 2)                                                                                  \
-        gemm_tile_gl<n, rs, C, FP4>(a_frag, b_frag, b_scale, KB, tc.rb0, tc.rbt, nb0, nb_valid, rowmap, ba,   \
-                                    bb, outp, N, limit, st0, st1, st2, st3, st4, st5, st6, st7);              \
-    } else {                                                                                                  \
-      gemm_tile<n, rs, C, FP4>(a_frag, b_frag, b_scale, KB, tc.rb0, tc.rbt, nb0, nb_valid, ba,                \
-                               static_cast<float *>(outp), N, st0, st1, st2, st3, epi);                       \
-    }                                                                                                         \
-  } while (0)
-#define MOE_TILE(n) MOE_TILE_RS(n, 1)
+  // the tile with n row blocks per wave and the waves in rs row groups
+  auto tile = [&](auto n_c, auto rs_c) {
+    constexpr int n = decltype(n_c)::value, rs = decltype(rs_c)::value;
+    if constexpr (n * rs <= C::RBT_MAX) {
+      if constexpr (GATE_UP) {
+        gemm_tile_gl<n, rs, C, FP4, STREAM>(a_frag, b_frag, b_scale, KB, tc.rb0, tc.rbt, nb0, nb_valid, rowmap,
+                                            ba, bb, outp, N, limit, st0, st1, st2, st3, st4, st5, st6, st7);
+      } else {
+        gemm_tile<n, rs, C, FP4, STREAM>(a_frag, b_frag, b_scale, KB, tc.rb0, tc.rbt, nb0, nb_valid, ba,
+                                         static_cast<float *>(outp), N, st0, st1, st2, st3, epi);
+      }
+    }
+  };
   // the last column tile, when only a quarter or half of the waves have columns in it
   const int rs = row_split_of(nb_valid, C::NW, C::NBW);
-  if (!GATE_UP && rs == 4) {  // gate_up comes in (gate, up) pairs of pairs: never a quarter
-    if (tc.rbt <= 4) MOE_TILE_RS(1, 4); else MOE_TILE_RS(2, 4);
-    return;
+  if constexpr (!GATE_UP) {  // gate_up comes in (gate, up) pairs of pairs: never a quarter
+    if (rs == 4) {
+      if (tc.rbt <= 4) tile(IC<1>{}, IC<4>{}); else tile(IC<2>{}, IC<4>{});
+      return;
+    }
   }
   if (rs == 2) {
     switch ((tc.rbt + 1) >> 1) {
-      case 1: MOE_TILE_RS(1, 2); break;
-      case 2: MOE_TILE_RS(2, 2); break;
-      case 3: MOE_TILE_RS(3, 2); break;
-      default: MOE_TILE_RS(4, 2); break;
+      case 1: tile(IC<1>{}, IC<2>{}); break;
+      case 2: tile(IC<2>{}, IC<2>{}); break;
+      case 3: tile(IC<3>{}, IC<2>{}); break;
+      default: tile(IC<4>{}, IC<2>{}); break;
     }
     return;
   }
   switch (tc.rbt) {
-    case 1: MOE_TILE(1); break;
-    case 2: MOE_TILE(2); break;
-    case 3: MOE_TILE(3); break;
-    case 4: MOE_TILE(4); break;
-    case 5: MOE_TILE(5); break;
-    case 6: MOE_TILE(6); break;
-    case 7: MOE_TILE(7); break;
-    default: MOE_TILE(8); break;
+    case 1: tile(IC<1>{}, IC<1>{}); break;
+    case 2: tile(IC<2>{}, IC<1>{}); break;
+    case 3: tile(IC<3>{}, IC<1>{}); break;
+    case 4: tile(IC<4>{}, IC<1>{}); break;
+    case 5: tile(IC<5>{}, IC<1>{}); break;
+    case 6: tile(IC<6>{}, IC<1>{}); break;
+    case 7: tile(IC<7>{}, IC<1>{}); break;
+    default: tile(IC<8>{}, IC<1>{}); break;
   }
-#undef MOE_TILE
-#undef MOE_TILE_RS
 }
 
 // 4 waves, one per SIMD, each 256 rows x 64 columns (8 x 2 accumulators = all
 // 256 accumulation registers); 256 x 256 tiles; 4 ring slots.
-using CfgGemm = GemmCfg<4, 2, 4>;
-static_assert(CfgGemm::RBT_MAX * kRowBlock == kTileRows && CfgGemm::TILE_NB == kGemmTileNb,
+using CfgFull = GemmCfg<4, 2, 4, 8, 1>;
+// MXFP4: tiles half as high, two workgroups per CU.  A step of MXFP4 weights is
+// 4 KB, so that a second tile of the same columns costs next to nothing, and the
+// decode, the fill and the epilogue of one workgroup run under the other's MFMAs.
+// us per layer call, full / half height (2880 x 2880, even routing): 32 experts,
+// 256 tokens 175 / 143, 512: 188 / 172, 1024: 242 / 242, 2048: 427 / 395, 4096:
+// 731 / 725; 128 experts, 768: 533 / 428, 2048: 621 / 551, 3072: 712 / 676.  With
+// bf16 weights (16 KB per step) it is the other way round where an expert then
+// takes two tiles: 1024 tokens 392 / 439, 6144 tokens and 128 experts 1639 / 1813.
+using CfgHalf = GemmCfg<4, 2, 4, 4, 2>;
+static_assert(CfgFull::RBT_MAX * kRowBlock == kTileRows && CfgHalf::RBT_MAX * kRowBlock == kHalfTileRows &&
+                  CfgFull::TILE_NB == kGemmTileNb && CfgHalf::TILE_NB == kGemmTileNb,
               "tile plan of build_plan");
 
+// Whether the expert matrices are read past the caches (non-temporal loads): while
+// most experts have one row tile their weights are read by one workgroup, and
+// lines that nobody reads again push the rows and the code out of L2.  us per
+// layer call, cached / past the caches: bf16 (tiles of 256 rows), 32 experts, 256
+// tokens 330 / 305, 512: 364 / 351, 1024: 392 / 374, 1536: 447 / 434; 128 experts,
+// 1024: 1234 / 1173, 6144 (192 rows per expert): 1639 / 1651; 8 experts, 256:
+// 143 / 135, 1024 (512 rows): 254 / 269.  MXFP4 (tiles of 128 rows), 32 experts,
+// 256 tokens 143 / 135, 512: 172 / 163, 1024 (128 rows): 242 / 245, 4096: 725 /
+// 750; 128 experts, 3072 (96 rows): 676 / 668.  MXFP4 in tiles of 256 rows gains
+// nothing (8 experts, 256 tokens 93 / 95).
+constexpr int kStreamRowsFull = 160, kStreamRowsHalf = 96;  // mean rows of an expert, at most
+static bool gemm_streams_weights(int T, int E, bool half) {
+  return T * kTopK <= (half ? kStreamRowsHalf : kStreamRowsFull) * E;
+}
+
 // w_scale == nullptr: w holds bf16 fragments; otherwise w holds MXFP4 chunks and
-// w_scale their scale bytes (pack_fp4_kernel).
+// w_scale their scale bytes (pack_fp4_kernel).  The plan is of tiles of plan.tile_rows.
 template <bool GATE_UP>
 static hipError_t launch_gemm(const void *a, const void *w, const uint16_t *w_scale, const float *ba,
                               const float *bb, const DispatchBuffers &d, void *out, int K, int N,
-                              float limit, int mt_cap, hipStream_t s) {
-  using C = CfgGemm;
+                              float limit, int T, int E, int tile_rows, hipStream_t s) {
   const int nb_total = (GATE_UP ? 2 * N : N) / kRowBlock;
-  const int n_ct = (nb_total + C::TILE_NB - 1) / C::TILE_NB;
-  const int grid = kXcds * xcd_tile_cap(mt_cap * n_ct);
+  const int n_ct = (nb_total + kGemmTileNb - 1) / kGemmTileNb;
+  const int grid = kXcds * xcd_tile_cap(gemm_tile_cap(T, E, tile_rows) * n_ct);
   const TileDesc *tiles = GATE_UP ? d.tiles_gate_up : d.tiles_down;
   const uint4 *af = static_cast<const uint4 *>(a), *wf = static_cast<const uint4 *>(w);
-  if (w_scale) {
-    grouped_gemm_kernel<C, GATE_UP, true><<<grid, C::THREADS, 0, s>>>(af, wf, w_scale, ba, bb, tiles, d.totals,
-                                                                      d.rowmap, out, K, N, limit);
+  // the full-height kernels take a plan of either height, the others one of half height
+  const bool half = w_scale && tile_rows == kHalfTileRows;
+  const bool stream = gemm_streams_weights(T, E, half);
+#define MOE_GEMM(C, FP4, STREAM)                                                                            \
+  grouped_gemm_kernel<C, GATE_UP, FP4, STREAM><<<grid, C::THREADS, 0, s>>>(af, wf, w_scale, ba, bb, tiles,  \
+                                                                           d.totals, d.rowmap, out, K, N, limit)
+  if (half) {
+    if (stream) MOE_GEMM(CfgHalf, true, true); else MOE_GEMM(CfgHalf, true, false);
+  } else if (w_scale) {
+    MOE_GEMM(CfgFull, true, false);
   } else {
-    grouped_gemm_kernel<C, GATE_UP, false><<<grid, C::THREADS, 0, s>>>(af, wf, nullptr, ba, bb, tiles, d.totals,
-                                                                       d.rowmap, out, K, N, limit);
+    if (stream) MOE_GEMM(CfgFull, false, true); else MOE_GEMM(CfgFull, false, false);
   }
+#undef MOE_GEMM
   return hipGetLastError();
 }
 
 hipError_t launch_gate_up(const uint16_t *x, const void *w1, const uint16_t *w1_scale, const float *b1g,
                           const float *b1u, const DispatchBuffers &d, uint16_t *act, int H, int IM,
-                          float limit, int mt_cap, hipStream_t s) {
-  return launch_gemm<true>(x, w1, w1_scale, b1g, b1u, d, act, H, IM, limit, mt_cap, s);
+                          float limit, int T, int E, int tile_rows, hipStream_t s) {
+  return launch_gemm<true>(x, w1, w1_scale, b1g, b1u, d, act, H, IM, limit, T, E, tile_rows, s);
 }
 
 hipError_t launch_down(const uint16_t *act, const void *w2, const uint16_t *w2_scale, const float *b2,
-                       const DispatchBuffers &d, float *y, int H, int IM, int mt_cap, hipStream_t s) {
-  return launch_gemm<false>(act, w2, w2_scale, b2, nullptr, d, y, IM, H, 0.f, mt_cap, s);
+                       const DispatchBuffers &d, float *y, int H, int IM, int T, int E, int tile_rows,
+                       hipStream_t s) {
+  return launch_gemm<false>(act, w2, w2_scale, b2, nullptr, d, y, IM, H, 0.f, T, E, tile_rows, s);
 }
 
 }  // namespace moe

@@ -65,6 +65,7 @@ struct moe_handle {
   int a_cap = 0;      // max assignments
   int a_pad_cap = 0;  // max padded rows
   int n_blk_cap = 0;
+  int plan_rows = kTileRows;  // tallest row tile of the last plan
   int disp_tokens = -1;  // batch of the last moe_dispatch (stage-level calls), -1: none
   bool gemms_done = false;  // moe_expert_gemms has run on that dispatch: y holds its rows
   bool distinct_ids = false;  // moe_set_distinct_ids: caller-supplied ids name an expert once per token
@@ -140,6 +141,15 @@ inline int down_col_tiles(const moe_handle *h) {
   return (h->Hp / kRowBlock + kGemmTileNb - 1) / kGemmTileNb;
 }
 
+// Plan of a batch for layers whose weights are all MXFP4 or not.  The kernels of
+// bf16 weights take a plan of either height (a caller may dispatch before it names the layer).
+int run_dispatch(moe_handle *h, const int *topk_i, const int *pos, int T, bool mxfp4, hipStream_t s) {
+  const int E = h->cfg.experts;
+  h->plan_rows = mxfp4 && half_tiles(T, E, gate_up_col_tiles(h)) ? kHalfTileRows : kTileRows;
+  HIP_TRY(launch_dispatch(topk_i, pos, T, E, gate_up_col_tiles(h), down_col_tiles(h), h->plan_rows, h->disp, s));
+  return MOE_OK;
+}
+
 // Stages 3-4 on the plan of the last dispatch: gate_up GEMM with the SwiGLU (it
 // reads the routed token rows itself, there is no gathered copy), down GEMM.
 // Leaves the per-assignment rows in h->y.
@@ -162,10 +172,10 @@ int run_gemms(moe_handle *h, int layer, const uint16_t *x, int T, const DirectId
     HIP_TRY(launch_stream_down(h->act, w2, lw.w2s, lw.b2, h->disp, h->y, h->Hp, h->IMp, tiles, direct, s));
     return MOE_OK;
   }
-  const int mt_cap = gemm_tile_cap(T, c.experts);
-  HIP_TRY(launch_gate_up(x, w1, lw.w1s, lw.b1g, lw.b1u, h->disp, h->act, h->Hp, h->IMp, c.swiglu_limit, mt_cap, s));
+  HIP_TRY(launch_gate_up(x, w1, lw.w1s, lw.b1g, lw.b1u, h->disp, h->act, h->Hp, h->IMp, c.swiglu_limit, T,
+                         c.experts, h->plan_rows, s));
   HIP_TRY(tm.mark(MOE_STAGE_DOWN));
-  HIP_TRY(launch_down(h->act, w2, lw.w2s, lw.b2, h->disp, h->y, h->Hp, h->IMp, mt_cap, s));
+  HIP_TRY(launch_down(h->act, w2, lw.w2s, lw.b2, h->disp, h->y, h->Hp, h->IMp, T, c.experts, h->plan_rows, s));
   return MOE_OK;
 }
 
@@ -193,12 +203,12 @@ int run_experts(moe_handle *h, int layer, const uint16_t *x, const int *pos, con
   // combine find their rows from the ids themselves
   const bool direct_plan = direct_plan_fits(T, max_rows, c.experts, h->a_pad_cap);
   const DirectIds direct{direct_plan ? topk_i : nullptr, pos, T, c.experts};
-  if (!direct_plan)
-    HIP_TRY(launch_dispatch(topk_i, pos, T, c.experts, gate_up_col_tiles(h), down_col_tiles(h), h->disp, s));
+  int rc = direct_plan ? MOE_OK : run_dispatch(h, topk_i, pos, T, h->layers[layer].w1q != nullptr, s);
+  if (rc != MOE_OK) return rc;
   h->unplanned = direct;
   h->disp_tokens = -1;  // the plan now belongs to this call, not to a moe_dispatch
   h->gemms_done = false;
-  int rc = run_gemms(h, layer, x, T, direct, s, tm);
+  rc = run_gemms(h, layer, x, T, direct, s, tm);
   if (rc != MOE_OK) return rc;
   return run_combine(h, topk_v, pos, T, out, accumulate, resid, s, tm);
 }
@@ -240,7 +250,7 @@ int moe_create(const moe_config *cfg, moe_handle **out) {
   }
   h->layers.resize(cfg->layers);
 
-  const int E = cfg->experts, H = cfg->hidden, IM = cfg->inter, T = cfg->max_tokens;
+  const int E = cfg->experts, H = cfg->hidden, T = cfg->max_tokens;
   h->a_cap = T * kTopK;
   h->a_pad_cap = ((h->a_cap + kTileGran * E + kTileGran - 1) / kTileGran) * kTileGran;
   // room for the fixed slots of the batches that run without a dispatch pass
@@ -260,7 +270,7 @@ int moe_create(const moe_config *cfg, moe_handle **out) {
   ALLOC(h->disp.info, (size_t)E);
   ALLOC(h->disp.totals, (size_t)kTotInts);
   {
-    const int mt_cap = gemm_tile_cap(T, E);  // row tiles at max_tokens, at most
+    const int mt_cap = gemm_tile_cap(T, E, kHalfTileRows);  // row tiles at max_tokens, at most
     h->disp.tile_cap_gate_up = mt_cap * gate_up_col_tiles(h);
     h->disp.tile_cap_down = mt_cap * down_col_tiles(h);
   }
@@ -467,8 +477,10 @@ int moe_dispatch(moe_handle *h, const int *topk_i, const int *pos, int n_tokens,
   if (n_tokens > h->cfg.max_tokens)
     return fail(MOE_ERR_CAPACITY, "n_tokens %d exceeds max_tokens %d", n_tokens, h->cfg.max_tokens);
   if (n_tokens > 0 && !topk_i) return fail(MOE_ERR_BAD_ARG, "null device pointer");
-  HIP_TRY(launch_dispatch(topk_i, pos, n_tokens, h->cfg.experts, gate_up_col_tiles(h),
-                          down_col_tiles(h), h->disp, static_cast<hipStream_t>(stream)));
+  bool mxfp4 = true;
+  for (const LayerWeights &lw : h->layers) mxfp4 = mxfp4 && !lw.w1;
+  const int rc = run_dispatch(h, topk_i, pos, n_tokens, mxfp4, static_cast<hipStream_t>(stream));
+  if (rc != MOE_OK) return rc;
   h->disp_tokens = n_tokens;
   h->gemms_done = false;
   h->unplanned.topk_i = nullptr;
@@ -481,9 +493,8 @@ int moe_get_dispatch(moe_handle *h, int *offsets, int *perm, int n_tokens, void 
     return fail(MOE_ERR_BAD_ARG, "n_tokens %d out of range", n_tokens);
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (h->unplanned.topk_i) {
-    const moe_config &c = h->cfg;
-    HIP_TRY(launch_dispatch(h->unplanned.topk_i, h->unplanned.pos, h->unplanned.T, c.experts,
-                            gate_up_col_tiles(h), down_col_tiles(h), h->disp, s));
+    const int rc = run_dispatch(h, h->unplanned.topk_i, h->unplanned.pos, h->unplanned.T, false, s);
+    if (rc != MOE_OK) return rc;
     h->unplanned.topk_i = nullptr;
   }
   if (offsets)

@@ -30,6 +30,7 @@ constexpr int kRowBlock = 32;   // rows of one MFMA fragment (v_mfma_f32_32x32x1
 constexpr int kFragK = 16;      // reduction depth of one fragment
 constexpr int kFragBytes = 1024;  // 64 lanes x 8 bf16
 constexpr int kTileRows = 256;  // tallest row tile of the grouped GEMMs
+constexpr int kHalfTileRows = 128;  // ... where two workgroups share a CU (MXFP4 weights, half_tiles)
 constexpr int kTileGran = 32;   // an expert's segment of padded rows is a multiple of one row block
 constexpr float kAlpha = 1.702f;  // run.cpp:709
 
@@ -141,8 +142,9 @@ struct DispatchBuffers {
   TileDesc *tiles_down;     // [tile_cap_down]    ... of the down GEMM
   int tile_cap_gate_up, tile_cap_down;
 };
+// tile_rows: tallest row tile of the plan (kTileRows or kHalfTileRows)
 hipError_t launch_dispatch(const int *topk_i, const int *pos, int T, int E, int n_ct_gate_up,
-                           int n_ct_down, const DispatchBuffers &d, hipStream_t s);
+                           int n_ct_down, int tile_rows, const DispatchBuffers &d, hipStream_t s);
 
 // Batches of at most kDirectTokens tokens run without a dispatch pass: the 256
 // threads of a workgroup hold one assignment each, so every workgroup of the
@@ -183,20 +185,30 @@ inline bool direct_plan_fits(int T, int max_rows, int E, int a_pad_cap) {
 constexpr int kCus = 256;
 constexpr int kStreamMeanRows = 20;
 inline bool stream_batch(int T, int E) { return T <= kDirectTokens || T * kTopK <= kStreamMeanRows * E; }
-// row tiles of the grouped GEMMs in all, at most: row blocks of 32 (stream.hip) or tiles of 256 rows (gemm.hip)
+// row tiles of the grouped GEMMs in all, at most: row blocks of 32 (stream.hip) or tiles of tile_rows (gemm.hip)
 inline int stream_tile_cap(int T, int E) {
   const int A = T * kTopK;
   return A < E ? A : (A / kRowBlock + E < A ? A / kRowBlock + E : A);
 }
-inline int gemm_tile_cap(int T, int E) { return T * kTopK / kTileRows + E; }
+inline int gemm_tile_cap(int T, int E, int tile_rows) { return T * kTopK / tile_rows + E; }
+// Height of the row tiles of a batch on MXFP4 weights (CfgHalf in gemm.hip has the
+// reason and times): half height where that gives the GPU its two workgroups per
+// CU.  With fewer tiles than that the full height keeps more columns' worth of work
+// in each (8 experts, 256 tokens: 93 us per layer call at full height, 104 at half;
+// 768 tokens, above the line: 183 / 181).
+inline bool half_tiles(int T, int E, int n_ct_gate_up) {
+  const int row_tiles = T * kTopK / kHalfTileRows > E ? T * kTopK / kHalfTileRows : E;
+  return (long long)row_tiles * n_ct_gate_up >= 2 * kCus;
+}
 // The first GEMM reads the routed token rows of x itself, through rowmap; there is
 // no gathered copy.  act holds the activation in the order the second GEMM of the
 // same file reads it: MFMA fragments (gemm.hip) or rows (stream.hip).
 hipError_t launch_gate_up(const uint16_t *x, const void *w1, const uint16_t *w1_scale, const float *b1g,
                           const float *b1u, const DispatchBuffers &d, uint16_t *act, int H, int IM,
-                          float limit, int mt_cap, hipStream_t s);
+                          float limit, int T, int E, int tile_rows, hipStream_t s);
 hipError_t launch_down(const uint16_t *act, const void *w2, const uint16_t *w2_scale, const float *b2,
-                       const DispatchBuffers &d, float *y, int H, int IM, int mt_cap, hipStream_t s);
+                       const DispatchBuffers &d, float *y, int H, int IM, int T, int E, int tile_rows,
+                       hipStream_t s);
 // tiles: experts that can have rows (ids.topk_i given) or row blocks of the plan, at most
 hipError_t launch_stream_gate_up(const uint16_t *x, const void *w1, const uint16_t *w1_scale, const float *b1g,
                                  const float *b1u, const DispatchBuffers &d, uint16_t *act, int H, int IM,

@@ -39,27 +39,6 @@
 #include "moe_internal.h"
 #include "swiglu.h"
 
-#ifndef PIN
-#define PIN
-#endif
-#ifndef OCC
-#define OCC 4
-#endif
-#ifndef D1
-#define D1 8
-#endif
-#ifndef D1B
-#define D1B 4
-#endif
-#ifndef D2
-#define D2 4
-#endif
-#ifndef D2B
-#define D2B 3
-#endif
-#ifndef NPV
-#define NPV 1
-#endif
 namespace moe {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));

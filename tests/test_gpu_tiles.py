@@ -1,0 +1,68 @@
+"""The grouped GEMMs at the edges of their row tiles: 256 rows, and 128 rows where
+the weights are MXFP4 and there are tiles enough; weights read through the caches
+and past them (few and many rows per expert); full, half and quarter column tiles.
+
+Bars as in test_gpu_parity.py: max-abs 2e-2 and rel-L2 1e-3 of the oracle on the
+same inputs; the two weight formats, whose tiles differ, bit for bit."""
+import numpy as np
+import pytest
+
+from gpt_oss_amd import abi, synth
+from oracle import binding as ob
+
+pytestmark = pytest.mark.gpu
+
+E = 32
+FEW = (1, 31, 32, 33, 63, 64, 65, 95, 96, 97, 127, 128, 129, 160, 161, 255, 256, 257)  # 1823 rows: 57 per expert
+MANY = FEW + (288, 383, 384, 385, 512, 513, 640, 800, 1024)  # 6752 rows: 211 per expert
+
+
+@pytest.mark.parametrize("rows", [FEW, MANY], ids=["few", "many"])
+@pytest.mark.parametrize("H,IM", [(64, 2048), (128, 2112), (192, 2080)])
+def test_row_tiles(rows, H, IM):
+    rng = np.random.default_rng(H + len(rows))
+    experts = rng.permutation(E)[:len(rows)]
+    ids = np.repeat(experts, rows).astype(np.int32)
+    T = -(-len(ids) // 4)
+    ids = rng.permutation(np.concatenate([ids, np.full(4 * T - len(ids), -1, np.int32)])).reshape(T, 4)
+    tv = rng.random((T, 4)).astype(np.float32)
+    sh = synth.LayerShape("tiles", T, H, IM, E)
+    x = synth.round_bf16(synth.make_activations(sh))
+    wr, br = (synth.round_bf16(a) for a in synth.make_router(sh))
+    b1k, s1, b1, b2k, s2, b2 = synth.make_experts_mxfp4(sh)
+    b1, b2 = synth.round_bf16(b1), synth.round_bf16(b2)
+    w1, w2 = ob.mxfp4_dequant(b1k, s1), ob.mxfp4_dequant(b2k, s2)
+    dx, dti = abi.DevBuf.from_numpy(synth.to_bf16_bits(x)), abi.DevBuf.from_numpy(ids)
+    dtv, dout = abi.DevBuf.from_numpy(tv), abi.DevBuf(T * H * 4)
+    got = []
+    for fp4 in (True, False):
+        m = abi.Moe(H, IM, E, max_tokens=T, swiglu_limit=sh.limit)
+        if fp4:
+            m.upload_layer_mxfp4(0, wr, br, b1k, s1, b1, b2k, s2, b2)
+        else:
+            m.upload_layer(0, wr, br, w1, b1, w2, b2)
+        dout.memset(0xFF)
+        m.experts(0, dx, None, dti, dtv, T, dout)
+        abi.sync()
+        got.append(dout.download((T, H), np.float32))
+        # stage by stage: the dispatch does not know the layer
+        dout.memset(0xFF)
+        m.dispatch(dti, None, T)
+        m.expert_gemms(0, dx, T)
+        m.combine(dtv, None, T, dout)
+        abi.sync()
+        got.append(dout.download((T, H), np.float32))
+        m.close()
+    for other in got[1:]:
+        assert np.array_equal(got[0], other)
+    # a token of every expert at least, and those of the tiles' last rows
+    some = np.unique(np.concatenate([np.nonzero((ids == e).any(1))[0][[0, -1]] for e in experts]))
+    want = np.zeros((len(some), H), np.float32)
+    for i, t in enumerate(some):
+        for k, e in enumerate(ids[t]):
+            if e >= 0:
+                want[i] += tv[t, k] * ob.expert_token(x[t], w1[e], b1[e], w2[e], b2[e], sh.limit,
+                                                      mode=ob.ROUND_ACT_BF16)
+    d = got[0][some] - want
+    assert np.abs(d).max() <= 2e-2 * max(1.0, float(np.abs(want).max()))
+    assert np.linalg.norm(d) <= 1e-3 * np.linalg.norm(want)
