@@ -146,7 +146,10 @@ inline int down_col_tiles(const moe_handle *h) {
 int run_dispatch(moe_handle *h, const int *topk_i, const int *pos, int T, bool mxfp4, hipStream_t s) {
   const int E = h->cfg.experts;
   h->plan_rows = mxfp4 && half_tiles(T, E, gate_up_col_tiles(h)) ? kHalfTileRows : kTileRows;
-  HIP_TRY(launch_dispatch(topk_i, pos, T, E, gate_up_col_tiles(h), down_col_tiles(h), h->plan_rows, h->disp, s));
+  // the kernels of stream.hip go by row blocks and need no tile tables
+  const bool tables = !stream_batch(T, E);
+  HIP_TRY(launch_dispatch(topk_i, pos, T, E, tables ? gate_up_col_tiles(h) : 0, tables ? down_col_tiles(h) : 0,
+                          h->plan_rows, h->disp, s));
   return MOE_OK;
 }
 

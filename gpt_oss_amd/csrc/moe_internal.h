@@ -177,13 +177,15 @@ inline bool direct_plan_fits(int T, int max_rows, int E, int a_pad_cap) {
 // average when every expert is active.  Those kernels take 32 rows per tile, and
 // an expert with more streams its weights again: measured on either side of the
 // line, us per layer call with the kernels of stream.hip and of gemm.hip:
-//   32 experts, MXFP4:  128 tokens 125 / 157, 192: 146 / 158, 256: 186 / 179
-//   32 experts, bf16:   128 tokens 297 / 319, 192: 325 / 319, 256: 471 / 332
-//   128 experts, MXFP4: 400 tokens 383 / 518, 800: 502 / 538, 1200: 698 / 562
-//   128 experts, bf16:  400 tokens 1057 / 1170, 800: 1354 / 1205
+//   32 experts, MXFP4:  96 tokens 110 / 121, 128: 121 / 121, 192: 149 / 132
+//   32 experts, bf16:   96 tokens 282 / 289, 128: 295 / 290, 192: 332 / 294
+//   128 experts, MXFP4: 384 tokens 374 / 386, 512: 402 / 386, 640: 432 / 400
+//   128 experts, bf16:  384 tokens 1047 / 1112, 512: 1110 / 1134, 640: 1177 / 1133
+// (Zipf routing, 256 tokens, 128 experts: 292 / 291 MXFP4, 804 / 730 bf16: there an
+// expert with many rows streams its weights several times; the host does not know.)
 // The rule knows nothing of the weights' format: both formats give the same bits.
 constexpr int kCus = 256;
-constexpr int kStreamMeanRows = 20;
+constexpr int kStreamMeanRows = 16;
 inline bool stream_batch(int T, int E) { return T <= kDirectTokens || T * kTopK <= kStreamMeanRows * E; }
 // row tiles of the grouped GEMMs in all, at most: row blocks of 32 (stream.hip) or tiles of tile_rows (gemm.hip)
 inline int stream_tile_cap(int T, int E) {

@@ -17,7 +17,7 @@ pytestmark = pytest.mark.gpu
 W = ("w_router", "b_router", "w_mlp1", "b_mlp1", "w_mlp2", "b_mlp2")
 
 
-@pytest.mark.parametrize("rows", [1, 16, 17, 32, 33, 64, 65, 150])
+@pytest.mark.parametrize("rows", [1, 16, 17, 32, 33, 64, 65, 128, 150])
 @pytest.mark.parametrize("H,IM", [(64, 64), (192, 320), (704, 64)])
 def test_rows_of_an_expert(rows, H, IM):
     """Every token names the experts 2, 30, 31 and 0: each has all the rows."""
