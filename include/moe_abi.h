@@ -183,12 +183,11 @@ int moe_experts(moe_handle *h, int layer, const uint16_t *x, const int *pos,
  * moe_expert_gemms): distinct != 0 says that the K ids of a token name K
  * different experts, which holds for any top-k selection, the reference's
  * included (run.cpp:388-421, utility/utility.cpp:273-365).  No expert then gets
- * more rows than the batch has tokens, and batches of up to 64 tokens run the
- * small-batch kernels (no dispatch pass, several workgroups per CU) as they do
- * under moe_forward.  Without the promise (the default) an expert may be named
- * in all K slots of every token and only batches of up to 16 tokens take that
- * path.  Ids that break the promise do not fault: rows beyond an expert's 64
- * are dropped.  Has no counterpart in the reference. */
+ * more rows than the batch has tokens, and batches of up to 64 tokens run
+ * without a dispatch pass as they do under moe_forward.  Without the promise
+ * (the default) an expert may be named in all K slots of every token and only
+ * batches of up to 16 tokens do.  Ids that break the promise do not fault: rows
+ * beyond an expert's 64 are dropped.  Has no counterpart in the reference. */
 int moe_set_distinct_ids(moe_handle *h, int distinct);
 
 /* moe_dispatch for callers that cannot allocate device memory: code under HIP
