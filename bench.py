@@ -270,7 +270,9 @@ def main():
     combine_bytes = A * H * 2 + T * H * 4
     mfma_tflops = flops_gate_up / t_gate_up / 1e12
     hbm_gbs = bytes_gate_up / t_gate_up / 1e9
-    kernel = "grouped_gemm_kernel<gate_up%s>" % (", MXFP4" if mxfp4 else "")
+    # few rows per expert: the kernels of stream.hip (stream_batch in moe_internal.h)
+    kernel = "%s<gate_up%s>" % ("stream_gemm_kernel" if T <= 64 or T * K <= 16 * E else "grouped_gemm_kernel",
+                                ", MXFP4" if mxfp4 else "")
     if BOUND[shape.name] == "mfma":
         roofline = {"bound": "mfma", "kernel": kernel, "achieved": mfma_tflops, "peak": PEAK_BF16_TFLOPS,
                     "unit": "TFLOP/s", "frac": mfma_tflops / PEAK_BF16_TFLOPS}
