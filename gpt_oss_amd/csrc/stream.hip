@@ -68,10 +68,11 @@ __device__ __forceinline__ void stream_slice(const uint4 *__restrict__ a_rows, i
   const int r = lane & 15, q = lane >> 4;
   const int piece = (q >> 1) + 2 * (q & 1);
   // addresses: a base that is the same for the whole wave and moves with the step,
-  // plus a 32-bit offset per lane that does not
-  uint32_t a_off[RG];
+  // plus an offset per lane that does not.  The rows' is 64 bits wide: the fixed
+  // slots of 256 experts reach 4 GiB from an intermediate size of 131 600 on.
+  size_t a_off[RG];
 #pragma unroll
-  for (int g = 0; g < RG; g++) a_off[g] = ((uint32_t)row[g] * (uint32_t)lda + piece) * 16u;
+  for (int g = 0; g < RG; g++) a_off[g] = ((size_t)row[g] * lda + piece) * 16;
   // bf16: fragment (block b, k block kb) is 64 pieces; this lane's piece of half hh is
   // kb = q & 1, (q >> 1) * 32 + 16 hh + r.  FP4: one chunk of 64 pieces per step.
   const uint32_t w_off = FP4 ? lane * 16u : ((q & 1) * 64 + (q >> 1) * 32 + r) * 16u;

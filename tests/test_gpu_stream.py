@@ -73,3 +73,46 @@ def test_two_pairs_of_columns_per_wave(T):
     assert np.abs(got - want).max() <= 2e-2 * max(1.0, float(np.abs(want).max()))
     m4.close()
     m16.close()
+
+
+def test_activation_past_4_gib():
+    """256 experts with fixed slots of 64 rows and an intermediate size at which the
+    last slot lies past 4 GiB of the activation: the first and the last expert (all
+    have the same matrices) give the oracle's rows.  The down GEMM's sums of 131616
+    products are compared at the bars above, which scale with the rows."""
+    E, H, IM, T = 256, 32, 131616, 3
+    assert (E - 1) * 64 * (IM // 64 * 64 + 64) * 2 > 2**32
+    rng = np.random.default_rng(5)
+
+    def codes(rows, cols, exp):
+        return (rng.integers(0, 256, (1, rows, cols // 32, 16), dtype=np.uint8),
+                rng.integers(exp, exp + 3, (1, rows, cols // 32), dtype=np.uint8))
+
+    (b1k, s1), (b2k, s2) = codes(2 * IM, H, 122), codes(H, IM, 114)
+    b1 = synth.round_bf16(rng.standard_normal((1, 2 * IM)).astype(np.float32) * 0.1)
+    b2 = synth.round_bf16(rng.standard_normal((1, H)).astype(np.float32) * 0.1)
+    x = synth.round_bf16(rng.standard_normal((T, H)).astype(np.float32))
+
+    def each(a):
+        return np.repeat(a, E, axis=0)
+
+    m = abi.Moe(H, IM, E, max_tokens=T, swiglu_limit=7.0)
+    m.upload_layer_mxfp4(0, np.zeros((E, H), np.float32), np.zeros(E, np.float32), each(b1k), each(s1), each(b1),
+                         each(b2k), each(s2), each(b2))
+    m.set_distinct_ids(True)
+    w1, w2 = ob.mxfp4_dequant(b1k, s1)[0], ob.mxfp4_dequant(b2k, s2)[0]
+    rows = np.stack([ob.expert_token(x[t], w1, b1[0], w2, b2[0], 7.0, mode=ob.ROUND_ACT_BF16) for t in range(T)])
+    tv = np.array([[0.1, 0.2, 0.3, 0.4]] * T, np.float32)
+    dx, dtv, dout = abi.DevBuf.from_numpy(synth.to_bf16_bits(x)), abi.DevBuf.from_numpy(tv), abi.DevBuf(T * H * 4)
+    got = []
+    for ids in ([0, 1, 2, 3], [255, 254, 253, 252], [0, 255, 128, 64]):
+        dti = abi.DevBuf.from_numpy(np.array([ids] * T, np.int32))
+        dout.memset(0xFF)
+        m.experts(0, dx, None, dti, dtv, T, dout)
+        abi.sync()
+        got.append(dout.download((T, H), np.float32))
+        d = got[-1] - rows
+        assert np.linalg.norm(d) <= 1e-3 * np.linalg.norm(rows), ids
+        assert np.abs(d).max() <= 2e-2 * max(1.0, float(np.abs(rows).max())), ids
+    assert np.array_equal(got[0], got[1]) and np.array_equal(got[0], got[2])
+    m.close()
