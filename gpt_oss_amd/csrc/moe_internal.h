@@ -174,15 +174,15 @@ inline bool direct_plan_fits(int T, int max_rows, int E, int a_pad_cap) {
 }
 // Batches in which the weights are a stream run the kernels of stream.hip: up to
 // kDirectTokens tokens, and up to kStreamMeanRows rows per active expert on
-// average when every expert is active.  Those kernels take 32 rows per tile, and
-// an expert with more streams its weights again: measured on either side of the
-// line, us per layer call with the kernels of stream.hip and of gemm.hip:
-//   32 experts, MXFP4:  96 tokens 110 / 121, 128: 121 / 121, 192: 149 / 132
-//   32 experts, bf16:   96 tokens 282 / 289, 128: 295 / 290, 192: 332 / 294
-//   128 experts, MXFP4: 384 tokens 374 / 386, 512: 402 / 386, 640: 432 / 400
-//   128 experts, bf16:  384 tokens 1047 / 1112, 512: 1110 / 1134, 640: 1177 / 1133
-// (Zipf routing, 256 tokens, 128 experts: 292 / 291 MXFP4, 804 / 730 bf16: there an
-// expert with many rows streams its weights several times; the host does not know.)
+// average when every expert is active.  Those kernels take 32 rows per tile, so an
+// expert with more is multiplied (and, with MXFP4, decoded) once per tile, by
+// workgroups that read its weights side by side (share_of in stream.hip).  On
+// either side of the line, us per moe_experts call at 2880 x 2880 with the kernels
+// of stream.hip / of gemm.hip, even routing and Zipf's (exponent 1.2):
+//   32 experts, MXFP4:  96 tokens 101 / 114, 101 / 122;  128: 107 / 108, 113 / 125;  192: 121 / 115, 124 / 156
+//   32 experts, bf16:   96 tokens 268 / 276, 272 / 281;  128: 281 / 276, 283 / 296;  192: 303 / 282, 327 / 308
+//   128 experts, MXFP4: 384 tokens 340 / 358, 324 / 369;  512: 372 / 361, 380 / 408;  640: 396 / 367, 427 / 429
+//   128 experts, bf16:  384 tokens 1017 / 1086, 1018 / 1024;  512: 1071 / 1084, 1111 / 1072;  640: 1129 / 1085, 1199 / 1114
 // The rule knows nothing of the weights' format: both formats give the same bits.
 constexpr int kCus = 256;
 constexpr int kStreamMeanRows = 16;

@@ -56,11 +56,35 @@ constexpr int kStreamTwoPairs = 1024;
 // Orders LDS traffic only: the loads in flight stay in flight.
 __device__ __forceinline__ void stream_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
+// 16 bytes of weights: past the caches where one workgroup reads them (measured,
+// see above), through them where several do at about the same time (share_of).
+template <bool SHARED>
+__device__ __forceinline__ u32x4 load_weights(const char *g) {
+  const u32x4 *v = reinterpret_cast<const u32x4 *>(g);
+  if constexpr (SHARED) return *v;
+  return __builtin_nontemporal_load(v);
+}
+
+// Place of workgroup l of an expert with nb tiles of rows and wgs tiles of columns:
+// eight column tiles at a time, their first row tiles, then their second ones, and
+// so on.  Workgroup ids are dealt round-robin to the XCDs, so the row tiles that
+// read the same weights run at about the same time on one XCD and the weights come
+// from HBM once.  With a row tile's workgroups wgs ids apart and every load past the
+// caches each tile fetched them for itself: 128 experts, bf16, Zipf routing (exponent
+// 1.2), us per moe_experts call at 256 tokens 958, with this order 888, at 512 tokens
+// 1294 and 1130; MXFP4 301 and 279, 415 and 380; even routing within 1 %.
+__device__ __forceinline__ void share_of(int l, int wgs, int nb, int &col, int &blk) {
+  const int g = l / (kXcds * nb), r = l - g * kXcds * nb;
+  const int width = min(kXcds, wgs - g * kXcds);
+  blk = r / width;
+  col = g * kXcds + r - blk * width;
+}
+
 // One wave's share of a tile: RG groups of 16 rows times NP pairs of column
 // blocks over the steps [ks0, ks0 + n) of 32 k.  a_rows: rows of lda 16-byte
 // pieces; row[g]: the row this lane feeds in group g.  np_valid: pairs inside
 // the matrix; one past it repeats the first, and its sums are not used.
-template <int NP, int RG, int D, bool FP4>
+template <int NP, int RG, int D, bool FP4, bool SHARED>
 __device__ __forceinline__ void stream_slice(const uint4 *__restrict__ a_rows, int lda, const int (&row)[RG],
                                              const uint4 *__restrict__ w, const uint16_t *__restrict__ ws, int KB,
                                              int np_valid, int ks0, int n, int lane, f32x4 (&acc)[NP][4][RG]) {
@@ -85,18 +109,16 @@ __device__ __forceinline__ void stream_slice(const uint4 *__restrict__ a_rows, i
 #pragma unroll
     for (int p = 0; p < NP; p++) {
       const size_t pair = p < np_valid ? p : 0;
-      // the weights are read once: they go past the caches (measured, see above)
       if (FP4) {
         const char *wb = reinterpret_cast<const char *>(w) + pair * KB * 512 + k * 1024;
         const char *sb = reinterpret_cast<const char *>(ws) + pair * KB * 32 + k * 64;
-        wq[d][p][0] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(wb + w_off));
+        wq[d][p][0] = load_weights<SHARED>(wb + w_off);
         sc[d][p] = *reinterpret_cast<const uint32_t *>(sb + s_off);
       } else {
         const char *wb = reinterpret_cast<const char *>(w) + pair * KB * 2048 + k * 2048;
 #pragma unroll
         for (int i = 0; i < 4; i++)
-          wq[d][p][i] = __builtin_nontemporal_load(
-              reinterpret_cast<const u32x4 *>(wb + (size_t)(i >> 1) * KB * 1024 + (i & 1) * 256 + w_off));
+          wq[d][p][i] = load_weights<SHARED>(wb + (size_t)(i >> 1) * KB * 1024 + (i & 1) * 256 + w_off);
       }
     }
     const char *ab = reinterpret_cast<const char *>(a_rows) + k * 64;
@@ -202,12 +224,13 @@ __device__ __forceinline__ void stream_finish(const f32x4 *part, const float *__
 // its own by ballot; workgroup i * wgs + c is column tile c of the i-th expert
 // with rows, so that the column tiles of the few experts a small batch reaches
 // spread over all XCDs.  Otherwise a tile is a row block of the plan's padded rows.
+// tiles: experts that have rows or row blocks, at most.
 template <int NP, bool GATE_UP, bool FP4, bool DIRECT>
 __global__ __launch_bounds__(kStreamKw * 64, NP == 1 ? 4 : 3) void stream_gemm_kernel(
     const uint4 *__restrict__ a_rows, const uint4 *__restrict__ w_frag, const uint16_t *__restrict__ w_scale,
     const float *__restrict__ bias_a, const float *__restrict__ bias_b, const int *__restrict__ rowmap,
     const int *__restrict__ blk_expert, const int *__restrict__ totals, int *__restrict__ inv,
-    void *__restrict__ outp, int K, int N, float limit, DirectIds ids) {
+    void *__restrict__ outp, int K, int N, float limit, int tiles, DirectIds ids) {
   constexpr int RG = kStreamRows / 16;
   __shared__ f32x4 part[kStreamKw * 4 * RG * 64];
   __shared__ int rows_sh[DIRECT ? kDirectSlotRows : kStreamRows];  // row of the tile -> token
@@ -216,20 +239,21 @@ __global__ __launch_bounds__(kStreamKw * 64, NP == 1 ? 4 : 3) void stream_gemm_k
   const int n_cols = GATE_UP ? 2 * N : N;
   const int pairs = n_cols / kStreamCols;
   const int wgs = (pairs + NP - 1) / NP;
-  const int ti = blockIdx.x / wgs, P = (blockIdx.x - ti * wgs) * NP;
-  const int np_valid = min(NP, pairs - P);
   const int KB = K / kFragK, steps = K / 32;
   const int per = (steps + kStreamKw - 1) / kStreamKw;
   const int ks0 = min(w * per, steps), n = min(per, steps - ks0);
-  int e, row0, count;
+  int e, row0, count, col;
+  bool shared;  // more than one tile of rows reads these weights
   if constexpr (DIRECT) {
     static_assert(kStreamKw * 64 == kDirectTokens * kTopK, "one thread per assignment");
     __shared__ uint32_t mask[8];
     __shared__ int cnt[kStreamKw];
     const int lane = tid & 63;
     const int mine = direct_expert_of(ids, tid);
+    const int ti = blockIdx.x / wgs;
+    col = blockIdx.x - ti * wgs;
     // the first column tile's workgroups also write where each assignment's row is, for the combine
-    const bool writes_inv = GATE_UP && P == 0 && blockIdx.y == 0;
+    const bool writes_inv = GATE_UP && col == 0 && blockIdx.y == 0;
     if (writes_inv && ti == 0 && mine < 0 && tid < ids.T * kTopK) inv[tid] = -1;
     if (tid < 8) mask[tid] = 0;
     stream_barrier();
@@ -262,6 +286,7 @@ __global__ __launch_bounds__(kStreamKw * 64, NP == 1 ? 4 : 3) void stream_gemm_k
     }
     count = __builtin_amdgcn_readfirstlane(min(count, kDirectSlotRows));
     row0 = e * kDirectSlotRows;
+    shared = count > kStreamRows;
     if (GATE_UP) {
       const int at = before + __popcll(bal & ((1ull << lane) - 1ull));
       if (mine == e && at < kDirectSlotRows) rows_sh[at] = tid / kTopK;
@@ -269,17 +294,29 @@ __global__ __launch_bounds__(kStreamKw * 64, NP == 1 ? 4 : 3) void stream_gemm_k
       stream_barrier();
     }
   } else {
-    if (ti >= totals[kTotRows] / kRowBlock) return;  // surplus workgroups of the upper-bound grid
+    // Row block ti is one of an expert's: its blocks (those among the 64 from `from`)
+    // stand in a row and share the wgs workgroups of each (share_of).
+    const int ti = blockIdx.x / wgs, from = ti & ~63;
     const int lane = tid & 63;
-    e = __builtin_amdgcn_readfirstlane(blk_expert[ti]);
-    row0 = ti * kRowBlock;
-    const int a = lane < kStreamRows ? rowmap[row0 + lane] : -1;
+    const int n_blk = totals[kTotRows] / kRowBlock;
+    const int be = blk_expert[min(from + lane, tiles - 1)];
+    int a = lane < kStreamRows ? rowmap[ti * kRowBlock + lane] : -1;  // asked for before it is known to be the one
+    if (ti >= n_blk) return;  // surplus workgroups of the upper-bound grid
+    e = __builtin_amdgcn_readlane(be, ti & 63);
+    const unsigned long long own = __ballot(be == e && from + lane < n_blk);
+    const int first = from + __builtin_ctzll(own), nb = __popcll(own);
+    int blk;
+    share_of(blockIdx.x - first * wgs, wgs, nb, col, blk);
+    shared = nb > 1;
+    row0 = (first + blk) * kRowBlock;
+    if (first + blk != ti) a = lane < kStreamRows ? rowmap[row0 + lane] : -1;
     count = __popcll(__ballot(a >= 0));  // the valid rows of a block come first
     if (GATE_UP) {
       if (w == 0 && lane < count) rows_sh[lane] = a / kTopK;
       stream_barrier();
     }
   }
+  const int P = col * NP, np_valid = min(NP, pairs - P);
   const size_t blk0 = (size_t)e * (n_cols / kRowBlock) + 2 * P;
   const uint4 *wp = w_frag + blk0 * (size_t)(KB * (FP4 ? 16 : 64));
   const uint16_t *sp = FP4 ? w_scale + blk0 * KB * 8 : nullptr;
@@ -299,10 +336,11 @@ __global__ __launch_bounds__(kStreamKw * 64, NP == 1 ? 4 : 3) void stream_gemm_k
       const int rr = r0 + min(16 * g + (lane & 15), rows - 1);
       row[g] = GATE_UP ? rows_sh[rr] : row0 + rr;
     }
-    auto tile = [&](auto g_c, auto d_c, const auto &tile_row) {
+    auto tile = [&](auto g_c, auto d_c, auto shared_c, const auto &tile_row) {
       constexpr int G = decltype(g_c)::value;
       f32x4 acc[NP][4][G];
-      stream_slice<NP, G, decltype(d_c)::value, FP4>(a_rows, K / 8, tile_row, wp, sp, KB, np_valid, ks0, n, lane, acc);
+      stream_slice<NP, G, decltype(d_c)::value, FP4, decltype(shared_c)::value>(a_rows, K / 8, tile_row, wp, sp, KB,
+                                                                                np_valid, ks0, n, lane, acc);
 #pragma unroll
       for (int p = 0; p < NP; p++) {
         if (p >= np_valid) break;
@@ -319,11 +357,14 @@ __global__ __launch_bounds__(kStreamKw * 64, NP == 1 ? 4 : 3) void stream_gemm_k
     // (more gain nothing: at 64 tokens and MXFP4 weights the same time with 4, 6 and 8)
     using One = std::integral_constant<int, 1>;
     using Two = std::integral_constant<int, 2>;
-    if (rows <= 16) {
-      const int one[1] = {row[0]};
-      tile(One{}, std::integral_constant<int, FP4 ? (NP == 1 ? 6 : 4) : 4>{}, one);
+    using DeepTwo = std::integral_constant<int, FP4 ? (NP == 1 ? 4 : 2) : 3>;
+    if (shared) {
+      tile(Two{}, DeepTwo{}, std::true_type{}, row);
+    } else if (rows > 16) {
+      tile(Two{}, DeepTwo{}, std::false_type{}, row);
     } else {
-      tile(Two{}, std::integral_constant<int, FP4 ? (NP == 1 ? 4 : 2) : 3>{}, row);
+      const int one[1] = {row[0]};
+      tile(One{}, std::integral_constant<int, FP4 ? (NP == 1 ? 6 : 4) : 4>{}, std::false_type{}, one);
     }
   }
 }
@@ -339,7 +380,7 @@ static hipError_t launch_stream_np(const uint4 *a, const uint4 *w, const uint16_
   const dim3 grid(tiles * ((pairs + NP - 1) / NP), two_tiles ? 2 : 1);
 #define MOE_STREAM(FP4, DIRECT)                                                 \
   stream_gemm_kernel<NP, GATE_UP, FP4, DIRECT><<<grid, kStreamKw * 64, 0, s>>>( \
-      a, w, w_scale, ba, bb, d.rowmap, d.blk_expert, d.totals, d.inv, out, K, N, limit, ids)
+      a, w, w_scale, ba, bb, d.rowmap, d.blk_expert, d.totals, d.inv, out, K, N, limit, tiles, ids)
   if constexpr (NP == 1) {
     if (!w_scale) {
       if (ids.topk_i) MOE_STREAM(false, true); else MOE_STREAM(false, false);

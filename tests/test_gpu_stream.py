@@ -75,6 +75,49 @@ def test_two_pairs_of_columns_per_wave(T):
     m16.close()
 
 
+def test_hot_experts_under_a_plan():
+    """512 tokens over 128 experts, most rows at a few of them: experts of two and
+    of many row blocks, one of them on both sides of the 64th block, single blocks
+    between them; column tiles that are no multiple of the eight XCDs, an odd number
+    of pairs.  MXFP4 (two pairs per wave) and bf16 (one) bit for bit, and the oracle
+    at the first and last token of every expert."""
+    E, H, IM, T = 128, 704, 384, 512
+    counts = {**{e: 33 for e in range(30)}, 30: 290, 31: 1, 32: 16, 33: 17, 34: 32, 35: 64, 100: 138, 127: 500}
+    assert sum(counts.values()) == 4 * T
+    rng = np.random.default_rng(12)
+    ids = rng.permutation(np.repeat(list(counts), list(counts.values())).astype(np.int32)).reshape(T, 4)
+    tv = rng.random((T, 4)).astype(np.float32)
+    sh = synth.LayerShape("hot", T, H, IM, E)
+    x = synth.round_bf16(synth.make_activations(sh))
+    wr, br = (synth.round_bf16(a) for a in synth.make_router(sh))
+    b1k, s1, b1, b2k, s2, b2 = synth.make_experts_mxfp4(sh)
+    b1, b2 = synth.round_bf16(b1), synth.round_bf16(b2)
+    w1, w2 = ob.mxfp4_dequant(b1k, s1), ob.mxfp4_dequant(b2k, s2)
+    dx, dti = abi.DevBuf.from_numpy(synth.to_bf16_bits(x)), abi.DevBuf.from_numpy(ids)
+    dtv, dout = abi.DevBuf.from_numpy(tv), abi.DevBuf(T * H * 4)
+    got = []
+    for fp4 in (True, False):
+        m = abi.Moe(H, IM, E, max_tokens=T, swiglu_limit=sh.limit)
+        if fp4:
+            m.upload_layer_mxfp4(0, wr, br, b1k, s1, b1, b2k, s2, b2)
+        else:
+            m.upload_layer(0, wr, br, w1, b1, w2, b2)
+        dout.memset(0xFF)
+        m.experts(0, dx, None, dti, dtv, T, dout)
+        abi.sync()
+        got.append(dout.download((T, H), np.float32))
+        m.close()
+    assert np.array_equal(got[0], got[1])
+    some = np.unique(np.concatenate([np.nonzero((ids == e).any(1))[0][[0, -1]] for e in counts]))
+    want = np.zeros((len(some), H), np.float32)
+    for i, t in enumerate(some):
+        for k, e in enumerate(ids[t]):
+            want[i] += tv[t, k] * ob.expert_token(x[t], w1[e], b1[e], w2[e], b2[e], sh.limit, mode=ob.ROUND_ACT_BF16)
+    d = got[0][some] - want
+    assert np.abs(d).max() <= 2e-2 * max(1.0, float(np.abs(want).max()))
+    assert np.linalg.norm(d) <= 1e-3 * np.linalg.norm(want)
+
+
 def test_activation_past_4_gib():
     """256 experts with fixed slots of 64 rows and an intermediate size at which the
     last slot lies past 4 GiB of the activation: the first and the last expert (all
