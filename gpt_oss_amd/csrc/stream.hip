@@ -5,7 +5,7 @@
 // A wave owns a pair of column blocks (64 columns) of one expert and a slice of
 // the reduction, and shares nothing with other waves until its slice is done: the
 // weights and the token rows go straight into registers, D steps of 32 k ahead,
-// there is no LDS stage, no barrier and no DMA in the loop.  The KW waves of a
+// there is no barrier and no DMA in the loop.  The KW waves of a
 // workgroup take the KW slices of the same columns and add their sums through
 // LDS at the end, in a fixed order.  Compared with one workgroup per 256 columns
 // whose waves walk the whole reduction in lock step (gemm_tile), a wave's chain
@@ -74,29 +74,53 @@ __device__ __forceinline__ u32x4 load_weights(const char *g) {
 // 1.2), us per moe_experts call at 256 tokens 958, with this order 888, at 512 tokens
 // 1294 and 1130; MXFP4 301 and 279, 415 and 380; even routing within 1 %.
 __device__ __forceinline__ void share_of(int l, int wgs, int nb, int &col, int &blk) {
+  col = l;
+  blk = 0;
+  if (nb == 1) return;
   const int g = l / (kXcds * nb), r = l - g * kXcds * nb;
   const int width = min(kXcds, wgs - g * kXcds);
   blk = r / width;
   col = g * kXcds + r - blk * width;
 }
 
+// The L1 serves four adjacent lanes at a time, 64 contiguous bytes in one access.  In
+// operand order adjacent lanes hold different rows, and a load of 16 rows of 64 bytes
+// takes 52 accesses (counted) instead of 16.  So, where there are more than a few rows,
+//   * token rows are loaded with four adjacent lanes to a row and put in operand order
+//     through a kilobyte of LDS that only the wave touches (STAGED; tiles of more than
+//     16 rows: below, the weights' loads are the more).  8 experts, 64 tokens, us per
+//     moe_experts call without / with: bf16 90.7 / 87.9, MXFP4 43.5 / 42.6;
+//   * gate_up leaves the activation in "quads" for the down GEMM (stream_act_quads):
+//     per 16 rows and step of 32 k a kilobyte, in it the pieces of 8 k of four rows side
+//     by side.  The byte of piece `piece` of row r:
+__device__ __forceinline__ uint32_t act_place(int r, int piece) { return (r >> 2) * 256u + piece * 64u + (r & 3) * 16u; }
+
 // One wave's share of a tile: RG groups of 16 rows times NP pairs of column
 // blocks over the steps [ks0, ks0 + n) of 32 k.  a_rows: rows of lda 16-byte
-// pieces; row[g]: the row this lane feeds in group g.  np_valid: pairs inside
+// pieces; row[g]: the row this lane loads in group g.  np_valid: pairs inside
 // the matrix; one past it repeats the first, and its sums are not used.
-template <int NP, int RG, int D, bool FP4, bool SHARED>
+// stage: RG KB of LDS that only this wave touches (STAGED).  quads: a_rows is an
+// activation in quads.
+template <int NP, int RG, int D, bool FP4, bool SHARED, bool STAGED>
 __device__ __forceinline__ void stream_slice(const uint4 *__restrict__ a_rows, int lda, const int (&row)[RG],
                                              const uint4 *__restrict__ w, const uint16_t *__restrict__ ws, int KB,
-                                             int np_valid, int ks0, int n, int lane, f32x4 (&acc)[NP][4][RG]) {
+                                             int np_valid, int ks0, int n, int lane, f32x4 *stage, bool quads,
+                                             f32x4 (&acc)[NP][4][RG]) {
   constexpr int WR = FP4 ? 1 : 4;  // 16-byte registers of weights per pair and step
   const int r = lane & 15, q = lane >> 4;
   const int piece = (q >> 1) + 2 * (q & 1);
+  // STAGED: lane 4 r + c loads piece (c - r / 4) % 4 of row r and writes it at its own
+  // place; the reads of one piece of 16 rows then fall on 16 different slots of 256 bytes.
+  const int own = ((lane & 3) - q) & 3, staged_at = 4 * r + ((piece + (r >> 2)) & 3);
   // addresses: a base that is the same for the whole wave and moves with the step,
   // plus an offset per lane that does not.  The rows' is 64 bits wide: the fixed
   // slots of 256 experts reach 4 GiB from an intermediate size of 131 600 on.
   size_t a_off[RG];
 #pragma unroll
-  for (int g = 0; g < RG; g++) a_off[g] = ((size_t)row[g] * lda + piece) * 16;
+  for (int g = 0; g < RG; g++)
+    a_off[g] = quads ? (size_t)(row[g] >> 4) * lda * 256 + act_place(row[g] & 15, piece)
+                     : ((size_t)row[g] * lda + (STAGED ? own : piece)) * 16;
+  const uint32_t a_step = quads ? 1024 : 64;
   // bf16: fragment (block b, k block kb) is 64 pieces; this lane's piece of half hh is
   // kb = q & 1, (q >> 1) * 32 + 16 hh + r.  FP4: one chunk of 64 pieces per step.
   const uint32_t w_off = FP4 ? lane * 16u : ((q & 1) * 64 + (q >> 1) * 32 + r) * 16u;
@@ -121,7 +145,7 @@ __device__ __forceinline__ void stream_slice(const uint4 *__restrict__ a_rows, i
           wq[d][p][i] = load_weights<SHARED>(wb + (size_t)(i >> 1) * KB * 1024 + (i & 1) * 256 + w_off);
       }
     }
-    const char *ab = reinterpret_cast<const char *>(a_rows) + k * 64;
+    const char *ab = reinterpret_cast<const char *>(a_rows) + k * a_step;
 #pragma unroll
     for (int g = 0; g < RG; g++) xa[d][g] = *reinterpret_cast<const u32x4 *>(ab + a_off[g]);
   };
@@ -132,6 +156,19 @@ __device__ __forceinline__ void stream_slice(const uint4 *__restrict__ a_rows, i
 #pragma unroll
       for (int g = 0; g < RG; g++) acc[p][i][g] = f32x4{0.f, 0.f, 0.f, 0.f};
   auto compute = [&](int d) {
+    u32x4 xf[RG];
+    if constexpr (STAGED) {
+      // (the LDS instructions of a wave are carried out in their order)
+#pragma unroll
+      for (int g = 0; g < RG; g++) stage[g * 64 + lane] = __builtin_bit_cast(f32x4, xa[d][g]);
+      __builtin_amdgcn_wave_barrier();
+#pragma unroll
+      for (int g = 0; g < RG; g++) xf[g] = __builtin_bit_cast(u32x4, stage[g * 64 + staged_at]);
+      __builtin_amdgcn_wave_barrier();
+    } else {
+#pragma unroll
+      for (int g = 0; g < RG; g++) xf[g] = xa[d][g];
+    }
 #pragma unroll
     for (int p = 0; p < NP; p++) {
       bf16x8 wf[4];  // 16 weight rows each: [2 * block + half]
@@ -160,7 +197,7 @@ __device__ __forceinline__ void stream_slice(const uint4 *__restrict__ a_rows, i
       for (int i = 0; i < 4; i++)
 #pragma unroll
         for (int g = 0; g < RG; g++)
-          acc[p][i][g] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[i], __builtin_bit_cast(bf16x8, xa[d][g]),
+          acc[p][i][g] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[i], __builtin_bit_cast(bf16x8, xf[g]),
                                                                  acc[p][i][g], 0, 0, 0);
     }
   };
@@ -191,7 +228,7 @@ __device__ __forceinline__ void stream_slice(const uint4 *__restrict__ a_rows, i
 template <int RG, bool GATE_UP>
 __device__ __forceinline__ void stream_finish(const f32x4 *part, const float *__restrict__ bias_a,
                                               const float *__restrict__ bias_b, int P, int row0, int rows,
-                                              void *__restrict__ outp, int ldo, float limit, int w, int lane) {
+                                              void *__restrict__ outp, int ldo, bool quads, float limit, int w, int lane) {
   const int r = lane & 15, q = lane >> 4;
   auto sum = [&](int i, int g) {
     f32x4 v = part[(i * RG + g) * 64 + lane];
@@ -209,8 +246,11 @@ __device__ __forceinline__ void stream_finish(const f32x4 *part, const float *__
       const f32x4 ga = sum(i, g) + bg, up = sum(2 + i, g) + (bu + 1.0f);
       const uint32_t lo = pack_bf16(swiglu_shifted(ga[0], up[0], limit), swiglu_shifted(ga[1], up[1], limit));
       const uint32_t hi = pack_bf16(swiglu_shifted(ga[2], up[2], limit), swiglu_shifted(ga[3], up[3], limit));
-      if (row < rows)
-        *reinterpret_cast<uint2 *>(static_cast<uint16_t *>(outp) + (size_t)(row0 + row) * ldo + j) = make_uint2(lo, hi);
+      // quads: columns [32 P, 32 P + 32) are a step of the down GEMM, these half of its piece 2 i + q / 2
+      const int ar = row0 + row;
+      const size_t at = quads ? ((size_t)(ar >> 4) * (ldo / 32) + P) * 1024 + act_place(ar & 15, 2 * i + (q >> 1)) + 8 * (q & 1)
+                              : ((size_t)ar * ldo + j) * 2;
+      if (row < rows) *reinterpret_cast<uint2 *>(static_cast<char *>(outp) + at) = make_uint2(lo, hi);
     } else {
       const int j = kStreamCols * P + 16 * i + 4 * q;
       const f32x4 v = sum(i, g) + *reinterpret_cast<const f32x4 *>(bias_a + j);
@@ -219,18 +259,87 @@ __device__ __forceinline__ void stream_finish(const f32x4 *part, const float *__
   }
 }
 
+// The ti-th expert that has rows, in *e (-1: there are fewer).  mine: the expert of
+// the assignment of thread tid, -1: none.  some: LDS.
+__device__ __forceinline__ void find_expert(unsigned long long *some, int mine, int ti, int E, int tid, int &e,
+                                            int &first, int &nb) {
+  uint32_t *mask = reinterpret_cast<uint32_t *>(some);
+  if (tid < 2 * kStreamKw) mask[tid] = 0;
+  stream_barrier();
+  if (mine >= 0) atomicOr(&mask[mine >> 5], 1u << (mine & 31));
+  stream_barrier();
+  e = -1;
+  int left = ti;
+  for (int ww = 0; ww < (E + 31) / 32; ww++) {
+    uint32_t m = __builtin_amdgcn_readfirstlane(mask[ww]);
+    const int c = __builtin_popcount(m);
+    if (left < c) {
+      for (int i = 0; i < left; i++) m &= m - 1;
+      e = ww * 32 + __builtin_ctz(m);
+      break;
+    }
+    left -= c;
+  }
+  e = __builtin_amdgcn_readfirstlane(e);
+  first = ti;
+  nb = 1;
+}
+
+// The same where an expert with more than 32 rows counts as two tiles: the expert of
+// the ti-th tile, its first tile and its tiles.  The tiles follow each other without
+// gaps: with two places for every expert the workgroups without work stand between
+// the others, and the CUs they are dealt to stay idle (8 experts, 48 tokens, MXFP4:
+// 54.1 us per moe_experts call instead of 42.6).
+__device__ __forceinline__ void find_tile(int *hist, unsigned long long *some, unsigned long long *more, int mine,
+                                          int ti, int tid, int &e, int &first, int &nb) {
+  static_assert(kDirectSlotRows <= 2 * kStreamRows, "two tiles per expert, at most");
+  const int lane = tid & 63;
+  hist[tid] = 0;  // expert -> rows
+  stream_barrier();
+  if (mine >= 0) atomicAdd(&hist[mine], 1);
+  stream_barrier();
+  {
+    const int rows = hist[tid];
+    const unsigned long long s = __ballot(rows > 0), m = __ballot(rows > kStreamRows);
+    if (lane == 0) {
+      some[tid >> 6] = s;
+      more[tid >> 6] = m;
+    }
+  }
+  stream_barrier();
+  e = -1;
+  first = 0;
+  nb = 1;
+  const unsigned long long below = (1ull << lane) - 1ull;
+#pragma unroll
+  for (int ww = 0; ww < kStreamKw; ww++) {
+    const unsigned long long s = some[ww], m = more[ww];
+    const int tiles = __builtin_amdgcn_readfirstlane(__popcll(s) + __popcll(m));
+    if (e < 0 && ti < first + tiles) {
+      // lane: expert 64 ww + lane
+      const int at = first + __popcll(s & below) + __popcll(m & below);
+      const int have = (int)(s >> lane & 1) + (int)(m >> lane & 1);
+      const int l = __builtin_ctzll(__ballot(at <= ti && ti < at + have));
+      e = ww * 64 + l;
+      first = __builtin_amdgcn_readlane(at, l);
+      nb = __builtin_amdgcn_readlane(have, l);
+    } else if (e < 0) {
+      first += tiles;
+    }
+  }
+}
+
 // DIRECT: there is no plan.  The workgroup reads the batch's ids (one per
-// thread), lists the experts that have rows in a bit mask and finds the rows of
-// its own by ballot; workgroup i * wgs + c is column tile c of the i-th expert
-// with rows, so that the column tiles of the few experts a small batch reaches
-// spread over all XCDs.  Otherwise a tile is a row block of the plan's padded rows.
-// tiles: experts that have rows or row blocks, at most.
+// thread), finds the expert of its tile and by ballot that expert's rows; workgroup
+// i * wgs + c is column tile c of tile i, so that the column tiles of the few experts a
+// small batch reaches spread over all XCDs.  Otherwise a tile is a row block of the
+// plan's padded rows.  tiles: tiles of rows, at most.
 template <int NP, bool GATE_UP, bool FP4, bool DIRECT>
 __global__ __launch_bounds__(kStreamKw * 64, NP == 1 ? 4 : 3) void stream_gemm_kernel(
     const uint4 *__restrict__ a_rows, const uint4 *__restrict__ w_frag, const uint16_t *__restrict__ w_scale,
     const float *__restrict__ bias_a, const float *__restrict__ bias_b, const int *__restrict__ rowmap,
     const int *__restrict__ blk_expert, const int *__restrict__ totals, int *__restrict__ inv,
-    void *__restrict__ outp, int K, int N, float limit, int tiles, DirectIds ids) {
+    void *__restrict__ outp, int K, int N, float limit, int tiles, bool quads, DirectIds ids) {
   constexpr int RG = kStreamRows / 16;
   __shared__ f32x4 part[kStreamKw * 4 * RG * 64];
   __shared__ int rows_sh[DIRECT ? kDirectSlotRows : kStreamRows];  // row of the tile -> token
@@ -244,35 +353,30 @@ __global__ __launch_bounds__(kStreamKw * 64, NP == 1 ? 4 : 3) void stream_gemm_k
   const int ks0 = min(w * per, steps), n = min(per, steps - ks0);
   int e, row0, count, col;
   bool shared;  // more than one tile of rows reads these weights
+  int r0 = 0, r_step = kStreamRows;  // the workgroup's rows among those from row0: 32 from r0, and so on
   if constexpr (DIRECT) {
     static_assert(kStreamKw * 64 == kDirectTokens * kTopK, "one thread per assignment");
-    __shared__ uint32_t mask[8];
-    __shared__ int cnt[kStreamKw];
+    __shared__ int hist[256], cnt[kStreamKw];
+    __shared__ unsigned long long some[kStreamKw], more[kStreamKw];
     const int lane = tid & 63;
     const int mine = direct_expert_of(ids, tid);
     const int ti = blockIdx.x / wgs;
-    col = blockIdx.x - ti * wgs;
     // the first column tile's workgroups also write where each assignment's row is, for the combine
-    const bool writes_inv = GATE_UP && col == 0 && blockIdx.y == 0;
-    if (writes_inv && ti == 0 && mine < 0 && tid < ids.T * kTopK) inv[tid] = -1;
-    if (tid < 8) mask[tid] = 0;
-    stream_barrier();
-    if (mine >= 0) atomicOr(&mask[mine >> 5], 1u << (mine & 31));
-    stream_barrier();
-    e = -1;
-    int left = ti;
-    for (int ww = 0; ww < (ids.E + 31) / 32; ww++) {
-      uint32_t m = __builtin_amdgcn_readfirstlane(mask[ww]);
-      const int c = __builtin_popcount(m);
-      if (left < c) {
-        for (int i = 0; i < left; i++) m &= m - 1;
-        e = ww * 32 + __builtin_ctz(m);
-        break;
-      }
-      left -= c;
+    if (GATE_UP && blockIdx.x == 0 && mine < 0 && tid < ids.T * kTopK) inv[tid] = -1;
+    int first, nb;  // the expert's first tile, and how many workgroups share its rows
+    if (ids.T <= kStreamRows) {
+      // (an expert with more than 32 rows, which ids that repeat one can make, keeps its one workgroup)
+      find_expert(some, mine, ti, ids.E, tid, e, first, nb);
+    } else {
+      find_tile(hist, some, more, mine, ti, tid, e, first, nb);
     }
-    e = __builtin_amdgcn_readfirstlane(e);
-    if (e < 0) return;  // fewer experts than the grid provides for
+    if (e < 0) return;  // fewer tiles than the grid provides for
+    int blk;
+    share_of(blockIdx.x - first * wgs, wgs, nb, col, blk);
+    shared = nb > 1;
+    r0 = blk * kStreamRows;
+    r_step = nb * kStreamRows;
+    const bool writes_inv = GATE_UP && col == 0 && blk == 0;
     const unsigned long long bal = __ballot(mine == e);
     if (lane == 0) cnt[w] = __popcll(bal);
     stream_barrier();
@@ -286,7 +390,6 @@ __global__ __launch_bounds__(kStreamKw * 64, NP == 1 ? 4 : 3) void stream_gemm_k
     }
     count = __builtin_amdgcn_readfirstlane(min(count, kDirectSlotRows));
     row0 = e * kDirectSlotRows;
-    shared = count > kStreamRows;
     if (GATE_UP) {
       const int at = before + __popcll(bal & ((1ull << lane) - 1ull));
       if (mine == e && at < kDirectSlotRows) rows_sh[at] = tid / kTopK;
@@ -322,49 +425,51 @@ __global__ __launch_bounds__(kStreamKw * 64, NP == 1 ? 4 : 3) void stream_gemm_k
   const uint16_t *sp = FP4 ? w_scale + blk0 * KB * 8 : nullptr;
   const float *ba = bias_a + (size_t)e * N;
   const float *bb = GATE_UP ? bias_b + (size_t)e * N : nullptr;
-  // (gridDim.y: workgroups that share an expert's tiles of 32 rows)
-  for (int r0 = blockIdx.y * kStreamRows; r0 < count; r0 += gridDim.y * kStreamRows) {
+  for (bool again = false; r0 < count; r0 += r_step, again = true) {
     const int rows = min(count - r0, kStreamRows);
     // (a second round is rare: keeps what depends on the lane from being computed
     // ahead of the loop and held, or spilled, through it)
     int lane = tid & 63;
     asm volatile("" : "+v"(lane));
-    // lanes past the last row repeat it; their sums are not stored
-    int row[RG];
-#pragma unroll
-    for (int g = 0; g < RG; g++) {
-      const int rr = r0 + min(16 * g + (lane & 15), rows - 1);
-      row[g] = GATE_UP ? rows_sh[rr] : row0 + rr;
-    }
-    auto tile = [&](auto g_c, auto d_c, auto shared_c, const auto &tile_row) {
+    auto tile = [&](auto g_c, auto d_c, auto shared_c) {
       constexpr int G = decltype(g_c)::value;
+      constexpr bool kStaged = GATE_UP && G > 1;
+      // lanes past the last row repeat it; their sums are not stored
+      int row[G];
+#pragma unroll
+      for (int g = 0; g < G; g++) {
+        const int rr = r0 + min(16 * g + (kStaged ? lane >> 2 : lane & 15), rows - 1);
+        row[g] = GATE_UP ? rows_sh[rr] : row0 + rr;
+      }
+      if (again) stream_barrier();  // the sums before have been read
       f32x4 acc[NP][4][G];
-      stream_slice<NP, G, decltype(d_c)::value, FP4, decltype(shared_c)::value>(a_rows, K / 8, tile_row, wp, sp, KB,
-                                                                                np_valid, ks0, n, lane, acc);
+      stream_slice<NP, G, decltype(d_c)::value, FP4, decltype(shared_c)::value, kStaged>(
+          a_rows, K / 8, row, wp, sp, KB, np_valid, ks0, n, lane, part + w * (4 * RG * 64), !GATE_UP && quads, acc);
 #pragma unroll
       for (int p = 0; p < NP; p++) {
         if (p >= np_valid) break;
-        if (p || r0 != (int)blockIdx.y * kStreamRows) stream_barrier();  // the sums before have been read
+        if (p) stream_barrier();  // the sums before have been read
 #pragma unroll
         for (int i = 0; i < 4; i++)
 #pragma unroll
           for (int g = 0; g < G; g++) part[((w * 4 + i) * G + g) * 64 + lane] = acc[p][i][g];
         stream_barrier();
-        stream_finish<G, GATE_UP>(part, ba, bb, P + p, row0 + r0, rows, outp, N, limit, w, lane);
+        stream_finish<G, GATE_UP>(part, ba, bb, P + p, row0 + r0, rows, outp, N, quads, limit, w, lane);
       }
     };
-    // steps ahead: as many as the registers of three or four waves per SIMD hold
-    // (more gain nothing: at 64 tokens and MXFP4 weights the same time with 4, 6 and 8)
+    // steps ahead: as many as the registers of three or four waves per SIMD hold (more gain
+    // nothing: at 64 tokens and 32 experts, MXFP4, the same time with 4, 6 and 8; fewer cost:
+    // two pairs of columns and up to 32 rows, 16 experts and 64 tokens, 2 steps 56.7 us per
+    // moe_experts call, 3 steps 55.3)
     using One = std::integral_constant<int, 1>;
     using Two = std::integral_constant<int, 2>;
-    using DeepTwo = std::integral_constant<int, FP4 ? (NP == 1 ? 4 : 2) : 3>;
+    using DeepTwo = std::integral_constant<int, FP4 ? (NP == 1 ? 4 : 3) : 3>;
     if (shared) {
-      tile(Two{}, DeepTwo{}, std::true_type{}, row);
+      tile(Two{}, DeepTwo{}, std::true_type{});
     } else if (rows > 16) {
-      tile(Two{}, DeepTwo{}, std::false_type{}, row);
+      tile(Two{}, DeepTwo{}, std::false_type{});
     } else {
-      const int one[1] = {row[0]};
-      tile(One{}, std::integral_constant<int, FP4 ? (NP == 1 ? 6 : 4) : 4>{}, std::false_type{}, one);
+      tile(One{}, std::integral_constant<int, FP4 ? (NP == 1 ? 6 : 4) : 4>{}, std::false_type{});
     }
   }
 }
@@ -372,15 +477,12 @@ __global__ __launch_bounds__(kStreamKw * 64, NP == 1 ? 4 : 3) void stream_gemm_k
 template <int NP, bool GATE_UP>
 static hipError_t launch_stream_np(const uint4 *a, const uint4 *w, const uint16_t *w_scale, const float *ba,
                                    const float *bb, const DispatchBuffers &d, void *out, int K, int N, float limit,
-                                   int tiles, const DirectIds &ids, hipStream_t s) {
+                                   int tiles, bool quads, const DirectIds &ids, hipStream_t s) {
   const int pairs = (GATE_UP ? 2 * N : N) / kStreamCols;
-  // Without a plan an expert may have two tiles: one workgroup takes both, one
-  // after the other, unless most experts are likely to have two.
-  const bool two_tiles = ids.topk_i && ids.T > kStreamRows && ids.T * kTopK > kStreamRows / 2 * ids.E;
-  const dim3 grid(tiles * ((pairs + NP - 1) / NP), two_tiles ? 2 : 1);
+  const int grid = tiles * ((pairs + NP - 1) / NP);
 #define MOE_STREAM(FP4, DIRECT)                                                 \
   stream_gemm_kernel<NP, GATE_UP, FP4, DIRECT><<<grid, kStreamKw * 64, 0, s>>>( \
-      a, w, w_scale, ba, bb, d.rowmap, d.blk_expert, d.totals, d.inv, out, K, N, limit, tiles, ids)
+      a, w, w_scale, ba, bb, d.rowmap, d.blk_expert, d.totals, d.inv, out, K, N, limit, tiles, quads, ids)
   if constexpr (NP == 1) {
     if (!w_scale) {
       if (ids.topk_i) MOE_STREAM(false, true); else MOE_STREAM(false, false);
@@ -395,24 +497,24 @@ static hipError_t launch_stream_np(const uint4 *a, const uint4 *w, const uint16_
 template <bool GATE_UP>
 static hipError_t launch_stream(const void *a, const void *w, const uint16_t *w_scale, const float *ba,
                                 const float *bb, const DispatchBuffers &d, void *out, int K, int N, float limit,
-                                int tiles, const DirectIds &ids, hipStream_t s) {
+                                int tiles, bool quads, const DirectIds &ids, hipStream_t s) {
   const uint4 *af = static_cast<const uint4 *>(a), *wf = static_cast<const uint4 *>(w);
   const int pairs = (GATE_UP ? 2 * N : N) / kStreamCols;
   if (w_scale && tiles * pairs >= kStreamTwoPairs)
-    return launch_stream_np<2, GATE_UP>(af, wf, w_scale, ba, bb, d, out, K, N, limit, tiles, ids, s);
-  return launch_stream_np<1, GATE_UP>(af, wf, w_scale, ba, bb, d, out, K, N, limit, tiles, ids, s);
+    return launch_stream_np<2, GATE_UP>(af, wf, w_scale, ba, bb, d, out, K, N, limit, tiles, quads, ids, s);
+  return launch_stream_np<1, GATE_UP>(af, wf, w_scale, ba, bb, d, out, K, N, limit, tiles, quads, ids, s);
 }
 
 hipError_t launch_stream_gate_up(const uint16_t *x, const void *w1, const uint16_t *w1_scale, const float *b1g,
                                  const float *b1u, const DispatchBuffers &d, uint16_t *act, int H, int IM,
-                                 float limit, int tiles, const DirectIds &ids, hipStream_t s) {
-  return launch_stream<true>(x, w1, w1_scale, b1g, b1u, d, act, H, IM, limit, tiles, ids, s);
+                                 float limit, int tiles, bool quads, const DirectIds &ids, hipStream_t s) {
+  return launch_stream<true>(x, w1, w1_scale, b1g, b1u, d, act, H, IM, limit, tiles, quads, ids, s);
 }
 
 hipError_t launch_stream_down(const uint16_t *act, const void *w2, const uint16_t *w2_scale, const float *b2,
-                              const DispatchBuffers &d, float *y, int H, int IM, int tiles, const DirectIds &ids,
-                              hipStream_t s) {
-  return launch_stream<false>(act, w2, w2_scale, b2, nullptr, d, y, IM, H, 0.f, tiles, ids, s);
+                              const DispatchBuffers &d, float *y, int H, int IM, int tiles, bool quads,
+                              const DirectIds &ids, hipStream_t s) {
+  return launch_stream<false>(act, w2, w2_scale, b2, nullptr, d, y, IM, H, 0.f, tiles, quads, ids, s);
 }
 
 }  // namespace moe

@@ -118,6 +118,69 @@ def test_hot_experts_under_a_plan():
     assert np.linalg.norm(d) <= 1e-3 * np.linalg.norm(want)
 
 
+@pytest.mark.parametrize("E,H,IM", [(32, 1728, 896), (8, 4416, 2240)])
+def test_tiles_of_both_formats(E, H, IM):
+    """Sizes at which an MXFP4 wave takes two pairs of columns (the down GEMM's last one
+    has one) and batches in which experts have one tile of rows, two tiles, and none
+    between them; a repeated expert that has 64 rows in a batch of 16 tokens; inactive
+    rows.  Without a plan and with one, MXFP4 and bf16: the same bits; the oracle at
+    the first and last rows and around the 16th and 32nd."""
+    sh = synth.LayerShape("both", 64, H, IM, E)
+    x = synth.round_bf16(synth.make_activations(sh))
+    wr, br = (synth.round_bf16(a) for a in synth.make_router(sh))
+    b1k, s1, b1, b2k, s2, b2 = synth.make_experts_mxfp4(sh)
+    b1, b2 = synth.round_bf16(b1), synth.round_bf16(b2)
+    w1, w2 = ob.mxfp4_dequant(b1k, s1), ob.mxfp4_dequant(b2k, s2)
+    m4, m16 = (abi.Moe(H, IM, E, max_tokens=64, swiglu_limit=sh.limit) for _ in range(2))
+    m4.upload_layer_mxfp4(0, wr, br, b1k, s1, b1, b2k, s2, b2)
+    m16.upload_layer(0, wr, br, w1, b1, w2, b2)
+    rng = np.random.default_rng(E)
+    dx, dout = abi.DevBuf.from_numpy(synth.to_bf16_bits(x)), abi.DevBuf(64 * H * 4)
+
+    def skewed(T):  # expert 3 in every token, 5 in most, two of the rest
+        ids = np.stack([rng.permutation([e for e in range(E) if e not in (3, 5)])[:4] for _ in range(T)]).astype(np.int32)
+        ids[:, 1] = 3
+        ids[rng.permutation(T)[:T * 3 // 4], 2] = 5
+        return ids
+
+    one = np.full((16, 4), E - 1, np.int32)
+    for ids in [skewed(T) for T in (16, 17, 32, 33, 48, 64)] + [one]:
+        T = len(ids)
+        tv = rng.random((T, 4)).astype(np.float32)
+        pos = np.zeros(T, np.int32)
+        if T == 48:
+            pos[4::7] = -1
+        dti, dtv, dpos = (abi.DevBuf.from_numpy(a) for a in (ids, tv, pos))
+        first = None
+        for m in (m4, m16):
+            for distinct in ((False,) if ids is one else (True, False)):
+                m.set_distinct_ids(distinct)
+                dout.memset(0xFF)
+                m.experts(0, dx, dpos, dti, dtv, T, dout)
+                abi.sync()
+                got = dout.download((T, H), np.float32)
+                first = got if first is None else first
+                assert np.array_equal(got, first), (T, distinct)
+            m.dispatch(dti, dpos, T)  # with a plan also where moe_experts has none
+            m.expert_gemms(0, dx, T)
+            dout.memset(0xFF)
+            m.combine(dtv, dpos, T, dout)
+            abi.sync()
+            assert np.array_equal(dout.download((T, H), np.float32), first), T
+        assert np.all(first[pos < 0] == 0)
+        some = [t for t in sorted({0, 15, 16, 31, 32, T - 1}) if t < T and pos[t] >= 0]
+        want = np.zeros((len(some), H), np.float32)
+        for i, t in enumerate(some):
+            y = {e: ob.expert_token(x[t], w1[e], b1[e], w2[e], b2[e], sh.limit, mode=ob.ROUND_ACT_BF16) for e in set(ids[t])}
+            for k, e in enumerate(ids[t]):
+                want[i] += tv[t, k] * y[e]
+        d = first[some] - want
+        assert np.abs(d).max() <= 2e-2 * max(1.0, float(np.abs(want).max())), T
+        assert np.linalg.norm(d) <= 1e-3 * np.linalg.norm(want), T
+    m4.close()
+    m16.close()
+
+
 def test_activation_past_4_gib():
     """256 experts with fixed slots of 64 rows and an intermediate size at which the
     last slot lies past 4 GiB of the activation: the first and the last expert (all
