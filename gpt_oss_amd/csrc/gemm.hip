@@ -814,9 +814,10 @@ static_assert(CfgFull::RBT_MAX * kRowBlock == kTileRows && CfgHalf::RBT_MAX * kR
 // 143 / 135, 1024 (512 rows): 254 / 269.  MXFP4 (tiles of 128 rows), 32 experts,
 // 256 tokens 143 / 135, 512: 172 / 163, 1024 (128 rows): 242 / 245, 4096: 725 /
 // 750; 128 experts, 3072 (96 rows): 676 / 668.  MXFP4 in tiles of 256 rows gains
-// nothing (8 experts, 256 tokens 93 / 95).
+// nothing (8 experts, 256 tokens 93 / 95).  cached: kCachedWeightBytes.
 constexpr int kStreamRowsFull = 160, kStreamRowsHalf = 96;  // mean rows of an expert, at most
-static bool gemm_streams_weights(int T, int E, bool half) {
+static bool gemm_streams_weights(int T, int E, bool half, bool cached) {
+  if (cached) return false;
   return T * kTopK <= (half ? kStreamRowsHalf : kStreamRowsFull) * E;
 }
 
@@ -825,7 +826,7 @@ static bool gemm_streams_weights(int T, int E, bool half) {
 template <bool GATE_UP>
 static hipError_t launch_gemm(const void *a, const void *w, const uint16_t *w_scale, const float *ba,
                               const float *bb, const DispatchBuffers &d, void *out, int K, int N,
-                              float limit, int T, int E, int tile_rows, hipStream_t s) {
+                              float limit, int T, int E, int tile_rows, bool cached, hipStream_t s) {
   const int nb_total = (GATE_UP ? 2 * N : N) / kRowBlock;
   const int n_ct = (nb_total + kGemmTileNb - 1) / kGemmTileNb;
   const int grid = kXcds * xcd_tile_cap(gemm_tile_cap(T, E, tile_rows) * n_ct);
@@ -833,7 +834,7 @@ static hipError_t launch_gemm(const void *a, const void *w, const uint16_t *w_sc
   const uint4 *af = static_cast<const uint4 *>(a), *wf = static_cast<const uint4 *>(w);
   // the full-height kernels take a plan of either height, the others one of half height
   const bool half = w_scale && tile_rows == kHalfTileRows;
-  const bool stream = gemm_streams_weights(T, E, half);
+  const bool stream = gemm_streams_weights(T, E, half, cached);
 #define MOE_GEMM(C, FP4, STREAM)                                                                            \
   grouped_gemm_kernel<C, GATE_UP, FP4, STREAM><<<grid, C::THREADS, 0, s>>>(af, wf, w_scale, ba, bb, tiles,  \
                                                                            d.totals, d.rowmap, out, K, N, limit)
@@ -850,14 +851,14 @@ static hipError_t launch_gemm(const void *a, const void *w, const uint16_t *w_sc
 
 hipError_t launch_gate_up(const uint16_t *x, const void *w1, const uint16_t *w1_scale, const float *b1g,
                           const float *b1u, const DispatchBuffers &d, uint16_t *act, int H, int IM,
-                          float limit, int T, int E, int tile_rows, hipStream_t s) {
-  return launch_gemm<true>(x, w1, w1_scale, b1g, b1u, d, act, H, IM, limit, T, E, tile_rows, s);
+                          float limit, int T, int E, int tile_rows, bool cached, hipStream_t s) {
+  return launch_gemm<true>(x, w1, w1_scale, b1g, b1u, d, act, H, IM, limit, T, E, tile_rows, cached, s);
 }
 
 hipError_t launch_down(const uint16_t *act, const void *w2, const uint16_t *w2_scale, const float *b2,
                        const DispatchBuffers &d, float *y, int H, int IM, int T, int E, int tile_rows,
-                       hipStream_t s) {
-  return launch_gemm<false>(act, w2, w2_scale, b2, nullptr, d, y, IM, H, 0.f, T, E, tile_rows, s);
+                       bool cached, hipStream_t s) {
+  return launch_gemm<false>(act, w2, w2_scale, b2, nullptr, d, y, IM, H, 0.f, T, E, tile_rows, cached, s);
 }
 
 }  // namespace moe

@@ -55,6 +55,7 @@ struct moe_handle {
   int Hp = 0, IMp = 0;  // hidden / inter as the GEMMs see them: padded to multiples of 64
   std::vector<LayerWeights> layers;
   size_t layer_bytes = 0;
+  size_t expert_bytes = 0;  // expert matrices of all uploaded layers
   size_t ws_bytes = 0;
 
   // routing produced by the router stage (or copied from the caller)
@@ -162,6 +163,7 @@ int run_gemms(moe_handle *h, int layer, const uint16_t *x, int T, const DirectId
   const LayerWeights &lw = h->layers[layer];
   const void *w1 = lw.w1q ? static_cast<const void *>(lw.w1q) : lw.w1;
   const void *w2 = lw.w2q ? static_cast<const void *>(lw.w2q) : lw.w2;
+  const bool cached = h->expert_bytes <= kCachedWeightBytes;
   HIP_TRY(tm.mark(MOE_STAGE_GATE_UP));
   if (h->Hp != c.hidden) {  // a hidden size that is not a multiple of 64: rows widened with zeros
     HIP_TRY(launch_pad_rows(x, h->x_pad, T, c.hidden, h->Hp, s));
@@ -171,15 +173,15 @@ int run_gemms(moe_handle *h, int layer, const uint16_t *x, int T, const DirectId
     const int tiles = direct.topk_i ? stream_direct_tile_cap(T, c.experts) : stream_tile_cap(T, c.experts);
     const bool quads = stream_act_quads(T, c.experts);
     HIP_TRY(launch_stream_gate_up(x, w1, lw.w1s, lw.b1g, lw.b1u, h->disp, h->act, h->Hp, h->IMp, c.swiglu_limit,
-                                  tiles, quads, direct, s));
+                                  tiles, quads, cached, direct, s));
     HIP_TRY(tm.mark(MOE_STAGE_DOWN));
-    HIP_TRY(launch_stream_down(h->act, w2, lw.w2s, lw.b2, h->disp, h->y, h->Hp, h->IMp, tiles, quads, direct, s));
+    HIP_TRY(launch_stream_down(h->act, w2, lw.w2s, lw.b2, h->disp, h->y, h->Hp, h->IMp, tiles, quads, cached, direct, s));
     return MOE_OK;
   }
   HIP_TRY(launch_gate_up(x, w1, lw.w1s, lw.b1g, lw.b1u, h->disp, h->act, h->Hp, h->IMp, c.swiglu_limit, T,
-                         c.experts, h->plan_rows, s));
+                         c.experts, h->plan_rows, cached, s));
   HIP_TRY(tm.mark(MOE_STAGE_DOWN));
-  HIP_TRY(launch_down(h->act, w2, lw.w2s, lw.b2, h->disp, h->y, h->Hp, h->IMp, T, c.experts, h->plan_rows, s));
+  HIP_TRY(launch_down(h->act, w2, lw.w2s, lw.b2, h->disp, h->y, h->Hp, h->IMp, T, c.experts, h->plan_rows, cached, s));
   return MOE_OK;
 }
 
@@ -420,6 +422,9 @@ int upload_layer(moe_handle *h, int layer, const float *w_router, const float *b
   (void)hipFree(stage);
   (void)hipFree(stage_b);
   if (rc == MOE_OK) lw.uploaded = true;
+  h->expert_bytes = 0;
+  for (const LayerWeights &l : h->layers)
+    if (l.uploaded) h->expert_bytes += (size_t)E * (p1 + p2) * (l.w1q ? 17 : 64) / 32;  // 17/32 byte per MXFP4 weight
   return rc;
 }
 

@@ -214,23 +214,32 @@ inline bool half_tiles(int T, int E, int n_ct_gate_up) {
   const int row_tiles = T * kTopK / kHalfTileRows > E ? T * kTopK / kHalfTileRows : E;
   return (long long)row_tiles * n_ct_gate_up >= 2 * kCus;
 }
+// Expert matrices up to this many bytes, over all layers of a handle, are read through
+// the caches whatever the batch: they then stay in the 256 MB memory-side cache from
+// one call to the next, which loads past the caches do not use.  us per moe_experts
+// call through / past the caches, 2880 x 2880: MXFP4, 64 tokens, 20 experts (265 MB)
+// 56.2 / 61.3, 22 (291 MB) 61.5 / 62.2, 24 (318 MB) 74.1 / 70.1, 32 (423 MB) 90.1 /
+// 81.4; bf16, 96 tokens, 4 experts (199 MB) 63.2 / 93.8, 6 (299 MB) 101.7 / 98.2, 8
+// 107.1 / 96.2.  Eight layers of 8 experts, 1440 x 1440, called in turn, 24 tokens:
+// MXFP4 (211 MB together) 18.7 / 20.7, bf16 (796 MB) 32.3 / 31.2.
+constexpr size_t kCachedWeightBytes = (size_t)256 << 20;
 // The first GEMM reads the routed token rows of x itself, through rowmap; there is
 // no gathered copy.  act holds the activation in the order the second GEMM of the
 // same file reads it: MFMA fragments (gemm.hip) or rows (stream.hip).
 hipError_t launch_gate_up(const uint16_t *x, const void *w1, const uint16_t *w1_scale, const float *b1g,
                           const float *b1u, const DispatchBuffers &d, uint16_t *act, int H, int IM,
-                          float limit, int T, int E, int tile_rows, hipStream_t s);
+                          float limit, int T, int E, int tile_rows, bool cached, hipStream_t s);
 hipError_t launch_down(const uint16_t *act, const void *w2, const uint16_t *w2_scale, const float *b2,
                        const DispatchBuffers &d, float *y, int H, int IM, int T, int E, int tile_rows,
-                       hipStream_t s);
+                       bool cached, hipStream_t s);
 // tiles: row tiles, at most (stream_direct_tile_cap with ids.topk_i, otherwise stream_tile_cap).
-// quads: order of act (stream_act_quads), the same for both.
+// quads: order of act (stream_act_quads), the same for both.  cached: kCachedWeightBytes.
 hipError_t launch_stream_gate_up(const uint16_t *x, const void *w1, const uint16_t *w1_scale, const float *b1g,
                                  const float *b1u, const DispatchBuffers &d, uint16_t *act, int H, int IM,
-                                 float limit, int tiles, bool quads, const DirectIds &ids, hipStream_t s);
+                                 float limit, int tiles, bool quads, bool cached, const DirectIds &ids, hipStream_t s);
 hipError_t launch_stream_down(const uint16_t *act, const void *w2, const uint16_t *w2_scale, const float *b2,
                               const DispatchBuffers &d, float *y, int H, int IM, int tiles, bool quads,
-                              const DirectIds &ids, hipStream_t s);
+                              bool cached, const DirectIds &ids, hipStream_t s);
 // ldy: floats per row of y (the padded hidden size)
 hipError_t launch_combine(const float *y, int ldy, const int *inv, const float *topk_v, const int *pos, float *out,
                           int T, int H, int accumulate, hipStream_t s);

@@ -22,10 +22,11 @@
 // Bound by HBM with bf16 weights; with MXFP4 weights the conversions, the rows'
 // loads through L1 and the few microseconds in which a launch fills and drains
 // show as well.  Measured at 2880 x 2880 and 32 experts, against the kernels this
-// replaces (us, gate_up + down): 24 tokens bf16 157 + 81 (6.8 and 6.6 TB/s; were
-// 199 + 105), 64 tokens MXFP4 50 + 29 (were 60 + 40), 1 token MXFP4 10 + 6 (27 +
-// 16).  What that rests on, by leaving it out: the weights' non-temporal loads
-// (bf16 174 + 90 with plain ones), two pairs of columns per wave that share the
+// replaced (us, gate_up + down): 24 tokens bf16, 30 experts named, 147 + 79 (6.8 and
+// 6.3 TB/s of weights; were 194 + 102), 64 tokens MXFP4 52 + 28 (were 59 + 39), 1
+// token MXFP4 10 + 6 (were 23 + 14).  What that rests on, by leaving it out, measured on a
+// batch that named all 32 experts (157 + 81; MXFP4 50 + 29): the weights' non-temporal
+// loads (bf16 174 + 90 with plain ones), two pairs of columns per wave that share the
 // rows they load (MXFP4 55 + 32 with one; where that would leave fewer than
 // kStreamTwoPairs workgroups of work, one), no refill loads past the slice's end
 // (MXFP4 57 + 32 with them).  The number of slices (1, 2 or 4) matters to the
@@ -56,12 +57,13 @@ constexpr int kStreamTwoPairs = 1024;
 // Orders LDS traffic only: the loads in flight stay in flight.
 __device__ __forceinline__ void stream_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
-// 16 bytes of weights: past the caches where one workgroup reads them (measured,
-// see above), through them where several do at about the same time (share_of).
-template <bool SHARED>
+// 16 bytes of weights: past the caches where one workgroup reads them and they are not
+// there from the call before (measured, see above), through them where several do at
+// about the same time (share_of) or all weights fit (kCachedWeightBytes).
+template <bool CACHED>
 __device__ __forceinline__ u32x4 load_weights(const char *g) {
   const u32x4 *v = reinterpret_cast<const u32x4 *>(g);
-  if constexpr (SHARED) return *v;
+  if constexpr (CACHED) return *v;
   return __builtin_nontemporal_load(v);
 }
 
@@ -99,12 +101,12 @@ __device__ __forceinline__ uint32_t act_place(int r, int piece) { return (r >> 2
 // blocks over the steps [ks0, ks0 + n) of 32 k.  a_rows: rows of lda 16-byte
 // pieces; row[g]: the row this lane loads in group g.  np_valid: pairs inside
 // the matrix; one past it repeats the first, and its sums are not used.
-// stage: RG KB of LDS that only this wave touches (STAGED).  quads: a_rows is an
+// stage: RG KB of LDS that only this wave touches (STAGED).  QUADS: a_rows is an
 // activation in quads.
-template <int NP, int RG, int D, bool FP4, bool SHARED, bool STAGED>
+template <int NP, int RG, int D, bool FP4, bool CACHED, bool STAGED, bool QUADS>
 __device__ __forceinline__ void stream_slice(const uint4 *__restrict__ a_rows, int lda, const int (&row)[RG],
                                              const uint4 *__restrict__ w, const uint16_t *__restrict__ ws, int KB,
-                                             int np_valid, int ks0, int n, int lane, f32x4 *stage, bool quads,
+                                             int np_valid, int ks0, int n, int lane, f32x4 *stage,
                                              f32x4 (&acc)[NP][4][RG]) {
   constexpr int WR = FP4 ? 1 : 4;  // 16-byte registers of weights per pair and step
   const int r = lane & 15, q = lane >> 4;
@@ -118,9 +120,8 @@ __device__ __forceinline__ void stream_slice(const uint4 *__restrict__ a_rows, i
   size_t a_off[RG];
 #pragma unroll
   for (int g = 0; g < RG; g++)
-    a_off[g] = quads ? (size_t)(row[g] >> 4) * lda * 256 + act_place(row[g] & 15, piece)
+    a_off[g] = QUADS ? (size_t)(row[g] >> 4) * lda * 256 + act_place(row[g] & 15, piece)
                      : ((size_t)row[g] * lda + (STAGED ? own : piece)) * 16;
-  const uint32_t a_step = quads ? 1024 : 64;
   // bf16: fragment (block b, k block kb) is 64 pieces; this lane's piece of half hh is
   // kb = q & 1, (q >> 1) * 32 + 16 hh + r.  FP4: one chunk of 64 pieces per step.
   const uint32_t w_off = FP4 ? lane * 16u : ((q & 1) * 64 + (q >> 1) * 32 + r) * 16u;
@@ -136,16 +137,16 @@ __device__ __forceinline__ void stream_slice(const uint4 *__restrict__ a_rows, i
       if (FP4) {
         const char *wb = reinterpret_cast<const char *>(w) + pair * KB * 512 + k * 1024;
         const char *sb = reinterpret_cast<const char *>(ws) + pair * KB * 32 + k * 64;
-        wq[d][p][0] = load_weights<SHARED>(wb + w_off);
+        wq[d][p][0] = load_weights<CACHED>(wb + w_off);
         sc[d][p] = *reinterpret_cast<const uint32_t *>(sb + s_off);
       } else {
         const char *wb = reinterpret_cast<const char *>(w) + pair * KB * 2048 + k * 2048;
 #pragma unroll
         for (int i = 0; i < 4; i++)
-          wq[d][p][i] = load_weights<SHARED>(wb + (size_t)(i >> 1) * KB * 1024 + (i & 1) * 256 + w_off);
+          wq[d][p][i] = load_weights<CACHED>(wb + (size_t)(i >> 1) * KB * 1024 + (i & 1) * 256 + w_off);
       }
     }
-    const char *ab = reinterpret_cast<const char *>(a_rows) + k * a_step;
+    const char *ab = reinterpret_cast<const char *>(a_rows) + k * (QUADS ? 1024 : 64);
 #pragma unroll
     for (int g = 0; g < RG; g++) xa[d][g] = *reinterpret_cast<const u32x4 *>(ab + a_off[g]);
   };
@@ -225,10 +226,10 @@ __device__ __forceinline__ void stream_slice(const uint4 *__restrict__ a_rows, i
 // Sum of the slices in their order, bias, SwiGLU and the rows out.  A unit is 16
 // columns (gate_up: 16 of gate and the same 16 of up) of one group of rows, in
 // which a lane holds four consecutive columns of one row; the waves share them.
-template <int RG, bool GATE_UP>
+template <int RG, bool GATE_UP, bool QUADS>
 __device__ __forceinline__ void stream_finish(const f32x4 *part, const float *__restrict__ bias_a,
                                               const float *__restrict__ bias_b, int P, int row0, int rows,
-                                              void *__restrict__ outp, int ldo, bool quads, float limit, int w, int lane) {
+                                              void *__restrict__ outp, int ldo, float limit, int w, int lane) {
   const int r = lane & 15, q = lane >> 4;
   auto sum = [&](int i, int g) {
     f32x4 v = part[(i * RG + g) * 64 + lane];
@@ -246,9 +247,9 @@ __device__ __forceinline__ void stream_finish(const f32x4 *part, const float *__
       const f32x4 ga = sum(i, g) + bg, up = sum(2 + i, g) + (bu + 1.0f);
       const uint32_t lo = pack_bf16(swiglu_shifted(ga[0], up[0], limit), swiglu_shifted(ga[1], up[1], limit));
       const uint32_t hi = pack_bf16(swiglu_shifted(ga[2], up[2], limit), swiglu_shifted(ga[3], up[3], limit));
-      // quads: columns [32 P, 32 P + 32) are a step of the down GEMM, these half of its piece 2 i + q / 2
+      // QUADS: columns [32 P, 32 P + 32) are a step of the down GEMM, these half of its piece 2 i + q / 2
       const int ar = row0 + row;
-      const size_t at = quads ? ((size_t)(ar >> 4) * (ldo / 32) + P) * 1024 + act_place(ar & 15, 2 * i + (q >> 1)) + 8 * (q & 1)
+      const size_t at = QUADS ? ((size_t)(ar >> 4) * (ldo / 32) + P) * 1024 + act_place(ar & 15, 2 * i + (q >> 1)) + 8 * (q & 1)
                               : ((size_t)ar * ldo + j) * 2;
       if (row < rows) *reinterpret_cast<uint2 *>(static_cast<char *>(outp) + at) = make_uint2(lo, hi);
     } else {
@@ -259,8 +260,8 @@ __device__ __forceinline__ void stream_finish(const f32x4 *part, const float *__
   }
 }
 
-// The ti-th expert that has rows, in *e (-1: there are fewer).  mine: the expert of
-// the assignment of thread tid, -1: none.  some: LDS.
+// The ti-th expert that has rows (-1: there are fewer).  mine: the expert of the
+// assignment of thread tid, -1: none.  some: LDS.
 __device__ __forceinline__ void find_expert(unsigned long long *some, int mine, int ti, int E, int tid, int &e,
                                             int &first, int &nb) {
   uint32_t *mask = reinterpret_cast<uint32_t *>(some);
@@ -333,13 +334,14 @@ __device__ __forceinline__ void find_tile(int *hist, unsigned long long *some, u
 // thread), finds the expert of its tile and by ballot that expert's rows; workgroup
 // i * wgs + c is column tile c of tile i, so that the column tiles of the few experts a
 // small batch reaches spread over all XCDs.  Otherwise a tile is a row block of the
-// plan's padded rows.  tiles: tiles of rows, at most.
-template <int NP, bool GATE_UP, bool FP4, bool DIRECT>
+// plan's padded rows.  tiles: tiles of rows, at most.  cached: the weights are read
+// through the caches (also those that several tiles of rows read).
+template <int NP, bool GATE_UP, bool FP4, bool DIRECT, bool QUADS>
 __global__ __launch_bounds__(kStreamKw * 64, NP == 1 ? 4 : 3) void stream_gemm_kernel(
     const uint4 *__restrict__ a_rows, const uint4 *__restrict__ w_frag, const uint16_t *__restrict__ w_scale,
     const float *__restrict__ bias_a, const float *__restrict__ bias_b, const int *__restrict__ rowmap,
     const int *__restrict__ blk_expert, const int *__restrict__ totals, int *__restrict__ inv,
-    void *__restrict__ outp, int K, int N, float limit, int tiles, bool quads, DirectIds ids) {
+    void *__restrict__ outp, int K, int N, float limit, int tiles, bool cached, DirectIds ids) {
   constexpr int RG = kStreamRows / 16;
   __shared__ f32x4 part[kStreamKw * 4 * RG * 64];
   __shared__ int rows_sh[DIRECT ? kDirectSlotRows : kStreamRows];  // row of the tile -> token
@@ -352,8 +354,7 @@ __global__ __launch_bounds__(kStreamKw * 64, NP == 1 ? 4 : 3) void stream_gemm_k
   const int per = (steps + kStreamKw - 1) / kStreamKw;
   const int ks0 = min(w * per, steps), n = min(per, steps - ks0);
   int e, row0, count, col;
-  bool shared;  // more than one tile of rows reads these weights
-  int r0 = 0, r_step = kStreamRows;  // the workgroup's rows among those from row0: 32 from r0, and so on
+  int r0 = 0;  // the tile's first row among those from row0
   if constexpr (DIRECT) {
     static_assert(kStreamKw * 64 == kDirectTokens * kTopK, "one thread per assignment");
     __shared__ int hist[256], cnt[kStreamKw];
@@ -363,9 +364,8 @@ __global__ __launch_bounds__(kStreamKw * 64, NP == 1 ? 4 : 3) void stream_gemm_k
     const int ti = blockIdx.x / wgs;
     // the first column tile's workgroups also write where each assignment's row is, for the combine
     if (GATE_UP && blockIdx.x == 0 && mine < 0 && tid < ids.T * kTopK) inv[tid] = -1;
-    int first, nb;  // the expert's first tile, and how many workgroups share its rows
-    if (ids.T <= kStreamRows) {
-      // (an expert with more than 32 rows, which ids that repeat one can make, keeps its one workgroup)
+    int first, nb;  // the expert's first tile and its tiles
+    if (ids.T * kTopK <= kStreamRows) {  // no expert has a second tile, whatever the ids
       find_expert(some, mine, ti, ids.E, tid, e, first, nb);
     } else {
       find_tile(hist, some, more, mine, ti, tid, e, first, nb);
@@ -373,9 +373,8 @@ __global__ __launch_bounds__(kStreamKw * 64, NP == 1 ? 4 : 3) void stream_gemm_k
     if (e < 0) return;  // fewer tiles than the grid provides for
     int blk;
     share_of(blockIdx.x - first * wgs, wgs, nb, col, blk);
-    shared = nb > 1;
+    cached |= nb > 1;
     r0 = blk * kStreamRows;
-    r_step = nb * kStreamRows;
     const bool writes_inv = GATE_UP && col == 0 && blk == 0;
     const unsigned long long bal = __ballot(mine == e);
     if (lane == 0) cnt[w] = __popcll(bal);
@@ -410,7 +409,7 @@ __global__ __launch_bounds__(kStreamKw * 64, NP == 1 ? 4 : 3) void stream_gemm_k
     const int first = from + __builtin_ctzll(own), nb = __popcll(own);
     int blk;
     share_of(blockIdx.x - first * wgs, wgs, nb, col, blk);
-    shared = nb > 1;
+    cached |= nb > 1;
     row0 = (first + blk) * kRowBlock;
     if (first + blk != ti) a = lane < kStreamRows ? rowmap[row0 + lane] : -1;
     count = __popcll(__ballot(a >= 0));  // the valid rows of a block come first
@@ -425,64 +424,64 @@ __global__ __launch_bounds__(kStreamKw * 64, NP == 1 ? 4 : 3) void stream_gemm_k
   const uint16_t *sp = FP4 ? w_scale + blk0 * KB * 8 : nullptr;
   const float *ba = bias_a + (size_t)e * N;
   const float *bb = GATE_UP ? bias_b + (size_t)e * N : nullptr;
-  for (bool again = false; r0 < count; r0 += r_step, again = true) {
-    const int rows = min(count - r0, kStreamRows);
-    // (a second round is rare: keeps what depends on the lane from being computed
-    // ahead of the loop and held, or spilled, through it)
-    int lane = tid & 63;
-    asm volatile("" : "+v"(lane));
-    auto tile = [&](auto g_c, auto d_c, auto shared_c) {
-      constexpr int G = decltype(g_c)::value;
-      constexpr bool kStaged = GATE_UP && G > 1;
-      // lanes past the last row repeat it; their sums are not stored
-      int row[G];
+  const int lane = tid & 63, rows = min(count - r0, kStreamRows);
+  auto tile = [&](auto g_c, auto d_c, auto cached_c) {
+    constexpr int G = decltype(g_c)::value;
+    constexpr bool kStaged = GATE_UP && G > 1;
+    // lanes past the last row repeat it; their sums are not stored
+    int row[G];
 #pragma unroll
-      for (int g = 0; g < G; g++) {
-        const int rr = r0 + min(16 * g + (kStaged ? lane >> 2 : lane & 15), rows - 1);
-        row[g] = GATE_UP ? rows_sh[rr] : row0 + rr;
-      }
-      if (again) stream_barrier();  // the sums before have been read
-      f32x4 acc[NP][4][G];
-      stream_slice<NP, G, decltype(d_c)::value, FP4, decltype(shared_c)::value, kStaged>(
-          a_rows, K / 8, row, wp, sp, KB, np_valid, ks0, n, lane, part + w * (4 * RG * 64), !GATE_UP && quads, acc);
-#pragma unroll
-      for (int p = 0; p < NP; p++) {
-        if (p >= np_valid) break;
-        if (p) stream_barrier();  // the sums before have been read
-#pragma unroll
-        for (int i = 0; i < 4; i++)
-#pragma unroll
-          for (int g = 0; g < G; g++) part[((w * 4 + i) * G + g) * 64 + lane] = acc[p][i][g];
-        stream_barrier();
-        stream_finish<G, GATE_UP>(part, ba, bb, P + p, row0 + r0, rows, outp, N, quads, limit, w, lane);
-      }
-    };
-    // steps ahead: as many as the registers of three or four waves per SIMD hold (more gain
-    // nothing: at 64 tokens and 32 experts, MXFP4, the same time with 4, 6 and 8; fewer cost:
-    // two pairs of columns and up to 32 rows, 16 experts and 64 tokens, 2 steps 56.7 us per
-    // moe_experts call, 3 steps 55.3)
-    using One = std::integral_constant<int, 1>;
-    using Two = std::integral_constant<int, 2>;
-    using DeepTwo = std::integral_constant<int, FP4 ? (NP == 1 ? 4 : 3) : 3>;
-    if (shared) {
-      tile(Two{}, DeepTwo{}, std::true_type{});
-    } else if (rows > 16) {
-      tile(Two{}, DeepTwo{}, std::false_type{});
-    } else {
-      tile(One{}, std::integral_constant<int, FP4 ? (NP == 1 ? 6 : 4) : 4>{}, std::false_type{});
+    for (int g = 0; g < G; g++) {
+      const int rr = r0 + min(16 * g + (kStaged ? lane >> 2 : lane & 15), rows - 1);
+      row[g] = GATE_UP ? rows_sh[rr] : row0 + rr;
     }
+    f32x4 acc[NP][4][G];
+    stream_slice<NP, G, decltype(d_c)::value, FP4, decltype(cached_c)::value, kStaged, !GATE_UP && QUADS>(
+        a_rows, K / 8, row, wp, sp, KB, np_valid, ks0, n, lane, part + w * (4 * RG * 64), acc);
+#pragma unroll
+    for (int p = 0; p < NP; p++) {
+      if (p >= np_valid) break;
+      if (p) stream_barrier();  // the sums before have been read
+#pragma unroll
+      for (int i = 0; i < 4; i++)
+#pragma unroll
+        for (int g = 0; g < G; g++) part[((w * 4 + i) * G + g) * 64 + lane] = acc[p][i][g];
+      stream_barrier();
+      stream_finish<G, GATE_UP, QUADS>(part, ba, bb, P + p, row0 + r0, rows, outp, N, limit, w, lane);
+    }
+  };
+  // steps ahead: as many as the registers of three or four waves per SIMD hold (more gain
+  // nothing: at 64 tokens and 32 experts, MXFP4, the same time with 4, 6 and 8; fewer cost:
+  // two pairs of columns and up to 32 rows, 16 experts and 64 tokens, 2 steps 56.7 us per
+  // moe_experts call, 3 steps 55.3)
+  using One = std::integral_constant<int, 1>;
+  using Two = std::integral_constant<int, 2>;
+  using DeepTwo = std::integral_constant<int, FP4 ? (NP == 1 ? 4 : 3) : 3>;
+  using DeepOne = std::integral_constant<int, FP4 ? (NP == 1 ? 6 : 4) : 4>;
+  if (rows > 16) {
+    if (cached) tile(Two{}, DeepTwo{}, std::true_type{}); else tile(Two{}, DeepTwo{}, std::false_type{});
+  } else {
+    if (cached) tile(One{}, DeepOne{}, std::true_type{}); else tile(One{}, DeepOne{}, std::false_type{});
   }
 }
 
 template <int NP, bool GATE_UP>
 static hipError_t launch_stream_np(const uint4 *a, const uint4 *w, const uint16_t *w_scale, const float *ba,
                                    const float *bb, const DispatchBuffers &d, void *out, int K, int N, float limit,
-                                   int tiles, bool quads, const DirectIds &ids, hipStream_t s) {
+                                   int tiles, bool quads, bool cached, const DirectIds &ids, hipStream_t s) {
   const int pairs = (GATE_UP ? 2 * N : N) / kStreamCols;
   const int grid = tiles * ((pairs + NP - 1) / NP);
-#define MOE_STREAM(FP4, DIRECT)                                                 \
-  stream_gemm_kernel<NP, GATE_UP, FP4, DIRECT><<<grid, kStreamKw * 64, 0, s>>>( \
-      a, w, w_scale, ba, bb, d.rowmap, d.blk_expert, d.totals, d.inv, out, K, N, limit, tiles, quads, ids)
+#define MOE_STREAM(FP4, DIRECT)                                                              \
+  do {                                                                                       \
+    if (quads)                                                                               \
+      stream_gemm_kernel<NP, GATE_UP, FP4, DIRECT, true><<<grid, kStreamKw * 64, 0, s>>>(    \
+          a, w, w_scale, ba, bb, d.rowmap, d.blk_expert, d.totals, d.inv, out, K, N, limit,  \
+          tiles, cached, ids);                                                               \
+    else                                                                                     \
+      stream_gemm_kernel<NP, GATE_UP, FP4, DIRECT, false><<<grid, kStreamKw * 64, 0, s>>>(   \
+          a, w, w_scale, ba, bb, d.rowmap, d.blk_expert, d.totals, d.inv, out, K, N, limit,  \
+          tiles, cached, ids);                                                               \
+  } while (0)
   if constexpr (NP == 1) {
     if (!w_scale) {
       if (ids.topk_i) MOE_STREAM(false, true); else MOE_STREAM(false, false);
@@ -497,24 +496,24 @@ static hipError_t launch_stream_np(const uint4 *a, const uint4 *w, const uint16_
 template <bool GATE_UP>
 static hipError_t launch_stream(const void *a, const void *w, const uint16_t *w_scale, const float *ba,
                                 const float *bb, const DispatchBuffers &d, void *out, int K, int N, float limit,
-                                int tiles, bool quads, const DirectIds &ids, hipStream_t s) {
+                                int tiles, bool quads, bool cached, const DirectIds &ids, hipStream_t s) {
   const uint4 *af = static_cast<const uint4 *>(a), *wf = static_cast<const uint4 *>(w);
   const int pairs = (GATE_UP ? 2 * N : N) / kStreamCols;
   if (w_scale && tiles * pairs >= kStreamTwoPairs)
-    return launch_stream_np<2, GATE_UP>(af, wf, w_scale, ba, bb, d, out, K, N, limit, tiles, quads, ids, s);
-  return launch_stream_np<1, GATE_UP>(af, wf, w_scale, ba, bb, d, out, K, N, limit, tiles, quads, ids, s);
+    return launch_stream_np<2, GATE_UP>(af, wf, w_scale, ba, bb, d, out, K, N, limit, tiles, quads, cached, ids, s);
+  return launch_stream_np<1, GATE_UP>(af, wf, w_scale, ba, bb, d, out, K, N, limit, tiles, quads, cached, ids, s);
 }
 
 hipError_t launch_stream_gate_up(const uint16_t *x, const void *w1, const uint16_t *w1_scale, const float *b1g,
                                  const float *b1u, const DispatchBuffers &d, uint16_t *act, int H, int IM,
-                                 float limit, int tiles, bool quads, const DirectIds &ids, hipStream_t s) {
-  return launch_stream<true>(x, w1, w1_scale, b1g, b1u, d, act, H, IM, limit, tiles, quads, ids, s);
+                                 float limit, int tiles, bool quads, bool cached, const DirectIds &ids, hipStream_t s) {
+  return launch_stream<true>(x, w1, w1_scale, b1g, b1u, d, act, H, IM, limit, tiles, quads, cached, ids, s);
 }
 
 hipError_t launch_stream_down(const uint16_t *act, const void *w2, const uint16_t *w2_scale, const float *b2,
                               const DispatchBuffers &d, float *y, int H, int IM, int tiles, bool quads,
-                              const DirectIds &ids, hipStream_t s) {
-  return launch_stream<false>(act, w2, w2_scale, b2, nullptr, d, y, IM, H, 0.f, tiles, quads, ids, s);
+                              bool cached, const DirectIds &ids, hipStream_t s) {
+  return launch_stream<false>(act, w2, w2_scale, b2, nullptr, d, y, IM, H, 0.f, tiles, quads, cached, ids, s);
 }
 
 }  // namespace moe

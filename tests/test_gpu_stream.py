@@ -17,6 +17,12 @@ pytestmark = pytest.mark.gpu
 W = ("w_router", "b_router", "w_mlp1", "b_mlp1", "w_mlp2", "b_mlp2")
 
 
+def past_the_caches(sh, fp4):
+    """Layers of this shape from which a handle holds more than 256 MiB of expert
+    matrices, which are then read past the caches."""
+    return int((256 << 20) / (3 * sh.hidden * sh.inter * sh.experts * (17 / 32 if fp4 else 2))) + 1
+
+
 @pytest.mark.parametrize("rows", [1, 16, 17, 32, 33, 64, 65, 128, 150])
 @pytest.mark.parametrize("H,IM", [(64, 64), (192, 320), (704, 64)])
 def test_rows_of_an_expert(rows, H, IM):
@@ -79,8 +85,8 @@ def test_hot_experts_under_a_plan():
     """512 tokens over 128 experts, most rows at a few of them: experts of two and
     of many row blocks, one of them on both sides of the 64th block, single blocks
     between them; column tiles that are no multiple of the eight XCDs, an odd number
-    of pairs.  MXFP4 (two pairs per wave) and bf16 (one) bit for bit, and the oracle
-    at the first and last token of every expert."""
+    of pairs.  MXFP4 (two pairs per wave) and bf16 (one), through the caches and past
+    them, bit for bit, and the oracle at the first and last token of every expert."""
     E, H, IM, T = 128, 704, 384, 512
     counts = {**{e: 33 for e in range(30)}, 30: 290, 31: 1, 32: 16, 33: 17, 34: 32, 35: 64, 100: 138, 127: 500}
     assert sum(counts.values()) == 4 * T
@@ -96,18 +102,20 @@ def test_hot_experts_under_a_plan():
     dx, dti = abi.DevBuf.from_numpy(synth.to_bf16_bits(x)), abi.DevBuf.from_numpy(ids)
     dtv, dout = abi.DevBuf.from_numpy(tv), abi.DevBuf(T * H * 4)
     got = []
-    for fp4 in (True, False):
-        m = abi.Moe(H, IM, E, max_tokens=T, swiglu_limit=sh.limit)
-        if fp4:
-            m.upload_layer_mxfp4(0, wr, br, b1k, s1, b1, b2k, s2, b2)
-        else:
-            m.upload_layer(0, wr, br, w1, b1, w2, b2)
+    for fp4, layers in ((True, 1), (False, 1), (True, past_the_caches(sh, True)), (False, past_the_caches(sh, False))):
+        m = abi.Moe(H, IM, E, max_tokens=T, swiglu_limit=sh.limit, layers=layers)
+        for i in range(layers):
+            if fp4:
+                m.upload_layer_mxfp4(i, wr, br, b1k, s1, b1, b2k, s2, b2)
+            else:
+                m.upload_layer(i, wr, br, w1, b1, w2, b2)
         dout.memset(0xFF)
         m.experts(0, dx, None, dti, dtv, T, dout)
         abi.sync()
         got.append(dout.download((T, H), np.float32))
         m.close()
-    assert np.array_equal(got[0], got[1])
+    for other in got[1:]:
+        assert np.array_equal(got[0], other)
     some = np.unique(np.concatenate([np.nonzero((ids == e).any(1))[0][[0, -1]] for e in counts]))
     want = np.zeros((len(some), H), np.float32)
     for i, t in enumerate(some):
@@ -123,16 +131,22 @@ def test_tiles_of_both_formats(E, H, IM):
     """Sizes at which an MXFP4 wave takes two pairs of columns (the down GEMM's last one
     has one) and batches in which experts have one tile of rows, two tiles, and none
     between them; a repeated expert that has 64 rows in a batch of 16 tokens; inactive
-    rows.  Without a plan and with one, MXFP4 and bf16: the same bits; the oracle at
-    the first and last rows and around the 16th and 32nd."""
+    rows.  Without a plan and with one, MXFP4 (through the caches and past them) and
+    bf16: the same bits; the oracle at the first and last rows and around the 16th
+    and 32nd."""
     sh = synth.LayerShape("both", 64, H, IM, E)
     x = synth.round_bf16(synth.make_activations(sh))
     wr, br = (synth.round_bf16(a) for a in synth.make_router(sh))
     b1k, s1, b1, b2k, s2, b2 = synth.make_experts_mxfp4(sh)
     b1, b2 = synth.round_bf16(b1), synth.round_bf16(b2)
     w1, w2 = ob.mxfp4_dequant(b1k, s1), ob.mxfp4_dequant(b2k, s2)
+    many = past_the_caches(sh, True)
+    assert many > 1 and past_the_caches(sh, False) == 1
     m4, m16 = (abi.Moe(H, IM, E, max_tokens=64, swiglu_limit=sh.limit) for _ in range(2))
+    m4s = abi.Moe(H, IM, E, max_tokens=64, swiglu_limit=sh.limit, layers=many)
     m4.upload_layer_mxfp4(0, wr, br, b1k, s1, b1, b2k, s2, b2)
+    for i in range(many):
+        m4s.upload_layer_mxfp4(i, wr, br, b1k, s1, b1, b2k, s2, b2)
     m16.upload_layer(0, wr, br, w1, b1, w2, b2)
     rng = np.random.default_rng(E)
     dx, dout = abi.DevBuf.from_numpy(synth.to_bf16_bits(x)), abi.DevBuf(64 * H * 4)
@@ -152,7 +166,7 @@ def test_tiles_of_both_formats(E, H, IM):
             pos[4::7] = -1
         dti, dtv, dpos = (abi.DevBuf.from_numpy(a) for a in (ids, tv, pos))
         first = None
-        for m in (m4, m16):
+        for m in (m4, m4s, m16):
             for distinct in ((False,) if ids is one else (True, False)):
                 m.set_distinct_ids(distinct)
                 dout.memset(0xFF)
@@ -177,8 +191,8 @@ def test_tiles_of_both_formats(E, H, IM):
         d = first[some] - want
         assert np.abs(d).max() <= 2e-2 * max(1.0, float(np.abs(want).max())), T
         assert np.linalg.norm(d) <= 1e-3 * np.linalg.norm(want), T
-    m4.close()
-    m16.close()
+    for m in (m4, m4s, m16):
+        m.close()
 
 
 def test_activation_past_4_gib():

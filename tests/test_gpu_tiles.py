@@ -1,6 +1,7 @@
 """The grouped GEMMs at the edges of their row tiles: 256 rows, and 128 rows where
 the weights are MXFP4 and there are tiles enough; weights read through the caches
-and past them (few and many rows per expert); full, half and quarter column tiles.
+and past them (few rows per expert and more than 256 MiB of matrices in the handle);
+full, half and quarter column tiles.
 
 Bars as in test_gpu_parity.py: max-abs 2e-2 and rel-L2 1e-3 of the oracle on the
 same inputs; the two weight formats, whose tiles differ, bit for bit."""
@@ -35,12 +36,14 @@ def test_row_tiles(rows, H, IM):
     dx, dti = abi.DevBuf.from_numpy(synth.to_bf16_bits(x)), abi.DevBuf.from_numpy(ids)
     dtv, dout = abi.DevBuf.from_numpy(tv), abi.DevBuf(T * H * 4)
     got = []
-    for fp4 in (True, False):
-        m = abi.Moe(H, IM, E, max_tokens=T, swiglu_limit=sh.limit)
-        if fp4:
-            m.upload_layer_mxfp4(0, wr, br, b1k, s1, b1, b2k, s2, b2)
-        else:
-            m.upload_layer(0, wr, br, w1, b1, w2, b2)
+    many = int((256 << 20) / (3 * H * IM * E * 17 / 32)) + 1  # MXFP4 layers from which the weights are read past the caches
+    for fp4, layers in ((True, 1), (False, 1), (True, many), (False, many * 17 // 64 + 1)):
+        m = abi.Moe(H, IM, E, max_tokens=T, swiglu_limit=sh.limit, layers=layers)
+        for i in range(layers):
+            if fp4:
+                m.upload_layer_mxfp4(i, wr, br, b1k, s1, b1, b2k, s2, b2)
+            else:
+                m.upload_layer(i, wr, br, w1, b1, w2, b2)
         dout.memset(0xFF)
         m.experts(0, dx, None, dti, dtv, T, dout)
         abi.sync()
