@@ -31,6 +31,9 @@ import numpy as np
 ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
+# copies of kDirectTokens and kStreamMeanRows in moe_internal.h (stream_batch), to name the
+# kernel of a batch; tests/test_abi_host.py compares them
+STREAM_TOKENS, STREAM_MEAN_ROWS = 64, 16
 PEAK_BF16_TFLOPS = 2500.0  # MI355X dense bf16 MFMA
 PEAK_HBM_GBS = 8000.0
 SETTLE_STEPS = 200  # untimed calls in front of the warm-up steps, see run_leg
@@ -270,9 +273,8 @@ def main():
     combine_bytes = A * H * 2 + T * H * 4
     mfma_tflops = flops_gate_up / t_gate_up / 1e12
     hbm_gbs = bytes_gate_up / t_gate_up / 1e9
-    # few rows per expert: the kernels of stream.hip (stream_batch in moe_internal.h)
-    kernel = "%s<gate_up%s>" % ("stream_gemm_kernel" if T <= 64 or T * K <= 16 * E else "grouped_gemm_kernel",
-                                ", MXFP4" if mxfp4 else "")
+    kernel = "%s<gate_up%s>" % ("stream_gemm_kernel" if T <= STREAM_TOKENS or T * K <= STREAM_MEAN_ROWS * E
+                                else "grouped_gemm_kernel", ", MXFP4" if mxfp4 else "")
     if BOUND[shape.name] == "mfma":
         roofline = {"bound": "mfma", "kernel": kernel, "achieved": mfma_tflops, "peak": PEAK_BF16_TFLOPS,
                     "unit": "TFLOP/s", "frac": mfma_tflops / PEAK_BF16_TFLOPS}

@@ -328,7 +328,13 @@ __device__ __forceinline__ void gemm_tile(const uint4 *__restrict__ a_frag,  // 
   // "Step s of the row operand has landed" as a bound on the vector-memory
   // counter.  The loads are issued in the order A(0) B(0) A(1) B(1) ... and
   // complete in that order, so all but the newest n outstanding means step s has
-  // landed with n = everything issued behind it.
+  // landed with n = everything issued behind it.  Open question: in a configuration
+  // since removed (ring of 7, two or three workgroups per CU, DMA of 32 bytes of
+  // scattered token rows, this mixed count of DMAs and register loads) whole tiles of
+  // wrong token rows were once seen, different from run to run, and the cause was never
+  // found.  The half-height kernels share three of those properties (two workgroups per
+  // CU, scattered DMA in gate_up, the mixed count); the tests that repeat calls at 512,
+  // 4096, 6144 and 7168 tokens are there to catch it.
   constexpr int WAIT_DMA_FILL = LPS * (R - 2) + LA;  // A(0), A(0..R-1) issued
   constexpr int WAIT_DMA_STEP = LPS * (R - 2);       // A(ks+1) at step ks
 
@@ -474,7 +480,7 @@ constexpr int kLineStages = 4;
 // Loads are issued in the order  B(0) B(1) B(2) A2(0) A2(1) A2(2) A2(3) | step 0:
 // B(3) | step 1: B(4) A2(4) | step 2: B(5) | step 3: B(6) A2(5) | ...  (R2 = RB =
 // 4).  The counted wait in the middle of a step leaves the newest 2 LB + LA2
-// loads in flight (see gemm_tile for the assumption): that covers A2(d+1), which
+// loads in flight (see gemm_tile for the assumption and the open question): that covers A2(d+1), which
 // an odd step 2d+1 needs, and B(ks+1), which every step's successor needs.  Even
 // steps need no barrier: they read a double stage that landed before the
 // previous odd step's barrier and refill nothing.

@@ -74,7 +74,7 @@ struct moe_handle {
   // moe_get_dispatch that asks for the plan afterwards.  topk_i == nullptr: none.
   DirectIds unplanned{nullptr, nullptr, 0, 0};
   // expert pipeline
-  uint16_t *act = nullptr;  // SwiGLU output, bf16: fragments or rows (stream_batch)
+  uint16_t *act = nullptr;  // SwiGLU output, bf16: fragments (gemm.hip), quads or rows (stream.hip)
   float *y = nullptr;       // down output [a_pad_cap, Hp]
   uint16_t *t_norm = nullptr;  // normalised rows of moe_block_forward [max_tokens, H], allocated on first use
   uint16_t *x_pad = nullptr;   // the batch's rows widened to Hp columns [max_tokens, Hp]; only where Hp != H
@@ -205,8 +205,8 @@ int run_experts(moe_handle *h, int layer, const uint16_t *x, const int *pos, con
                 StageTimer &tm, uint16_t *resid = nullptr) {
   const moe_config &c = h->cfg;
   HIP_TRY(tm.mark(MOE_STAGE_DISPATCH));
-  // a batch of at most 64 tokens needs no dispatch pass: the GEMMs and the
-  // combine find their rows from the ids themselves
+  // a batch of at most 64 tokens needs no dispatch pass: the GEMMs find their rows
+  // from the ids themselves, and the first of them leaves inv for the combine
   const bool direct_plan = direct_plan_fits(T, max_rows, c.experts, h->a_pad_cap);
   const DirectIds direct{direct_plan ? topk_i : nullptr, pos, T, c.experts};
   int rc = direct_plan ? MOE_OK : run_dispatch(h, topk_i, pos, T, h->layers[layer].w1q != nullptr, s);

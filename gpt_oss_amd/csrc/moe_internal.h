@@ -225,7 +225,7 @@ inline bool half_tiles(int T, int E, int n_ct_gate_up) {
 constexpr size_t kCachedWeightBytes = (size_t)256 << 20;
 // The first GEMM reads the routed token rows of x itself, through rowmap; there is
 // no gathered copy.  act holds the activation in the order the second GEMM of the
-// same file reads it: MFMA fragments (gemm.hip) or rows (stream.hip).
+// same file reads it: MFMA fragments (gemm.hip), quads or rows (stream.hip).
 hipError_t launch_gate_up(const uint16_t *x, const void *w1, const uint16_t *w1_scale, const float *b1g,
                           const float *b1u, const DispatchBuffers &d, uint16_t *act, int H, int IM,
                           float limit, int T, int E, int tile_rows, bool cached, hipStream_t s);

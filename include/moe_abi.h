@@ -14,6 +14,14 @@
  * common/defines.h:94-102); the host shim turns a non-zero status into that
  * behaviour.
  *
+ * Bits: a call gives the same bits every time, whichever of the entry points
+ * below makes it and whether the expert matrices were uploaded as MXFP4 or as
+ * their fp32 expansion.  A row's sums are the same in batches of any size on one
+ * side of the line to which the weights-bound kernels are used (64 tokens, or 16
+ * rows per expert on average, n_tokens * K <= 16 * experts); across it they are
+ * taken in another order and differ by fp32 rounding, which can move a rounding
+ * of the bf16 activation.  n_tokens counts the inactive rows.
+ *
  * A handle belongs to one device and one host thread at a time.  Calls on one
  * handle are asynchronous on the given stream and never synchronise with the
  * host; all routing counts and offsets stay on the device.

@@ -106,3 +106,15 @@ def test_bench_refuses_more_than_one_gpu_and_needs_a_gpu():
         r = subprocess.run([sys.executable, os.path.join(root, "bench.py"), "--steps", "1", "--warmup", "0"],
                            capture_output=True, text=True, timeout=120)
         assert r.returncode == 3 and "no CPU fallback" in r.stderr and r.stdout.strip() == ""
+
+
+def test_bench_names_kernels_by_the_librarys_rule():
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+    def value(path, name):
+        text = open(os.path.join(root, path)).read()
+        return int(re.search(name, text)[1])
+
+    header = "gpt_oss_amd/csrc/moe_internal.h"
+    assert value("bench.py", r"STREAM_TOKENS, STREAM_MEAN_ROWS = (\d+)") == value(header, r"kDirectTokens = (\d+)")
+    assert value("bench.py", r"STREAM_TOKENS, STREAM_MEAN_ROWS = \d+, (\d+)") == value(header, r"kStreamMeanRows = (\d+)")

@@ -314,18 +314,17 @@ def test_all_tokens_on_four_experts_and_tiny_batches(c2):
         check_outputs(R, L2, x, None, np.arange(T))
 
 
-@pytest.mark.parametrize("T", [5, 6, 16, 17, 64, 65, 128, 129, 256, 257])
+@pytest.mark.parametrize("T", [5, 6, 8, 9, 16, 17, 47, 48, 64, 65, 128, 129, 256, 257])
 def test_batch_size_boundaries(c2, T):
-    """Either side of the sizes at which the library changes its plan: up to 64
-    rows per expert the GEMMs run in their small-batch configuration and gate_up
-    reads the token rows itself, up to 128 tokens several workgroups share a
-    router tile, up to 256 tokens the dispatch is one workgroup, up to 5 tokens
-    (at 32 experts and 12 column tiles) the down GEMM's reduction is split over
-    two workgroups per tile.
+    """Either side of the sizes at which the library changes its plan at 32 experts:
+    up to 8 tokens no expert can have a second tile of rows, from 48 on the
+    activation is left in quads for the down GEMM, up to 64 there is no dispatch
+    pass, up to 128 (16 rows per expert) the GEMMs stream the weights, up to 256 the
+    dispatch is one workgroup.
     moe_forward bounds the rows per expert by T, moe_experts (whose ids come from
     the caller) by 4 T unless the caller promises distinct ids, so between 17
-    and 64 tokens the two entry points take different configurations for the
-    same work: same bits required, with the promise and without."""
+    and 64 tokens the two entry points run with and without a plan for the same
+    work: same bits required, with the promise and without."""
     sh, L, m = c2
     x = L["x"][500:500 + T]
     R = abi.run_layer(m, 0, x, None)
@@ -340,8 +339,6 @@ def test_batch_size_boundaries(c2, T):
             m.experts(0, dx, None, dti, dtv, T, dout, accumulate=False)
             abi.sync()
             got = dout.download((T, sh.hidden), np.float32)
-            # (at this shape only batches of up to 5 tokens split the reduction, and those run the
-            # small-batch configuration with or without the promise)
             assert np.array_equal(got, R["out"]), f"distinct={distinct}"
     finally:
         m.set_distinct_ids(False)
@@ -407,8 +404,8 @@ def test_c5_mxfp4_ingest():
 @pytest.mark.parametrize("T", [5, 33, 64])
 def test_small_batches_without_dispatch_pass(c2, T):
     """Up to 64 tokens moe_forward launches no dispatch kernels: the workgroups
-    of the GEMMs and of the combine find their rows from the expert ids
-    themselves, in fixed slots of 64 rows per expert.  The staged entry points
+    of the GEMMs find their rows from the expert ids themselves, in fixed slots of
+    64 rows per expert, and the first GEMM leaves the rows' places for the combine.  The staged entry points
     (moe_dispatch, moe_expert_gemms, moe_combine) keep the planned path, so the
     same batch through both must give the same bits -- with inactive rows too,
     which come out as zeros, are left alone in accumulate mode, and whose
@@ -418,7 +415,7 @@ def test_small_batches_without_dispatch_pass(c2, T):
     x = L["x"][900:900 + T]
     pos = np.where(np.random.default_rng(T).random(T) < 0.3, -1, 3).astype(np.int32)
     pos[0] = 3
-    m.set_distinct_ids(True)  # the staged calls then run the small-batch configuration up to 64 tokens, too
+    m.set_distinct_ids(True)
     for p in (None, pos):
         R = abi.run_layer(m, 0, x, p)
         check_routing(R, L, x, p, sh.experts)
@@ -449,12 +446,10 @@ def test_small_batches_without_dispatch_pass(c2, T):
 
 
 def test_small_batches_repeat_bit_for_bit():
-    """Batches of at most 64 tokens take paths of their own (one-workgroup
-    dispatch, gate_up reading the token rows through the row map, GEMMs built
-    for several workgroups per CU).  Twelve calls in a row must give the same
-    bits, with MXFP4 and with bf16 weights, and the two must agree (the MXFP4
-    values are exact in bf16): a row operand read before it had landed showed
-    as whole token rows that differed from run to run."""
+    """Batches of at most 64 tokens take a path of their own (no dispatch pass, the
+    kernels of stream.hip).  Twelve calls in a row must give the same bits, with
+    MXFP4 and with bf16 weights, and the two must agree (the MXFP4 values are exact
+    in bf16)."""
     sh = synth.CONFIGS["c5"]
     wr, br = (synth.round_bf16(a) for a in synth.make_router(sh))
     b1k, s1, b1, b2k, s2, b2 = synth.make_experts_mxfp4(sh)
@@ -486,7 +481,7 @@ def test_ffn_block_in_place(c2, T):
     bf16 stream.  The norm is checked through the routing it leads to (bit-exact
     offsets and permutation need bit-exact normalised rows up to near-ties), the
     result against the oracle's composition of the same steps.  48 tokens take
-    the small-batch path, whose gate_up reads the normalised rows directly."""
+    the path without a dispatch pass."""
     sh, L, m = c2
     rng = np.random.default_rng(21)
     x = synth.round_bf16((rng.standard_normal((T, sh.hidden)) * rng.uniform(0.5, 4.0, (T, 1))).astype(np.float32))
@@ -529,7 +524,7 @@ def test_forward_replays_from_a_hip_graph(c2, T):
     """moe_forward allocates nothing, never synchronises and clears its buffers
     with kernels, so a caller may capture it.  Three replays, with eager calls
     and synchronisations of the program's own in between, must each reproduce the
-    eager result bit for bit.  48 tokens take the small-batch kernels."""
+    eager result bit for bit.  48 tokens take the kernels of stream.hip."""
     import ctypes as C
     hip = C.CDLL("libamdhip64.so")
 

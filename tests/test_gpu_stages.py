@@ -44,10 +44,7 @@ def test_stage_entry_points_compose(T):
     sh = synth.LayerShape("s", T, 320, 128, 13)
     L = bf16_layer(sh, seed=5)
     m = make_moe(sh, L, T)
-    # the router's ids are four different experts per token: with that said, the staged
-    # calls run the configuration moe_forward runs (same bits also at 40 tokens, where
-    # with so few column tiles the small-batch down GEMM sums its reduction in two parts)
-    m.set_distinct_ids(True)
+    m.set_distinct_ids(True)  # the router's ids are four different experts per token
     pos = np.zeros(T, np.int32)
     pos[3::7] = -1
     base = abi.run_layer(m, 0, L["x"], pos)
@@ -82,9 +79,9 @@ def test_stage_entry_points_compose(T):
 def test_caller_routing_with_distinct_ids(T):
     """moe_set_distinct_ids: with the promise that a token's ids are four
     different experts, moe_experts bounds the rows per expert by T as
-    moe_forward does and takes the small-batch kernels up to 64 tokens: the bits
-    of moe_forward.  Without it the bound is 4 T and the full-height kernels
-    run: the same bits, too."""
+    moe_forward does and needs no dispatch pass up to 64 tokens: the bits of
+    moe_forward.  Without it the bound is 4 T and the same kernels run on a plan:
+    the same bits, too."""
     sh = synth.LayerShape("d", T, 2880, 320, 32)
     L = bf16_layer(sh, seed=8)
     m = make_moe(sh, L, 128)
@@ -96,8 +93,6 @@ def test_caller_routing_with_distinct_ids(T):
     dti, dtv = abi.DevBuf.from_numpy(base["topk_i"]), abi.DevBuf.from_numpy(base["topk_v"])
     dout = abi.DevBuf(T * sh.hidden * 4)
     def same(got, distinct):
-        # at this shape only batches of up to 5 tokens split the down GEMM's reduction, and
-        # those run the small-batch configuration with or without the promise
         assert np.array_equal(got, base["out"]), f"distinct={distinct}"
 
     for distinct in (False, True, False):
@@ -123,7 +118,7 @@ def test_reference_7m_model_shape():
     """The reference's smallest model (export_model_bin/gpt-oss-7m/config.json:
     hidden 32, intermediate 64, 32 experts): sizes that are multiples of 32 but
     not of 64 are padded inside the library.  Whole layer, FFN block and MXFP4
-    upload against the oracle; batches on both sides of the small-batch limit."""
+    upload against the oracle; batches on both sides of 64 tokens."""
     for H, IM, E in ((32, 64, 32), (96, 96, 32), (32, 32, 8)):
         for T in (1, 50, 64, 300, 1100):
             sh = synth.LayerShape("7m", T, H, IM, E)
@@ -335,7 +330,9 @@ def test_large_batches_repeat_bit_for_bit():
     tile height and both narrow last column tiles (row split 2 in gate_up, 4 in
     down); twelve calls in a row must give the same bits, with bf16 and with
     MXFP4 weights, so must 7168 tokens under Zipf routing (one expert with 28
-    row tiles), and so must the FFN block at 48 tokens."""
+    row tiles), 512 tokens with either format, whose weights go past the caches
+    (MXFP4: tiles of 128 rows, two workgroups per CU), and so must the FFN block
+    at 48 tokens."""
     sh = synth.CONFIGS["c2"]
     T = sh.tokens
     wr, br = (synth.round_bf16(a) for a in synth.make_router(sh))
@@ -360,6 +357,14 @@ def test_large_batches_repeat_bit_for_bit():
                 first = got
                 assert np.isfinite(got).all()
             assert np.array_equal(got, first), f"call {i}: a repeated call gave other bits"
+    few = 512
+    for m in (m16, m4):
+        for i in range(12):
+            dout.memset(0xFF)
+            m.forward(0, dx, None, few, dout)
+            abi.sync()
+            got = dout.download((few, sh.hidden), np.float32)
+            assert np.array_equal(got, first[:few]), f"{few} tokens, call {i}: other bits"
     # 7168 tokens with Zipf routing: up to 28 row tiles on one expert, the deepest XCD ranges
     z = synth.CONFIGS["c3b"]
     T3 = z.tokens
@@ -402,8 +407,8 @@ def test_large_batches_repeat_bit_for_bit():
 @pytest.mark.parametrize("T", [3, 100])
 def test_padded_shape_and_split_reduction_replay_from_a_hip_graph(T):
     """moe_forward at a hidden size that needs padding (one more kernel per call,
-    the row widening) and, at 3 tokens, with the down GEMM's reduction split over
-    two workgroups per tile: captured once, replayed three times with eager
+    the row widening), at 3 tokens (no dispatch pass, the reductions split over the
+    waves of a workgroup) and at 100: captured once, replayed three times with eager
     calls of another size in between, every replay bit-identical to the eager
     result."""
     import ctypes as C

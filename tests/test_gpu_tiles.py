@@ -69,3 +69,37 @@ def test_row_tiles(rows, H, IM):
     d = got[0][some] - want
     assert np.abs(d).max() <= 2e-2 * max(1.0, float(np.abs(want).max()))
     assert np.linalg.norm(d) <= 1e-3 * np.linalg.norm(want)
+
+
+@pytest.mark.parametrize("n_experts,IM,T", [(16, 2880, 735), (16, 2880, 736), (32, 2048, 768), (32, 2048, 769),
+                                            (32, 2048, 1280), (32, 2048, 1281)])
+def test_sides_of_the_lines(n_experts, IM, T):
+    """Either side of the line to tiles of 128 rows (MXFP4, 16 experts, 23 column
+    tiles: 736 tokens) and of the lines up to which weights that exceed 256 MiB are
+    read past the caches (96 rows per expert in tiles of 128, 160 in tiles of 256):
+    the two weight formats bit for bit, and the oracle."""
+    H = 64
+    sh = synth.LayerShape("lines", T, H, IM, n_experts)
+    x = synth.round_bf16(synth.make_activations(sh))
+    wr, br = (synth.round_bf16(a) for a in synth.make_router(sh))
+    b1k, s1, b1, b2k, s2, b2 = synth.make_experts_mxfp4(sh)
+    b1, b2 = synth.round_bf16(b1), synth.round_bf16(b2)
+    w1, w2 = ob.mxfp4_dequant(b1k, s1), ob.mxfp4_dequant(b2k, s2)
+    many = int((256 << 20) / (3 * H * IM * n_experts * 17 / 32)) + 1
+    got = []
+    for fp4, layers in ((True, many), (False, many * 17 // 64 + 1)):
+        m = abi.Moe(H, IM, n_experts, max_tokens=T, swiglu_limit=sh.limit, layers=layers)
+        for i in range(layers):
+            if fp4:
+                m.upload_layer_mxfp4(i, wr, br, b1k, s1, b1, b2k, s2, b2)
+            else:
+                m.upload_layer(i, wr, br, w1, b1, w2, b2)
+        got.append(abi.run_layer(m, layers - 1, x, None)["out"])
+        m.close()
+    assert np.array_equal(got[0], got[1])
+    rows = np.arange(0, T, T // 15)
+    want = ob.moe_layer(np.ascontiguousarray(x[rows]), None, wr, br, w1, b1, w2, b2, 4, sh.limit,
+                        mode=ob.ROUND_ACT_BF16 | ob.PAR_TOKENS)
+    d = got[0][rows] - want
+    assert np.abs(d).max() <= 2e-2 * max(1.0, float(np.abs(want).max()))
+    assert np.linalg.norm(d) <= 1e-3 * np.linalg.norm(want)
