@@ -171,11 +171,10 @@ int run_gemms(moe_handle *h, int layer, const uint16_t *x, int T, const DirectId
   }
   if (stream_batch(T, c.experts)) {
     const int tiles = direct.topk_i ? stream_direct_tile_cap(T, c.experts) : stream_tile_cap(T, c.experts);
-    const bool quads = stream_act_quads(T, c.experts);
     HIP_TRY(launch_stream_gate_up(x, w1, lw.w1s, lw.b1g, lw.b1u, h->disp, h->act, h->Hp, h->IMp, c.swiglu_limit,
-                                  tiles, quads, cached, direct, s));
+                                  tiles, T, c.experts, cached, direct, s));
     HIP_TRY(tm.mark(MOE_STAGE_DOWN));
-    HIP_TRY(launch_stream_down(h->act, w2, lw.w2s, lw.b2, h->disp, h->y, h->Hp, h->IMp, tiles, quads, cached, direct, s));
+    HIP_TRY(launch_stream_down(h->act, w2, lw.w2s, lw.b2, h->disp, h->y, h->Hp, h->IMp, tiles, T, c.experts, cached, direct, s));
     return MOE_OK;
   }
   HIP_TRY(launch_gate_up(x, w1, lw.w1s, lw.b1g, lw.b1u, h->disp, h->act, h->Hp, h->IMp, c.swiglu_limit, T,

@@ -197,13 +197,6 @@ inline int stream_direct_tile_cap(int T, int E) {
   const int A = T * kTopK;
   return (A < E ? A : E) + A / (kRowBlock + 1);
 }
-// Order of act between the two GEMMs of stream.hip: in quads (act_place), or rows where
-// few rows share an expert, whose pieces then stand in fewer cache lines.  us per
-// moe_experts call, rows / quads, MXFP4: 128 experts, 24 tokens (0.75 rows per expert)
-// 140.8 / 143.1, 64 (2): 220 / 222, 256 (8): 305 / 302; 32 experts, 48 (6): 77.1 /
-// 76.6, 128 (16): 103.8 / 100.8; 8 experts, 32 (16): 39.0 / 36.7, 64 (32): 48.6 / 42.9.
-// bf16 gains less: 8 experts, 64 tokens 92.6 / 87.8.
-inline bool stream_act_quads(int T, int E) { return T * kTopK >= 6 * E; }
 inline int gemm_tile_cap(int T, int E, int tile_rows) { return T * kTopK / tile_rows + E; }
 // Height of the row tiles of a batch on MXFP4 weights (CfgHalf in gemm.hip has the
 // reason and times): half height where that gives the GPU its two workgroups per
@@ -233,12 +226,13 @@ hipError_t launch_down(const uint16_t *act, const void *w2, const uint16_t *w2_s
                        const DispatchBuffers &d, float *y, int H, int IM, int T, int E, int tile_rows,
                        bool cached, hipStream_t s);
 // tiles: row tiles, at most (stream_direct_tile_cap with ids.topk_i, otherwise stream_tile_cap).
-// quads: order of act (stream_act_quads), the same for both.  cached: kCachedWeightBytes.
+// T, E: tokens and experts of the batch, the same for both (the order of act between them follows from these).
+// cached: kCachedWeightBytes.
 hipError_t launch_stream_gate_up(const uint16_t *x, const void *w1, const uint16_t *w1_scale, const float *b1g,
                                  const float *b1u, const DispatchBuffers &d, uint16_t *act, int H, int IM,
-                                 float limit, int tiles, bool quads, bool cached, const DirectIds &ids, hipStream_t s);
+                                 float limit, int tiles, int T, int E, bool cached, const DirectIds &ids, hipStream_t s);
 hipError_t launch_stream_down(const uint16_t *act, const void *w2, const uint16_t *w2_scale, const float *b2,
-                              const DispatchBuffers &d, float *y, int H, int IM, int tiles, bool quads,
+                              const DispatchBuffers &d, float *y, int H, int IM, int tiles, int T, int E,
                               bool cached, const DirectIds &ids, hipStream_t s);
 // ldy: floats per row of y (the padded hidden size)
 hipError_t launch_combine(const float *y, int ldy, const int *inv, const float *topk_v, const int *pos, float *out,

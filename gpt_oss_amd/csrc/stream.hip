@@ -27,8 +27,7 @@
 // token MXFP4 10 + 6 (were 23 + 14).  What that rests on, by leaving it out, measured on a
 // batch that named all 32 experts (157 + 81; MXFP4 50 + 29): the weights' non-temporal
 // loads (bf16 174 + 90 with plain ones), two pairs of columns per wave that share the
-// rows they load (MXFP4 55 + 32 with one; where that would leave fewer than
-// kStreamTwoPairs workgroups of work, one), no refill loads past the slice's end
+// rows they load (MXFP4 55 + 32 with one; kStreamTwoPairs), no refill loads past the slice's end
 // (MXFP4 57 + 32 with them).  The number of slices (1, 2 or 4) matters to the
 // small launches only.
 //
@@ -51,8 +50,23 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 constexpr int kStreamKw = 4;     // waves of a workgroup = slices of the reduction
 constexpr int kStreamCols = 64;  // columns of a pair of column blocks
 constexpr int kStreamRows = 32;  // rows of a tile, at most
-// MXFP4: with this many column tiles of one pair or more, a wave takes two pairs
-constexpr int kStreamTwoPairs = 1024;
+// MXFP4: with this many column tiles of one pair or more, and more than this many
+// tokens, a wave takes two pairs.  What they save are loads of rows, which are few in a
+// batch of a few tokens, and with half as many workgroups the last ones leave more CUs
+// idle.  us per moe_experts call, one pair / two, even routing: 128 experts, 6 tokens
+// 54.9 / 60.1, 24: 136.4 / 140.8, 64: 219 / 218, 128: 277.6 / 268.5; Zipf's (exponent
+// 1.2) 6: 39.3 / 42.4, 24: 89 / 89, 32: 95.6 / 91.8, 64: 164.6 / 156.8; 32 experts, 6
+// tokens 45.6 / 47.5, 24: 73.2 / 73.5, 48: 78.9 / 77.2, 128: 114.4 / 100.6; 16 experts, 24
+// tokens 41.1 / 43.5, 64: 47.6 / 48.7.  Few column tiles, eight layers of 8 experts: 24
+// tokens (900 in gate_up) 33.9 / 34.2, 32 (990) 37.3 / 37.7, 48 (1170) 42.6 / 41.3.
+constexpr int kStreamTwoPairs = 1024, kStreamTwoPairsTokens = 24;
+// Order of act between the two GEMMs: in quads (act_place) from this many rows per
+// expert on; with fewer in rows, whose pieces then stand in fewer cache lines.  us per
+// moe_experts call, rows / quads, MXFP4: 128 experts, 24 tokens (0.75 rows per expert)
+// 140.8 / 143.1, 64 (2): 220 / 222, 256 (8): 305 / 302; 32 experts, 48 (6): 77.1 /
+// 76.6, 128 (16): 103.8 / 100.8; 8 experts, 32 (16): 39.0 / 36.7, 64 (32): 48.6 / 42.9.
+// bf16 gains less: 8 experts, 64 tokens 92.6 / 87.8.
+constexpr int kStreamQuadRows = 6;
 
 // Orders LDS traffic only: the loads in flight stay in flight.
 __device__ __forceinline__ void stream_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
@@ -92,7 +106,7 @@ __device__ __forceinline__ void share_of(int l, int wgs, int nb, int &col, int &
 //     through a kilobyte of LDS that only the wave touches (STAGED; tiles of more than
 //     16 rows: below, the weights' loads are the more).  8 experts, 64 tokens, us per
 //     moe_experts call without / with: bf16 90.7 / 87.9, MXFP4 43.5 / 42.6;
-//   * gate_up leaves the activation in "quads" for the down GEMM (stream_act_quads):
+//   * gate_up leaves the activation in "quads" for the down GEMM (kStreamQuadRows):
 //     per 16 rows and step of 32 k a kilobyte, in it the pieces of 8 k of four rows side
 //     by side.  The byte of piece `piece` of row r:
 __device__ __forceinline__ uint32_t act_place(int r, int piece) { return (r >> 2) * 256u + piece * 64u + (r & 3) * 16u; }
@@ -468,12 +482,12 @@ __global__ __launch_bounds__(kStreamKw * 64, NP == 1 ? 4 : 3) void stream_gemm_k
 template <int NP, bool GATE_UP>
 static hipError_t launch_stream_np(const uint4 *a, const uint4 *w, const uint16_t *w_scale, const float *ba,
                                    const float *bb, const DispatchBuffers &d, void *out, int K, int N, float limit,
-                                   int tiles, bool quads, bool cached, const DirectIds &ids, hipStream_t s) {
+                                   int tiles, int T, int E, bool cached, const DirectIds &ids, hipStream_t s) {
   const int pairs = (GATE_UP ? 2 * N : N) / kStreamCols;
   const int grid = tiles * ((pairs + NP - 1) / NP);
 #define MOE_STREAM(FP4, DIRECT)                                                              \
   do {                                                                                       \
-    if (quads)                                                                               \
+    if (T * kTopK >= kStreamQuadRows * E)                                                    \
       stream_gemm_kernel<NP, GATE_UP, FP4, DIRECT, true><<<grid, kStreamKw * 64, 0, s>>>(    \
           a, w, w_scale, ba, bb, d.rowmap, d.blk_expert, d.totals, d.inv, out, K, N, limit,  \
           tiles, cached, ids);                                                               \
@@ -496,24 +510,24 @@ static hipError_t launch_stream_np(const uint4 *a, const uint4 *w, const uint16_
 template <bool GATE_UP>
 static hipError_t launch_stream(const void *a, const void *w, const uint16_t *w_scale, const float *ba,
                                 const float *bb, const DispatchBuffers &d, void *out, int K, int N, float limit,
-                                int tiles, bool quads, bool cached, const DirectIds &ids, hipStream_t s) {
+                                int tiles, int T, int E, bool cached, const DirectIds &ids, hipStream_t s) {
   const uint4 *af = static_cast<const uint4 *>(a), *wf = static_cast<const uint4 *>(w);
   const int pairs = (GATE_UP ? 2 * N : N) / kStreamCols;
-  if (w_scale && tiles * pairs >= kStreamTwoPairs)
-    return launch_stream_np<2, GATE_UP>(af, wf, w_scale, ba, bb, d, out, K, N, limit, tiles, quads, cached, ids, s);
-  return launch_stream_np<1, GATE_UP>(af, wf, w_scale, ba, bb, d, out, K, N, limit, tiles, quads, cached, ids, s);
+  if (w_scale && tiles * pairs >= kStreamTwoPairs && T > kStreamTwoPairsTokens)
+    return launch_stream_np<2, GATE_UP>(af, wf, w_scale, ba, bb, d, out, K, N, limit, tiles, T, E, cached, ids, s);
+  return launch_stream_np<1, GATE_UP>(af, wf, w_scale, ba, bb, d, out, K, N, limit, tiles, T, E, cached, ids, s);
 }
 
 hipError_t launch_stream_gate_up(const uint16_t *x, const void *w1, const uint16_t *w1_scale, const float *b1g,
                                  const float *b1u, const DispatchBuffers &d, uint16_t *act, int H, int IM,
-                                 float limit, int tiles, bool quads, bool cached, const DirectIds &ids, hipStream_t s) {
-  return launch_stream<true>(x, w1, w1_scale, b1g, b1u, d, act, H, IM, limit, tiles, quads, cached, ids, s);
+                                 float limit, int tiles, int T, int E, bool cached, const DirectIds &ids, hipStream_t s) {
+  return launch_stream<true>(x, w1, w1_scale, b1g, b1u, d, act, H, IM, limit, tiles, T, E, cached, ids, s);
 }
 
 hipError_t launch_stream_down(const uint16_t *act, const void *w2, const uint16_t *w2_scale, const float *b2,
-                              const DispatchBuffers &d, float *y, int H, int IM, int tiles, bool quads,
+                              const DispatchBuffers &d, float *y, int H, int IM, int tiles, int T, int E,
                               bool cached, const DirectIds &ids, hipStream_t s) {
-  return launch_stream<false>(act, w2, w2_scale, b2, nullptr, d, y, IM, H, 0.f, tiles, quads, cached, ids, s);
+  return launch_stream<false>(act, w2, w2_scale, b2, nullptr, d, y, IM, H, 0.f, tiles, T, E, cached, ids, s);
 }
 
 }  // namespace moe

@@ -55,10 +55,10 @@ def test_rows_of_an_expert(rows, H, IM):
     m.close()
 
 
-@pytest.mark.parametrize("T", [2, 40, 65])
+@pytest.mark.parametrize("T", [2, 24, 40, 65])
 def test_two_pairs_of_columns_per_wave(T):
-    """128 experts and nine pairs of columns: MXFP4 waves take two pairs each from
-    40 tokens on (the last of a row has one), one pair at 2 tokens."""
+    """128 experts and nine pairs of columns: MXFP4 waves take two pairs each
+    from 25 tokens on (the last of a row has one), one pair up to 24."""
     sh = synth.LayerShape("pairs", T, 576, 576, 128)
     x = synth.round_bf16(synth.make_activations(sh))
     wr, br = (synth.round_bf16(a) for a in synth.make_router(sh))
