@@ -179,10 +179,12 @@ inline bool direct_plan_fits(int T, int max_rows, int E, int a_pad_cap) {
 // workgroups that read its weights side by side (share_of in stream.hip).  On
 // either side of the line, us per moe_experts call at 2880 x 2880 with the kernels
 // of stream.hip / of gemm.hip, even routing and Zipf's (exponent 1.2):
-//   32 experts, MXFP4:  96 tokens 101 / 114, 101 / 122;  128: 107 / 108, 113 / 125;  192: 121 / 115, 124 / 156
-//   32 experts, bf16:   96 tokens 268 / 276, 272 / 281;  128: 281 / 276, 283 / 296;  192: 303 / 282, 327 / 308
-//   128 experts, MXFP4: 384 tokens 340 / 358, 324 / 369;  512: 372 / 361, 380 / 408;  640: 396 / 367, 427 / 429
-//   128 experts, bf16:  384 tokens 1017 / 1086, 1018 / 1024;  512: 1071 / 1084, 1111 / 1072;  640: 1129 / 1085, 1199 / 1114
+//   32 experts, MXFP4:  96 tokens 98 / 113, 103 / 121;  128: 103 / 113, 109 / 141;  192: 113 / 114, 117 / 138
+//   32 experts, bf16:   96 tokens 263 / 277, 261 / 285;  128: 272 / 278, 270 / 291;  192: 288 / 282, 305 / 321
+//   128 experts, MXFP4: 384 tokens 342 / 367, 314 / 356;  512: 364 / 370, 372 / 424;  768: 391 / 379, 436 / 451
+//   128 experts, bf16:  384 tokens 993 / 1087, 942 / 988;  512: 1027 / 1087, 1088 / 1122;  768: 1111 / 1098, 1210 / 1168
+//   8 experts, 96 tokens: MXFP4 48 / 52, 49 / 60;  bf16 117 / 96, 101 / 106;  128 tokens, bf16: 135 / 106, 132 / 111
+// Up to the line neither format loses under either routing; past it bf16 does.
 // The rule knows nothing of the weights' format: both formats give the same bits.
 constexpr int kCus = 256;
 constexpr int kStreamMeanRows = 16;
