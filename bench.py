@@ -274,7 +274,7 @@ def main():
     mfma_tflops = flops_gate_up / t_gate_up / 1e12
     hbm_gbs = bytes_gate_up / t_gate_up / 1e9
     kernel = "%s<gate_up%s>" % ("stream_gemm_kernel" if T <= STREAM_TOKENS or T * K <= STREAM_MEAN_ROWS * E
-                                else "grouped_gemm_kernel", ", MXFP4" if mxfp4 else "")
+                                else "grouped_gemm_kernel" if mxfp4 else "bf16_gemm_kernel", ", MXFP4" if mxfp4 else "")
     if BOUND[shape.name] == "mfma":
         roofline = {"bound": "mfma", "kernel": kernel, "achieved": mfma_tflops, "peak": PEAK_BF16_TFLOPS,
                     "unit": "TFLOP/s", "frac": mfma_tflops / PEAK_BF16_TFLOPS}

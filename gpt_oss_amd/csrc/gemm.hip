@@ -1,5 +1,5 @@
-// Grouped expert GEMMs on the bf16 matrix cores (v_mfma_f32_32x32x16_bf16,
-// fp32 accumulate).  Replaces mlp1_kernel / mlp1_120b_kernel
+// Grouped expert GEMMs with MXFP4 weights on the bf16 matrix cores
+// (v_mfma_f32_32x32x16_bf16, fp32 accumulate).  Replaces mlp1_kernel / mlp1_120b_kernel
 // (matmul/matmul.cpp:1023-1465) with the clamped SwiGLU in the epilogue
 // (utility/utility.cpp:1108-1125; formula of run.cpp:709-726) and
 // mlp2_kernel_noatomic / mlp2_120b_kernel (matmul/matmul.cpp:1470-1914).
@@ -11,7 +11,8 @@
 // operand of gate_up is the token rows themselves, bf16 row-major, found through
 // the dispatch's row map: there is no gathered copy (gemm_tile_gl).
 //
-// Batches with few rows per expert run the kernels of stream.hip instead.
+// Batches with few rows per expert run the kernels of stream.hip instead, bf16 weights
+// those of gemm_bf16.hip.
 //
 // Tiling.  A workgroup of NW waves owns a tile of (RBT*32) rows x
 // (NW*NBW*32) columns of one expert.  The waves split the columns only: each
@@ -19,18 +20,14 @@
 // 1..8 following the expert's row count (see build_plan in dispatch.hip), so a ragged
 // segment pads to at most 31 rows and MFMA work follows the real rows.
 //
-// Feeding the matrix cores.  A step of 32 k needs 32 KB per CU, and one CU
-// takes data in from L2 at about 45 GB/s with 100 KB in flight and 55-60 GB/s
-// with 200 KB, so the design keeps many bytes in flight:
+// Feeding the matrix cores.  Many bytes are kept in flight:
 //   * the row operand (shared by all waves) goes straight into an R-stage LDS
 //     ring by DMA (global_load_lds_dwordx4), R-1 steps ahead of the MFMAs;
 //   * the column operand is private to a wave in this layout, so it never
 //     touches LDS: it is loaded into an R-slot ring of VGPRs, R-1 steps ahead.
-// R is 4 (3 steps x 32 KB = 96 KB in flight
-// per CU: measured against 3, 5, 6 and 7, a deeper ring gains nothing in the
-// main loop and costs the time its longer fill takes at the start of every
-// tile, 0.7 % of the layer per stage at 4096 tokens; with 3 the main loop
-// starves).  These loads
+// R is 4 (measured against 3, 5, 6 and 7 on bf16 weights, which these kernels ran as
+// well: a deeper ring gains nothing in the main loop and its longer fill costs at the
+// start of every tile; with 3 the main loop starves).  These loads
 // complete in the order they were issued, so waiting for "all but the newest n"
 // (s_waitcnt vmcnt(n)) picks out exactly the step that is needed next and
 // leaves the later ones in flight.
@@ -188,14 +185,13 @@ struct GemmCfg {
   static constexpr int EPI_WAVE = 32 * EPI_LD / 4;       // uint4 per wave of epilogue buffer
 };
 
-// FP4: the column operand is MXFP4 as packed by pack_fp4_kernel: per pair of
+// The column operand is MXFP4 as packed by pack_fp4_kernel: per pair of
 // column blocks and step of 32 k one 16-byte chunk per lane (blocks 2P and 2P+1,
 // each [k block 0: 8 nibbles][k block 1: 8 nibbles] of the lane's row) and two
 // scale bytes per row.  A step of 32 k is exactly one MXFP4 block, so one scale
 // serves both of its k blocks.  The nibbles become bf16 MFMA operands in
 // registers (v_cvt_scalef32_pk_bf16_fp4: two values and their scale per
-// instruction, exact); everything else is the bf16 kernel, which then takes in
-// 4.25 KB instead of 16 KB of weights per CU and step.
+// instruction, exact).
 //
 // RS (row split) > 1 serves the last column tile of a matrix whose width is not
 // a multiple of the tile's: only NW / RS waves would have columns there, so the
@@ -206,10 +202,10 @@ struct GemmCfg {
 //
 // gemm_tile is the down GEMM; gate_up, whose row operand is scattered, is
 // gemm_tile_gl below.
-template <int RBT, int RS, typename C, bool FP4, bool STREAM>
+template <int RBT, int RS, typename C, bool STREAM>
 __device__ __forceinline__ void gemm_tile(const uint4 *__restrict__ a_frag,  // [rb][KB][64]
-                                          const uint4 *__restrict__ b_frag,  // expert: [nb][KB][64], FP4: [nb/2][KB/2][64]
-                                          const uint16_t *__restrict__ b_scale,  // FP4: expert's [nb/2][KB/2][32] byte pairs
+                                          const uint4 *__restrict__ b_frag,  // expert's [nb/2][KB/2][64] chunks
+                                          const uint16_t *__restrict__ b_scale,  // expert's [nb/2][KB/2][32] byte pairs
                                           int KB, int rb0, int rbt, int nb0, int nb_valid,
                                           const float *__restrict__ bias,  // expert's
                                           float *__restrict__ y, int out_ld,
@@ -234,12 +230,12 @@ __device__ __forceinline__ void gemm_tile(const uint4 *__restrict__ a_frag,  // 
   static_assert(KPS == 2, "the step is software-pipelined as two k blocks");
   constexpr int A_CH = RBT * RS * KPS;       // 1 KB chunks of the row operand per step
   constexpr int LA = (A_CH + NW - 1) / NW;   // DMA loads per wave per step (a short last pass repeats a chunk)
-  constexpr int LB = FP4 ? 2 : NBW * KPS;    // register loads per wave per step
+  constexpr int LB = 2;                      // register loads per wave per step (nibbles, scales)
   constexpr int LPS = LA + LB;
   static_assert(LPS * (R - 2) + LA <= 63, "vmcnt is a 6-bit counter");
-  static_assert(!FP4 || NBW == 2, "an MXFP4 chunk holds the pair of column blocks of one wave");
+  static_assert(NBW == 2, "an MXFP4 chunk holds the pair of column blocks of one wave");
   constexpr int NM = RBT * NBW;              // MFMAs per k block
-  constexpr int DEC = FP4 ? NBW : 0;         // decode items per k block (one column block each)
+  constexpr int DEC = NBW;         // decode items per k block (one column block each)
   constexpr int SIDE1 = (RBT + LB + DEC + NM - 1) / NM;  // side items per MFMA, k block 0
   constexpr int SIDE2 = (LA + RBT + DEC + NM - 1) / NM;  // ... k block 1
   const int tid = threadIdx.x;
@@ -261,17 +257,9 @@ __device__ __forceinline__ void gemm_tile(const uint4 *__restrict__ a_frag,  // 
   const uint4 *a_src = a_frag + (size_t)rb0 * KB * 64 + lane;
   // Column blocks past the end of the matrix (last column tile only) re-load
   // the last valid block; their products are never stored.
-  const uint4 *b_src[NBW];
-  const uint16_t *s_src = nullptr;
-  if (FP4) {
-    const size_t pair = (size_t)((nb0 + min(cw * NBW, nb_valid - NBW)) >> 1);
-    b_src[0] = b_frag + pair * n_steps * 64 + lane;
-    s_src = b_scale + pair * n_steps * 32 + (lane & 31);
-  } else {
-#pragma unroll
-    for (int j = 0; j < NBW; j++)
-      b_src[j] = b_frag + (size_t)(nb0 + min(cw * NBW + j, nb_valid - 1)) * KB * 64 + lane;
-  }
+  const size_t pair = (size_t)((nb0 + min(cw * NBW, nb_valid - NBW)) >> 1);
+  const uint4 *b_src = b_frag + pair * n_steps * 64 + lane;
+  const uint16_t *s_src = b_scale + pair * n_steps * 32 + (lane & 31);
 
   // Row operand: chunk c of a step (c = pass*NW + wave) is row block c / KPS, k block c % KPS.
   auto issue_a = [&](uint4 *st, int ks, int m) {
@@ -279,28 +267,23 @@ __device__ __forceinline__ void gemm_tile(const uint4 *__restrict__ a_frag,  // 
     const int blk = RS == 1 ? c / KPS : min(c / KPS, rbt - 1);
     dma_to_lds_16(a_src + ((size_t)blk * KB + ks * KPS + c % KPS) * 64, st + c * 64);
   };
-  // Column operand: register m of a slot is column block m / KPS, k block m % KPS.
-  // FP4: load 0 of a slot is the chunk of nibbles, load 1 the two scale bytes.
-  u32x4 bq[R][FP4 ? 1 : LB];
+  // Column operand: load 0 of a slot is the chunk of nibbles, load 1 the two scale bytes.
+  u32x4 bq[R];
   uint32_t bsc[R];
   auto issue_b = [&](int slot, int ks, int m) {
-    if (FP4) {
-      if (m == 0) {
-        bq[slot][0] = load_cols<STREAM>(b_src[0] + (size_t)ks * 64);
-      } else {
-        bsc[slot] = s_src[(size_t)ks * 32];
-      }
+    if (m == 0) {
+      bq[slot] = load_cols<STREAM>(b_src + (size_t)ks * 64);
     } else {
-      bq[slot][m] = load_cols<STREAM>(b_src[m / KPS] + (size_t)(ks * KPS + m % KPS) * 64);
+      bsc[slot] = s_src[(size_t)ks * 32];
     }
   };
-  // FP4: the decoded operands of the step at hand, [column block][k block].
+  // The decoded operands of the step at hand, [column block][k block].
   // Those of k block 0 are decoded during the previous step's second half,
   // those of k block 1 during this step's first half.
   bf16x8 bdec[NBW][KPS];
   auto decode = [&](int slot, int j, int kk) {
     const float scale = __uint_as_float(((bsc[slot] >> (8 * j)) & 0xffu) << 23);  // 2^(s - 127)
-    const uint32_t nib = bq[slot][0][j * KPS + kk];
+    const uint32_t nib = bq[slot][j * KPS + kk];
     const bf16x2 p0 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(nib, scale, 0);
     const bf16x2 p1 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(nib, scale, 1);
     const bf16x2 p2 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(nib, scale, 2);
@@ -315,14 +298,6 @@ __device__ __forceinline__ void gemm_tile(const uint4 *__restrict__ a_frag,  // 
   };
   auto mma = [](bf16x8 rows, bf16x8 colv, f32x16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(rows, colv, c, 0, 0, 0);
-  };
-  // column operand of (slot, column block j, k block kk)
-  auto cols_of = [&](int slot, int j, int kk) {
-    if constexpr (FP4) {
-      return bdec[j][kk];
-    } else {
-      return __builtin_bit_cast(bf16x8, bq[slot][j * KPS + kk]);
-    }
   };
   static_assert(R >= 3 && R <= 4, "up to four stage arrays are passed in");
   // "Step s of the row operand has landed" as a bound on the vector-memory
@@ -362,10 +337,8 @@ __device__ __forceinline__ void gemm_tile(const uint4 *__restrict__ a_frag,  // 
   lds_barrier();
 #pragma unroll
   for (int i = 0; i < RBT; i++) read_a(ring.p[0], 0, 0, i);
-  if (FP4) {
 #pragma unroll
-    for (int j = 0; j < NBW; j++) decode(0, j, 0);
-  }
+  for (int j = 0; j < NBW; j++) decode(0, j, 0);
 
   // Step ks, slot u = ks % R:
   //   [MFMAs of k block 0 | read row fragments of k block 1, load B(ks+R-1) into slot u-1]
@@ -396,7 +369,7 @@ __device__ __forceinline__ void gemm_tile(const uint4 *__restrict__ a_frag,  // 
           decode(u, t - RBT - LB, 1);
         }
       }
-      acc[m / NBW][m % NBW] = mma(fa[0][m / NBW], cols_of(u, m % NBW, 0), acc[m / NBW][m % NBW]);
+      acc[m / NBW][m % NBW] = mma(fa[0][m / NBW], bdec[m % NBW][0], acc[m / NBW][m % NBW]);
       __builtin_amdgcn_sched_barrier(0);
     }
     WAIT_VMCNT(WAIT_DMA_STEP);
@@ -414,7 +387,7 @@ __device__ __forceinline__ void gemm_tile(const uint4 *__restrict__ a_frag,  // 
           decode((u + 1) % R, t - LA - RBT, 0);  // landed: the wait above covers it
         }
       }
-      acc[m / NBW][m % NBW] = mma(fa[1][m / NBW], cols_of(u, m % NBW, 1), acc[m / NBW][m % NBW]);
+      acc[m / NBW][m % NBW] = mma(fa[1][m / NBW], bdec[m % NBW][1], acc[m / NBW][m % NBW]);
       __builtin_amdgcn_sched_barrier(0);
     }
   };
@@ -484,7 +457,7 @@ constexpr int kLineStages = 4;
 // an odd step 2d+1 needs, and B(ks+1), which every step's successor needs.  Even
 // steps need no barrier: they read a double stage that landed before the
 // previous odd step's barrier and refill nothing.
-template <int RBT, int RS, typename C, bool FP4, bool STREAM>
+template <int RBT, int RS, typename C, bool STREAM>
 __device__ __forceinline__ void gemm_tile_gl(const uint4 *__restrict__ x_rows,  // token rows [T][KB * 2] of 16 bytes
                                              const uint4 *__restrict__ b_frag,
                                              const uint16_t *__restrict__ b_scale, int KB, int rb0, int rbt,
@@ -500,10 +473,10 @@ __device__ __forceinline__ void gemm_tile_gl(const uint4 *__restrict__ x_rows,  
   static_assert(KPS == 2 && NW == 4 && RB == 4 && C::RBT_MAX <= 8 && (RS == 1 || RS == 2), "shape of the line gather");
   constexpr int NB = RBT * RS;                // row blocks staged per step
   constexpr int LA2 = NB;                     // DMA loads per wave and double step: one per row block
-  constexpr int LB = FP4 ? 2 : NBW * KPS;     // register loads per wave and step
-  static_assert(!FP4 || NBW == 2, "an MXFP4 chunk holds the pair of column blocks of one wave");
+  constexpr int LB = 2;                       // register loads per wave and step (nibbles, scales)
+  static_assert(NBW == 2, "an MXFP4 chunk holds the pair of column blocks of one wave");
   constexpr int NM = RBT * NBW;               // MFMAs per k block
-  constexpr int DEC = FP4 ? NBW : 0;
+  constexpr int DEC = NBW;
   static_assert(R2 >= 3, "with 2 double stages an odd step would have to wait for all but 2 * LB loads");
   constexpr int WAIT_FILL = (R2 - 1) * LA2;  // the loads behind A2(0) in the first filling
   constexpr int WAIT_MID = 2 * LB + LA2;                                     // see the steps
@@ -560,39 +533,27 @@ __device__ __forceinline__ void gemm_tile_gl(const uint4 *__restrict__ x_rows,  
         lane_rd[par][kk] = sub * 64 + (4 * (row8 >> 1) + 2 * (par ^ (sub & 1)) + (row8 & 1)) * 4 +
                            ((kk * 2 + h + (row8 >> 1)) & 3);
   }
-  const uint4 *b_src[NBW];
-  const uint16_t *s_src = nullptr;
-  if (FP4) {
-    const size_t pair = (size_t)((nb0 + min(cw * NBW, nb_valid - NBW)) >> 1);
-    b_src[0] = b_frag + pair * n_steps * 64 + lane;
-    s_src = b_scale + pair * n_steps * 32 + (lane & 31);
-  } else {
-#pragma unroll
-    for (int j = 0; j < NBW; j++)
-      b_src[j] = b_frag + (size_t)(nb0 + min(cw * NBW + j, nb_valid - 1)) * KB * 64 + lane;
-  }
+  const size_t pair = (size_t)((nb0 + min(cw * NBW, nb_valid - NBW)) >> 1);
+  const uint4 *b_src = b_frag + pair * n_steps * 64 + lane;
+  const uint16_t *s_src = b_scale + pair * n_steps * 32 + (lane & 31);
 
   // double step jd of row block m into double stage slot d
   auto issue_a2 = [&](int d, int jd, int m) {
     dma_to_lds_16(x_rows + lane_src[m] + jd * 8, arr[2 * d + (m >= 4 ? 1 : 0)] + ((m & 3) * 4 + w) * 64);
   };
-  u32x4 bq[RB][FP4 ? 1 : LB];
+  u32x4 bq[RB];
   uint32_t bsc[RB];
   auto issue_b = [&](int slot, int ks, int m) {
-    if (FP4) {
-      if (m == 0) {
-        bq[slot][0] = load_cols<STREAM>(b_src[0] + (size_t)ks * 64);
-      } else {
-        bsc[slot] = s_src[(size_t)ks * 32];
-      }
+    if (m == 0) {
+      bq[slot] = load_cols<STREAM>(b_src + (size_t)ks * 64);
     } else {
-      bq[slot][m] = load_cols<STREAM>(b_src[m / KPS] + (size_t)(ks * KPS + m % KPS) * 64);
+      bsc[slot] = s_src[(size_t)ks * 32];
     }
   };
   bf16x8 bdec[NBW][KPS];
   auto decode = [&](int slot, int j, int kk) {
     const float scale = __uint_as_float(((bsc[slot] >> (8 * j)) & 0xffu) << 23);
-    const uint32_t nib = bq[slot][0][j * KPS + kk];
+    const uint32_t nib = bq[slot][j * KPS + kk];
     const bf16x2 p0 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(nib, scale, 0);
     const bf16x2 p1 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(nib, scale, 1);
     const bf16x2 p2 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(nib, scale, 2);
@@ -607,13 +568,6 @@ __device__ __forceinline__ void gemm_tile_gl(const uint4 *__restrict__ x_rows,  
   };
   auto mma = [](bf16x8 rows, bf16x8 colv, f32x16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(colv, rows, c, 0, 0, 0);
-  };
-  auto cols_of = [&](int slot, int j, int kk) {
-    if constexpr (FP4) {
-      return bdec[j][kk];
-    } else {
-      return __builtin_bit_cast(bf16x8, bq[slot][j * KPS + kk]);
-    }
   };
 
   // one double step of the row operand / one step of the column operand, all of the wave's loads
@@ -655,10 +609,8 @@ __device__ __forceinline__ void gemm_tile_gl(const uint4 *__restrict__ x_rows,  
   lds_barrier();
 #pragma unroll
   for (int i = 0; i < RBT; i++) read_a(0, 0, 0, 0, i);
-  if (FP4) {
 #pragma unroll
-    for (int j = 0; j < NBW; j++) decode(0, j, 0);
-  }
+  for (int j = 0; j < NBW; j++) decode(0, j, 0);
 
   // Step ks = 2 jd + par, u = ks mod PERIOD: column slot u % RB, double stage (u / 2) % R2.
   auto step = [&](auto u_c, int ks) {
@@ -682,7 +634,7 @@ __device__ __forceinline__ void gemm_tile_gl(const uint4 *__restrict__ x_rows,  
           decode(slot, t - RBT - LB, 1);
         }
       }
-      acc[m / NBW][m % NBW] = mma(fa[0][m / NBW], cols_of(slot, m % NBW, 0), acc[m / NBW][m % NBW]);
+      acc[m / NBW][m % NBW] = mma(fa[0][m / NBW], bdec[m % NBW][0], acc[m / NBW][m % NBW]);
       __builtin_amdgcn_sched_barrier(0);
     }
     // Every step says in its middle what has landed, as a count: all but the
@@ -709,7 +661,7 @@ __device__ __forceinline__ void gemm_tile_gl(const uint4 *__restrict__ x_rows,  
           decode((slot + 1) % RB, t - LAX - RBT, 0);
         }
       }
-      acc[m / NBW][m % NBW] = mma(fa[1][m / NBW], cols_of(slot, m % NBW, 1), acc[m / NBW][m % NBW]);
+      acc[m / NBW][m % NBW] = mma(fa[1][m / NBW], bdec[m % NBW][1], acc[m / NBW][m % NBW]);
       __builtin_amdgcn_sched_barrier(0);
     }
   };
@@ -726,7 +678,7 @@ __device__ __forceinline__ void gemm_tile_gl(const uint4 *__restrict__ x_rows,  
   gate_up_epilogue<RBT, RS, C>(acc, outp, out_ld, limit, rb0, rbt, nb0, nb_valid, cw, rg, lane);
 }
 
-template <typename C, bool GATE_UP, bool FP4, bool STREAM>
+template <typename C, bool GATE_UP, bool STREAM>
 __global__ __launch_bounds__(C::THREADS, C::WGS) void grouped_gemm_kernel(
     const uint4 *__restrict__ a_frag, const uint4 *__restrict__ w_frag,
     const uint16_t *__restrict__ w_scale,
@@ -748,9 +700,9 @@ __global__ __launch_bounds__(C::THREADS, C::WGS) void grouped_gemm_kernel(
   if (!locate_tile(tiles, totals + (GATE_UP ? kTotBoundsGateUp : kTotBoundsDown), tc)) return;
   const int nb0 = tc.nt * C::TILE_NB;
   const int nb_valid = min(C::TILE_NB, nb_total - nb0);
-  // per expert: bf16 nb_total * KB fragments of 1 KB; MXFP4 (nb_total/2) * (KB/2) chunks of 1 KB
-  const uint4 *b_frag = w_frag + (size_t)tc.e * nb_total * KB * (FP4 ? 16 : 64);
-  const uint16_t *b_scale = FP4 ? w_scale + (size_t)tc.e * nb_total * KB * 8 : nullptr;
+  // per expert (nb_total/2) * (KB/2) chunks of 1 KB
+  const uint4 *b_frag = w_frag + (size_t)tc.e * nb_total * KB * 16;
+  const uint16_t *b_scale = w_scale + (size_t)tc.e * nb_total * KB * 8;
   const float *ba = bias_a + (size_t)tc.e * N;
   const float *bb = GATE_UP ? bias_b + (size_t)tc.e * N : nullptr;
   // the tile with n row blocks per wave and the waves in rs row groups
@@ -758,10 +710,10 @@ __global__ __launch_bounds__(C::THREADS, C::WGS) void grouped_gemm_kernel(
     constexpr int n = decltype(n_c)::value, rs = decltype(rs_c)::value;
     if constexpr (n * rs <= C::RBT_MAX) {
       if constexpr (GATE_UP) {
-        gemm_tile_gl<n, rs, C, FP4, STREAM>(a_frag, b_frag, b_scale, KB, tc.rb0, tc.rbt, nb0, nb_valid, rowmap,
+        gemm_tile_gl<n, rs, C, STREAM>(a_frag, b_frag, b_scale, KB, tc.rb0, tc.rbt, nb0, nb_valid, rowmap,
                                             ba, bb, outp, N, limit, st0, st1, st2, st3, st4, st5, st6, st7);
       } else {
-        gemm_tile<n, rs, C, FP4, STREAM>(a_frag, b_frag, b_scale, KB, tc.rb0, tc.rbt, nb0, nb_valid, ba,
+        gemm_tile<n, rs, C, STREAM>(a_frag, b_frag, b_scale, KB, tc.rb0, tc.rbt, nb0, nb_valid, ba,
                                          static_cast<float *>(outp), N, st0, st1, st2, st3, epi);
       }
     }
@@ -798,14 +750,12 @@ __global__ __launch_bounds__(C::THREADS, C::WGS) void grouped_gemm_kernel(
 // 4 waves, one per SIMD, each 256 rows x 64 columns (8 x 2 accumulators = all
 // 256 accumulation registers); 256 x 256 tiles; 4 ring slots.
 using CfgFull = GemmCfg<4, 2, 4, 8, 1>;
-// MXFP4: tiles half as high, two workgroups per CU.  A step of MXFP4 weights is
+// Tiles half as high, two workgroups per CU.  A step of MXFP4 weights is
 // 4 KB, so that a second tile of the same columns costs next to nothing, and the
 // decode, the fill and the epilogue of one workgroup run under the other's MFMAs.
 // us per layer call, full / half height (2880 x 2880, even routing): 32 experts,
 // 256 tokens 175 / 143, 512: 188 / 172, 1024: 242 / 242, 2048: 427 / 395, 4096:
-// 731 / 725; 128 experts, 768: 533 / 428, 2048: 621 / 551, 3072: 712 / 676.  With
-// bf16 weights (16 KB per step) it is the other way round where an expert then
-// takes two tiles: 1024 tokens 392 / 439, 6144 tokens and 128 experts 1639 / 1813.
+// 731 / 725; 128 experts, 768: 533 / 428, 2048: 621 / 551, 3072: 712 / 676.
 using CfgHalf = GemmCfg<4, 2, 4, 4, 2>;
 static_assert(CfgFull::RBT_MAX * kRowBlock == kTileRows && CfgHalf::RBT_MAX * kRowBlock == kHalfTileRows &&
                   CfgFull::TILE_NB == kGemmTileNb && CfgHalf::TILE_NB == kGemmTileNb,
@@ -827,8 +777,7 @@ static bool gemm_streams_weights(int T, int E, bool half, bool cached) {
   return T * kTopK <= (half ? kStreamRowsHalf : kStreamRowsFull) * E;
 }
 
-// w_scale == nullptr: w holds bf16 fragments; otherwise w holds MXFP4 chunks and
-// w_scale their scale bytes (pack_fp4_kernel).  The plan is of tiles of plan.tile_rows.
+// w holds MXFP4 chunks and w_scale their scale bytes (pack_fp4_kernel).  The plan is of tiles of tile_rows.
 template <bool GATE_UP>
 static hipError_t launch_gemm(const void *a, const void *w, const uint16_t *w_scale, const float *ba,
                               const float *bb, const DispatchBuffers &d, void *out, int K, int N,
@@ -839,18 +788,14 @@ static hipError_t launch_gemm(const void *a, const void *w, const uint16_t *w_sc
   const TileDesc *tiles = GATE_UP ? d.tiles_gate_up : d.tiles_down;
   const uint4 *af = static_cast<const uint4 *>(a), *wf = static_cast<const uint4 *>(w);
   // the full-height kernels take a plan of either height, the others one of half height
-  const bool half = w_scale && tile_rows == kHalfTileRows;
+  const bool half = tile_rows == kHalfTileRows;
   const bool stream = gemm_streams_weights(T, E, half, cached);
-#define MOE_GEMM(C, FP4, STREAM)                                                                            \
-  grouped_gemm_kernel<C, GATE_UP, FP4, STREAM><<<grid, C::THREADS, 0, s>>>(af, wf, w_scale, ba, bb, tiles,  \
-                                                                           d.totals, d.rowmap, out, K, N, limit)
-  if (half) {
-    if (stream) MOE_GEMM(CfgHalf, true, true); else MOE_GEMM(CfgHalf, true, false);
-  } else if (w_scale) {
-    MOE_GEMM(CfgFull, true, false);
-  } else {
-    if (stream) MOE_GEMM(CfgFull, false, true); else MOE_GEMM(CfgFull, false, false);
-  }
+#define MOE_GEMM(C, STREAM)                                                                                 \
+  grouped_gemm_kernel<C, GATE_UP, STREAM><<<grid, C::THREADS, 0, s>>>(af, wf, w_scale, ba, bb, tiles, d.totals, \
+                                                                      d.rowmap, out, K, N, limit)
+  if (!half) MOE_GEMM(CfgFull, false);
+  else if (stream) MOE_GEMM(CfgHalf, true);
+  else MOE_GEMM(CfgHalf, false);
 #undef MOE_GEMM
   return hipGetLastError();
 }
@@ -858,12 +803,17 @@ static hipError_t launch_gemm(const void *a, const void *w, const uint16_t *w_sc
 hipError_t launch_gate_up(const uint16_t *x, const void *w1, const uint16_t *w1_scale, const float *b1g,
                           const float *b1u, const DispatchBuffers &d, uint16_t *act, int H, int IM,
                           float limit, int T, int E, int tile_rows, bool cached, hipStream_t s) {
+  if (!w1_scale)
+    return launch_bf16_gate_up(x, w1, b1g, b1u, d, act, H, IM, limit, T, E, tile_rows,
+                               gemm_streams_weights(T, E, false, cached), s);
   return launch_gemm<true>(x, w1, w1_scale, b1g, b1u, d, act, H, IM, limit, T, E, tile_rows, cached, s);
 }
 
 hipError_t launch_down(const uint16_t *act, const void *w2, const uint16_t *w2_scale, const float *b2,
                        const DispatchBuffers &d, float *y, int H, int IM, int T, int E, int tile_rows,
                        bool cached, hipStream_t s) {
+  if (!w2_scale)
+    return launch_bf16_down(act, w2, b2, d, y, H, IM, T, E, tile_rows, gemm_streams_weights(T, E, false, cached), s);
   return launch_gemm<false>(act, w2, w2_scale, b2, nullptr, d, y, IM, H, 0.f, T, E, tile_rows, cached, s);
 }
 

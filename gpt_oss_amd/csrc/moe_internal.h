@@ -227,6 +227,13 @@ hipError_t launch_gate_up(const uint16_t *x, const void *w1, const uint16_t *w1_
 hipError_t launch_down(const uint16_t *act, const void *w2, const uint16_t *w2_scale, const float *b2,
                        const DispatchBuffers &d, float *y, int H, int IM, int T, int E, int tile_rows,
                        bool cached, hipStream_t s);
+// bf16 weights (gemm_bf16.hip; launch_gate_up and launch_down call them), a plan of either height.
+// stream: weights past the caches.
+hipError_t launch_bf16_gate_up(const uint16_t *x, const void *w1, const float *b1g, const float *b1u,
+                               const DispatchBuffers &d, uint16_t *act, int H, int IM, float limit, int T, int E,
+                               int tile_rows, bool stream, hipStream_t s);
+hipError_t launch_bf16_down(const uint16_t *act, const void *w2, const float *b2, const DispatchBuffers &d, float *y,
+                            int H, int IM, int T, int E, int tile_rows, bool stream, hipStream_t s);
 // tiles: row tiles, at most (stream_direct_tile_cap with ids.topk_i, otherwise stream_tile_cap).
 // T, E: tokens and experts of the batch, the same for both (the order of act between them follows from these).
 // cached: kCachedWeightBytes.

@@ -103,3 +103,62 @@ def test_sides_of_the_lines(n_experts, IM, T):
     d = got[0][rows] - want
     assert np.abs(d).max() <= 2e-2 * max(1.0, float(np.abs(want).max()))
     assert np.linalg.norm(d) <= 1e-3 * np.linalg.norm(want)
+
+
+@pytest.mark.parametrize("H,IM", [(64, 64), (256, 320), (448, 64), (320, 384), (576, 448)])
+def test_reduction_depths(H, IM):
+    """Reductions of 1 to 9 double steps of 64, shorter and longer than the rings of
+    the loads in front of them, under row tiles of 1 to 8 blocks and full, three-quarter,
+    half and quarter column tiles: the weight formats bit for bit, and the oracle."""
+    rng = np.random.default_rng(H + IM)
+    rows = rng.permutation([1, 33, 65, 97, 129, 161, 193, 225, 256, 300, 385, 15])
+    n_experts = len(rows)
+    ids = np.repeat(np.arange(n_experts), rows).astype(np.int32)
+    T = -(-len(ids) // 4)
+    ids = rng.permutation(np.concatenate([ids, np.full(4 * T - len(ids), -1, np.int32)])).reshape(T, 4)
+    tv = rng.random((T, 4)).astype(np.float32)
+    sh = synth.LayerShape("depths", T, H, IM, n_experts)
+    x = synth.round_bf16(synth.make_activations(sh))
+    wr, br = (synth.round_bf16(a) for a in synth.make_router(sh))
+    b1k, s1, b1, b2k, s2, b2 = synth.make_experts_mxfp4(sh)
+    b1, b2 = synth.round_bf16(b1), synth.round_bf16(b2)
+    w1, w2 = ob.mxfp4_dequant(b1k, s1), ob.mxfp4_dequant(b2k, s2)
+    dx, dti = abi.DevBuf.from_numpy(synth.to_bf16_bits(x)), abi.DevBuf.from_numpy(ids)
+    dtv, dout = abi.DevBuf.from_numpy(tv), abi.DevBuf(T * H * 4)
+    got = []
+    for fp4 in (True, False):
+        m = abi.Moe(H, IM, n_experts, max_tokens=T, swiglu_limit=sh.limit)
+        if fp4:
+            m.upload_layer_mxfp4(0, wr, br, b1k, s1, b1, b2k, s2, b2)
+        else:
+            m.upload_layer(0, wr, br, w1, b1, w2, b2)
+        for _ in range(3):
+            dout.memset(0xFF)
+            m.experts(0, dx, None, dti, dtv, T, dout)
+            abi.sync()
+            got.append(dout.download((T, H), np.float32))
+        m.close()
+    # a handle with layers of both formats: the dispatch plans tiles of 256 rows for either
+    m = abi.Moe(H, IM, n_experts, max_tokens=T, swiglu_limit=sh.limit, layers=2)
+    m.upload_layer_mxfp4(0, wr, br, b1k, s1, b1, b2k, s2, b2)
+    m.upload_layer(1, wr, br, w1, b1, w2, b2)
+    for layer in (0, 1):
+        dout.memset(0xFF)
+        m.dispatch(dti, None, T)
+        m.expert_gemms(layer, dx, T)
+        m.combine(dtv, None, T, dout)
+        abi.sync()
+        got.append(dout.download((T, H), np.float32))
+    m.close()
+    for other in got[1:]:
+        assert np.array_equal(got[0], other)
+    some = np.unique(np.concatenate([np.nonzero((ids == e).any(1))[0][[0, -1]] for e in range(n_experts)]))
+    want = np.zeros((len(some), H), np.float32)
+    for i, t in enumerate(some):
+        for k, e in enumerate(ids[t]):
+            if e >= 0:
+                want[i] += tv[t, k] * ob.expert_token(x[t], w1[e], b1[e], w2[e], b2[e], sh.limit,
+                                                      mode=ob.ROUND_ACT_BF16)
+    d = got[0][some] - want
+    assert np.abs(d).max() <= 2e-2 * max(1.0, float(np.abs(want).max()))
+    assert np.linalg.norm(d) <= 1e-3 * np.linalg.norm(want)
