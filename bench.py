@@ -34,6 +34,7 @@ sys.path.insert(0, ROOT)
 # copies of kDirectTokens and kStreamMeanRows in moe_internal.h (stream_batch), to name the
 # kernel of a batch; tests/test_abi_host.py compares them
 STREAM_TOKENS, STREAM_MEAN_ROWS = 64, 16
+FP4_MANY_ROWS = 64  # and MXFP4 weights with this many rows per expert those of gemm_fp4.hip
 PEAK_BF16_TFLOPS = 2500.0  # MI355X dense bf16 MFMA
 PEAK_HBM_GBS = 8000.0
 SETTLE_STEPS = 200  # untimed calls in front of the warm-up steps, see run_leg
@@ -274,7 +275,8 @@ def main():
     mfma_tflops = flops_gate_up / t_gate_up / 1e12
     hbm_gbs = bytes_gate_up / t_gate_up / 1e9
     kernel = "%s<gate_up%s>" % ("stream_gemm_kernel" if T <= STREAM_TOKENS or T * K <= STREAM_MEAN_ROWS * E
-                                else "grouped_gemm_kernel" if mxfp4 else "bf16_gemm_kernel", ", MXFP4" if mxfp4 else "")
+                                else "bf16_gemm_kernel" if not mxfp4 else
+                                "fp4_gemm_kernel" if T * K >= FP4_MANY_ROWS * E else "grouped_gemm_kernel", ", MXFP4" if mxfp4 else "")
     if BOUND[shape.name] == "mfma":
         roofline = {"bound": "mfma", "kernel": kernel, "achieved": mfma_tflops, "peak": PEAK_BF16_TFLOPS,
                     "unit": "TFLOP/s", "frac": mfma_tflops / PEAK_BF16_TFLOPS}

@@ -200,14 +200,27 @@ inline int stream_direct_tile_cap(int T, int E) {
   return (A < E ? A : E) + A / (kRowBlock + 1);
 }
 inline int gemm_tile_cap(int T, int E, int tile_rows) { return T * kTopK / tile_rows + E; }
-// Height of the row tiles of a batch on MXFP4 weights (CfgHalf in gemm.hip has the
-// reason and times): half height where that gives the GPU its two workgroups per
-// CU.  With fewer tiles than that the full height keeps more columns' worth of work
-// in each (8 experts, 256 tokens: 93 us per layer call at full height, 104 at half;
-// 768 tokens, above the line: 183 / 181).
-inline bool half_tiles(int T, int E, int n_ct_gate_up) {
+// MXFP4 weights: whether the kernels of gemm_fp4.hip (tiles of 128 rows, products of 16 x 16
+// x 32) run rather than those of gemm.hip (128 or 256 rows, 32 x 32 x 16).  They do where
+// the products are the time: many rows per expert on average, of all experts.  us per layer call at 2880
+// x 2880, gemm.hip / gemm_fp4.hip: 32 experts, 150 tokens (19 rows) 120 / 125, 256 (32) 136 / 138,
+// 512 (64) 174 / 162; 16 experts, 300 (75) 107 / 105, 450 (112) 135 / 122; 128 experts, 600 (19) 385 /
+// 397, 3072 (96) 688 / 655.  With a workgroup on every CU or fewer, a wave has its SIMD to
+// itself and the smaller products' instructions show until experts have more than one tile:
+// 8 experts, 150 tokens (75 rows) 70 / 76, 256 (128) 93 / 99, 300 (150) 105 / 100, 400 128 / 115; 4
+// experts, 100 (100) 78 / 86, 150 (150) 88 / 75.  w1_rows: rows of an expert's gate_up matrix.
+constexpr int kFp4ManyRows = 64;
+inline bool fp4_many_rows(int T, int E, int w1_rows) {
+  const int n_ct = (w1_rows / kRowBlock + kGemmTileNb - 1) / kGemmTileNb;
+  return T * kTopK > kHalfTileRows * E || (T * kTopK >= kFp4ManyRows * E && E * n_ct > kCus);
+}
+// Height of the row tiles of a batch on MXFP4 weights: half where the kernels of gemm_fp4.hip run,
+// and where it gives the GPU two workgroups per CU (CfgHalf in gemm.hip has the reason).  With
+// fewer tiles than that the full height keeps more columns' worth of work in each.
+inline bool half_tiles(int T, int E, int w1_rows) {
+  const int n_ct = (w1_rows / kRowBlock + kGemmTileNb - 1) / kGemmTileNb;
   const int row_tiles = T * kTopK / kHalfTileRows > E ? T * kTopK / kHalfTileRows : E;
-  return (long long)row_tiles * n_ct_gate_up >= 2 * kCus;
+  return fp4_many_rows(T, E, w1_rows) || (long long)row_tiles * n_ct >= 2 * kCus;
 }
 // Expert matrices up to this many bytes, over all layers of a handle, are read through
 // the caches whatever the batch: they then stay in the 256 MB memory-side cache from
@@ -234,6 +247,12 @@ hipError_t launch_bf16_gate_up(const uint16_t *x, const void *w1, const float *b
                                int tile_rows, bool stream, hipStream_t s);
 hipError_t launch_bf16_down(const uint16_t *act, const void *w2, const float *b2, const DispatchBuffers &d, float *y,
                             int H, int IM, int T, int E, int tile_rows, bool stream, hipStream_t s);
+// MXFP4 weights with many rows per expert (gemm_fp4.hip; likewise), a plan of kHalfTileRows.
+hipError_t launch_fp4_gate_up(const uint16_t *x, const void *w1, const uint16_t *w1_scale, const float *b1g,
+                              const float *b1u, const DispatchBuffers &d, uint16_t *act, int H, int IM, float limit,
+                              int T, int E, bool stream, hipStream_t s);
+hipError_t launch_fp4_down(const uint16_t *act, const void *w2, const uint16_t *w2_scale, const float *b2,
+                           const DispatchBuffers &d, float *y, int H, int IM, int T, int E, bool stream, hipStream_t s);
 // tiles: row tiles, at most (stream_direct_tile_cap with ids.topk_i, otherwise stream_tile_cap).
 // T, E: tokens and experts of the batch, the same for both (the order of act between them follows from these).
 // cached: kCachedWeightBytes.
