@@ -671,13 +671,13 @@ static_assert(CfgFull::RBT_MAX * kRowBlock == kTileRows && CfgHalf::RBT_MAX * kR
 // most experts have one row tile their weights are read by one workgroup, and
 // lines that nobody reads again push the rows and the code out of L2.  us per
 // layer call, cached / past the caches: bf16 (tiles of 256 rows), 32 experts, 256
-// tokens 330 / 305, 512: 364 / 351, 1024: 392 / 374, 1536: 447 / 434; 128 experts,
-// 1024: 1234 / 1173, 6144 (192 rows per expert): 1639 / 1651; 8 experts, 256:
-// 143 / 135, 1024 (512 rows): 254 / 269.  MXFP4 (tiles of 128 rows), 32 experts,
-// 256 tokens 143 / 135, 512: 172 / 163, 1024 (128 rows): 242 / 245, 4096: 725 /
-// 750; 128 experts, 3072 (96 rows): 676 / 668.  MXFP4 in tiles of 256 rows gains
+// tokens 330 / 305, 512: 364 / 351, 1024: 392 / 374, 1536 (192 rows per expert): 433 / 414, 2048
+// (256): 525 / 512, 2560: 603 / 607, 4096: 831 / 845; 128 experts, 1024: 1234 / 1173, 6144 (192): 1631 /
+// 1632; 8 experts, 400 (200): 159 / 153, 600 (300): 191 / 195, 1000: 242 / 244.  Tiles of 128 rows
+// (measured with MXFP4), 32 experts, 256 tokens 143 / 135, 512: 172 / 163, 1024 (128 rows): 242 / 245,
+// 4096: 725 / 750; 128 experts, 3072 (96 rows): 676 / 668.  MXFP4 in tiles of 256 rows gains
 // nothing (8 experts, 256 tokens 93 / 95).  cached: kCachedWeightBytes.
-constexpr int kStreamRowsFull = 160, kStreamRowsHalf = 96;  // mean rows of an expert, at most
+constexpr int kStreamRowsFull = 256, kStreamRowsHalf = 96;  // mean rows of an expert, at most
 static bool gemm_streams_weights(int T, int E, bool half, bool cached) {
   if (cached) return false;
   return T * kTopK <= (half ? kStreamRowsHalf : kStreamRowsFull) * E;
@@ -711,7 +711,7 @@ hipError_t launch_gate_up(const uint16_t *x, const void *w1, const uint16_t *w1_
                           float limit, int T, int E, int tile_rows, bool cached, hipStream_t s) {
   if (!w1_scale)
     return launch_bf16_gate_up(x, w1, b1g, b1u, d, act, H, IM, limit, T, E, tile_rows,
-                               gemm_streams_weights(T, E, false, cached), s);
+                               gemm_streams_weights(T, E, tile_rows == kHalfTileRows, cached), s);
   if (tile_rows == kHalfTileRows && fp4_many_rows(T, E, 2 * IM))
     return launch_fp4_gate_up(x, w1, w1_scale, b1g, b1u, d, act, H, IM, limit, T, E,
                               gemm_streams_weights(T, E, true, cached), s);
@@ -722,7 +722,7 @@ hipError_t launch_down(const uint16_t *act, const void *w2, const uint16_t *w2_s
                        const DispatchBuffers &d, float *y, int H, int IM, int T, int E, int tile_rows,
                        bool cached, hipStream_t s) {
   if (!w2_scale)
-    return launch_bf16_down(act, w2, b2, d, y, H, IM, T, E, tile_rows, gemm_streams_weights(T, E, false, cached), s);
+    return launch_bf16_down(act, w2, b2, d, y, H, IM, T, E, tile_rows, gemm_streams_weights(T, E, tile_rows == kHalfTileRows, cached), s);
   if (tile_rows == kHalfTileRows && fp4_many_rows(T, E, 2 * IM))
     return launch_fp4_down(act, w2, w2_scale, b2, d, y, H, IM, T, E, gemm_streams_weights(T, E, true, cached), s);
   return launch_gemm<false>(act, w2, w2_scale, b2, nullptr, d, y, IM, H, 0.f, T, E, tile_rows, cached, s);

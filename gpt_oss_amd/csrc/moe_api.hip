@@ -146,7 +146,8 @@ inline int down_col_tiles(const moe_handle *h) {
 // bf16 weights take a plan of either height (a caller may dispatch before it names the layer).
 int run_dispatch(moe_handle *h, const int *topk_i, const int *pos, int T, bool mxfp4, hipStream_t s) {
   const int E = h->cfg.experts;
-  h->plan_rows = mxfp4 && half_tiles(T, E, 2 * h->IMp) ? kHalfTileRows : kTileRows;
+  const bool half = mxfp4 ? half_tiles(T, E, 2 * h->IMp) : bf16_half_tiles(T, E, h->Hp, h->IMp);
+  h->plan_rows = half ? kHalfTileRows : kTileRows;
   // the kernels of stream.hip go by row blocks and need no tile tables
   const bool tables = !stream_batch(T, E);
   HIP_TRY(launch_dispatch(topk_i, pos, T, E, tables ? gate_up_col_tiles(h) : 0, tables ? down_col_tiles(h) : 0,

@@ -222,6 +222,29 @@ inline bool half_tiles(int T, int E, int w1_rows) {
   const int row_tiles = T * kTopK / kHalfTileRows > E ? T * kTopK / kHalfTileRows : E;
   return fp4_many_rows(T, E, w1_rows) || (long long)row_tiles * n_ct >= 2 * kCus;
 }
+// bf16 weights: whether row tiles of 128 rows in place of 256 are expected to be quicker.  They stream an
+// expert's weights more often, so they pay only where the tall tiles leave CUs without work, in either
+// GEMM.  The estimate: an expert has half a tile more than its rows fill on average; a tile takes the time of 4
+// + (its row blocks) steps of its reduction; the CUs take tiles in rounds.  us per layer call, 256 rows / 128:
+// 4 experts, 2880 x 2880, 150 tokens 89 / 71; 4 experts, 1024 x 2048, 500 tokens 85 / 62; 512 x 512, 8 experts,
+// 1000 tokens 51 / 43, 32 experts, 700 tokens 50 / 45; 256 x 1440, 32 experts, 1000 tokens, Zipf's
+// routing 72 / 60.  Where the estimate says 256 rows: 8 experts, 2880 x 2880, 256 tokens 129 / 152, 400 156 /
+// 162, 600 182 / 215; 16 experts, 700 tokens 240 / 266; 8 experts, 512 x 512, 7000 tokens 92 / 96 (3000, a
+// close call, 59 / 56).  128 rows have to be a tenth quicker by the estimate.
+inline bool bf16_half_tiles(int T, int E, int H, int IM) {
+  const int A = T * kTopK;
+  const float blocks = (float)A / kRowBlock + 0.5f * E;
+  auto time = [&](int tile_rows) {
+    float tiles = (float)A / tile_rows + 0.5f * E;
+    if (tiles < E) tiles = (float)E;
+    auto rounds = [&](int cols) {
+      const int n = (int)(tiles * ((cols / kRowBlock + kGemmTileNb - 1) / kGemmTileNb));
+      return (float)((n + kCus - 1) / kCus);
+    };
+    return (4.f + blocks / tiles) * (H * rounds(2 * IM) + IM * rounds(H));
+  };
+  return time(kHalfTileRows) < 0.9f * time(kTileRows);
+}
 // Expert matrices up to this many bytes, over all layers of a handle, are read through
 // the caches whatever the batch: they then stay in the 256 MB memory-side cache from
 // one call to the next, which loads past the caches do not use.  us per moe_experts

@@ -72,11 +72,11 @@ def test_row_tiles(rows, H, IM):
 
 
 @pytest.mark.parametrize("n_experts,IM,T", [(16, 2880, 735), (16, 2880, 736), (32, 2048, 768), (32, 2048, 769),
-                                            (32, 2048, 1280), (32, 2048, 1281)])
+                                            (32, 2048, 1280), (32, 2048, 1281), (32, 2048, 2048), (32, 2048, 2049)])
 def test_sides_of_the_lines(n_experts, IM, T):
     """Either side of the line to tiles of 128 rows (MXFP4, 16 experts, 23 column
     tiles: 736 tokens) and of the lines up to which weights that exceed 256 MiB are
-    read past the caches (96 rows per expert in tiles of 128, 160 in tiles of 256):
+    read past the caches (96 rows per expert in tiles of 128, 256 in tiles of 256):
     the two weight formats bit for bit, and the oracle."""
     H = 64
     sh = synth.LayerShape("lines", T, H, IM, n_experts)
@@ -160,5 +160,45 @@ def test_reduction_depths(H, IM):
                 want[i] += tv[t, k] * ob.expert_token(x[t], w1[e], b1[e], w2[e], b2[e], sh.limit,
                                                       mode=ob.ROUND_ACT_BF16)
     d = got[0][some] - want
+    assert np.abs(d).max() <= 2e-2 * max(1.0, float(np.abs(want).max()))
+    assert np.linalg.norm(d) <= 1e-3 * np.linalg.norm(want)
+
+
+@pytest.mark.parametrize("n_experts,H,IM,T", [(16, 64, 2880, 255), (16, 64, 2880, 256), (8, 64, 2880, 256), (8, 64, 2880, 257),
+                                              (8, 512, 512, 1927), (8, 512, 512, 1928), (8, 512, 512, 3856)])
+def test_sides_of_the_product_lines(n_experts, H, IM, T):
+    """Either side of the lines between the products of the MXFP4 kernels (64 rows per
+    expert, and 128 where there is at most a workgroup per CU) and between row tiles of 128
+    and 256 rows under bf16 weights: the two weight formats, which cross none of these
+    together, bit for bit, stage by stage as well, and the oracle."""
+    sh = synth.LayerShape("products", T, H, IM, n_experts)
+    x = synth.round_bf16(synth.make_activations(sh))
+    wr, br = (synth.round_bf16(a) for a in synth.make_router(sh))
+    b1k, s1, b1, b2k, s2, b2 = synth.make_experts_mxfp4(sh)
+    b1, b2 = synth.round_bf16(b1), synth.round_bf16(b2)
+    w1, w2 = ob.mxfp4_dequant(b1k, s1), ob.mxfp4_dequant(b2k, s2)
+    dx = abi.DevBuf.from_numpy(synth.to_bf16_bits(x))
+    dti, dtv, dout = abi.DevBuf(T * 16), abi.DevBuf(T * 16), abi.DevBuf(T * H * 4)
+    got = []
+    for fp4 in (True, False):
+        m = abi.Moe(H, IM, n_experts, max_tokens=T, swiglu_limit=sh.limit)
+        if fp4:
+            m.upload_layer_mxfp4(0, wr, br, b1k, s1, b1, b2k, s2, b2)
+        else:
+            m.upload_layer(0, wr, br, w1, b1, w2, b2)
+        got.append(abi.run_layer(m, 0, x, None)["out"])
+        m.router(0, dx, None, T, None, dti, dtv)
+        m.dispatch(dti, None, T)
+        m.expert_gemms(0, dx, T)
+        m.combine(dtv, None, T, dout)
+        abi.sync()
+        got.append(dout.download((T, H), np.float32))
+        m.close()
+    for other in got[1:]:
+        assert np.array_equal(got[0], other)
+    rows = np.arange(0, T, max(1, T // 15))
+    want = ob.moe_layer(np.ascontiguousarray(x[rows]), None, wr, br, w1, b1, w2, b2, 4, sh.limit,
+                        mode=ob.ROUND_ACT_BF16 | ob.PAR_TOKENS)
+    d = got[0][rows] - want
     assert np.abs(d).max() <= 2e-2 * max(1.0, float(np.abs(want).max()))
     assert np.linalg.norm(d) <= 1e-3 * np.linalg.norm(want)
