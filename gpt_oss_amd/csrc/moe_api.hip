@@ -155,6 +155,12 @@ int run_dispatch(moe_handle *h, const int *topk_i, const int *pos, int T, bool m
   return MOE_OK;
 }
 
+// Scratch of the router inside a whole-layer call: the down GEMM's rows, which are written later in the
+// same call.  (moe_router has none: calls of it on several streams may overlap.)
+float *router_scratch(const moe_handle *h, int T) {
+  return (size_t)T * (h->E_pad + 4) <= (size_t)h->a_pad_cap * h->Hp ? h->y : nullptr;
+}
+
 // Stages 3-4 on the plan of the last dispatch: gate_up GEMM with the SwiGLU (it
 // reads the routed token rows itself, there is no gathered copy), down GEMM.
 // Leaves the per-assignment rows in h->y.
@@ -476,7 +482,7 @@ int moe_router(moe_handle *h, int layer, const uint16_t *x, const int *pos, int 
   if (n_tokens == 0) return MOE_OK;
   const LayerWeights &lw = h->layers[layer];
   HIP_TRY(launch_router(x, pos, lw.wr, lw.br, lw.br + h->E_pad, n_tokens, h->cfg.hidden, h->cfg.experts,
-                        h->E_pad, score, topk_i, topk_v, static_cast<hipStream_t>(stream)));
+                        h->E_pad, score, topk_i, topk_v, nullptr, static_cast<hipStream_t>(stream)));
   return MOE_OK;
 }
 
@@ -574,7 +580,7 @@ int moe_forward(moe_handle *h, int layer, const uint16_t *x, const int *pos, int
   StageTimer tm(h, s);
   HIP_TRY(tm.mark(MOE_STAGE_ROUTER));
   HIP_TRY(launch_router(x, pos, lw.wr, lw.br, lw.br + h->E_pad, n_tokens, h->cfg.hidden, h->cfg.experts,
-                        h->E_pad, nullptr, h->topk_i, h->topk_v, s));
+                        h->E_pad, nullptr, h->topk_i, h->topk_v, router_scratch(h, n_tokens), s));
   rc = run_experts(h, layer, x, pos, h->topk_i, h->topk_v, n_tokens, n_tokens, out, accumulate, s, tm);
   if (rc == MOE_OK) tm.done();
   return rc;
@@ -622,7 +628,7 @@ int moe_block_forward(moe_handle *h, int layer, uint16_t *x, const int *pos, int
   HIP_TRY(tm.mark(MOE_STAGE_ROUTER));  // the norm is counted with the router stage
   HIP_TRY(launch_rmsnorm(x, lw.rms_w, pos, h->t_norm, n_tokens, h->cfg.hidden, s));
   HIP_TRY(launch_router(h->t_norm, pos, lw.wr, lw.br, lw.br + h->E_pad, n_tokens, h->cfg.hidden,
-                        h->cfg.experts, h->E_pad, nullptr, h->topk_i, h->topk_v, s));
+                        h->cfg.experts, h->E_pad, nullptr, h->topk_i, h->topk_v, router_scratch(h, n_tokens), s));
   rc = run_experts(h, layer, h->t_norm, pos, h->topk_i, h->topk_v, n_tokens, n_tokens, nullptr, 0, s, tm,
                    x);
   if (rc == MOE_OK) tm.done();

@@ -124,9 +124,13 @@ hipError_t launch_pad_rows(const uint16_t *x, uint16_t *xp, int T, int H, int Hp
 // bound that decides which tokens need exact fp64 logits.
 hipError_t launch_router_stats(const float *w_src, const float *b_src, int E, int H, float *rstat,
                                hipStream_t s);
+// first: scratch for T * (E_pad + 4) floats that no other call uses meanwhile, or nullptr.  With it, batches of up to
+// kSplitRouterTokens tokens at more than 64 experts run the first pass on E_pad / 16 times as many
+// workgroups and a launch of their own; the results are the same bits.
+constexpr int kSplitRouterTokens = 1024;
 hipError_t launch_router(const uint16_t *x, const int *pos, const uint16_t *wr, const float *br,
                          const float *rstat, int T, int H, int E, int E_pad, float *score, int *topk_i,
-                         float *topk_v, hipStream_t s);
+                         float *topk_v, float *first, hipStream_t s);
 
 struct DispatchBuffers {
   int *blk_counts;    // [n_blk, E]

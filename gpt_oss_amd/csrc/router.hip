@@ -164,11 +164,16 @@ __device__ __forceinline__ void unpack8(const uint4 v, float (&f)[8]) {
 // Its WPC waves split the reduction dimension in chunks of 32 (wave w takes
 // chunks w, w + WPC, ...); D register sets of loads run ahead of the MFMAs.
 // rstat[0] = max_e |w_e| (slightly inflated), rstat[1] = max_e |b_e|.
-template <int NT, int WPC, int MT, int D, int FLUSH>
+//
+// SPLIT: the first pass has run (router_logits_kernel), `first` holds its logits
+// [T][E_pad], then its partial sums of squares [T][kSplitWaves].
+constexpr int kSplitWaves = 4;
+template <int NT, int WPC, int MT, int D, int FLUSH, bool SPLIT>
 __global__ __launch_bounds__(WPC * 64) void router_kernel(
     const uint16_t *__restrict__ x, const int *__restrict__ pos, const uint16_t *__restrict__ wr,
     const float *__restrict__ br, const float *__restrict__ rstat, int T, int H, int E,
-    float *__restrict__ score, int *__restrict__ topk_i, float *__restrict__ topk_v) {
+    float *__restrict__ score, int *__restrict__ topk_i, float *__restrict__ topk_v,
+    const float *__restrict__ first) {
   constexpr int E_pad = NT * 16;
   constexpr int TOK = MT * 16;
   // selection: LPT lanes per token, each owning PER experts; SW waves take part.
@@ -183,8 +188,9 @@ __global__ __launch_bounds__(WPC * 64) void router_kernel(
   constexpr int NBLK = MT * NT;
   constexpr int GB = 32 / WPC < NBLK ? 32 / WPC : NBLK;
   static_assert(WPC >= 2 && NBLK % GB == 0, "groups of the cross-wave sum");
-  __shared__ double part[WPC / 2][GB][4][64];  // [wave][block][reg][lane]
-  __shared__ float sumsq[WPC][TOK];
+  __shared__ double part[SPLIT ? 1 : WPC / 2][GB][4][64];  // [wave][block][reg][lane]
+  constexpr int SQ = SPLIT ? kSplitWaves : WPC;
+  __shared__ float sumsq[SQ][TOK];
   __shared__ __attribute__((aligned(16))) float logits[TOK][LOG_LD];
   __shared__ float posted[RANKED ? TOK : 1][2 * (kTopK + 1)];  // ranked_top's lists
   __shared__ unsigned short tasks[TOK * E_pad];  // (token in tile) * E_pad + expert
@@ -207,6 +213,16 @@ __global__ __launch_bounds__(WPC * 64) void router_kernel(
   const bool active = w < SW && t < T && !(pos && pos[min(t, T - 1)] < 0);
   const float wn_max = rstat[0], bmax = rstat[1];
 
+  if constexpr (SPLIT) {
+    // rows of tokens past the batch are not looked at
+    for (int idx = tid; idx < TOK * E_pad / 4; idx += WPC * 64) {
+      const int tt = idx / (E_pad / 4), e = idx % (E_pad / 4) * 4;
+      const float4 f = *reinterpret_cast<const float4 *>(first + (size_t)min(tok0 + tt, T - 1) * E_pad + e);
+      logits[tt][e] = f.x; logits[tt][e + 1] = f.y; logits[tt][e + 2] = f.z; logits[tt][e + 3] = f.w;
+    }
+    if (tid < TOK * SQ) sumsq[tid % SQ][tid / SQ] = first[(size_t)T * E_pad + (size_t)min(tok0 + tid / SQ, T - 1) * SQ + tid % SQ];
+    __syncthreads();
+  } else {
   f32x4 acc32[MT][NT], nrm[MT];
   double acc64[MT][NT][4];
 #pragma unroll
@@ -315,6 +331,7 @@ __global__ __launch_bounds__(WPC * 64) void router_kernel(
     }
     __syncthreads();
   }
+  }
 
   // Pass 2, selection: LPT lanes per token.
   bool undecided = false;
@@ -334,7 +351,7 @@ __global__ __launch_bounds__(WPC * 64) void router_kernel(
     if (active) {
       float ss = 0.f;
 #pragma unroll
-      for (int ww = 0; ww < WPC; ww++) ss += sumsq[ww][tr];
+      for (int ww = 0; ww < SQ; ww++) ss += sumsq[ww][tr];
       // bound on |first-pass logit - exact logit|: the accumulation error plus
       // the two float roundings (sum -> float, + bias) of either arithmetic
       const float err0 = router_gamma(FLUSH) * sqrtf(ss * 1.002f) * wn_max;
@@ -460,6 +477,76 @@ __global__ __launch_bounds__(WPC * 64) void router_kernel(
   }
 }
 
+// The first pass of router_kernel<., 4, 1, ., 1> with a workgroup per 16 tokens and BLOCK of 16
+// experts: with all 128 or 256 experts to a workgroup one CU takes in the whole router
+// matrix (0.74 MB at 128 experts and 2880 columns, 12 us and more), and a small batch has few
+// of them.  The same chunks to the same four waves and the same order of the sums: the same
+// bits.  Written to `first` (see SPLIT), which a second launch reads.  us at 128 experts and
+// 2880 columns, one kernel / both launches: 6 tokens 16.7 / 5.0 + 6.3, 200 tokens 32.5 / 7.7 + 17.2 (the
+// rest is the second pass of a few undecided tokens).
+template <int D>
+__global__ __launch_bounds__(kSplitWaves * 64) void router_logits_kernel(
+    const uint16_t *__restrict__ x, const uint16_t *__restrict__ wr, const float *__restrict__ br, int T, int H,
+    int E_pad, float *__restrict__ first) {
+  __shared__ double part[kSplitWaves / 2][4][64];
+  const int tid = threadIdx.x;
+  const int lane = tid & 63, w = tid >> 6;
+  const int row = lane & 15, g = lane >> 4;
+  const int tok0 = blockIdx.x * 16, n = blockIdx.y;
+  const int kc_total = H / 32;
+  const float bias = br[16 * n + row];
+  const uint16_t *xrow = x + (size_t)min(tok0 + row, T - 1) * H + g * 8;
+  const uint16_t *wlane = wr + ((size_t)n * kc_total * 64 + lane) * 8;
+  f32x4 nrm = {0.f, 0.f, 0.f, 0.f};
+  double acc64[4] = {0.0, 0.0, 0.0, 0.0};
+  uint4 xs[D], wq[D];
+  auto load = [&](int d, int c) {
+    const int cc = min(c, kc_total - 1);  // only the first D loads of a wave can lie past the end
+    xs[d] = *reinterpret_cast<const uint4 *>(xrow + cc * 32);
+    wq[d] = *reinterpret_cast<const uint4 *>(wlane + (size_t)cc * 512);
+  };
+#pragma unroll
+  for (int d = 0; d < D; d++) load(d, w + d * kSplitWaves);
+  for (int c0 = w; c0 < kc_total; c0 += D * kSplitWaves) {
+#pragma unroll
+    for (int d = 0; d < D; d++) {
+      const int c = c0 + d * kSplitWaves;
+      if (c < kc_total) {  // the same for the whole wave
+        const bf16x8 xa = __builtin_bit_cast(bf16x8, xs[d]);
+        const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+        const f32x4 p = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa, __builtin_bit_cast(bf16x8, wq[d]), zero, 0, 0, 0);
+        nrm = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa, xa, nrm, 0, 0, 0);
+        if (c + D * kSplitWaves < kc_total) load(d, c + D * kSplitWaves);
+#pragma unroll
+        for (int i = 0; i < 4; i++) acc64[i] += (double)p[i];
+      }
+    }
+  }
+  if (n == 0 && (row >> 2) == g && tok0 + row < T) {
+    const int i = row & 3;
+    first[(size_t)T * E_pad + (size_t)(tok0 + row) * kSplitWaves + w] =
+        i == 0 ? nrm[0] : (i == 1 ? nrm[1] : (i == 2 ? nrm[2] : nrm[3]));
+  }
+  if (w >= kSplitWaves / 2) {
+#pragma unroll
+    for (int i = 0; i < 4; i++) part[w - kSplitWaves / 2][i][lane] = acc64[i];
+  }
+  __syncthreads();
+  if (w < kSplitWaves / 2) {
+#pragma unroll
+    for (int i = 0; i < 4; i++) part[w][i][lane] += acc64[i];
+  }
+  __syncthreads();
+  // thread -> register w of lane l: token 4 * (l / 16) + w, expert 16 n + l % 16
+  double sd = 0.0;
+#pragma unroll
+  for (int ww = 0; ww < kSplitWaves / 2; ww++) sd += part[ww][w][lane];
+  float f = (float)sd;  // run.cpp:368
+  f += bias;            // run.cpp:669-671
+  const int t = tok0 + 4 * g + w;
+  if (t < T) first[(size_t)t * E_pad + 16 * n + row] = f;
+}
+
 // Statistics of a layer's router for the error bound of the first pass:
 // rstat[0] = max_e |w_e|_2 over the bf16-rounded weights (inflated by 1e-3 for
 // the rounding of this very sum), rstat[1] = max_e |b_e|.  One workgroup.
@@ -499,7 +586,7 @@ hipError_t launch_router_stats(const float *w_src, const float *b_src, int E, in
 template <int NT>
 static hipError_t launch_router_nt(const uint16_t *x, const int *pos, const uint16_t *wr,
                                    const float *br, const float *rstat, int T, int H, int E,
-                                   float *score, int *topk_i, float *topk_v, hipStream_t s) {
+                                   float *score, int *topk_i, float *topk_v, float *first, hipStream_t s) {
   // As fine a split of the reduction as the registers allow: more waves keep
   // more loads in flight, and small batches still occupy the SIMDs.  D register
   // sets of 4 * (MT + NT) registers each run ahead.
@@ -513,27 +600,36 @@ static hipError_t launch_router_nt(const uint16_t *x, const int *pos, const uint
   // Every workgroup streams the whole router matrix through its CU; at 128
   // experts a workgroup takes two tiles of 16 tokens so that half as many do
   // (at 256 the accumulators of two tiles no longer fit the registers).
+  if constexpr (NT >= 8) {
+    static_assert(WPC == kSplitWaves, "router_logits_kernel adds up what router_kernel does, in its order");
+    if (first && T <= kSplitRouterTokens) {
+      router_logits_kernel<8><<<dim3((T + 15) / 16, NT), kSplitWaves * 64, 0, s>>>(x, wr, br, T, H, NT * 16, first);
+      router_kernel<NT, 8, 1, 1, FLUSH, true><<<(T + 15) / 16, 8 * 64, 0, s>>>(x, pos, wr, br, rstat, T, H, E, score,
+                                                                              topk_i, topk_v, first);
+      return hipGetLastError();
+    }
+  }
   if (NT == 8 && T > 256 * 16) {
     constexpr int MT = NT == 8 ? 2 : 1;
-    router_kernel<NT, WPC, MT, D, FLUSH><<<(T + 16 * MT - 1) / (16 * MT), WPC * 64, 0, s>>>(
-        x, pos, wr, br, rstat, T, H, E, score, topk_i, topk_v);
+    router_kernel<NT, WPC, MT, D, FLUSH, false><<<(T + 16 * MT - 1) / (16 * MT), WPC * 64, 0, s>>>(
+        x, pos, wr, br, rstat, T, H, E, score, topk_i, topk_v, nullptr);
   } else {
-    router_kernel<NT, WPC, 1, D, FLUSH><<<(T + 15) / 16, WPC * 64, 0, s>>>(x, pos, wr, br, rstat, T, H, E,
-                                                                          score, topk_i, topk_v);
+    router_kernel<NT, WPC, 1, D, FLUSH, false><<<(T + 15) / 16, WPC * 64, 0, s>>>(x, pos, wr, br, rstat, T, H, E,
+                                                                                 score, topk_i, topk_v, nullptr);
   }
   return hipGetLastError();
 }
 
 hipError_t launch_router(const uint16_t *x, const int *pos, const uint16_t *wr, const float *br,
                          const float *rstat, int T, int H, int E, int E_pad, float *score, int *topk_i,
-                         float *topk_v, hipStream_t s) {
+                         float *topk_v, float *first, hipStream_t s) {
   if (T <= 0) return hipSuccess;
   switch (E_pad / 16) {
-    case 1: return launch_router_nt<1>(x, pos, wr, br, rstat, T, H, E, score, topk_i, topk_v, s);
-    case 2: return launch_router_nt<2>(x, pos, wr, br, rstat, T, H, E, score, topk_i, topk_v, s);
-    case 4: return launch_router_nt<4>(x, pos, wr, br, rstat, T, H, E, score, topk_i, topk_v, s);
-    case 8: return launch_router_nt<8>(x, pos, wr, br, rstat, T, H, E, score, topk_i, topk_v, s);
-    case 16: return launch_router_nt<16>(x, pos, wr, br, rstat, T, H, E, score, topk_i, topk_v, s);
+    case 1: return launch_router_nt<1>(x, pos, wr, br, rstat, T, H, E, score, topk_i, topk_v, first, s);
+    case 2: return launch_router_nt<2>(x, pos, wr, br, rstat, T, H, E, score, topk_i, topk_v, first, s);
+    case 4: return launch_router_nt<4>(x, pos, wr, br, rstat, T, H, E, score, topk_i, topk_v, first, s);
+    case 8: return launch_router_nt<8>(x, pos, wr, br, rstat, T, H, E, score, topk_i, topk_v, first, s);
+    case 16: return launch_router_nt<16>(x, pos, wr, br, rstat, T, H, E, score, topk_i, topk_v, first, s);
     default: return hipErrorInvalidValue;
   }
 }

@@ -448,3 +448,29 @@ def test_padded_shape_and_split_reduction_replay_from_a_hip_graph(T):
         hip.hipGraphExecDestroy(gexec)
         hip.hipGraphDestroy(graph)
         hip.hipStreamDestroy(stream)
+
+
+@pytest.mark.parametrize("E,H", [(100, 96), (128, 2880), (200, 320)])
+def test_split_router_gives_the_same_bits(E, H):
+    """More than 64 experts: the router of the whole-layer calls runs its first pass as a launch
+    of its own up to 1024 tokens, moe_router in one kernel; ids, weights and so the layer agree bit
+    for bit, on either side of the line, with inactive rows and near ties among the tokens."""
+    for T in (1, 6, 17, 64, 200, 1023, 1024, 1025):
+        sh = synth.LayerShape("r", T, H, 64, E)
+        L = bf16_layer(sh, seed=T)
+        L["w_router"][E // 2] = L["w_router"][3]  # two experts that always tie but for the bias
+        m = make_moe(sh, L, T)
+        m.set_distinct_ids(True)
+        pos = np.zeros(T, np.int32)
+        pos[2::5] = -1
+        base = abi.run_layer(m, 0, L["x"], pos)["out"]
+        dx, dpos = abi.DevBuf.from_numpy(synth.to_bf16_bits(L["x"])), abi.DevBuf.from_numpy(pos)
+        dti, dtv, dout = abi.DevBuf(T * 16), abi.DevBuf(T * 16), abi.DevBuf(T * H * 4)
+        dout.memset(0)
+        m.router(0, dx, dpos, T, None, dti, dtv)
+        m.experts(0, dx, dpos, dti, dtv, T, dout)
+        abi.sync()
+        assert np.array_equal(dout.download((T, H), np.float32), base)
+        ids = dti.download((T, 4), np.int32)
+        assert (ids[pos >= 0] >= 0).all() and (ids[pos < 0] == -1).all()
+        m.close()

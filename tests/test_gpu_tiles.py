@@ -74,8 +74,8 @@ def test_row_tiles(rows, H, IM):
 @pytest.mark.parametrize("n_experts,IM,T", [(16, 2880, 735), (16, 2880, 736), (32, 2048, 768), (32, 2048, 769),
                                             (32, 2048, 1280), (32, 2048, 1281), (32, 2048, 2048), (32, 2048, 2049)])
 def test_sides_of_the_lines(n_experts, IM, T):
-    """Either side of the line to tiles of 128 rows (MXFP4, 16 experts, 23 column
-    tiles: 736 tokens) and of the lines up to which weights that exceed 256 MiB are
+    """Tiles of 128 rows under MXFP4 weights (16 experts, 23 column tiles, 735 and 736
+    tokens) and either side of the lines up to which weights that exceed 256 MiB are
     read past the caches (96 rows per expert in tiles of 128, 256 in tiles of 256):
     the two weight formats bit for bit, and the oracle."""
     H = 64
