@@ -167,7 +167,17 @@ __device__ __forceinline__ int build_plan(int count, int E, int n_ct_gate_up, in
     }
     if (info_out) *info_out = inf;
   }
-  if (!write_global) {  // (the same for the whole workgroup)
+  const bool tables = n_ct_gate_up > 0;
+  if (write_global && !tables && e == 0) {
+    offsets[E] = tot_count;
+    totals[kTotTiles] = tot_mt;
+    totals[kTotRows] = tot_pad;
+    totals[kTotAssign] = tot_count;
+  }
+  // Without column tiles (stream.hip) the XCDs' ranges are of no tiles: their search and its
+  // divisions are left out (us per call, 128 experts, 200 tokens 313.8 / 310.0; 512 x 512, 32 experts, 128
+  // tokens 35.7 / 33.8).
+  if (!write_global || !tables) {  // (the same for the whole workgroup)
     *ex_count_out = ex_count;
     if (tot_count_out) *tot_count_out = tot_count;
     return ex_pad;

@@ -126,7 +126,9 @@ hipError_t launch_router_stats(const float *w_src, const float *b_src, int E, in
                                hipStream_t s);
 // first: scratch for T * (E_pad + 4) floats that no other call uses meanwhile, or nullptr.  With it, batches of up to
 // kSplitRouterTokens tokens at more than 64 experts run the first pass on E_pad / 16 times as many
-// workgroups and a launch of their own; the results are the same bits.
+// workgroups and a launch of their own; the results are the same bits.  us per layer call without / with at 128
+// experts: 16 tokens 127.7 / 122.1, 512 383 / 377, 1024 445 / 441, 1500 473 / 474, 4096 816 / 826; 512 x 512,
+// 2000 tokens 70.6 / 72.9.
 constexpr int kSplitRouterTokens = 1024;
 hipError_t launch_router(const uint16_t *x, const int *pos, const uint16_t *wr, const float *br,
                          const float *rstat, int T, int H, int E, int E_pad, float *score, int *topk_i,
