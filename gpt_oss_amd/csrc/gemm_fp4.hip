@@ -256,9 +256,9 @@ __device__ __forceinline__ void gemm_tile(const uint4 *__restrict__ a_frag,  // 
   for (int n = 0; n < kDecodeParts; n++) decode(0, 0, 0, n);
 
   // Step ks, slot u = ks % R:
-  //   [MFMAs of k block 0 | read row fragments of k block 1, load B(ks+R-1) into slot u-1]
+  //   [first half of the row groups | decode column block 1, read the second half, load B(ks+R-1) into slot u-1]
   //   wait until step ks+1 has arrived, barrier
-  //   [MFMAs of k block 1 | DMA A(ks+R) into stage u, read row fragments of step ks+1]
+  //   [second half | DMA A(ks+R) into stage u, read the first half of step ks+1, decode its column block 0]
   // The side work is spread over the MFMAs so that it issues in their shadow.
   // Every step is the same straight code with the same count in its wait: the
   // refills of the tile's last R-1 steps, for which there is nothing left to
@@ -347,15 +347,13 @@ __device__ __forceinline__ void gemm_tile(const uint4 *__restrict__ a_frag,  // 
 // the main loop a quarter more, and 64 bytes of 16 rows an eighth.
 //
 // So the row operand is staged in double steps: a double stage holds 64 k of
-// all rows of the tile (two 16 KB arrays: row blocks 0-3 and 4-7), R2 of them
-// form the ring, and the refill comes every other step.  Wave w fetches rows
+// all rows of the tile (16 KB), R2 of them form the ring, and the refill comes every other step.  Wave w fetches rows
 // 8w .. 8w+7 of every row block; inside its kilobyte a lane holds one 16-byte
 // piece of one of the 8 rows, and WHICH is chosen so that (a) the four lanes of
-// a quad read 64 contiguous bytes of one row and (b) the MFMA operand reads
-// (lane = row, all lanes the same piece) find 8 consecutive rows on the 8
-// different 16-byte slots of 128 bytes of LDS and 16 consecutive rows on the 16
-// of 256 bytes: quad Q = 4 * (row / 2) + 2 * (half of the line ^ w % 2) + row % 2,
-// and lane j of the quad holds piece (j - row / 2) mod 4 of that half.
+// a quad read 64 contiguous bytes of one row and (b) the MFMA operand reads (16 lanes
+// to a piece of 8 k) find 16 different slots of 256 bytes, whichever of the four pieces'
+// lanes the LDS serves side by side: quad Q = 4 * (row / 2) + 2 * (half of the line ^ w % 2)
+// + row % 2, and lane j of the quad holds piece j ^ (row / 2) of that half.
 //
 // The column operand keeps its ring of RB register slots of one step each.
 // Loads are issued in the order  B(0) B(1) B(2) A2(0) A2(1) A2(2) A2(3) | step 0:

@@ -74,7 +74,7 @@ struct moe_handle {
   // moe_get_dispatch that asks for the plan afterwards.  topk_i == nullptr: none.
   DirectIds unplanned{nullptr, nullptr, 0, 0};
   // expert pipeline
-  uint16_t *act = nullptr;  // SwiGLU output, bf16: fragments (gemm.hip), quads or rows (stream.hip)
+  uint16_t *act = nullptr;  // SwiGLU output, bf16: fragments (gemm*.hip), quads or rows (stream.hip)
   float *y = nullptr;       // down output [a_pad_cap, Hp]
   uint16_t *t_norm = nullptr;  // normalised rows of moe_block_forward [max_tokens, H], allocated on first use
   uint16_t *x_pad = nullptr;   // the batch's rows widened to Hp columns [max_tokens, Hp]; only where Hp != H

@@ -56,7 +56,7 @@ __global__ void pack_weight_kernel(const float *__restrict__ src, uint4 *__restr
 // in its high nibble; a nibble indexes {0, .5, 1, 1.5, 2, 3, 4, 6} and their
 // negatives, and the scale byte s multiplies by 2^(s - 127).  The weights stay
 // in this format on the device, re-ordered for the GEMMs that decode them in
-// registers (gemm_tile with FP4).  Per pair of row blocks (2P, 2P+1) and step of 32 k (one
+// registers (gemm.hip, gemm_fp4.hip, stream.hip).  Per pair of row blocks (2P, 2P+1) and step of 32 k (one
 // MXFP4 block): a 16-byte chunk per lane l = (row n = l % 32, half h = l / 32),
 //   bytes 0-3   row of block 2P,   k block 0: elements 8h .. 8h+7  = source bytes 4h .. 4h+3
 //   bytes 4-7   row of block 2P,   k block 1: elements 16+8h ..    = source bytes 8+4h ..

@@ -1,6 +1,6 @@
 // Grouped expert GEMMs of the batches in which the weights are a stream: few rows
 // per expert, so the time is that of reading the weights once.  Same contract as
-// the kernels of gemm.hip (matmul/matmul.cpp:1023-1914, SwiGLU of run.cpp:709-726).
+// the kernels of gemm.hip, gemm_bf16.hip and gemm_fp4.hip (matmul/matmul.cpp:1023-1914, SwiGLU of run.cpp:709-726).
 //
 // A wave owns a pair of column blocks (64 columns) of one expert and a slice of
 // the reduction, and shares nothing with other waves until its slice is done: the
