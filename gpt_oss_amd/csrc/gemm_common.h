@@ -22,6 +22,18 @@ __device__ __forceinline__ void static_for(F &&f) {
   static_for_impl(f, std::make_integer_sequence<int, N>{});
 }
 
+// f(IC<0>{}), ..., f(IC<left-1>{}) for left <= N, each inside the condition of the one before it: no
+// path leaves out a step in front of one that runs.
+template <int N, int U = 0, typename F>
+__device__ __forceinline__ void static_left(int left, F &&f) {
+  if constexpr (U < N) {
+    if (left > U) {
+      f(IC<U>{});
+      static_left<N, U + 1>(left, f);
+    }
+  }
+}
+
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
