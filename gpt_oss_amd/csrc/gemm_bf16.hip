@@ -57,9 +57,12 @@ static_assert(kTileRows == 8 * kRowBlock && kGemmTileNb == 8, "tile plan of buil
 // ---- 16 bytes per lane from global memory to LDS, lane l at lds + 16 l ----
 // In assembly, because the compiler, which does not know one stage from another here,
 // would make every LDS read wait for all of them.  There is no output register; the
-// waits are the counted ones below and the barriers.  m0 is used for nothing else.
+// waits are the counted ones below and the barriers.  m0 is named as written, which the
+// compiler remarks on, as on any register that it does not allocate.
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
 __device__ __forceinline__ void dma_lanes(uint32_t lds, const char *g) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(g) : "memory");
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(g) : "m0", "memory");
 }
 // ... from base + lane_off + OFF, where OFF counts on both sides.  STREAM: past the caches
 // (gemm_streams_weights).
@@ -68,12 +71,13 @@ __device__ __forceinline__ void dma_wave(uint32_t lds, const char *base, uint32_
   if constexpr (STREAM)
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 offset:%3 nt" ::"s"(lds), "v"(lane_off),
                  "s"(base), "n"(OFF)
-                 : "memory");
+                 : "m0", "memory");
   else
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 offset:%3" ::"s"(lds), "v"(lane_off),
                  "s"(base), "n"(OFF)
-                 : "memory");
+                 : "m0", "memory");
 }
+#pragma clang diagnostic pop
 typedef __attribute__((address_space(3))) const u32x4 lds_u32x4;
 typedef __attribute__((address_space(3))) const char lds_char;
 __device__ __forceinline__ bf16x8 lds_operand(uint32_t byte, int off) {

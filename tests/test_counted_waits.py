@@ -3,6 +3,7 @@ LDS ring by counting: "all but the newest n loads have landed".  That holds only
 lie behind the awaited ones, and the compiler drops a register load that nothing reads.  So the
 counts are checked against the loads that are in the built library, along every path through
 the disassembled kernels, without a GPU."""
+import glob
 import os
 import re
 import shutil
@@ -120,3 +121,15 @@ def test_waits_leave_no_awaited_row_in_flight(kernels):
         assert not lax, f"{name}: waits that leave awaited rows in flight (instruction: loads too many): {lax}"
         checked += len(found)
     assert checked >= 100
+
+
+def test_assembly_names_m0_where_it_writes_it():
+    """A DMA's LDS address goes into m0: assembly that writes it has to tell the compiler, which may
+    hold something of its own there."""
+    writes = 0
+    for path in sorted(glob.glob(os.path.join(build.CSRC, "*.hip")) + glob.glob(os.path.join(build.CSRC, "*.h"))):
+        for m in re.finditer(r"\basm\s+volatile\s*\((.*?)\);", open(path).read(), re.S):
+            if re.search(r"s_mov_b32 m0", m[1]):
+                writes += 1
+                assert '"m0"' in m[1].rsplit(":", 1)[1], f"{os.path.basename(path)}: {m[1]}"
+    assert writes
