@@ -31,16 +31,26 @@ import numpy as np
 ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
-# copies of kDirectTokens and kStreamMeanRows in moe_internal.h (stream_batch), to name the
-# kernel of a batch; tests/test_abi_host.py compares them
+# the line of stream_batch in moe_internal.h (kDirectTokens, kStreamMeanRows), and the
+# rule of its fp4_many_rows below, to name the kernel of a batch; tests/test_abi_host.py compares them
 STREAM_TOKENS, STREAM_MEAN_ROWS = 64, 16
-FP4_MANY_ROWS = 64  # and MXFP4 weights with this many rows per expert those of gemm_fp4.hip
 PEAK_BF16_TFLOPS = 2500.0  # MI355X dense bf16 MFMA
 PEAK_HBM_GBS = 8000.0
 SETTLE_STEPS = 200  # untimed calls in front of the warm-up steps, see run_leg
 # which roofline binds the gate_up GEMM of a workload: rows per expert
 # (4 T / E) against the machine balance of 312 flop per byte
 BOUND = {"c2": "mfma", "c3a": "hbm", "c3b": "mfma", "c4": "hbm", "c5": "hbm", "d4": "mfma"}
+
+
+def gemm_kernel(T: int, K: int, E: int, IM: int, mxfp4: bool) -> str:
+    """Name of the kernel of a batch's grouped GEMMs."""
+    if T <= STREAM_TOKENS or T * K <= STREAM_MEAN_ROWS * E:
+        return "stream_gemm_kernel"
+    if not mxfp4:
+        return "bf16_gemm_kernel"
+    col_tiles = -(-2 * (-(-IM // 64) * 64) // 256)
+    many = T * K > 128 * E or (T * K >= 64 * E and E * col_tiles > 256)
+    return "fp4_gemm_kernel" if many else "grouped_gemm_kernel"
 
 
 def cpu_model() -> str:
@@ -274,9 +284,7 @@ def main():
     combine_bytes = A * H * 2 + T * H * 4
     mfma_tflops = flops_gate_up / t_gate_up / 1e12
     hbm_gbs = bytes_gate_up / t_gate_up / 1e9
-    kernel = "%s<gate_up%s>" % ("stream_gemm_kernel" if T <= STREAM_TOKENS or T * K <= STREAM_MEAN_ROWS * E
-                                else "bf16_gemm_kernel" if not mxfp4 else
-                                "fp4_gemm_kernel" if T * K >= FP4_MANY_ROWS * E else "grouped_gemm_kernel", ", MXFP4" if mxfp4 else "")
+    kernel = "%s<gate_up%s>" % (gemm_kernel(T, K, E, IM, mxfp4), ", MXFP4" if mxfp4 else "")
     if BOUND[shape.name] == "mfma":
         roofline = {"bound": "mfma", "kernel": kernel, "achieved": mfma_tflops, "peak": PEAK_BF16_TFLOPS,
                     "unit": "TFLOP/s", "frac": mfma_tflops / PEAK_BF16_TFLOPS}

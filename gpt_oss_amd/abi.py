@@ -27,7 +27,7 @@ SYMBOLS = [
     "moe_profile_read", "moe_weight_bytes", "moe_workspace_bytes", "moe_last_error",
     "moe_version", "moe_dev_alloc", "moe_dev_free", "moe_dev_upload", "moe_dev_download",
     "moe_dev_memset", "moe_dev_sync", "moe_dev_count", "moe_time_forward", "moe_time_forward_each",
-    "moe_yardstick_mfma", "moe_yardstick_hbm",
+    "moe_yardstick_mfma", "moe_yardstick_hbm", "moe_batch_kernel",
 ]
 
 
@@ -84,6 +84,8 @@ def lib() -> C.CDLL:
         L.moe_dev_memset.argtypes = [vp, ci, C.c_size_t]
         L.moe_time_forward.argtypes = [vp, ci, vp, vp, ci, vp, ci, ci, C.POINTER(cf)]
         L.moe_time_forward_each.argtypes = [vp, ci, vp, vp, ci, vp, ci, C.POINTER(cf)]
+        L.moe_batch_kernel.argtypes = [C.POINTER(MoeConfig), ci, ci, C.POINTER(C.c_char_p), C.POINTER(ci),
+                                       C.POINTER(ci)]
         L.moe_yardstick_mfma.argtypes = [ci, ci, ci, C.POINTER(C.c_double), C.POINTER(C.c_double)]
         L.moe_yardstick_hbm.argtypes = [C.c_size_t, ci, C.POINTER(C.c_double), C.POINTER(C.c_double)]
         _lib = L
@@ -145,6 +147,14 @@ def dispatch_static(topk_i, pos, n_tokens, n_experts, offsets, perm, stream=None
     """moe_dispatch_static: no handle, no allocation; device buffers in and out."""
     check(lib().moe_dispatch_static(_p(topk_i), _p(pos), n_tokens, n_experts, _p(offsets), _p(perm),
                                     stream))
+
+
+def batch_kernel(hidden, inter, experts, tokens, mxfp4, layers=1):
+    """(kernel name, rows of a row tile, weights past the caches?) of a batch's grouped GEMMs; no GPU needed."""
+    cfg = MoeConfig(hidden, inter, experts, 4, layers, max(tokens, 1), 7.0)
+    name, rows, past = C.c_char_p(), C.c_int(), C.c_int()
+    check(lib().moe_batch_kernel(C.byref(cfg), int(bool(mxfp4)), tokens, C.byref(name), C.byref(rows), C.byref(past)))
+    return name.value.decode(), rows.value, bool(past.value)
 
 
 def yardstick_mfma(n_workgroups: int = 256, iters: int = 20000, data: int = 1):

@@ -680,39 +680,21 @@ static_assert(CfgFull::RBT_MAX * kRowBlock == kTileRows && CfgHalf::RBT_MAX * kR
 
 }  // namespace
 
-// Whether the expert matrices are read past the caches (non-temporal loads): while
-// most experts have one row tile their weights are read by one workgroup, and
-// lines that nobody reads again push the rows and the code out of L2.  us per
-// layer call, cached / past the caches: bf16 (tiles of 256 rows), 32 experts, 256
-// tokens 330 / 305, 512: 364 / 351, 1024: 392 / 374, 1536 (192 rows per expert): 433 / 414, 2048
-// (256): 525 / 512, 2560: 603 / 607, 4096: 831 / 845; 128 experts, 1024: 1234 / 1173, 6144 (192): 1631 /
-// 1632; 8 experts, 400 (200): 159 / 153, 600 (300): 191 / 195, 1000: 242 / 244.  Tiles of 128 rows
-// (measured with MXFP4), 32 experts, 256 tokens 143 / 135, 512: 172 / 163, 1024 (128 rows): 242 / 245,
-// 4096: 725 / 750; 128 experts, 3072 (96 rows): 676 / 668.  MXFP4 in tiles of 256 rows gains
-// nothing (8 experts, 256 tokens 93 / 95).  cached: kCachedWeightBytes.
-constexpr int kStreamRowsFull = 256, kStreamRowsHalf = 96;  // mean rows of an expert, at most
-static bool gemm_streams_weights(int T, int E, bool half, bool cached) {
-  if (cached) return false;
-  return T * kTopK <= (half ? kStreamRowsHalf : kStreamRowsFull) * E;
-}
-
 // w holds MXFP4 chunks and w_scale their scale bytes (pack_fp4_kernel).  The plan is of tiles of tile_rows.
 template <bool GATE_UP>
 static hipError_t launch_gemm(const void *a, const void *w, const uint16_t *w_scale, const float *ba,
                               const float *bb, const DispatchBuffers &d, void *out, int K, int N,
-                              float limit, int T, int E, int tile_rows, bool cached, hipStream_t s) {
+                              float limit, int T, int E, int tile_rows, bool stream, hipStream_t s) {
   const int nb_total = (GATE_UP ? 2 * N : N) / kRowBlock;
   const int n_ct = (nb_total + kGemmTileNb - 1) / kGemmTileNb;
   const int grid = kXcds * xcd_tile_cap(gemm_tile_cap(T, E, tile_rows) * n_ct);
   const TileDesc *tiles = GATE_UP ? d.tiles_gate_up : d.tiles_down;
   const uint4 *af = static_cast<const uint4 *>(a), *wf = static_cast<const uint4 *>(w);
   // the full-height kernels take a plan of either height, the others one of half height
-  const bool half = tile_rows == kHalfTileRows;
-  const bool stream = gemm_streams_weights(T, E, half, cached);
 #define MOE_GEMM(C, STREAM)                                                                                 \
   grouped_gemm_kernel<C, GATE_UP, STREAM><<<grid, C::THREADS, 0, s>>>(af, wf, w_scale, ba, bb, tiles, d.totals, \
                                                                       d.rowmap, out, K, N, limit)
-  if (!half) MOE_GEMM(CfgFull, false);
+  if (tile_rows != kHalfTileRows) MOE_GEMM(CfgFull, false);
   else if (stream) MOE_GEMM(CfgHalf, true);
   else MOE_GEMM(CfgHalf, false);
 #undef MOE_GEMM
@@ -723,24 +705,22 @@ hipError_t launch_gate_up(const uint16_t *x, const void *w1, const uint16_t *w1_
                           const float *b1u, const DispatchBuffers &d, uint16_t *act, int H, int IM,
                           float limit, int T, int E, int tile_rows, bool cached, hipStream_t s) {
   if (H % 64 || IM % 64) return hipErrorInvalidValue;  // the kernels take steps of 32 in pairs
-  if (!w1_scale)
-    return launch_bf16_gate_up(x, w1, b1g, b1u, d, act, H, IM, limit, T, E, tile_rows,
-                               gemm_streams_weights(T, E, tile_rows == kHalfTileRows, cached), s);
-  if (tile_rows == kHalfTileRows && fp4_many_rows(T, E, 2 * IM))
-    return launch_fp4_gate_up(x, w1, w1_scale, b1g, b1u, d, act, H, IM, limit, T, E,
-                              gemm_streams_weights(T, E, true, cached), s);
-  return launch_gemm<true>(x, w1, w1_scale, b1g, b1u, d, act, H, IM, limit, T, E, tile_rows, cached, s);
+  const TileRoute r = tile_route(T, E, 2 * IM, w1_scale != nullptr, tile_rows, cached);
+  if (r.kernel == kBf16Tiles)
+    return launch_bf16_gate_up(x, w1, b1g, b1u, d, act, H, IM, limit, T, E, tile_rows, r.past_caches, s);
+  if (r.kernel == kFp4ManyTiles)
+    return launch_fp4_gate_up(x, w1, w1_scale, b1g, b1u, d, act, H, IM, limit, T, E, r.past_caches, s);
+  return launch_gemm<true>(x, w1, w1_scale, b1g, b1u, d, act, H, IM, limit, T, E, tile_rows, r.past_caches, s);
 }
 
 hipError_t launch_down(const uint16_t *act, const void *w2, const uint16_t *w2_scale, const float *b2,
                        const DispatchBuffers &d, float *y, int H, int IM, int T, int E, int tile_rows,
                        bool cached, hipStream_t s) {
   if (H % 64 || IM % 64) return hipErrorInvalidValue;  // the kernels take steps of 32 in pairs
-  if (!w2_scale)
-    return launch_bf16_down(act, w2, b2, d, y, H, IM, T, E, tile_rows, gemm_streams_weights(T, E, tile_rows == kHalfTileRows, cached), s);
-  if (tile_rows == kHalfTileRows && fp4_many_rows(T, E, 2 * IM))
-    return launch_fp4_down(act, w2, w2_scale, b2, d, y, H, IM, T, E, gemm_streams_weights(T, E, true, cached), s);
-  return launch_gemm<false>(act, w2, w2_scale, b2, nullptr, d, y, IM, H, 0.f, T, E, tile_rows, cached, s);
+  const TileRoute r = tile_route(T, E, 2 * IM, w2_scale != nullptr, tile_rows, cached);
+  if (r.kernel == kBf16Tiles) return launch_bf16_down(act, w2, b2, d, y, H, IM, T, E, tile_rows, r.past_caches, s);
+  if (r.kernel == kFp4ManyTiles) return launch_fp4_down(act, w2, w2_scale, b2, d, y, H, IM, T, E, r.past_caches, s);
+  return launch_gemm<false>(act, w2, w2_scale, b2, nullptr, d, y, IM, H, 0.f, T, E, tile_rows, r.past_caches, s);
 }
 
 }  // namespace moe

@@ -134,6 +134,11 @@ struct StageTimer {
   }
 };
 
+// bytes of a layer's expert matrices on the device (17/32 of a byte per MXFP4 weight)
+inline size_t expert_matrix_bytes(int E, int Hp, int IMp, bool mxfp4) {
+  return (size_t)E * 3 * IMp * Hp * (mxfp4 ? 17 : 64) / 32;
+}
+
 // column tiles of the two grouped GEMMs (tiles are kGemmTileNb blocks of 32 columns wide)
 inline int gate_up_col_tiles(const moe_handle *h) {
   return (2 * h->IMp / kRowBlock + kGemmTileNb - 1) / kGemmTileNb;
@@ -146,8 +151,7 @@ inline int down_col_tiles(const moe_handle *h) {
 // bf16 weights take a plan of either height (a caller may dispatch before it names the layer).
 int run_dispatch(moe_handle *h, const int *topk_i, const int *pos, int T, bool mxfp4, hipStream_t s) {
   const int E = h->cfg.experts;
-  const bool half = mxfp4 ? half_tiles(T, E, 2 * h->IMp) : bf16_half_tiles(T, E, h->Hp, h->IMp);
-  h->plan_rows = half ? kHalfTileRows : kTileRows;
+  h->plan_rows = plan_tile_rows(T, E, h->Hp, h->IMp, mxfp4);
   // the kernels of stream.hip go by row blocks and need no tile tables
   const bool tables = !stream_batch(T, E);
   HIP_TRY(launch_dispatch(topk_i, pos, T, E, tables ? gate_up_col_tiles(h) : 0, tables ? down_col_tiles(h) : 0,
@@ -430,7 +434,7 @@ int upload_layer(moe_handle *h, int layer, const float *w_router, const float *b
   if (rc == MOE_OK) lw.uploaded = true;
   h->expert_bytes = 0;
   for (const LayerWeights &l : h->layers)
-    if (l.uploaded) h->expert_bytes += (size_t)E * (p1 + p2) * (l.w1q ? 17 : 64) / 32;  // 17/32 byte per MXFP4 weight
+    if (l.uploaded) h->expert_bytes += expert_matrix_bytes(E, Hp, IMp, l.w1q != nullptr);
   return rc;
 }
 
@@ -672,6 +676,27 @@ int moe_profile_read(moe_handle *h, float *ms, int *n_calls) {
   for (int st = 0; st < MOE_NUM_STAGES; st++)
     ms[st] = h->prof_recorded ? (float)(sum[st] / h->prof_recorded) : 0.f;
   if (n_calls) *n_calls = h->prof_recorded;
+  return MOE_OK;
+}
+
+int moe_batch_kernel(const moe_config *cfg, int mxfp4, int n_tokens, const char **kernel, int *tile_rows,
+                     int *past_caches) {
+  if (!cfg || !kernel || !tile_rows || !past_caches) return fail(MOE_ERR_BAD_ARG, "null argument");
+  if (cfg->hidden <= 0 || cfg->inter <= 0 || cfg->experts <= 0 || cfg->layers <= 0 || n_tokens < 0 ||
+      (long long)n_tokens * kTopK > (1ll << 28))
+    return fail(MOE_ERR_BAD_ARG, "moe_batch_kernel: sizes must be positive, n_tokens in range");
+  const int T = n_tokens, E = cfg->experts, Hp = padded_dim(cfg->hidden), IMp = padded_dim(cfg->inter);
+  const bool cached = cfg->layers * expert_matrix_bytes(E, Hp, IMp, mxfp4 != 0) <= kCachedWeightBytes;
+  if (stream_batch(T, E)) {
+    *kernel = "stream_gemm_kernel";
+    *tile_rows = kRowBlock;
+    *past_caches = !cached;
+    return MOE_OK;
+  }
+  *tile_rows = plan_tile_rows(T, E, Hp, IMp, mxfp4 != 0);
+  const TileRoute r = tile_route(T, E, 2 * IMp, mxfp4 != 0, *tile_rows, cached);
+  *kernel = r.kernel == kBf16Tiles ? "bf16_gemm_kernel" : (r.kernel == kFp4Tiles ? "grouped_gemm_kernel" : "fp4_gemm_kernel");
+  *past_caches = r.past_caches;
   return MOE_OK;
 }
 

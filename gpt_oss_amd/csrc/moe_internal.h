@@ -251,6 +251,36 @@ inline bool bf16_half_tiles(int T, int E, int H, int IM) {
   };
   return time(kHalfTileRows) < 0.9f * time(kTileRows);
 }
+// Whether the expert matrices are read past the caches (non-temporal loads): while
+// most experts have one row tile their weights are read by one workgroup, and
+// lines that nobody reads again push the rows and the code out of L2.  us per
+// layer call, cached / past the caches: bf16 (tiles of 256 rows), 32 experts, 256
+// tokens 330 / 305, 512: 364 / 351, 1024: 392 / 374, 1536 (192 rows per expert): 433 / 414, 2048
+// (256): 525 / 512, 2560: 603 / 607, 4096: 831 / 845; 128 experts, 1024: 1234 / 1173, 6144 (192): 1631 /
+// 1632; 8 experts, 400 (200): 159 / 153, 600 (300): 191 / 195, 1000: 242 / 244.  Tiles of 128 rows
+// (measured with MXFP4), 32 experts, 256 tokens 143 / 135, 512: 172 / 163, 1024 (128 rows): 242 / 245,
+// 4096: 725 / 750; 128 experts, 3072 (96 rows): 676 / 668.  MXFP4 in tiles of 256 rows gains
+// nothing (8 experts, 256 tokens 93 / 95).  cached: kCachedWeightBytes.
+constexpr int kStreamRowsFull = 256, kStreamRowsHalf = 96;  // mean rows of an expert, at most
+inline bool gemm_streams_weights(int T, int E, bool half, bool cached) {
+  if (cached) return false;
+  return T * kTopK <= (half ? kStreamRowsHalf : kStreamRowsFull) * E;
+}
+// Row tiles of a plan, and what runs on it.
+inline int plan_tile_rows(int T, int E, int H, int IM, bool mxfp4) {
+  return (mxfp4 ? half_tiles(T, E, 2 * IM) : bf16_half_tiles(T, E, H, IM)) ? kHalfTileRows : kTileRows;
+}
+enum TileKernel { kBf16Tiles /* gemm_bf16.hip */, kFp4Tiles /* gemm.hip */, kFp4ManyTiles /* gemm_fp4.hip */ };
+struct TileRoute {
+  TileKernel kernel;
+  bool past_caches;
+};
+inline TileRoute tile_route(int T, int E, int w1_rows, bool mxfp4, int tile_rows, bool cached) {
+  const bool half = tile_rows == kHalfTileRows;
+  if (!mxfp4) return {kBf16Tiles, gemm_streams_weights(T, E, half, cached)};
+  return {half && fp4_many_rows(T, E, w1_rows) ? kFp4ManyTiles : kFp4Tiles,
+          half && gemm_streams_weights(T, E, half, cached)};
+}
 // Expert matrices up to this many bytes, over all layers of a handle, are read through
 // the caches whatever the batch: they then stay in the 256 MB memory-side cache from
 // one call to the next, which loads past the caches do not use.  us per moe_experts

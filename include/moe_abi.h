@@ -244,6 +244,13 @@ int moe_combine(moe_handle *h, const float *topk_v, const int *pos, int n_tokens
 int moe_profile_enable(moe_handle *h, int n_calls);
 int moe_profile_read(moe_handle *h, float *ms, int *n_calls);
 
+/* The grouped-GEMM kernel that a batch of n_tokens runs under moe_forward, for reports and
+ * tests: its name in a profile, the rows of its tallest row tiles, and whether it reads the
+ * expert matrices past the caches, with all layers of cfg uploaded in one format (mxfp4 != 0:
+ * MXFP4).  Needs neither a handle nor a GPU.  Has no counterpart in the reference. */
+int moe_batch_kernel(const moe_config *cfg, int mxfp4, int n_tokens, const char **kernel,
+                     int *tile_rows, int *past_caches);
+
 /* Sizes the kernels work with, for reports: number of row tiles the last
  * dispatch produced is data dependent and stays on the device; these are the
  * static figures. */

@@ -118,3 +118,26 @@ def test_bench_names_kernels_by_the_librarys_rule():
     header = "gpt_oss_amd/csrc/moe_internal.h"
     assert value("bench.py", r"STREAM_TOKENS, STREAM_MEAN_ROWS = (\d+)") == value(header, r"kDirectTokens = (\d+)")
     assert value("bench.py", r"STREAM_TOKENS, STREAM_MEAN_ROWS = \d+, (\d+)") == value(header, r"kStreamMeanRows = (\d+)")
+
+
+@pytest.mark.parametrize("E", [4, 8, 12, 32, 128, 256])
+@pytest.mark.parametrize("IM", [32, 512, 1440, 2880])
+def test_bench_names_the_kernel_that_runs(E, IM):
+    """bench.py's name of a batch's kernel is that of the library's own rule, on both sides of
+    every line (16 and 64 rows per expert, 128 where there is at most a workgroup per CU)."""
+    import bench
+    for rows in (1, 15, 16, 17, 63, 64, 65, 100, 127, 128, 129, 500):
+        for T in {max(1, rows * E // 4 + d) for d in (-1, 0, 1)} | {64, 65}:
+            for mxfp4 in (False, True):
+                name = abi.batch_kernel(2880, IM, E, T, mxfp4)[0]
+                assert bench.gemm_kernel(T, 4, E, IM, mxfp4) == name, (T, mxfp4)
+
+
+def test_batch_kernel_rejects_bad_arguments():
+    cfg = abi.MoeConfig(256, 256, 8, 4, 1, 64, 7.0)
+    name, rows, past = C.c_char_p(), C.c_int(), C.c_int()
+    L = abi.lib()
+    assert L.moe_batch_kernel(None, 0, 1, C.byref(name), C.byref(rows), C.byref(past)) == -1
+    assert L.moe_batch_kernel(C.byref(cfg), 0, 1, None, C.byref(rows), C.byref(past)) == -1
+    assert L.moe_batch_kernel(C.byref(cfg), 0, -1, C.byref(name), C.byref(rows), C.byref(past)) == -1
+    assert L.moe_batch_kernel(C.byref(cfg), 0, 0, C.byref(name), C.byref(rows), C.byref(past)) == 0
