@@ -151,7 +151,7 @@ inline int down_col_tiles(const moe_handle *h) {
 // bf16 weights take a plan of either height (a caller may dispatch before it names the layer).
 int run_dispatch(moe_handle *h, const int *topk_i, const int *pos, int T, bool mxfp4, hipStream_t s) {
   const int E = h->cfg.experts;
-  h->plan_rows = plan_tile_rows(T, E, h->Hp, h->IMp, mxfp4);
+  h->plan_rows = plan_tile_rows(T, E, h->Hp, h->IMp, mxfp4, h->expert_bytes <= kCachedWeightBytes);
   // the kernels of stream.hip go by row blocks and need no tile tables
   const bool tables = !stream_batch(T, E);
   HIP_TRY(launch_dispatch(topk_i, pos, T, E, tables ? gate_up_col_tiles(h) : 0, tables ? down_col_tiles(h) : 0,
@@ -693,7 +693,7 @@ int moe_batch_kernel(const moe_config *cfg, int mxfp4, int n_tokens, const char 
     *past_caches = !cached;
     return MOE_OK;
   }
-  *tile_rows = plan_tile_rows(T, E, Hp, IMp, mxfp4 != 0);
+  *tile_rows = plan_tile_rows(T, E, Hp, IMp, mxfp4 != 0, cached);
   const TileRoute r = tile_route(T, E, 2 * IMp, mxfp4 != 0, *tile_rows, cached);
   *kernel = r.kernel == kBf16Tiles ? "bf16_gemm_kernel" : (r.kernel == kFp4Tiles ? "grouped_gemm_kernel" : "fp4_gemm_kernel");
   *past_caches = r.past_caches;

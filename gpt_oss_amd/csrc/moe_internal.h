@@ -230,14 +230,19 @@ inline bool half_tiles(int T, int E, int w1_rows) {
 }
 // bf16 weights: whether row tiles of 128 rows in place of 256 are expected to be quicker.  They stream an
 // expert's weights more often, so they pay only where the tall tiles leave CUs without work, in either
-// GEMM.  The estimate: an expert has half a tile more than its rows fill on average; a tile takes the time of 4
-// + (its row blocks) steps of its reduction; the CUs take tiles in rounds.  us per layer call, 256 rows / 128:
-// 4 experts, 2880 x 2880, 150 tokens 89 / 71; 4 experts, 1024 x 2048, 500 tokens 85 / 62; 512 x 512, 8 experts,
-// 1000 tokens 51 / 43, 32 experts, 700 tokens 50 / 45; 256 x 1440, 32 experts, 1000 tokens, Zipf's
-// routing 72 / 60.  Where the estimate says 256 rows: 8 experts, 2880 x 2880, 256 tokens 129 / 152, 400 156 /
-// 162, 600 182 / 215; 16 experts, 700 tokens 240 / 266; 8 experts, 512 x 512, 7000 tokens 92 / 96 (3000, a
+// GEMM, and where the weights come out of the memory-side cache (cached: kCachedWeightBytes).  The estimate: an
+// expert has half a tile more than its rows fill on average; a tile takes the time of 4 + (its row blocks)
+// steps of its reduction; the CUs take tiles in rounds.  us per layer call, 256 rows / 128: 4
+// experts, 2880 x 2880, 145 tokens 88 / 70, 256 124 / 81; 1024 x 1024, 8 experts, 1800 tokens 96 / 79; 256 x
+// 1440, 8 experts, 1000 tokens 63 / 51, 32 experts, 1440 tokens, Zipf's routing 74 / 61; 512 x 512, 32 experts,
+// 1000 tokens 57 / 49.  Where the estimate says 256 rows: 8 experts, 512 x 512, 7000 tokens 92 / 96 (3000, a
 // close call, 59 / 56).  128 rows have to be a tenth quicker by the estimate.
-inline bool bf16_half_tiles(int T, int E, int H, int IM) {
+// From HBM a round more or less, which the host cannot foresee, costs more than the rule gains: where it
+// says 128, at 2880 x 2880, even / Zipf's routing: 8 experts, 520 tokens 0.94 / 1.00 of the time with 256, 221
+// 1.00 / 1.13, 1200 1.05 / 0.97; 10 experts, 450 1.10 / 0.96; 12 experts, 360 0.96 / 0.95, 480 1.18 /
+// 0.95; 14 experts, 460 1.26 / 1.10; 24 experts, 640 0.98 / 1.12.
+inline bool bf16_half_tiles(int T, int E, int H, int IM, bool cached) {
+  if (!cached) return false;
   const int A = T * kTopK;
   const float blocks = (float)A / kRowBlock + 0.5f * E;
   auto time = [&](int tile_rows) {
@@ -257,18 +262,18 @@ inline bool bf16_half_tiles(int T, int E, int H, int IM) {
 // layer call, cached / past the caches: bf16 (tiles of 256 rows), 32 experts, 256
 // tokens 330 / 305, 512: 364 / 351, 1024: 392 / 374, 1536 (192 rows per expert): 433 / 414, 2048
 // (256): 525 / 512, 2560: 603 / 607, 4096: 831 / 845; 128 experts, 1024: 1234 / 1173, 6144 (192): 1631 /
-// 1632; 8 experts, 400 (200): 159 / 153, 600 (300): 191 / 195, 1000: 242 / 244.  Tiles of 128 rows
-// (measured with MXFP4), 32 experts, 256 tokens 143 / 135, 512: 172 / 163, 1024 (128 rows): 242 / 245,
-// 4096: 725 / 750; 128 experts, 3072 (96 rows): 676 / 668.  MXFP4 in tiles of 256 rows gains
-// nothing (8 experts, 256 tokens 93 / 95).  cached: kCachedWeightBytes.
-constexpr int kStreamRowsFull = 256, kStreamRowsHalf = 96;  // mean rows of an expert, at most
-inline bool gemm_streams_weights(int T, int E, bool half, bool cached) {
-  if (cached) return false;
-  return T * kTopK <= (half ? kStreamRowsHalf : kStreamRowsFull) * E;
+// 1632; 8 experts, 400 (200): 159 / 153, 600 (300): 191 / 195, 1000: 242 / 244.  MXFP4 in tiles of 128 rows,
+// 32 experts, 256 tokens 143 / 135, 512: 172 / 163, 1024 (128 rows): 242 / 245, 4096: 725 / 750; 128 experts, 3072
+// (96 rows): 676 / 668.  MXFP4 in tiles of 256 rows gains nothing (8 experts, 256 tokens 93 / 95), and
+// bf16 has tiles of 128 rows only where the caches hold the matrices.  cached: kCachedWeightBytes.
+constexpr int kStreamRowsBf16 = 256, kStreamRowsFp4 = 96;  // mean rows of an expert, at most
+inline bool gemm_streams_weights(int T, int E, bool mxfp4, int tile_rows, bool cached) {
+  if (cached || tile_rows != (mxfp4 ? kHalfTileRows : kTileRows)) return false;
+  return T * kTopK <= (mxfp4 ? kStreamRowsFp4 : kStreamRowsBf16) * E;
 }
 // Row tiles of a plan, and what runs on it.
-inline int plan_tile_rows(int T, int E, int H, int IM, bool mxfp4) {
-  return (mxfp4 ? half_tiles(T, E, 2 * IM) : bf16_half_tiles(T, E, H, IM)) ? kHalfTileRows : kTileRows;
+inline int plan_tile_rows(int T, int E, int H, int IM, bool mxfp4, bool cached) {
+  return (mxfp4 ? half_tiles(T, E, 2 * IM) : bf16_half_tiles(T, E, H, IM, cached)) ? kHalfTileRows : kTileRows;
 }
 enum TileKernel { kBf16Tiles /* gemm_bf16.hip */, kFp4Tiles /* gemm.hip */, kFp4ManyTiles /* gemm_fp4.hip */ };
 struct TileRoute {
@@ -276,10 +281,9 @@ struct TileRoute {
   bool past_caches;
 };
 inline TileRoute tile_route(int T, int E, int w1_rows, bool mxfp4, int tile_rows, bool cached) {
-  const bool half = tile_rows == kHalfTileRows;
-  if (!mxfp4) return {kBf16Tiles, gemm_streams_weights(T, E, half, cached)};
-  return {half && fp4_many_rows(T, E, w1_rows) ? kFp4ManyTiles : kFp4Tiles,
-          half && gemm_streams_weights(T, E, half, cached)};
+  const bool past_caches = gemm_streams_weights(T, E, mxfp4, tile_rows, cached);
+  if (!mxfp4) return {kBf16Tiles, past_caches};
+  return {tile_rows == kHalfTileRows && fp4_many_rows(T, E, w1_rows) ? kFp4ManyTiles : kFp4Tiles, past_caches};
 }
 // Expert matrices up to this many bytes, over all layers of a handle, are read through
 // the caches whatever the batch: they then stay in the 256 MB memory-side cache from

@@ -141,3 +141,19 @@ def test_batch_kernel_rejects_bad_arguments():
     assert L.moe_batch_kernel(C.byref(cfg), 0, 1, None, C.byref(rows), C.byref(past)) == -1
     assert L.moe_batch_kernel(C.byref(cfg), 0, -1, C.byref(name), C.byref(rows), C.byref(past)) == -1
     assert L.moe_batch_kernel(C.byref(cfg), 0, 0, C.byref(name), C.byref(rows), C.byref(past)) == 0
+
+
+@pytest.mark.parametrize("H,IM,E,T,layers,rows", [
+    # bf16 matrices that the caches do not hold: tall tiles always
+    (2880, 2880, 8, 221, 1, 256), (2880, 2880, 10, 412, 1, 256), (2880, 2880, 12, 480, 1, 256), (2880, 2880, 14, 460, 1, 256),
+    (2880, 2880, 24, 640, 1, 256), (2880, 2880, 32, 4096, 1, 256), (512, 512, 32, 1000, 24, 256),
+    # that they hold: by the estimate
+    (2880, 2880, 4, 145, 1, 128), (2880, 2880, 4, 256, 1, 128), (1024, 1024, 8, 1800, 1, 128), (256, 1440, 8, 1000, 1, 128),
+    (512, 512, 32, 1000, 1, 128), (512, 512, 8, 7000, 1, 256),
+])
+def test_height_of_bf16_row_tiles(H, IM, E, T, layers, rows):
+    """Batches that lose by the other height (times in moe_internal.h)."""
+    name, got, past = abi.batch_kernel(H, IM, E, T, False, layers)
+    assert (name, got) == ("bf16_gemm_kernel", rows)
+    held = layers * E * 6 * H * IM <= 256 << 20
+    assert past == (not held and 4 * T <= 256 * E)
