@@ -125,11 +125,28 @@ hipError_t launch_pad_rows(const uint16_t *x, uint16_t *xp, int T, int H, int Hp
 hipError_t launch_router_stats(const float *w_src, const float *b_src, int E, int H, float *rstat,
                                hipStream_t s);
 // first: scratch for T * (E_pad + 4) floats that no other call uses meanwhile, or nullptr.  With it, batches of up to
-// kSplitRouterTokens tokens at more than 64 experts run the first pass on E_pad / 16 times as many
-// workgroups and a launch of their own; the results are the same bits.  us per layer call without / with at 128
-// experts: 16 tokens 127.7 / 122.1, 512 383 / 377, 1024 445 / 441, 1500 473 / 474, 4096 816 / 826; 512 x 512,
-// 2000 tokens 70.6 / 72.9.
-constexpr int kSplitRouterTokens = 1024;
+// split_router_tokens at more than 64 experts run the first pass on E_pad / 16 times as many
+// workgroups and a launch of their own; the results are the same bits.  That pays where one workgroup
+// would take long over the router matrix: the more the longer its rows, and the less the more workgroups
+// there are anyway.  Time of a layer call (MXFP4 experts) with the launch over that without:
+//   128 experts   tokens 1   40    200   400   600   1024
+//     256 columns    1.03  1.05  1.01  1.01  1.05  1.03
+//     512            1.01  1.00  1.00  0.98  1.01  1.01
+//     768            0.97  0.99  0.99  0.99  1.01  1.01
+//     1024           0.93  0.98  0.98  0.98  1.02  0.99
+//     1440           0.92  0.97  0.97  0.98  0.99  0.99
+//     2880           0.84  0.97  0.98  0.98  0.99  0.99   (4096 tokens 1.01)
+//   256 experts
+//     128            0.95  0.98  0.97  1.01  1.03  1.05
+//     256            0.92  0.96  0.96  0.99  1.01  1.04
+//     384            0.89  0.92  0.94  0.96  0.99  1.01
+//     2880           0.67  0.95  0.97  0.98  0.98  0.99
+inline int split_router_tokens(int E_pad, int H) {
+  if (E_pad < 128) return 0;
+  if (H > 1024) return 1024;
+  if (E_pad == 128) return H >= 768 ? 400 : 0;
+  return H >= 256 ? 400 : 200;
+}
 hipError_t launch_router(const uint16_t *x, const int *pos, const uint16_t *wr, const float *br,
                          const float *rstat, int T, int H, int E, int E_pad, float *score, int *topk_i,
                          float *topk_v, float *first, hipStream_t s);

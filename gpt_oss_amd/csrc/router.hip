@@ -602,7 +602,7 @@ static hipError_t launch_router_nt(const uint16_t *x, const int *pos, const uint
   // (at 256 the accumulators of two tiles no longer fit the registers).
   if constexpr (NT >= 8) {
     static_assert(WPC == kSplitWaves, "router_logits_kernel adds up what router_kernel does, in its order");
-    if (first && T <= kSplitRouterTokens) {
+    if (first && T <= split_router_tokens(NT * 16, H)) {
       router_logits_kernel<8><<<dim3((T + 15) / 16, NT), kSplitWaves * 64, 0, s>>>(x, wr, br, T, H, NT * 16, first);
       router_kernel<NT, 8, 1, 1, FLUSH, true><<<(T + 15) / 16, 8 * 64, 0, s>>>(x, pos, wr, br, rstat, T, H, E, score,
                                                                               topk_i, topk_v, first);

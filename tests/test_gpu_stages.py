@@ -450,12 +450,13 @@ def test_padded_shape_and_split_reduction_replay_from_a_hip_graph(T):
         hip.hipStreamDestroy(stream)
 
 
-@pytest.mark.parametrize("E,H", [(100, 96), (128, 2880), (200, 320)])
+@pytest.mark.parametrize("E,H", [(100, 96), (100, 768), (128, 2880), (200, 320), (256, 128)])
 def test_split_router_gives_the_same_bits(E, H):
     """More than 64 experts: the router of the whole-layer calls runs its first pass as a launch
-    of its own up to 1024 tokens, moe_router in one kernel; ids, weights and so the layer agree bit
-    for bit, on either side of the line, with inactive rows and near ties among the tokens."""
-    for T in (1, 6, 17, 64, 200, 1023, 1024, 1025):
+    of its own up to 200, 400 or 1024 tokens (split_router_tokens; at 96 columns never), moe_router in one
+    kernel; ids, weights and so the layer agree bit for bit, on either side of the line, with
+    inactive rows and near ties among the tokens."""
+    for T in (1, 6, 17, 64, 200, 201, 400, 401, 1023, 1024, 1025):
         sh = synth.LayerShape("r", T, H, 64, E)
         L = bf16_layer(sh, seed=T)
         L["w_router"][E // 2] = L["w_router"][3]  # two experts that always tie but for the bias

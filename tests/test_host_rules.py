@@ -1,0 +1,33 @@
+"""Rules of the launches that no entry point tells of, compiled from moe_internal.h for the host alone."""
+import ctypes as C
+import os
+import subprocess
+
+import pytest
+
+from gpt_oss_amd import build
+
+SOURCE = """
+#include "%s/moe_internal.h"
+extern "C" int split_router_tokens(int E_pad, int H) { return moe::split_router_tokens(E_pad, H); }
+""" % build.CSRC
+
+
+@pytest.fixture(scope="module")
+def rules(tmp_path_factory):
+    if not os.path.exists(build.HIPCC):
+        pytest.skip("no hipcc")
+    d = tmp_path_factory.mktemp("rules")
+    (d / "rules.hip").write_text(SOURCE)
+    subprocess.run([build.HIPCC, "--offload-host-only", "-std=c++17", "-O1", "-fPIC", "-shared", "-Wno-everything",
+                    str(d / "rules.hip"), "-o", str(d / "rules.so")], check=True)
+    return C.CDLL(str(d / "rules.so"))
+
+
+@pytest.mark.parametrize("E_pad,H,tokens", [(16, 2880, 0), (64, 2880, 0), (128, 256, 0), (128, 736, 0), (128, 768, 400),
+                                            (128, 1024, 400), (128, 1440, 1024), (128, 2880, 1024), (256, 128, 200),
+                                            (256, 256, 400), (256, 512, 400), (256, 2880, 1024)])
+def test_router_splits_where_it_gains(rules, E_pad, H, tokens):
+    """The router's first pass as a launch of its own costs small matrices more than it gains
+    (times in moe_internal.h)."""
+    assert rules.split_router_tokens(E_pad, H) == tokens
