@@ -347,6 +347,12 @@ hipError_t launch_combine(const float *y, int ldy, const int *inv, const float *
                           int T, int H, int accumulate, hipStream_t s);
 hipError_t launch_combine_residual(const float *y, int ldy, const int *inv, const float *topk_v, const int *pos,
                                    uint16_t *x, int T, int H, hipStream_t s);
+// Whether the norm takes a wave per token instead of a workgroup: rows that a wave's registers
+// hold, and of those beyond one piece per thread only with tokens enough for a workgroup on every
+// CU.  moe_block_forward, wave / workgroup: 7168 tokens, 64 columns 46.5 / 51.5 us, 256 0.93, 512 0.95, 1024
+// 0.98 of the time; 768 to 1024 columns, 2000 tokens 0.98, 1000 0.99, 8 to 64 tokens 1.02 to 1.03.
+constexpr int kNormHeld = 2;  // 16-byte pieces of the row per thread
+inline bool norm_wave_per_token(int T, int H) { return H <= 64 * 8 || (H <= 64 * 8 * kNormHeld && T >= 4 * kCus); }
 hipError_t launch_rmsnorm(const uint16_t *x, const float *weight, const int *pos, uint16_t *t_out,
                           int T, int H, hipStream_t s);
 

@@ -11,18 +11,23 @@
 
 namespace moe {
 
-// One workgroup per token, 8 elements (16 bytes) per thread and pass.  Bound by latency: row
-// and weight are asked for at once and the row stays in registers (up to 4096 elements;
-// longer ones read the rest again).  A wave per token walked the row twice: 6 tokens
-// 7.8 us, 200 tokens 9.3, 4096 tokens 16.0; now 4.5, 5.4 and 15.0.
+// THREADS per token, 8 elements (16 bytes) per thread and pass: a workgroup, or a wave for rows short
+// enough for its registers.  Bound by latency: row and weight are asked for at once and the
+// row stays in registers (up to 16 elements per thread; longer ones read the rest again).  At 2880
+// columns a wave per token, which walked the row twice, took 7.8 us for 6 tokens, 9.3 for 200, 16.0 for 4096; a
+// workgroup 4.5, 5.4 and 15.0.  With short rows a workgroup is mostly idle threads: a call of
+// moe_block_forward with 7168 tokens took 51 us instead of 47 at 64 columns, 69 instead of 64 at 256, 107
+// instead of 101 at 512.
+template <int THREADS>
 __global__ __launch_bounds__(256) void rmsnorm_kernel(const uint16_t *__restrict__ x,
                                                      const float *__restrict__ weight,
                                                      const int *__restrict__ pos,
-                                                     uint16_t *__restrict__ t_out, int H) {
-  constexpr int HELD = 2;
-  __shared__ double sh_ss[4];
-  const int tid = threadIdx.x;
-  const int t = blockIdx.x;
+                                                     uint16_t *__restrict__ t_out, int T, int H) {
+  constexpr int HELD = kNormHeld;
+  static_assert(THREADS == 64 || THREADS == 256, "a wave or a workgroup");
+  const int tid = threadIdx.x % THREADS;
+  const int t = blockIdx.x * (256 / THREADS) + threadIdx.x / THREADS;
+  if (t >= T) return;             // (waves of a short last workgroup)
   if (pos && pos[t] < 0) return;  // the row takes part in nothing downstream
   const uint4 *row = reinterpret_cast<const uint4 *>(x + (size_t)t * H);
   const int chunks = H / 8;
@@ -30,7 +35,7 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(const uint16_t *__restrict
   float4 w0[HELD], w1[HELD];
 #pragma unroll
   for (int i = 0; i < HELD; i++) {
-    const int c = tid + 256 * i;
+    const int c = tid + THREADS * i;
     held[i] = make_uint4(0u, 0u, 0u, 0u);
     if (c < chunks) {
       held[i] = row[c];
@@ -50,12 +55,15 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(const uint16_t *__restrict
   };
 #pragma unroll
   for (int i = 0; i < HELD; i++) add(held[i]);
-  for (int c = tid + 256 * HELD; c < chunks; c += 256) add(row[c]);
+  for (int c = tid + THREADS * HELD; c < chunks; c += THREADS) add(row[c]);
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) ss += __shfl_xor(ss, off, 64);
-  if ((tid & 63) == 0) sh_ss[tid >> 6] = ss;
-  __syncthreads();
-  ss = ((sh_ss[0] + sh_ss[1]) + sh_ss[2]) + sh_ss[3];
+  if constexpr (THREADS > 64) {
+    __shared__ double sh_ss[THREADS / 64];
+    if ((tid & 63) == 0) sh_ss[tid >> 6] = ss;
+    __syncthreads();
+    ss = ((sh_ss[0] + sh_ss[1]) + sh_ss[2]) + sh_ss[3];
+  }
   ss /= (double)H;
   ss += (double)1e-5f;
   const float narrowed = (float)ss;
@@ -77,8 +85,8 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(const uint16_t *__restrict
   };
 #pragma unroll
   for (int i = 0; i < HELD; i++)
-    if (tid + 256 * i < chunks) put(tid + 256 * i, held[i], w0[i], w1[i]);
-  for (int c = tid + 256 * HELD; c < chunks; c += 256)
+    if (tid + THREADS * i < chunks) put(tid + THREADS * i, held[i], w0[i], w1[i]);
+  for (int c = tid + THREADS * HELD; c < chunks; c += THREADS)
     put(c, row[c], *reinterpret_cast<const float4 *>(weight + 8 * c), *reinterpret_cast<const float4 *>(weight + 8 * c + 4));
 }
 
@@ -106,7 +114,10 @@ hipError_t launch_pad_rows(const uint16_t *x, uint16_t *xp, int T, int H, int Hp
 
 hipError_t launch_rmsnorm(const uint16_t *x, const float *weight, const int *pos, uint16_t *t_out,
                           int T, int H, hipStream_t s) {
-  rmsnorm_kernel<<<T, 256, 0, s>>>(x, weight, pos, t_out, H);
+  if (norm_wave_per_token(T, H))
+    rmsnorm_kernel<64><<<(T + 3) / 4, 256, 0, s>>>(x, weight, pos, t_out, T, H);
+  else
+    rmsnorm_kernel<256><<<T, 256, 0, s>>>(x, weight, pos, t_out, T, H);
   return hipGetLastError();
 }
 

@@ -475,3 +475,36 @@ def test_split_router_gives_the_same_bits(E, H):
         ids = dti.download((T, 4), np.int32)
         assert (ids[pos >= 0] >= 0).all() and (ids[pos < 0] == -1).all()
         m.close()
+
+
+@pytest.mark.parametrize("H", [32, 480, 512, 544, 1024, 1056, 4096, 4128])
+def test_norm_at_the_edges_of_its_threads(H):
+    """Rows of the norm at the edges of a wave's and a workgroup's pieces and held registers, and
+    token counts that leave a last workgroup short: the router behind it finds the oracle's ids (which
+    takes the oracle's normalised rows, but for near ties), the block the oracle's result."""
+    rng = np.random.default_rng(H)
+    for T in (1, 3, 65, 70) + ((1023, 1026) if H in (544, 1024) else ()):
+        sh = synth.LayerShape("n", T, H, 64, 8)
+        L = bf16_layer(sh, seed=H + T)
+        m = make_moe(sh, L, T)
+        x = synth.round_bf16((L["x"] * rng.uniform(0.5, 4.0, (T, 1))).astype(np.float32))
+        rw = synth.round_bf16((1 + 0.1 * rng.standard_normal(H)).astype(np.float32))
+        pos = np.zeros(T, np.int32)
+        pos[2::3] = -1
+        m.upload_norm(0, rw)
+        dx = abi.DevBuf.from_numpy(synth.to_bf16_bits(x))
+        m.block_forward(0, dx, abi.DevBuf.from_numpy(pos), T)
+        doff, dperm = abi.DevBuf(9 * 4), abi.DevBuf(T * 16)
+        m.get_dispatch(doff, dperm, T)
+        abi.sync()
+        _, ti, _ = ob.router(ob.round_to_bf16(ob.rmsnorm(x, rw)), pos, L["w_router"], L["b_router"], 4)
+        off, perm, _ = ob.dispatch(ti, pos, 8)
+        assert np.array_equal(doff.download((9,), np.int32), off)
+        assert np.array_equal(dperm.download((T * 4,), np.int32)[:off[-1]], perm)
+        got = synth.from_bf16_bits(dx.download((T, H), np.uint16))
+        rows = np.arange(T)[-70:]
+        want, _ = ob.ffn_block(np.ascontiguousarray(x[rows]), np.ascontiguousarray(pos[rows]), rw, *[L[k] for k in W], 4,
+                               sh.limit, mode=ob.ROUND_ACT_BF16 | ob.PAR_TOKENS)
+        assert np.all(np.abs(got[rows] - want) <= 2e-2 + 2.0 ** -7 * np.abs(want)), T  # one bf16 step on top of the layer's bar
+        assert np.array_equal(got[pos < 0], x[pos < 0])
+        m.close()

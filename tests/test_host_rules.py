@@ -10,6 +10,7 @@ from gpt_oss_amd import build
 SOURCE = """
 #include "%s/moe_internal.h"
 extern "C" int split_router_tokens(int E_pad, int H) { return moe::split_router_tokens(E_pad, H); }
+extern "C" int norm_wave_per_token(int T, int H) { return moe::norm_wave_per_token(T, H); }
 """ % build.CSRC
 
 
@@ -31,3 +32,10 @@ def test_router_splits_where_it_gains(rules, E_pad, H, tokens):
     """The router's first pass as a launch of its own costs small matrices more than it gains
     (times in moe_internal.h)."""
     assert rules.split_router_tokens(E_pad, H) == tokens
+
+
+@pytest.mark.parametrize("T,H,wave", [(1, 32, 1), (7168, 256, 1), (1, 512, 1), (64, 544, 0), (1023, 1024, 0),
+                                      (1024, 1024, 1), (7168, 1056, 0), (7168, 2880, 0)])
+def test_norm_of_short_rows_takes_a_wave(rules, T, H, wave):
+    """A workgroup per token of short rows is mostly idle threads (times in norm.hip)."""
+    assert rules.norm_wave_per_token(T, H) == wave
