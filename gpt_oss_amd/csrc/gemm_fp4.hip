@@ -229,7 +229,7 @@ __device__ __forceinline__ void gemm_tile(const uint4 *__restrict__ a_frag,  // 
   // (in a ring of 4 the second is the last that runs, and reads no further rows).  The half-height
   // kernels share three of those properties (two workgroups per CU, scattered DMA in
   // gate_up, the mixed count).  tests/test_counted_waits.py holds the counts against the built code,
-  // and the tests that repeat calls at 512, 4096, 6144 and 7168 tokens look for other bits.
+  // and test_large_batches_repeat_bit_for_bit looks for other bits in all of them.
   constexpr int WAIT_DMA_FILL = LPS * (R - 2) + LA;  // A(0), A(0..R-1) issued
   constexpr int WAIT_DMA_STEP = LPS * (R - 2);       // B(ks+1), and with it A(ks+1), at step ks
 

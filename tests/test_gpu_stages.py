@@ -325,14 +325,13 @@ def test_router_nan_row():
 # ---------------- repeatability of the large-batch kernels ----------------
 
 def test_large_batches_repeat_bit_for_bit():
-    """The GEMMs' main loop waits for its operands by counting outstanding loads
-    (loads complete in issue order).  4096 tokens at the 20B shape run every
-    tile height and both narrow last column tiles (row split 2 in gate_up, 4 in
-    down); twelve calls in a row must give the same bits, with bf16 and with
-    MXFP4 weights, so must 7168 tokens under Zipf routing (one expert with 28
-    row tiles), 512 tokens with either format, whose weights go past the caches
-    (MXFP4: tiles of 128 rows, two workgroups per CU), and so must the FFN block
-    at 48 tokens."""
+    """The GEMMs' main loop waits for its operands by counting outstanding loads (loads
+    complete in issue order).  Twelve calls in a row must give the same bits, with bf16 and with
+    MXFP4 weights: 4096 tokens at the 20B shape, which run every tile height and both narrow
+    last column tiles (row split 2 in gate_up, 4 in down); 7168 tokens under Zipf routing (one
+    expert with 28 row tiles of 256); 512 and 256 tokens, whose weights go past the caches; 200 tokens
+    at 8 experts.  With MXFP4 these are all three of its tile kernels: tiles of 128 rows, two
+    workgroups per CU, with either product, and tiles of 256.  So must the FFN block at 48 tokens."""
     sh = synth.CONFIGS["c2"]
     T = sh.tokens
     wr, br = (synth.round_bf16(a) for a in synth.make_router(sh))
@@ -357,30 +356,54 @@ def test_large_batches_repeat_bit_for_bit():
                 first = got
                 assert np.isfinite(got).all()
             assert np.array_equal(got, first), f"call {i}: a repeated call gave other bits"
-    few = 512
-    for m in (m16, m4):
+    kernels = set()
+    for few in (512, 256):
+        for m, fp4 in ((m16, False), (m4, True)):
+            kernels.add(abi.batch_kernel(sh.hidden, sh.inter, sh.experts, few, fp4)[:2])
+            for i in range(12):
+                dout.memset(0xFF)
+                m.forward(0, dx, None, few, dout)
+                abi.sync()
+                got = dout.download((few, sh.hidden), np.float32)
+                assert np.array_equal(got, first[:few]), f"{few} tokens, MXFP4 {fp4}, call {i}: other bits"
+    # 8 experts: one workgroup per CU
+    m8 = abi.Moe(sh.hidden, sh.inter, 8, max_tokens=200, swiglu_limit=sh.limit, layers=2)
+    w1, w2 = ob.mxfp4_dequant(b1k[:8], s1[:8]), ob.mxfp4_dequant(b2k[:8], s2[:8])
+    m8.upload_layer_mxfp4(0, wr[:8], br[:8], b1k[:8], s1[:8], b1[:8], b2k[:8], s2[:8], b2[:8])
+    m8.upload_layer(1, wr[:8], br[:8], w1, b1[:8], w2, b2[:8])
+    del w1, w2
+    first8 = None
+    for layer in (0, 1):
+        kernels.add(abi.batch_kernel(sh.hidden, sh.inter, 8, 200, layer == 0, 2)[:2])
         for i in range(12):
             dout.memset(0xFF)
-            m.forward(0, dx, None, few, dout)
+            m8.forward(layer, dx, None, 200, dout)
             abi.sync()
-            got = dout.download((few, sh.hidden), np.float32)
-            assert np.array_equal(got, first[:few]), f"{few} tokens, call {i}: other bits"
+            got = dout.download((200, sh.hidden), np.float32)
+            if first8 is None:
+                first8 = got
+                assert np.isfinite(got).all()
+            assert np.array_equal(got, first8), f"8 experts, layer {layer}, call {i}: other bits"
+    m8.close()
+    assert kernels == {("bf16_gemm_kernel", 256), ("grouped_gemm_kernel", 128), ("grouped_gemm_kernel", 256),
+                       ("fp4_gemm_kernel", 128)}
     # 7168 tokens with Zipf routing: up to 28 row tiles on one expert, the deepest XCD ranges
     z = synth.CONFIGS["c3b"]
     T3 = z.tokens
     m4.close()
-    mz = abi.Moe(z.hidden, z.inter, z.experts, max_tokens=T3, swiglu_limit=z.limit)
+    mz = abi.Moe(z.hidden, z.inter, z.experts, max_tokens=T3, swiglu_limit=z.limit, layers=2)
     wrz, brz = (synth.round_bf16(a) for a in synth.make_router(z))
     w1, w2 = ob.mxfp4_dequant(b1k, s1), ob.mxfp4_dequant(b2k, s2)
     mz.upload_layer(0, wrz, brz, w1, b1, w2, b2)
+    mz.upload_layer_mxfp4(1, wrz, brz, b1k, s1, b1, b2k, s2, b2)
     del w1, w2
     xz = synth.round_bf16(synth.make_activations(z))
     dxz = abi.DevBuf.from_numpy(synth.to_bf16_bits(xz))
     doz = abi.DevBuf(T3 * z.hidden * 4)
     firstz = None
-    for i in range(12):
+    for i in range(24):
         doz.memset(0xFF)
-        mz.forward(0, dxz, None, T3, doz)
+        mz.forward(i // 12, dxz, None, T3, doz)
         abi.sync()
         got = doz.download((T3, z.hidden), np.float32)
         if firstz is None:

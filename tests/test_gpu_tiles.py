@@ -1,7 +1,8 @@
-"""The grouped GEMMs at the edges of their row tiles: 256 rows, and 128 rows where
-the weights are MXFP4 and there are tiles enough; weights read through the caches
-and past them (few rows per expert and more than 256 MiB of matrices in the handle);
-full, half and quarter column tiles.
+"""The grouped GEMMs at the edges of their row tiles: of 256 and of 128 rows with either
+weight format and, with MXFP4, either product; weights read through the caches and
+past them (few rows per expert and more than 256 MiB of matrices in the handle);
+full, half and quarter column tiles.  Which kernel a case runs is asserted, so that a
+line moved elsewhere cannot empty it.
 
 Bars as in test_gpu_parity.py: max-abs 2e-2 and rel-L2 1e-3 of the oracle on the
 same inputs; the two weight formats, whose tiles differ, bit for bit."""
@@ -14,8 +15,12 @@ from oracle import binding as ob
 pytestmark = pytest.mark.gpu
 
 E = 32
-FEW = (1, 31, 32, 33, 63, 64, 65, 95, 96, 97, 127, 128, 129, 160, 161, 255, 256, 257)  # 1823 rows: 57 per expert
-MANY = FEW + (288, 383, 384, 385, 512, 513, 640, 800, 1024)  # 6752 rows: 211 per expert
+FEW = (1, 31, 32, 33, 63, 64, 65, 95, 96, 97, 127, 128, 129, 160, 161, 256, 257)  # 1795 rows: 56 per expert
+MANY = FEW + (255, 288, 383, 384, 385, 512, 513, 640, 800, 1024)  # 6979 rows: 218 per expert
+BF16, FP4, FP4_MANY = "bf16_gemm_kernel", "grouped_gemm_kernel", "fp4_gemm_kernel"
+# kernel, rows of a tile, past the caches: MXFP4 and bf16 weights that the caches hold, then that they do not
+ROUTES = {FEW: [(FP4, 128, False), (BF16, 256, False), (FP4, 128, True), (BF16, 256, True)],
+          MANY: [(FP4_MANY, 128, False), (BF16, 128, False), (FP4_MANY, 128, False), (BF16, 256, True)]}
 
 
 @pytest.mark.parametrize("rows", [FEW, MANY], ids=["few", "many"])
@@ -37,7 +42,8 @@ def test_row_tiles(rows, H, IM):
     dtv, dout = abi.DevBuf.from_numpy(tv), abi.DevBuf(T * H * 4)
     got = []
     many = int((256 << 20) / (3 * H * IM * E * 17 / 32)) + 1  # MXFP4 layers from which the weights are read past the caches
-    for fp4, layers in ((True, 1), (False, 1), (True, many), (False, many * 17 // 64 + 1)):
+    for (fp4, layers), route in zip(((True, 1), (False, 1), (True, many), (False, many * 17 // 64 + 1)), ROUTES[rows]):
+        assert abi.batch_kernel(H, IM, E, T, fp4, layers) == route
         m = abi.Moe(H, IM, E, max_tokens=T, swiglu_limit=sh.limit, layers=layers)
         for i in range(layers):
             if fp4:
@@ -71,13 +77,16 @@ def test_row_tiles(rows, H, IM):
     assert np.linalg.norm(d) <= 1e-3 * np.linalg.norm(want)
 
 
-@pytest.mark.parametrize("n_experts,IM,T", [(16, 2880, 735), (16, 2880, 736), (32, 2048, 768), (32, 2048, 769),
-                                            (32, 2048, 1280), (32, 2048, 1281), (32, 2048, 2048), (32, 2048, 2049)])
-def test_sides_of_the_lines(n_experts, IM, T):
-    """Tiles of 128 rows under MXFP4 weights (16 experts, 23 column tiles, 735 and 736
-    tokens) and either side of the lines up to which weights that exceed 256 MiB are
-    read past the caches (96 rows per expert in tiles of 128, 256 in tiles of 256):
-    the two weight formats bit for bit, and the oracle."""
+@pytest.mark.parametrize("n_experts,IM,T,fp4_route,bf16_route", [
+    (22, 2880, 300, (FP4, 256, False), (BF16, 256, True)), (23, 2880, 300, (FP4, 128, True), (BF16, 256, True)),
+    (32, 2048, 511, (FP4, 128, True), (BF16, 256, True)), (32, 2048, 512, (FP4_MANY, 128, True), (BF16, 256, True)),
+    (32, 2048, 768, (FP4_MANY, 128, True), (BF16, 256, True)), (32, 2048, 769, (FP4_MANY, 128, False), (BF16, 256, True)),
+    (32, 2048, 2048, (FP4_MANY, 128, False), (BF16, 256, True)), (32, 2048, 2049, (FP4_MANY, 128, False), (BF16, 256, False))])
+def test_sides_of_the_lines(n_experts, IM, T, fp4_route, bf16_route):
+    """Matrices that exceed 256 MiB, on either side of the lines to tiles of 128 rows under
+    MXFP4 weights (512 tiles of one row tile per expert), to the other product (64 rows per
+    expert), and up to which weights are read past the caches (96 rows per expert with MXFP4,
+    256 with bf16): the two weight formats bit for bit, and the oracle."""
     H = 64
     sh = synth.LayerShape("lines", T, H, IM, n_experts)
     x = synth.round_bf16(synth.make_activations(sh))
@@ -87,7 +96,8 @@ def test_sides_of_the_lines(n_experts, IM, T):
     w1, w2 = ob.mxfp4_dequant(b1k, s1), ob.mxfp4_dequant(b2k, s2)
     many = int((256 << 20) / (3 * H * IM * n_experts * 17 / 32)) + 1
     got = []
-    for fp4, layers in ((True, many), (False, many * 17 // 64 + 1)):
+    for fp4, layers, route in ((True, many, fp4_route), (False, many * 17 // 64 + 1, bf16_route)):
+        assert abi.batch_kernel(H, IM, n_experts, T, fp4, layers) == route
         m = abi.Moe(H, IM, n_experts, max_tokens=T, swiglu_limit=sh.limit, layers=layers)
         for i in range(layers):
             if fp4:
@@ -105,14 +115,20 @@ def test_sides_of_the_lines(n_experts, IM, T):
     assert np.linalg.norm(d) <= 1e-3 * np.linalg.norm(want)
 
 
-@pytest.mark.parametrize("H,IM", [(64, 64), (256, 320), (448, 64), (320, 384), (576, 448)])
-def test_reduction_depths(H, IM):
-    """Reductions of 1 to 9 double steps of 64, shorter and longer than the rings of
-    the loads in front of them, under row tiles of 1 to 8 blocks and full, three-quarter,
-    half and quarter column tiles: the weight formats bit for bit, and the oracle."""
+@pytest.mark.parametrize("H,IM,n_experts,fp4_route,bf16_rows", [
+    (H, IM, n, r, b) for H, IM in ((64, 64), (256, 320), (448, 64), (320, 384), (576, 448))
+    for n, r, b in ((12, (FP4_MANY, 128), 128), (32, (FP4, 256), 256)) + (((176, (FP4, 128), 256),) if IM > 64 else ())])
+def test_reduction_depths(H, IM, n_experts, fp4_route, bf16_rows):
+    """Reductions of 1 to 9 double steps of 64, shorter and longer than the rings of the
+    loads in front of them, under full, three-quarter, half and quarter column tiles and
+    every height of row tile: 12 experts give tiles of 1 to 4 blocks in either format, 32 of 1 to 8,
+    176 of 1 to 4 with MXFP4 under the product of few rows per expert.  The weight
+    formats bit for bit, and the oracle."""
     rng = np.random.default_rng(H + IM)
-    rows = rng.permutation([1, 33, 65, 97, 129, 161, 193, 225, 256, 300, 385, 15])
-    n_experts = len(rows)
+    rows = [1, 33, 65, 97, 129, 161, 193, 225, 256, 300, 385, 15]
+    if n_experts == 176:
+        rows += [17] * 100
+    rows = rng.permutation(rows + [0] * (n_experts - len(rows)))
     ids = np.repeat(np.arange(n_experts), rows).astype(np.int32)
     T = -(-len(ids) // 4)
     ids = rng.permutation(np.concatenate([ids, np.full(4 * T - len(ids), -1, np.int32)])).reshape(T, 4)
@@ -125,6 +141,8 @@ def test_reduction_depths(H, IM):
     w1, w2 = ob.mxfp4_dequant(b1k, s1), ob.mxfp4_dequant(b2k, s2)
     dx, dti = abi.DevBuf.from_numpy(synth.to_bf16_bits(x)), abi.DevBuf.from_numpy(ids)
     dtv, dout = abi.DevBuf.from_numpy(tv), abi.DevBuf(T * H * 4)
+    assert abi.batch_kernel(H, IM, n_experts, T, True)[:2] == fp4_route
+    assert abi.batch_kernel(H, IM, n_experts, T, False)[:2] == (BF16, bf16_rows)
     got = []
     for fp4 in (True, False):
         m = abi.Moe(H, IM, n_experts, max_tokens=T, swiglu_limit=sh.limit)
@@ -138,7 +156,7 @@ def test_reduction_depths(H, IM):
             abi.sync()
             got.append(dout.download((T, H), np.float32))
         m.close()
-    # a handle with layers of both formats: the dispatch plans tiles of 256 rows for either
+    # a handle with layers of both formats: the dispatch plans tiles of bf16's height for either
     m = abi.Moe(H, IM, n_experts, max_tokens=T, swiglu_limit=sh.limit, layers=2)
     m.upload_layer_mxfp4(0, wr, br, b1k, s1, b1, b2k, s2, b2)
     m.upload_layer(1, wr, br, w1, b1, w2, b2)
@@ -152,7 +170,7 @@ def test_reduction_depths(H, IM):
     m.close()
     for other in got[1:]:
         assert np.array_equal(got[0], other)
-    some = np.unique(np.concatenate([np.nonzero((ids == e).any(1))[0][[0, -1]] for e in range(n_experts)]))
+    some = np.unique(np.concatenate([np.nonzero((ids == e).any(1))[0][[0, -1]] for e in np.nonzero(rows)[0]]))
     want = np.zeros((len(some), H), np.float32)
     for i, t in enumerate(some):
         for k, e in enumerate(ids[t]):
@@ -164,13 +182,17 @@ def test_reduction_depths(H, IM):
     assert np.linalg.norm(d) <= 1e-3 * np.linalg.norm(want)
 
 
-@pytest.mark.parametrize("n_experts,H,IM,T", [(16, 64, 2880, 255), (16, 64, 2880, 256), (8, 64, 2880, 256), (8, 64, 2880, 257),
-                                              (8, 512, 512, 1927), (8, 512, 512, 1928), (8, 512, 512, 3856)])
-def test_sides_of_the_product_lines(n_experts, H, IM, T):
+@pytest.mark.parametrize("n_experts,H,IM,T,fp4_route,bf16_rows", [
+    (16, 64, 2880, 255, (FP4, 256), 256), (16, 64, 2880, 256, (FP4_MANY, 128), 256),
+    (8, 64, 2880, 256, (FP4, 256), 128), (8, 64, 2880, 257, (FP4_MANY, 128), 128),
+    (8, 512, 512, 1927, (FP4_MANY, 128), 128), (8, 512, 512, 1928, (FP4_MANY, 128), 256), (8, 512, 512, 3856, (FP4_MANY, 128), 128)])
+def test_sides_of_the_product_lines(n_experts, H, IM, T, fp4_route, bf16_rows):
     """Either side of the lines between the products of the MXFP4 kernels (64 rows per
     expert, and 128 where there is at most a workgroup per CU) and between row tiles of 128
-    and 256 rows under bf16 weights: the two weight formats, which cross none of these
-    together, bit for bit, stage by stage as well, and the oracle."""
+    and 256 rows under bf16 weights: the two weight formats bit for bit, stage by
+    stage as well, and the oracle."""
+    assert abi.batch_kernel(H, IM, n_experts, T, True)[:2] == fp4_route
+    assert abi.batch_kernel(H, IM, n_experts, T, False)[:2] == (BF16, bf16_rows)
     sh = synth.LayerShape("products", T, H, IM, n_experts)
     x = synth.round_bf16(synth.make_activations(sh))
     wr, br = (synth.round_bf16(a) for a in synth.make_router(sh))
