@@ -28,6 +28,7 @@ SYMBOLS = [
     "moe_version", "moe_dev_alloc", "moe_dev_free", "moe_dev_upload", "moe_dev_download",
     "moe_dev_memset", "moe_dev_sync", "moe_dev_count", "moe_time_forward", "moe_time_forward_each",
     "moe_yardstick_mfma", "moe_yardstick_hbm", "moe_batch_kernel",
+    "moe_yardstick_mfma_16x16x32",
 ]
 
 
@@ -87,6 +88,7 @@ def lib() -> C.CDLL:
         L.moe_batch_kernel.argtypes = [C.POINTER(MoeConfig), ci, ci, C.POINTER(C.c_char_p), C.POINTER(ci),
                                        C.POINTER(ci)]
         L.moe_yardstick_mfma.argtypes = [ci, ci, ci, C.POINTER(C.c_double), C.POINTER(C.c_double)]
+        L.moe_yardstick_mfma_16x16x32.argtypes = L.moe_yardstick_mfma.argtypes
         L.moe_yardstick_hbm.argtypes = [C.c_size_t, ci, C.POINTER(C.c_double), C.POINTER(C.c_double)]
         _lib = L
     return _lib
@@ -157,11 +159,11 @@ def batch_kernel(hidden, inter, experts, tokens, mxfp4, layers=1):
     return name.value.decode(), rows.value, bool(past.value)
 
 
-def yardstick_mfma(n_workgroups: int = 256, iters: int = 20000, data: int = 1):
-    """(TFLOP/s, shader GHz) of a register-resident v_mfma_f32_32x32x16_bf16 loop.
-    data: 0 zeros, 1 operands of unit scale, 2 unit scale against scale 0.02."""
+def yardstick_mfma(n_workgroups: int = 256, iters: int = 20000, data: int = 1, small: bool = False):
+    """(TFLOP/s, shader GHz) of a register-resident v_mfma_f32_32x32x16_bf16 loop, or with small
+    v_mfma_f32_16x16x32_bf16.  data: 0 zeros, 1 operands of unit scale, 2 unit scale against scale 0.02."""
     tf, ghz = C.c_double(), C.c_double()
-    check(lib().moe_yardstick_mfma(n_workgroups, iters, int(data), C.byref(tf), C.byref(ghz)))
+    check((lib().moe_yardstick_mfma_16x16x32 if small else lib().moe_yardstick_mfma)(n_workgroups, iters, int(data), C.byref(tf), C.byref(ghz)))
     return float(tf.value), float(ghz.value)
 
 

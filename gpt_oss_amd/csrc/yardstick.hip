@@ -1,5 +1,5 @@
 // Measured denominators for the rooflines the benchmark reports: what THIS GPU
-// sustains on the instruction the grouped GEMMs are built from, and on a plain
+// sustains on the instructions the grouped GEMMs are built from, and on a plain
 // stream through HBM.  The published peaks (2.5 PFLOP/s dense bf16 at the
 // nominal clock, 8 TB/s) are quoted next to them; these say how much of the
 // distance to those is the kernels' and how much is the machine's.  They play
@@ -9,6 +9,8 @@
 //
 // Nothing here is used by the layer; the entry points allocate and free their
 // own buffers and synchronise with the host.
+#include <type_traits>
+
 #include "moe_internal.h"
 
 namespace moe {
@@ -16,26 +18,33 @@ namespace {
 
 typedef __bf16 ybf16x8 __attribute__((ext_vector_type(8)));
 typedef float yf32x16 __attribute__((ext_vector_type(16)));
+typedef float yf32x4 __attribute__((ext_vector_type(4)));
 
-// 4 waves per workgroup, one per SIMD, each with 16 independent accumulators of
-// v_mfma_f32_32x32x16_bf16 (all 256 accumulation registers; the instruction of gemm.hip.  16x16x32,
-// that of gemm_bf16.hip and gemm_fp4.hip, takes less power: 2030 against 1810 TFLOP/s) and
-// no memory traffic at all.  The operands are pseudo-random values (data 1: unit
+// v_mfma_f32_32x32x16_bf16 (SMALL false: the instruction of gemm.hip) from 4 waves per workgroup, one per
+// SIMD, each with 16 independent accumulators (all 256 accumulation registers), or
+// v_mfma_f32_16x16x32_bf16 (SMALL: that of gemm_bf16.hip and gemm_fp4.hip, which takes less power) from 8 waves
+// with 32 accumulators, as the bf16 kernel has them, and no memory traffic at all.  The operands are pseudo-random values (data 1: unit
 // scale; data 2: unit scale against a scale of 0.02, as activations meet
 // weights in the layer) or zeros (data 0): the clock the matrix cores sustain
 // depends on how many bits toggle.  out[2*wg] = shader clocks, out[2*wg+1] = ticks of the
 // constant 100 MHz clock spent in the loop by the workgroup's first wave.
-__global__ __launch_bounds__(256) void mfma_loop_kernel(int iters, int data, unsigned long long *out,
+template <bool SMALL>
+struct MfmaLoop {
+  static constexpr int THREADS = SMALL ? 512 : 256, NA = SMALL ? 8 : 2, NB = SMALL ? 4 : 2, ACCS = SMALL ? 32 : 16;
+};
+template <bool SMALL>
+__global__ __launch_bounds__(MfmaLoop<SMALL>::THREADS) void mfma_loop_kernel(int iters, int data, unsigned long long *out,
                                                         float *sink) {
-  yf32x16 acc[16];
+  using C = MfmaLoop<SMALL>;
+  typename std::conditional<SMALL, yf32x4, yf32x16>::type acc[C::ACCS];
 #pragma unroll
-  for (int i = 0; i < 16; i++)
+  for (int i = 0; i < C::ACCS; i++)
 #pragma unroll
-    for (int q = 0; q < 16; q++) acc[i][q] = 0.f;
-  ybf16x8 a[2], b[2];
-  uint32_t s = 0x9e3779b9u * (blockIdx.x * 256u + threadIdx.x + 1u);
+    for (int q = 0; q < (SMALL ? 4 : 16); q++) acc[i][q] = 0.f;
+  ybf16x8 a[C::NA], b[C::NB];
+  uint32_t s = 0x9e3779b9u * (blockIdx.x * (uint32_t)C::THREADS + threadIdx.x + 1u);
 #pragma unroll
-  for (int h = 0; h < 2; h++)
+  for (int h = 0; h < C::NA; h++)
 #pragma unroll
     for (int j = 0; j < 8; j++) {
       float u = 0.f, v = 0.f;  // sums of four uniform variates on [-1, 1): bell-shaped, variance 4/3
@@ -49,18 +58,20 @@ __global__ __launch_bounds__(256) void mfma_loop_kernel(int iters, int data, uns
       // data 1: both operands of unit scale; data 2: as the layer's GEMMs see them,
       // activations of unit scale against weights of scale 0.02; data 0: zeros
       a[h][j] = (__bf16)(data ? 0.866f * u : 0.f);
-      b[h][j] = (__bf16)(data == 1 ? 0.866f * v : (data == 2 ? 0.0173f * v : 0.f));
+      if (h < C::NB) b[h][j] = (__bf16)(data == 1 ? 0.866f * v : (data == 2 ? 0.0173f * v : 0.f));
     }
   const unsigned long long c0 = clock64(), t0 = wall_clock64();
   for (int it = 0; it < iters; it++) {
 #pragma unroll
-    for (int i = 0; i < 16; i++)
-      acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i & 1], b[(i >> 1) & 1], acc[i], 0, 0, 0);
+    for (int i = 0; i < C::ACCS; i++) {
+      if constexpr (SMALL) acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i >> 2], b[i & 3], acc[i], 0, 0, 0);
+      else acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i & 1], b[(i >> 1) & 1], acc[i], 0, 0, 0);
+    }
   }
   const unsigned long long c1 = clock64(), t1 = wall_clock64();
   float r = 0.f;
 #pragma unroll
-  for (int i = 0; i < 16; i++) r += acc[i][0];
+  for (int i = 0; i < C::ACCS; i++) r += acc[i][0];
   if (r == 123.456f) sink[0] = r;  // keeps the loop alive
   if (threadIdx.x == 0) {
     out[2 * blockIdx.x] = c1 - c0;
@@ -116,13 +127,8 @@ __global__ __launch_bounds__(256) void read_kernel(const uint4 *__restrict__ src
     }                                                                                                \
   } while (0)
 
-}  // namespace
-}  // namespace moe
-
-using namespace moe;
-
-extern "C" int moe_yardstick_mfma(int n_workgroups, int iters, int data, double *tflops,
-                                  double *shader_ghz) {
+template <bool SMALL>
+int yardstick_mfma(int n_workgroups, int iters, int data, double *tflops, double *shader_ghz) {
   if (n_workgroups < 1 || n_workgroups > 4096 || iters < 1 || iters > (1 << 22) || !tflops)
     return set_error(MOE_ERR_BAD_ARG, "moe_yardstick_mfma: bad arguments");
   int rc = MOE_OK;
@@ -136,10 +142,10 @@ extern "C" int moe_yardstick_mfma(int n_workgroups, int iters, int data, double 
   Y_TRY(hipEventCreate(&e0));
   Y_TRY(hipEventCreate(&e1));
   // an untimed launch of the same length first: the clocks settle under load
-  mfma_loop_kernel<<<n_workgroups, 256>>>(iters, data, out, sink);
+  mfma_loop_kernel<SMALL><<<n_workgroups, MfmaLoop<SMALL>::THREADS>>>(iters, data, out, sink);
   Y_TRY(hipGetLastError());
   Y_TRY(hipEventRecord(e0, nullptr));
-  mfma_loop_kernel<<<n_workgroups, 256>>>(iters, data, out, sink);
+  mfma_loop_kernel<SMALL><<<n_workgroups, MfmaLoop<SMALL>::THREADS>>>(iters, data, out, sink);
   Y_TRY(hipGetLastError());
   Y_TRY(hipEventRecord(e1, nullptr));
   Y_TRY(hipEventSynchronize(e1));
@@ -151,7 +157,8 @@ extern "C" int moe_yardstick_mfma(int n_workgroups, int iters, int data, double 
       clk += (double)host[2 * i];
       ticks += (double)host[2 * i + 1];
     }
-    const double flop = (double)n_workgroups * 4 * iters * 16 * 2.0 * 32 * 32 * 16;
+    const double flop = (double)n_workgroups * (MfmaLoop<SMALL>::THREADS / 64) * iters * MfmaLoop<SMALL>::ACCS * 2.0 *
+                        (SMALL ? 16 * 16 * 32 : 32 * 32 * 16);
     *tflops = flop / (ms * 1e-3) / 1e12;
     if (shader_ghz) *shader_ghz = ticks > 0 ? clk / (ticks * 10.0) : 0.0;  // 100 MHz ticks -> ns
   }
@@ -162,6 +169,19 @@ done:
   (void)hipFree(out);
   (void)hipFree(sink);
   return rc;
+}
+
+}  // namespace
+}  // namespace moe
+
+using namespace moe;
+
+extern "C" int moe_yardstick_mfma(int n_workgroups, int iters, int data, double *tflops, double *shader_ghz) {
+  return yardstick_mfma<false>(n_workgroups, iters, data, tflops, shader_ghz);
+}
+
+extern "C" int moe_yardstick_mfma_16x16x32(int n_workgroups, int iters, int data, double *tflops, double *shader_ghz) {
+  return yardstick_mfma<true>(n_workgroups, iters, data, tflops, shader_ghz);
 }
 
 extern "C" int moe_yardstick_hbm(size_t bytes, int iters, double *copy_gbs, double *read_gbs) {

@@ -297,12 +297,17 @@ int moe_time_forward_each(moe_handle *h, int layer, const uint16_t *x,
  * scale of 0.02, as activations meet weights in the layer; data 0: zeros (the
  * clock the matrix cores sustain depends on the bits that toggle).  Returns
  * TFLOP/s over the launch and the mean shader clock in GHz during the loop.
+ * moe_yardstick_mfma_16x16x32: the same with v_mfma_f32_16x16x32_bf16, the
+ * instruction of the bf16 tile kernels and of MXFP4 batches with many rows per
+ * expert, on 8 waves with 32 accumulators each, iters x 32 per wave.
  *
  * moe_yardstick_hbm: a copy kernel and a read-only kernel over `bytes` of
  * device memory (choose it well above the 256 MB memory-side cache), iters
  * launches each; copy_gbs counts bytes read plus bytes written. */
 int moe_yardstick_mfma(int n_workgroups, int iters, int data, double *tflops,
                        double *shader_ghz);
+int moe_yardstick_mfma_16x16x32(int n_workgroups, int iters, int data,
+                                double *tflops, double *shader_ghz);
 int moe_yardstick_hbm(size_t bytes, int iters, double *copy_gbs, double *read_gbs);
 
 #ifdef __cplusplus

@@ -531,3 +531,10 @@ def test_norm_at_the_edges_of_its_threads(H):
         assert np.all(np.abs(got[rows] - want) <= 2e-2 + 2.0 ** -7 * np.abs(want)), T  # one bf16 step on top of the layer's bar
         assert np.array_equal(got[pos < 0], x[pos < 0])
         m.close()
+
+
+def test_yardstick_of_the_other_product_runs():
+    """v_mfma_f32_16x16x32_bf16 from registers, as test_yardsticks_run."""
+    tf, ghz = abi.yardstick_mfma(256, 2000, data=2, small=True)
+    tf0, _ = abi.yardstick_mfma(256, 2000, data=0, small=True)
+    assert 200 < tf < 2600 and 0.5 < ghz < 3.0 and tf0 > 0.9 * tf
