@@ -670,9 +670,10 @@ using CfgFull = GemmCfg<4, 2, 4, 8, 1>;
 // Tiles half as high, two workgroups per CU.  A step of MXFP4 weights is
 // 4 KB, so that a second tile of the same columns costs next to nothing, and the
 // decode, the fill and the epilogue of one workgroup run under the other's MFMAs.
-// us per layer call, full / half height (2880 x 2880, even routing): 32 experts,
-// 256 tokens 175 / 143, 512: 188 / 172, 1024: 242 / 242, 2048: 427 / 395, 4096:
-// 731 / 725; 128 experts, 768: 533 / 428, 2048: 621 / 551, 3072: 712 / 676.
+// us per layer call, full / half height (2880 x 2880, even routing): 32 experts, 256
+// tokens 175 / 143; 128 experts, 768: 533 / 428.  Runs where an expert has 17 to 63 rows
+// on average and there are 512 tiles of one row tile per expert (32 experts: 129 to 511 tokens);
+// with more rows gemm_fp4.hip has the same tiles and the other product.
 using CfgHalf = GemmCfg<4, 2, 4, 4, 2>;
 static_assert(CfgFull::RBT_MAX * kRowBlock == kTileRows && CfgHalf::RBT_MAX * kRowBlock == kHalfTileRows &&
                   CfgFull::TILE_NB == kGemmTileNb && CfgHalf::TILE_NB == kGemmTileNb,

@@ -21,18 +21,22 @@
 // for more than it takes in that time (six loads behind every second barrier: 489
 // instead of 476 us for gate_up at 4096 tokens and 32 experts).
 //
-// What bounds it.  At thousands of tokens the package's power: the kernel loses clock,
-// 2.4 to 1.7 GHz, whenever all CUs multiply, and variants that keep the matrix cores
-// busier (workgroups that stay and load the next tile under the epilogue of the last
-// one: no time between tiles at all) run at a lower clock and take as long.  So what
-// counts is the energy of a product.  v_mfma_f32_16x16x32_bf16 takes less than
-// 32x32x16 (from registers alone, all CUs, random operands: 2030 against 1810 TFLOP/s)
-// and gives the same bits.  us per layer call at 2880 x 2880, 32 x 32 x 16 with the
-// columns through registers and four waves, which this replaced / the same with
-// 16 x 16 x 32 / this: 4096 tokens, 32 experts 830 / 816 / 808; 7168, Zipf's routing
-// (exponent 1.2) 1406 / 1347 / 1323; 6144, 128 experts 1662 / 1649 / 1645; 512, Zipf's
-// 366 / 367 / 362; 672 of 896 rows active 345 / 344 / 342.  With few rows per expert it
-// is HBM: a tile's fill and epilogue are not under its stream.
+// What bounds it.  At thousands of tokens two things, neither of them alone.  The tile
+// plan: the flops of 4096 tokens at 32 experts take 457 + 276 us as ragged experts and 402 +
+// 220 as four dense ones (the same kernel and operands; down's 948 tiles are 3.7 rounds of the
+// CUs, 768 are 3).  The clock, which falls from 2.4 to 1.7-2.1 GHz whenever all CUs multiply
+// numbers that toggle: with zero weights the ragged experts take 408 + 252.  So the
+// energy of a product counts.  v_mfma_f32_16x16x32_bf16 takes less than 32x32x16 (from
+// registers alone, all CUs: 2030-2050 against 1810-1830 TFLOP/s with operands of unit scale,
+// 1955-1994 against 1670-1840 with weights of 0.02) and gives the same bits.  Workgroups that
+// stay and load the next tile under the epilogue of the last one spend no time between
+// tiles, but their steps take longer, 1033 instead of 931 clocks.  us per layer call at
+// 2880 x 2880, 32 x 32 x 16 with the columns through registers and four waves, which this replaced / the
+// same with 16 x 16 x 32 / this: 4096 tokens, 32 experts 830 / 816 / 808; 7168, Zipf's routing
+// (exponent 1.2) 1406 / 1347 / 1323.  6144 tokens at 128 experts (1662 / 1649 / 1645), 512 tokens, Zipf's (366 /
+// 367 / 362), and 672 of 896 rows active (345 / 344 / 342) gained no more than two runs of one
+// side differ.  With few rows per expert it is HBM: a tile's fill and epilogue are not under
+// its stream.
 #include <type_traits>
 
 #include "moe_internal.h"

@@ -2,10 +2,9 @@
 // kernels of gemm.hip (whose header has the data layout, the tiling, the tile order and
 // the loads) at tiles of 128 rows with v_mfma_f32_16x16x32_bf16 in place of 32x32x16.
 //
-// At thousands of tokens the package's power is the bound: the clock falls from 2.4 to 1.7 GHz
-// whenever all CUs multiply, so that the energy of a product counts.  From registers
-// alone, with random operands on all CUs, 16x16x32 runs at 2030 TFLOP/s and 32x32x16 at 1810;
-// the sums are the same bits.  us per layer call, 32x32x16 / this: 32 experts, 512 tokens 174 / 162,
+// At thousands of tokens the clock falls from 2.4 to 1.7-2.1 GHz whenever all CUs multiply, so
+// that the energy of a product counts.  From registers alone, on all CUs, 16x16x32 runs at
+// 2030-2050 TFLOP/s and 32x32x16 at 1810-1830 (operands of unit scale); the sums are the same bits.  us per layer call, 32x32x16 / this: 32 experts, 512 tokens 174 / 162,
 // 4096: 745 / 695; 7168, Zipf's routing (exponent 1.2) 1215 / 1128; 128 experts, 3072: 688 / 655.
 // Where the time is that of loads the smaller products are more instructions for nothing (fp4_many_rows).
 #include "gemm_common.h"

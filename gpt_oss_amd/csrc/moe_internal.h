@@ -231,7 +231,10 @@ inline int gemm_tile_cap(int T, int E, int tile_rows) { return T * kTopK / tile_
 // 397, 3072 (96) 688 / 655.  With a workgroup on every CU or fewer, a wave has its SIMD to
 // itself and the smaller products' instructions show until experts have more than one tile:
 // 8 experts, 150 tokens (75 rows) 70 / 76, 256 (128) 93 / 99, 300 (150) 105 / 100, 400 128 / 115; 4
-// experts, 100 (100) 78 / 86, 150 (150) 88 / 75.  w1_rows: rows of an expert's gate_up matrix.
+// experts, 100 (100) 78 / 86, 150 (150) 88 / 75.  Over 500 batches of 4 to 128 experts, sides of 512 to 2880, even
+// and Zipf's routing, from 64 rows on, the time is 0.7 to 1.02 of that with gemm.hip, but for: 32 experts,
+// 1024 x 2048 and 512 x 2048 (two workgroups per CU exactly), 64 to 80 rows 1.03 to 1.04; 4 experts, 2880 x
+// 2880, 260 to 380 rows (276 tiles on 256 CUs) 1.00 to 1.10.  w1_rows: rows of an expert's gate_up matrix.
 constexpr int kFp4ManyRows = 64;
 inline bool fp4_many_rows(int T, int E, int w1_rows) {
   const int n_ct = (w1_rows / kRowBlock + kGemmTileNb - 1) / kGemmTileNb;
