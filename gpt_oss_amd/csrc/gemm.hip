@@ -47,7 +47,7 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 // Epilogue of the gate_up GEMM: SwiGLU of the (gate, up) accumulator pairs, bf16,
 // stored in the fragment order the down GEMM reads as its row operand.
-template <int RBT, int RS, typename C>
+template <int RBT, int RS, typename C, bool STREAM>
 __device__ __forceinline__ void gate_up_epilogue(const f32x16 (&acc)[RBT][C::NBW], void *__restrict__ outp,
                                                  int out_ld, float limit, int rb0, int rbt, int nb0,
                                                  int nb_valid, int cw, int rg, int lane) {
@@ -61,7 +61,7 @@ __device__ __forceinline__ void gate_up_epilogue(const f32x16 (&acc)[RBT][C::NBW
   // fragment lane (g % 2)*32 + t of k block g / 2.  One exchange between the
   // lane halves (v_permlane32_swap) per dword completes the 16 bytes of every
   // fragment lane; nothing goes through LDS.
-  uint4 *act = reinterpret_cast<uint4 *>(outp);
+  u32x4 *act = reinterpret_cast<u32x4 *>(outp);
   const int kb2_total = out_ld / kFragK;
   const int P0 = (nb0 + cw * NBW) >> 1;                // first pair of this wave
   const int pairs_valid = (nb_valid - cw * NBW) >> 1;  // >= 1 here
@@ -80,13 +80,13 @@ __device__ __forceinline__ void gate_up_epilogue(const f32x16 (&acc)[RBT][C::NBW
               swiglu_shifted(acc[i][2 * p][4 * g + 2 * d], acc[i][2 * p + 1][4 * g + 2 * d], limit),
               swiglu_shifted(acc[i][2 * p][4 * g + 2 * d + 1], acc[i][2 * p + 1][4 * g + 2 * d + 1],
                              limit));
-      uint4 *dst = act + ((size_t)(rb0 + blk) * kb2_total + 2 * (P0 + p)) * 64 + lane;
+      u32x4 *dst = act + ((size_t)(rb0 + blk) * kb2_total + 2 * (P0 + p)) * 64 + lane;
 #pragma unroll
       for (int kb = 0; kb < 2; kb++) {
         // upper lane half of registers 8kb .. 8kb+3 <-> lower lane half of 8kb+4 .. 8kb+7
         const u32x2 s0 = __builtin_amdgcn_permlane32_swap(pk[2 * kb][0], pk[2 * kb + 1][0], false, false);
         const u32x2 s1 = __builtin_amdgcn_permlane32_swap(pk[2 * kb][1], pk[2 * kb + 1][1], false, false);
-        if (p < pairs_valid) dst[kb * 64] = make_uint4(s0[0], s1[0], s0[1], s1[1]);
+        if (p < pairs_valid) store_output<STREAM>(&dst[kb * 64], u32x4{s0[0], s1[0], s0[1], s1[1]});
       }
     }
   }
@@ -335,9 +335,9 @@ __device__ __forceinline__ void gemm_tile(const uint4 *__restrict__ a_frag,  // 
       const int idx = t * 64 + lane;
       const int r = idx / (NBW * 8);
       const int c4 = idx % (NBW * 8);
-      const float4 v = *reinterpret_cast<const float4 *>(ef + r * LD + 4 * c4);
+      const f32x4 v = *reinterpret_cast<const f32x4 *>(ef + r * LD + 4 * c4);
       if (cw * NBW + c4 / 8 < nb_valid)
-        *reinterpret_cast<float4 *>(y + (row0 + r) * out_ld + col0 + 4 * c4) = v;
+        store_output<STREAM>(reinterpret_cast<f32x4 *>(y + (row0 + r) * out_ld + col0 + 4 * c4), v);
     }
   }
 }
@@ -592,7 +592,7 @@ __device__ __forceinline__ void gemm_tile_gl(const uint4 *__restrict__ x_rows,  
   static_left<LEFT>(n_steps - ks0, [&](auto u_c) { step(u_c, IC<1>{}, ks0 + decltype(u_c)::value); });
 
   if (cw * NBW >= nb_valid) return;  // a wave without columns (last column tile only)
-  gate_up_epilogue<RBT, RS, C>(acc, outp, out_ld, limit, rb0, rbt, nb0, nb_valid, cw, rg, lane);
+  gate_up_epilogue<RBT, RS, C, STREAM>(acc, outp, out_ld, limit, rb0, rbt, nb0, nb_valid, cw, rg, lane);
 }
 
 template <typename C, bool GATE_UP, bool STREAM>

@@ -309,14 +309,14 @@ __device__ __forceinline__ void wave_tile(const Tile &t, uint32_t lds0) {
     if constexpr (GATE_UP) {
       // bf16 fragments, as the down GEMM reads them: one exchange of 16-lane rows between the two
       // row groups of a block per dword gives every lane 8 consecutive columns of a row.
-      uint4 *act = reinterpret_cast<uint4 *>(t.out);
+      u32x4 *act = reinterpret_cast<u32x4 *>(t.out);
       const int kb2_total = t.N / kFragK;
       const int P0 = (t.nb0 >> 1) + wn;
 #pragma unroll
       for (int i = 0; i < RBW; i++) {
         const int blk = i * S + rg;
         if (S > 2 && blk >= t.rbt) break;
-        uint4 *dst = act + ((size_t)(t.rb0 + blk) * kb2_total + 2 * P0) * 64 + lane;
+        u32x4 *dst = act + ((size_t)(t.rb0 + blk) * kb2_total + 2 * P0) * 64 + lane;
 #pragma unroll
         for (int c = 0; c < 2; c++) {
           uint32_t pk[2][2];
@@ -328,7 +328,7 @@ __device__ __forceinline__ void wave_tile(const Tile &t, uint32_t lds0) {
                                    swiglu_shifted(acc[2 * i + h][c][2 * d + 1], acc[2 * i + h][c + 2][2 * d + 1], t.limit));
           const u32x2 s0 = __builtin_amdgcn_permlane16_swap(pk[0][0], pk[1][0], false, false);
           const u32x2 s1 = __builtin_amdgcn_permlane16_swap(pk[0][1], pk[1][1], false, false);
-          dst[c * 64] = make_uint4(s0[0], s1[0], s0[1], s1[1]);
+          store_output<STREAM>(&dst[c * 64], u32x4{s0[0], s1[0], s0[1], s1[1]});
         }
       }
     } else {
@@ -349,8 +349,8 @@ __device__ __forceinline__ void wave_tile(const Tile &t, uint32_t lds0) {
               const f32x4 u = acc[2 * i + h][c], v = acc[2 * i + h][c + 1];
               const u32x2 x = __builtin_amdgcn_permlane16_swap(__float_as_uint(u[q]), __float_as_uint(v[q]), false, false);
               float *dst = y + ((size_t)(t.rb0 + blk) * kRowBlock + 16 * h + row + q) * t.N + col + 16 * c;
-              dst[0] = __uint_as_float(x[0]);
-              dst[4 * (size_t)t.N] = __uint_as_float(x[1]);
+              store_output<STREAM>(dst, __uint_as_float(x[0]));
+              store_output<STREAM>(dst + 4 * (size_t)t.N, __uint_as_float(x[1]));
             }
       }
     }

@@ -37,6 +37,7 @@ __device__ __forceinline__ void static_left(int left, F &&f) {
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));

@@ -12,8 +12,6 @@
 namespace moe {
 namespace {
 
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-
 // The product of 16 rows and 16 columns over 32 k.  The weights are the first operand,
 // so a lane ends with four consecutive columns of one row.
 __device__ __forceinline__ void mma(f32x4 &acc, bf16x8 rows, bf16x8 cols) {
