@@ -48,6 +48,13 @@ struct PlanOut {
   TileDesc *tiles_gate_up, *tiles_down;
   int tile_cap_gate_up, tile_cap_down;
   int tile_rb;  // row blocks of the tallest tile
+  int nb[2];    // column blocks of an expert's matrices, gate_up and down (0: no tile tables)
+  bool wide;    // tile_width
+  // column tiles of GEMM g over an expert whose tallest tile has so many row blocks
+  __device__ __forceinline__ int col_tiles(int g, int height) const {
+    const int width = tile_width(height, wide);
+    return (nb[g] + width - 1) / width;
+  }
 };
 
 // The tiles of expert ee in the tile sequences of both GEMMs.  An expert's row
@@ -61,16 +68,17 @@ struct PlanOut {
 // down GEMM's 1.75 -> 1.51 GB, durations unchanged; experts with up to
 // kRowTileGroup row tiles (even routing at 4096 tokens) are laid out as before.
 // One wave; its lanes run over the expert's tiles of both GEMMs in one sweep.
-__device__ __forceinline__ void write_expert_tiles(int ee, int nmt, int rbe, int exe, int rowblk, int first,
-                                                   int lane, int n_ct_gate_up, int n_ct_down,
-                                                   const PlanOut &out) {
+__device__ __forceinline__ void write_expert_tiles(int ee, int nmt, int rbe, int exe, int rowblk, int first_up,
+                                                   int first_down, int lane, const PlanOut &out) {
   if (nmt == 0) return;
-  const int n_up = nmt * n_ct_gate_up, n = n_up + nmt * n_ct_down;
+  const int height = rbe + (exe ? 1 : 0), width = tile_width(height, out.wide);
+  const int n_ct_up = out.col_tiles(0, height), n_ct_down = out.col_tiles(1, height);
+  const int n_up = nmt * n_ct_up, n = n_up + nmt * n_ct_down;
   for (int ii = lane; ii < n; ii += 64) {
     const bool g = ii >= n_up;
     const int i = g ? ii - n_up : ii;
-    const int L = first * (g ? n_ct_down : n_ct_gate_up) + i;
-    const int n_ct = g ? n_ct_down : n_ct_gate_up;
+    const int L = (g ? first_down : first_up) + i;
+    const int n_ct = g ? n_ct_down : n_ct_up;
     const int n_grp = (nmt + kRowTileGroup - 1) / kRowTileGroup;
     const int gs = nmt / n_grp, gx = nmt - gs * n_grp;  // the first gx groups hold gs + 1 row tiles
     const int big = gx * (gs + 1) * n_ct;               // tiles of those groups
@@ -88,8 +96,9 @@ __device__ __forceinline__ void write_expert_tiles(int ee, int nmt, int rbe, int
     const int mt = grp * gs + min(grp, gx) + (r - nt * gsz);
     TileDesc d;
     d.e = ee;
-    d.nt = nt;
-    d.rbt = rbe + (mt < exe ? 1 : 0);
+    d.nb0 = nt * width;
+    d.nbt = (uint16_t)min(width, out.nb[g] - nt * width);
+    d.rbt = (uint16_t)(rbe + (mt < exe ? 1 : 0));
     d.rb0 = rowblk + mt * rbe + min(mt, exe);
     if (L < (g ? out.tile_cap_down : out.tile_cap_gate_up)) (g ? out.tiles_down : out.tiles_gate_up)[L] = d;
   }
@@ -98,14 +107,14 @@ __device__ __forceinline__ void write_expert_tiles(int ee, int nmt, int rbe, int
 // write_global: this workgroup stores the plan (offsets, per-expert records,
 // totals, XCD bounds); the others only need the values returned to them.
 // with_tiles: this workgroup also writes the tile tables of all experts.
-__device__ __forceinline__ int build_plan(int count, int E, int n_ct_gate_up, int n_ct_down,
-                                          const PlanOut &out, bool with_tiles, int *ex_count_out,
+__device__ __forceinline__ int build_plan(int count, int E, const PlanOut &out, bool with_tiles, int *ex_count_out,
                                           int *tot_count_out = nullptr, bool write_global = true,
                                           ExpertInfo *info_out = nullptr) {
-  __shared__ int sh_wave[4][4];  // [wave][quantity]: the waves' sums
+  constexpr int kSums = 6;
+  __shared__ int sh_wave[4][kSums];  // [wave][quantity]: the waves' sums
   __shared__ int sh_nmt[256], sh_rb[256], sh_extra[256], sh_rowblk[256];
-  __shared__ int sh_cost[257];   // exclusive prefix of the experts' cost per column tile
-  __shared__ int sh_tiles[257];  // exclusive prefix of their row tiles
+  __shared__ int sh_cost[257];      // exclusive prefix of the experts' cost
+  __shared__ int sh_tiles[2][257];  // exclusive prefix of their tiles in either GEMM
   __shared__ int sh_bound[2][kXcds + 1];
   const int e = threadIdx.x;
   const int lane = e & 63;
@@ -117,29 +126,33 @@ __device__ __forceinline__ int build_plan(int count, int E, int n_ct_gate_up, in
   const int n_mt = (n_rb + out.tile_rb - 1) / out.tile_rb;
   const int rb = n_mt ? n_rb / n_mt : 0;
   const int extra = n_mt ? n_rb - rb * n_mt : 0;
-  // cost of one column tile's worth of the expert's row tiles
+  const int height = rb + (extra ? 1 : 0);
+  const int n_up = n_mt * out.col_tiles(0, height), n_down = n_mt * out.col_tiles(1, height);
+  // cost of kGemmTileNb column blocks' worth of the expert's row tiles: of tiles of any width, whose cost goes by it
   const int cost = n_mt * (kCostPerTile + kCostPerRowBlock * rb) + kCostPerRowBlock * extra;
-  // Exclusive prefix sums over the experts of four quantities at once: rows,
-  // padded rows, row tiles, cost.  In a wave by lane shifts, across the four
+  // Exclusive prefix sums over the experts of six quantities at once: rows,
+  // padded rows, row tiles, cost, tiles of either GEMM.  In a wave by lane shifts, across the four
   // waves through LDS.
-  const int own[4] = {count, n_rb * kRowBlock, n_mt, cost};
-  int incl[4] = {own[0], own[1], own[2], own[3]};
+  const int own[kSums] = {count, n_rb * kRowBlock, n_mt, cost, n_up, n_down};
+  int incl[kSums];
+#pragma unroll
+  for (int i = 0; i < kSums; i++) incl[i] = own[i];
 #pragma unroll
   for (int off = 1; off < 64; off <<= 1) {
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
+    for (int i = 0; i < kSums; i++) {
       const int up = __shfl_up(incl[i], off, 64);
       if (lane >= off) incl[i] += up;
     }
   }
   if (lane == 63) {
 #pragma unroll
-    for (int i = 0; i < 4; i++) sh_wave[w][i] = incl[i];
+    for (int i = 0; i < kSums; i++) sh_wave[w][i] = incl[i];
   }
   __syncthreads();
-  int ex[4], tot[4];
+  int ex[kSums], tot[kSums];
 #pragma unroll
-  for (int i = 0; i < 4; i++) {
+  for (int i = 0; i < kSums; i++) {
     int below = 0, all = 0;
 #pragma unroll
     for (int ww = 0; ww < 4; ww++) {
@@ -160,14 +173,15 @@ __device__ __forceinline__ int build_plan(int count, int E, int n_ct_gate_up, in
     inf.rb = rb;
     inf.tile_base = ex_mt;
     inf.extra = extra;
-    inf.pad_[0] = inf.pad_[1] = 0;
+    inf.tiles0[0] = ex[4];
+    inf.tiles0[1] = ex[5];
     if (e < E && write_global) {
       offsets[e] = ex_count;
       info[e] = inf;
     }
     if (info_out) *info_out = inf;
   }
-  const bool tables = n_ct_gate_up > 0;
+  const bool tables = out.nb[0] > 0;
   if (write_global && !tables && e == 0) {
     offsets[E] = tot_count;
     totals[kTotTiles] = tot_mt;
@@ -183,14 +197,16 @@ __device__ __forceinline__ int build_plan(int count, int E, int n_ct_gate_up, in
     return ex_pad;
   }
   sh_cost[e] = ex_cost;
-  sh_tiles[e] = ex_mt;
+  sh_tiles[0][e] = ex[4];
+  sh_tiles[1][e] = ex[5];
   sh_nmt[e] = n_mt;
   sh_rb[e] = rb;
   sh_extra[e] = extra;
   sh_rowblk[e] = ex_pad / kRowBlock;
   if (e == 0) {
     sh_cost[256] = tot_cost;
-    sh_tiles[256] = tot_mt;
+    sh_tiles[0][256] = tot[4];
+    sh_tiles[1][256] = tot[5];
     offsets[E] = tot_count;
     totals[kTotTiles] = tot_mt;
     totals[kTotRows] = tot_pad;
@@ -202,29 +218,24 @@ __device__ __forceinline__ int build_plan(int count, int E, int n_ct_gate_up, in
   // reaches x/8 of the total (an expert's tiles taken as equally dear: their heights differ by one block at most).
   if (e < 2 * (kXcds + 1)) {
     const int g = e / (kXcds + 1), x = e % (kXcds + 1);
-    const int n_ct = g ? n_ct_down : n_ct_gate_up;
-    const int total_tiles = tot_mt * n_ct;
+    const int total_tiles = tot[4 + g];
     int bound;
     if (x == 0) {
       bound = 0;
     } else if (x == kXcds) {
       bound = total_tiles;
     } else {
-      const long long target = (long long)tot_cost * n_ct * x / kXcds;
+      const long long target = (long long)tot_cost * x;  // kXcds times the cost in front of the boundary
       // last expert whose first tile starts at or before the target
       int lo = 0, hi = 255;
       while (lo < hi) {
         const int mid = (lo + hi + 1) >> 1;
-        if ((long long)sh_cost[mid] * n_ct <= target) lo = mid; else hi = mid - 1;
+        if ((long long)sh_cost[mid] * kXcds <= target) lo = mid; else hi = mid - 1;
       }
       const int c_e = sh_cost[lo + 1] - sh_cost[lo];  // > 0: the search stops on an expert with tiles
-      const int m_e = sh_tiles[lo + 1] - sh_tiles[lo];
-      long long rest = target - (long long)sh_cost[lo] * n_ct;
-      const int ct = c_e ? (int)(rest / c_e) : 0;
-      rest -= (long long)ct * c_e;
-      // row tiles inside the column tile: average cost is close enough
-      const int mt = c_e ? (int)(rest * m_e / c_e) : 0;
-      bound = sh_tiles[lo] * n_ct + min(ct, n_ct) * m_e + min(mt, m_e);
+      const int n_e = sh_tiles[g][lo + 1] - sh_tiles[g][lo];
+      const long long rest = target - (long long)sh_cost[lo] * kXcds;
+      bound = sh_tiles[g][lo] + (c_e ? min((int)(rest * n_e / ((long long)c_e * kXcds)), n_e) : 0);
       bound = min(bound, total_tiles);
     }
     sh_bound[g][x] = bound;
@@ -233,14 +244,13 @@ __device__ __forceinline__ int build_plan(int count, int E, int n_ct_gate_up, in
   // workgroups instead, which are many).  The waves take the experts in turn.
   if (with_tiles) {
     for (int ee = w; ee < E; ee += 4)
-      write_expert_tiles(ee, sh_nmt[ee], sh_rb[ee], sh_extra[ee], sh_rowblk[ee], sh_tiles[ee], lane,
-                         n_ct_gate_up, n_ct_down, out);
+      write_expert_tiles(ee, sh_nmt[ee], sh_rb[ee], sh_extra[ee], sh_rowblk[ee], sh_tiles[0][ee], sh_tiles[1][ee],
+                         lane, out);
   }
   __syncthreads();
   // keep every range within what the launch grid provides for (xcd_tile_cap)
   if (e < 2) {
-    const int n_ct = e ? n_ct_down : n_ct_gate_up;
-    const int total_tiles = tot_mt * n_ct;
+    const int total_tiles = tot[4 + e];
     const int cap = xcd_tile_cap(total_tiles);
     int *bounds = totals + (e ? kTotBoundsDown : kTotBoundsGateUp);
     int prev = 0;
@@ -324,7 +334,7 @@ __device__ __forceinline__ void wave_ranks_for(int E, const int (&id)[kTopK], in
 __global__ __launch_bounds__(kDispThreads) void dispatch_scatter_kernel(
     const int *__restrict__ topk_i, const int *__restrict__ pos, int T, int E,
     const int *__restrict__ blk_counts, int n_blk, int *__restrict__ perm, int *__restrict__ rowmap,
-    int *__restrict__ inv, int *__restrict__ blk_expert, int n_ct_gate_up, int n_ct_down, PlanOut plan) {
+    int *__restrict__ inv, int *__restrict__ blk_expert, PlanOut plan) {
   __shared__ int wave_cnt[kDispThreads / 64][256];
   __shared__ int sh_base[256], sh_off[256], sh_row0[256];
   __shared__ ExpertInfo sh_info[256];
@@ -356,7 +366,7 @@ __global__ __launch_bounds__(kDispThreads) void dispatch_scatter_kernel(
   }
   int ex_count;
   ExpertInfo inf;
-  const int row0 = build_plan(count, E, n_ct_gate_up, n_ct_down, plan, /*with_tiles=*/false, &ex_count, nullptr,
+  const int row0 = build_plan(count, E, plan, /*with_tiles=*/false, &ex_count, nullptr,
                               /*write_global=*/blockIdx.x == 0, &inf);
   sh_base[tid] = base;
   sh_off[tid] = ex_count;
@@ -370,8 +380,7 @@ __global__ __launch_bounds__(kDispThreads) void dispatch_scatter_kernel(
   // experts in turn.
   for (int ee = blockIdx.x * (kDispThreads / 64) + w; ee < E; ee += gridDim.x * (kDispThreads / 64)) {
     const ExpertInfo f = sh_info[ee];
-    write_expert_tiles(ee, f.n_mt, f.rb, f.extra, f.row0 / kRowBlock, f.tile_base, lane, n_ct_gate_up,
-                       n_ct_down, plan);
+    write_expert_tiles(ee, f.n_mt, f.rb, f.extra, f.row0 / kRowBlock, f.tiles0[0], f.tiles0[1], lane, plan);
   }
 #pragma unroll
   for (int k = 0; k < kTopK; k++)
@@ -403,8 +412,7 @@ __global__ __launch_bounds__(kDispThreads) void dispatch_scatter_kernel(
 constexpr int kSmallRounds = 1;
 
 __global__ __launch_bounds__(kDispThreads) void dispatch_small_kernel(
-    const int *__restrict__ topk_i, const int *__restrict__ pos, int T, int E, int n_ct_gate_up,
-    int n_ct_down, PlanOut out, int *__restrict__ perm, int *__restrict__ rowmap,
+    const int *__restrict__ topk_i, const int *__restrict__ pos, int T, int E, PlanOut out, int *__restrict__ perm, int *__restrict__ rowmap,
     int *__restrict__ inv, int *__restrict__ blk_expert) {
   __shared__ int hist[kSmallRounds][256];  // per round and expert: count, then exclusive base
   __shared__ int sh_off[256], sh_row0[256];
@@ -442,7 +450,7 @@ __global__ __launch_bounds__(kDispThreads) void dispatch_small_kernel(
     count += c;
   }
   int ex_count, tot_count;
-  const int row0 = build_plan(tid < E ? count : 0, E, n_ct_gate_up, n_ct_down, out, /*with_tiles=*/true, &ex_count, &tot_count);
+  const int row0 = build_plan(tid < E ? count : 0, E, out, /*with_tiles=*/true, &ex_count, &tot_count);
   sh_off[tid] = ex_count;
   sh_row0[tid] = row0;
   // -1 where the scatter below writes nothing: the padding rows of the experts
@@ -539,8 +547,8 @@ __global__ __launch_bounds__(256) void combine_kernel(const float *__restrict__ 
   }
 }
 
-hipError_t launch_dispatch(const int *topk_i, const int *pos, int T, int E, int n_ct_gate_up,
-                           int n_ct_down, int tile_rows, const DispatchBuffers &d, hipStream_t s) {
+hipError_t launch_dispatch(const int *topk_i, const int *pos, int T, int E, int nb_gate_up, int nb_down,
+                           int tile_rows, bool wide, const DispatchBuffers &d, hipStream_t s) {
   const int n_blk = (T + kDispThreads - 1) / kDispThreads;
   // Rows of the padded space this batch can reach: every expert rounds its
   // rows up to a multiple of 32.
@@ -556,16 +564,19 @@ hipError_t launch_dispatch(const int *topk_i, const int *pos, int T, int E, int 
   plan.tile_cap_gate_up = d.tile_cap_gate_up;
   plan.tile_cap_down = d.tile_cap_down;
   plan.tile_rb = tile_rows / kRowBlock;
+  plan.nb[0] = nb_gate_up;
+  plan.nb[1] = nb_down;
+  plan.wide = wide;
   if (n_blk <= kSmallRounds) {
     // small batches: one workgroup does both passes, one launch fewer
-    dispatch_small_kernel<<<1, kDispThreads, 0, s>>>(topk_i, pos, T, E, n_ct_gate_up, n_ct_down, plan,
-                                                     d.perm, d.rowmap, d.inv, d.blk_expert);
+    dispatch_small_kernel<<<1, kDispThreads, 0, s>>>(topk_i, pos, T, E, plan, d.perm,
+                                                     d.rowmap, d.inv, d.blk_expert);
     return hipGetLastError();
   }
   dispatch_count_kernel<<<n_blk, kDispThreads, 0, s>>>(topk_i, pos, T, E, d.blk_counts, d.rowmap,
                                                        fill_rows, d.perm);
   dispatch_scatter_kernel<<<n_blk, kDispThreads, 0, s>>>(topk_i, pos, T, E, d.blk_counts, n_blk, d.perm,
-                                                         d.rowmap, d.inv, d.blk_expert, n_ct_gate_up, n_ct_down, plan);
+                                                         d.rowmap, d.inv, d.blk_expert, plan);
   return hipGetLastError();
 }
 
@@ -670,7 +681,7 @@ extern "C" int moe_dispatch_static(const int *topk_i, const int *pos, int n_toke
   // no GEMM follows: with no column tiles the plan kernel writes no tile tables
   d.tiles_gate_up = d.tiles_down = nullptr;
   d.tile_cap_gate_up = d.tile_cap_down = 0;
-  const hipError_t el = launch_dispatch(topk_i, pos, n_tokens, n_experts, 0, 0, kTileRows, d, static_cast<hipStream_t>(stream));
+  const hipError_t el = launch_dispatch(topk_i, pos, n_tokens, n_experts, 0, 0, kTileRows, false, d, static_cast<hipStream_t>(stream));
   if (el != hipSuccess)
     return set_error(MOE_ERR_HIP, "dispatch launch failed: %s", hipGetErrorString(el));
   return MOE_OK;

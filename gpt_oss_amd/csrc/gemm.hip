@@ -615,8 +615,7 @@ __global__ __launch_bounds__(C::THREADS, C::WGS) void grouped_gemm_kernel(
   const int nb_total = (GATE_UP ? 2 * N : N) / kRowBlock;  // weight row blocks per expert
   TileDesc tc;
   if (!locate_tile(tiles, totals + (GATE_UP ? kTotBoundsGateUp : kTotBoundsDown), tc)) return;
-  const int nb0 = tc.nt * C::TILE_NB;
-  const int nb_valid = min(C::TILE_NB, nb_total - nb0);
+  const int nb0 = tc.nb0, nb_valid = tc.nbt;
   // per expert (nb_total/2) * (KB/2) chunks of 1 KB
   const uint4 *b_frag = w_frag + (size_t)tc.e * nb_total * KB * 16;
   const uint16_t *b_scale = w_scale + (size_t)tc.e * nb_total * KB * 8;
@@ -685,10 +684,10 @@ static_assert(CfgFull::RBT_MAX * kRowBlock == kTileRows && CfgHalf::RBT_MAX * kR
 template <bool GATE_UP>
 static hipError_t launch_gemm(const void *a, const void *w, const uint16_t *w_scale, const float *ba,
                               const float *bb, const DispatchBuffers &d, void *out, int K, int N,
-                              float limit, int T, int E, int tile_rows, bool stream, hipStream_t s) {
+                              float limit, int T, int E, int tile_rows, bool wide, bool stream, hipStream_t s) {
   const int nb_total = (GATE_UP ? 2 * N : N) / kRowBlock;
   const int n_ct = (nb_total + kGemmTileNb - 1) / kGemmTileNb;
-  const int grid = kXcds * xcd_tile_cap(gemm_tile_cap(T, E, tile_rows) * n_ct);
+  const dim3 grid(kXcds * xcd_tile_cap(gemm_tile_cap(T, E, tile_rows) * n_ct), wide ? 2 : 1);
   const TileDesc *tiles = GATE_UP ? d.tiles_gate_up : d.tiles_down;
   const uint4 *af = static_cast<const uint4 *>(a), *wf = static_cast<const uint4 *>(w);
   // the full-height kernels take a plan of either height, the others one of half height
@@ -704,24 +703,24 @@ static hipError_t launch_gemm(const void *a, const void *w, const uint16_t *w_sc
 
 hipError_t launch_gate_up(const uint16_t *x, const void *w1, const uint16_t *w1_scale, const float *b1g,
                           const float *b1u, const DispatchBuffers &d, uint16_t *act, int H, int IM,
-                          float limit, int T, int E, int tile_rows, bool cached, hipStream_t s) {
+                          float limit, int T, int E, int tile_rows, bool wide, bool cached, hipStream_t s) {
   if (H % 64 || IM % 64) return hipErrorInvalidValue;  // the kernels take steps of 32 in pairs
   const TileRoute r = tile_route(T, E, 2 * IM, w1_scale != nullptr, tile_rows, cached);
   if (r.kernel == kBf16Tiles)
-    return launch_bf16_gate_up(x, w1, b1g, b1u, d, act, H, IM, limit, T, E, tile_rows, r.past_caches, s);
+    return launch_bf16_gate_up(x, w1, b1g, b1u, d, act, H, IM, limit, T, E, tile_rows, wide, r.past_caches, s);
   if (r.kernel == kFp4ManyTiles)
-    return launch_fp4_gate_up(x, w1, w1_scale, b1g, b1u, d, act, H, IM, limit, T, E, r.past_caches, s);
-  return launch_gemm<true>(x, w1, w1_scale, b1g, b1u, d, act, H, IM, limit, T, E, tile_rows, r.past_caches, s);
+    return launch_fp4_gate_up(x, w1, w1_scale, b1g, b1u, d, act, H, IM, limit, T, E, wide, r.past_caches, s);
+  return launch_gemm<true>(x, w1, w1_scale, b1g, b1u, d, act, H, IM, limit, T, E, tile_rows, wide, r.past_caches, s);
 }
 
 hipError_t launch_down(const uint16_t *act, const void *w2, const uint16_t *w2_scale, const float *b2,
                        const DispatchBuffers &d, float *y, int H, int IM, int T, int E, int tile_rows,
-                       bool cached, hipStream_t s) {
+                       bool wide, bool cached, hipStream_t s) {
   if (H % 64 || IM % 64) return hipErrorInvalidValue;  // the kernels take steps of 32 in pairs
   const TileRoute r = tile_route(T, E, 2 * IM, w2_scale != nullptr, tile_rows, cached);
-  if (r.kernel == kBf16Tiles) return launch_bf16_down(act, w2, b2, d, y, H, IM, T, E, tile_rows, r.past_caches, s);
-  if (r.kernel == kFp4ManyTiles) return launch_fp4_down(act, w2, w2_scale, b2, d, y, H, IM, T, E, r.past_caches, s);
-  return launch_gemm<false>(act, w2, w2_scale, b2, nullptr, d, y, IM, H, 0.f, T, E, tile_rows, r.past_caches, s);
+  if (r.kernel == kBf16Tiles) return launch_bf16_down(act, w2, b2, d, y, H, IM, T, E, tile_rows, wide, r.past_caches, s);
+  if (r.kernel == kFp4ManyTiles) return launch_fp4_down(act, w2, w2_scale, b2, d, y, H, IM, T, E, wide, r.past_caches, s);
+  return launch_gemm<false>(act, w2, w2_scale, b2, nullptr, d, y, IM, H, 0.f, T, E, tile_rows, wide, r.past_caches, s);
 }
 
 }  // namespace moe

@@ -8,7 +8,9 @@
 // block more and one less, so that every SIMD has the same work and the tile's rows
 // still pad to at most 31.  In the last column tile of a matrix whose width is not a
 // multiple of 256 fewer waves have columns; they then take every fourth or eighth row
-// block (S).
+// block (S).  A tile of up to six row blocks may have 320 columns (bf16_wide_tiles has when, and the
+// figures): 60 of the 64 blocks of sums that the registers hold, in the same 160 KB of rings.  Its last two column
+// blocks are two waves' of either half of the rows, so that every SIMD still has the same work.
 //
 // Feeding the matrix cores.  Both operands go through LDS by DMA, and a wave reads 8 KB
 // of rows and 4 KB of columns per step of 32 k (LDS reads run at 226 bytes per clock and
@@ -51,12 +53,20 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kWaves = 8, kThreads = kWaves * 64;
-constexpr int kRowBlockBytes = 4096;                          // a double step (64 k) of a row block in LDS
-constexpr uint32_t kColSlot = 16384, kColSlots = 4;           // a step (32 k) of 8 column blocks
-constexpr uint32_t kRowRing = kColSlot * kColSlots;           // the rows' ring stands behind the columns'
-constexpr uint32_t kRowStage = 8 * kRowBlockBytes, kRowStages = 3;
-constexpr uint32_t kLds = kRowRing + kRowStage * kRowStages;  // 160 KB
-static_assert(kTileRows == 8 * kRowBlock && kGemmTileNb == 8, "tile plan of build_plan");
+constexpr int kRowBlockBytes = 4096;  // a double step (64 k) of a row block in LDS
+constexpr int kColBlockBytes = 2048;  // a step (32 k) of a column block
+constexpr uint32_t kColSlots = 4, kRowStages = 3;
+// The rings of a tile of up to W column blocks and H row blocks, the rows' behind the columns'.
+template <int W, int H>
+struct Rings {
+  static constexpr uint32_t ColSlot = W * kColBlockBytes, RowRing = ColSlot * kColSlots;
+  static constexpr uint32_t RowStage = H * kRowBlockBytes, End = RowRing + RowStage * kRowStages;
+};
+using Square = Rings<8, 8>;
+using Wide = Rings<10, 6>;
+constexpr uint32_t kLds = Square::End;  // 160 KB
+static_assert(Wide::End <= kLds, "rings");
+static_assert(kTileRows == 8 * kRowBlock, "tile plan of build_plan");
 
 // ---- 16 bytes per lane from global memory to LDS, lane l at lds + 16 l ----
 // In assembly, because the compiler, which does not know one stage from another here,
@@ -106,29 +116,34 @@ struct Tile {
 };
 
 // A wave's share of a tile: RBW row blocks (rg, rg + S, ...; one past the tile's last repeats
-// it and is not stored) times 2 column blocks.  LA: its loads of rows per double step.
-template <int RBW, int LA, int S, bool GATE_UP, bool STREAM>
+// it and is not stored) times NU units of columns.  A unit is what ends as 32 columns of down (a column
+// block) or 16 of the activation (half a pair of gate and up blocks): units 2 wn and 2 wn + 1, and with
+// NU = 3 unit 8 + wx.  LA: its loads of rows per double step, LB: of columns per step.
+template <int RBW, int LA, int S, int NU, int LB, typename R, bool GATE_UP, bool STREAM>
 __device__ __forceinline__ void wave_tile(const Tile &t, uint32_t lds0) {
-  constexpr int NBW = 2, LB = 2;
+  constexpr int NC = 2 * NU;  // groups of 16 columns: gate_up: the units' gates, then their ups; down: the units' halves
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wn = w % (kWaves / S), rg = w / (kWaves / S);
+  // waves 0, 1 and 6, 7 of a tile of ten blocks have the third units, one on each SIMD (wave w runs on SIMD w % 4)
+  const int wx = R::ColSlot == Wide::ColSlot ? (wn & 1) : wn;
   const int sub = w & 3, lg = w >> 2;  // DMA: quarter `sub` of row blocks lg, lg + 2, ...
   const int KB = t.KB, n_steps = KB >> 1, last = n_steps - 1, last_d = (n_steps >> 1) - 1;
   constexpr int RB1 = RBW ? RBW : 1;
+  auto unit = [&](int j) { return j < 2 ? 2 * wn + j : 8 + wx; };
 
   // The accumulators start from the bias.  gate_up's weights are the first operand: lane
-  // 16 q + r of columns c ends with columns 16 c + 4 q .. + 3 of row r, the gate (c < 2) and the
-  // up (c + 2) of a pair of blocks in the same lane (see pack_weight_kernel).  down's rows
+  // 16 q + r of group c ends with columns 4 q .. + 3 of row r, the gate (c < NU) and the
+  // up (c + NU) of a unit in the same lane (see pack_weight_kernel).  down's rows
   // are: the lane ends with rows 4 q .. + 3 of column r, for stores of whole lines.
-  f32x4 bias[4];
+  f32x4 bias[NC];
 #pragma unroll
-  for (int c = 0; c < 4; c++) {
+  for (int c = 0; c < NC; c++) {
     if constexpr (GATE_UP) {
-      const int P = min((t.nb0 >> 1) + wn, ((t.nb0 + t.nb_valid) >> 1) - 1);
-      bias[c] = *reinterpret_cast<const f32x4 *>((c < 2 ? t.ba : t.bb) + kRowBlock * P + 16 * (c & 1) + 4 * (lane >> 4));
+      const int u = t.nb0 + min(unit(c % NU), t.nb_valid - 1);
+      bias[c] = *reinterpret_cast<const f32x4 *>((c < NU ? t.ba : t.bb) + 16 * u + 4 * (lane >> 4));
     } else {
-      const float v = t.ba[kRowBlock * (t.nb0 + min(wn * NBW + (c >> 1), t.nb_valid - 1)) + 16 * (c & 1) + (lane & 15)];
+      const float v = t.ba[kRowBlock * (t.nb0 + min(unit(c >> 1), t.nb_valid - 1)) + 16 * (c & 1) + (lane & 15)];
       bias[c] = f32x4{v, v, v, v};
     }
   }
@@ -174,16 +189,22 @@ __device__ __forceinline__ void wave_tile(const Tile &t, uint32_t lds0) {
         rd_a[par][h] = lds0 + rg * kRowBlockBytes + (2 * par + (p4 >> 1)) * 1024 + ((p4 & 1) * 32 + r) * 16;
       }
     }
-  const uint32_t rd_b = lds0 + wn * (NBW * 2048) + (p4 >> 1) * 1024 + ((p4 & 1) * 32 + r16) * 16;
+  // a pair's blocks of gate and up stand side by side, and a group of 16 is a half of either
+  const uint32_t rd_lane = lds0 + (p4 >> 1) * 1024 + ((p4 & 1) * 32 + r16) * 16;
+  const uint32_t rd_b = rd_lane + wn * (2 * kColBlockBytes);
+  const uint32_t rd_x = rd_lane + (GATE_UP ? (8 + (wx & ~1)) * kColBlockBytes + (wx & 1) * 256 : (8 + wx) * kColBlockBytes);
   const char *b_src = t.b + (size_t)(t.nb0 + min(w, t.nb_valid - 1)) * KB * 1024;
+  const char *x_src = t.b + ((size_t)(t.nb0 + min(8 + (w >> 1), t.nb_valid - 1)) * KB + (w & 1)) * 1024;
   const uint32_t lane16 = lane * 16;
-  const uint32_t dst_a = lds0 + lg * kRowBlockBytes + sub * 1024, dst_b = lds0 + w * 2048;
+  const uint32_t dst_a = lds0 + lg * kRowBlockBytes + sub * 1024, dst_b = lds0 + w * kColBlockBytes;
+  const uint32_t dst_x = lds0 + 8 * kColBlockBytes + w * 1024;
 
   auto issue_a = [&](uint32_t stage, int m) { dma_lanes(dst_a + stage + m * 2 * kRowBlockBytes, a_src[m]); };
-  auto issue_b = [&](uint32_t slot, int ks, int kk) {
-    const char *p = b_src + (size_t)ks * 2048;
-    if (kk == 0) dma_wave<0, STREAM>(dst_b + slot, p, lane16);
-    else dma_wave<kFragBytes, STREAM>(dst_b + slot, p, lane16);
+  auto issue_b = [&](uint32_t slot, int ks, int n) {
+    const size_t at = (size_t)ks * kColBlockBytes;
+    if (n == 0) dma_wave<0, STREAM>(dst_b + slot, b_src + at, lane16);
+    else if (n == 1) dma_wave<kFragBytes, STREAM>(dst_b + slot, b_src + at, lane16);
+    else dma_wave<0, STREAM>(dst_x + slot, x_src + at, lane16);
   };
   auto adv_a = [&](int jd_next) {
     const int d = jd_next <= last_d ? A_STEP : 0;
@@ -191,71 +212,75 @@ __device__ __forceinline__ void wave_tile(const Tile &t, uint32_t lds0) {
     for (int m = 0; m < LA; m++) a_src[m] += d;
   };
   constexpr int G = 2 * RBW;        // groups of 16 rows
-  f32x4 acc[2 * RB1][4];
-  bf16x8 fa[2][RB1], fb[2][4];      // fa: first and second half of the groups; fb: steps of either parity
+  f32x4 acc[2 * RB1][NC];
+  bf16x8 fa[2][RB1], fb[2][NC];     // fa: first and second half of the groups; fb: steps of either parity
   auto read_a = [&](uint32_t stage, int par, int hf, int i) {
     const int g = hf * RBW + i;
     fa[hf][i] = lds_operand(rd_a[par][g & 1] + stage, (g >> 1) * S * kRowBlockBytes);
   };
-  auto read_b = [&](uint32_t slot, int par, int c) { fb[par][c] = lds_operand(rd_b + slot, (c >> 1) * 2048 + (c & 1) * 256); };
+  auto read_b = [&](uint32_t slot, int par, int c) {
+    const int j = GATE_UP ? c % NU : c >> 1, second = GATE_UP ? c / NU : c & 1;  // unit; its up, its second half
+    if (j == 2) fb[par][c] = lds_operand(rd_x + slot, second * (GATE_UP ? kColBlockBytes : 256));
+    else fb[par][c] = lds_operand(rd_b + slot, GATE_UP ? second * kColBlockBytes + j * 256 : j * kColBlockBytes + second * 256);
+  };
 #pragma unroll
   for (int g = 0; g < G; g++)
 #pragma unroll
-    for (int c = 0; c < 4; c++) acc[g][c] = GATE_UP && c >= 2 ? bias[c] + 1.0f : bias[c];
+    for (int c = 0; c < NC; c++) acc[g][c] = GATE_UP && c >= NU ? bias[c] + 1.0f : bias[c];
   WAIT_VMCNT(0);  // bias and row map: from here on the counter belongs to the loads of A and B
   __builtin_amdgcn_sched_barrier(0);
   // First filling: A(0) B(0) B(1) A(1) B(2) and what the steps before step 0 would have asked for
   // of B(3) and A(2).
   auto fill_a = [&](int d) {
 #pragma unroll
-    for (int m = 0; m < LA; m++) issue_a(kRowRing + d * kRowStage, m);
+    for (int m = 0; m < LA; m++) issue_a(R::RowRing + d * R::RowStage, m);
     adv_a(d + 1);
   };
   auto fill_b = [&](int ks) {
-    issue_b(ks * kColSlot, min(ks, last), 0);
-    issue_b(ks * kColSlot, min(ks, last), 1);
+#pragma unroll
+    for (int n = 0; n < LB; n++) issue_b(ks * R::ColSlot, min(ks, last), n);
   };
   fill_a(0);
   fill_b(0);
   fill_b(1);
   fill_a(1);
   fill_b(2);
-  issue_b(3 * kColSlot, min(3, last), 0);
-  if (LA > 0) issue_a(kRowRing + 2 * kRowStage, 0);
+  issue_b(3 * R::ColSlot, min(3, last), 0);
+  if (LA > 0) issue_a(R::RowRing + 2 * R::RowStage, 0);
   WAIT_VMCNT(LA + (LA > 0) + 2 * LB + 1);  // A(0), B(0)
   lds_barrier();
   if constexpr (RBW > 0) {
 #pragma unroll
-    for (int c = 0; c < 4; c++) read_b(0, 0, c);
+    for (int c = 0; c < NC; c++) read_b(0, 0, c);
 #pragma unroll
-    for (int i = 0; i < RBW; i++) read_a(kRowRing, 0, 0, i);
+    for (int i = 0; i < RBW; i++) read_a(R::RowRing, 0, 0, i);
   }
-  uint32_t sa = kRowRing, sb = 0;
-  constexpr int NM = RBW * 4;  // MFMAs of half a step
+  uint32_t sa = R::RowRing, sb = 0;
+  constexpr int NM = RBW * NC;  // MFMAs of half a step
   auto mma = [&](int par, int hf, int m) {
-    const int i = m / 4, c = m % 4, g = hf * RBW + i;
+    const int i = m / NC, c = m % NC, g = hf * RBW + i;
     if constexpr (GATE_UP) acc[g][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[par][c], fa[hf][i], acc[g][c], 0, 0, 0);
     else acc[g][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[hf][i], fb[par][c], acc[g][c], 0, 0, 0);
   };
   // Step ks = 2 jd + par: the products of the first half of the row groups, barrier, those of the
-  // second.  Meanwhile the operands of the next half are read, and one load of columns and one
-  // of rows go out: B(ks + 4) k block 0 behind the barrier of step ks, k block 1 before that of
+  // second.  Meanwhile the operands of the next half are read, and one or two loads of columns and one
+  // of rows go out: B(ks + 4)'s first behind the barrier of step ks, its others before that of
   // step ks + 1; A(jd + 3) m = 0 behind the barrier of the odd step 2 jd + 1, m = 1, 2, 3 in the
   // halves that follow.  At the barrier of step ks B(ks + 1) has to have landed, and at an odd one
   // A(jd + 1).  Behind B(ks + 1) an even step has issued twice B, m = 1, 2, 3 of A(jd + 1) and m =
   // 0, 1 of A(jd + 2); behind A(jd + 1) an odd one twice B and A(jd + 2).  Every step
   // is the same code with the same counts: past the tile's end the refills load its last step again,
   // hits that nobody reads.  The wave ends with those in flight; s_endpgm waits for them.
-  constexpr int WAIT_EVEN = 4 + (LA > 1) + (LA > 2) + (LA > 3) + (LA > 0) + (LA > 1);
-  constexpr int WAIT_ODD = 4 + LA;
+  constexpr int WAIT_EVEN = 2 * LB + (LA > 1) + (LA > 2) + (LA > 3) + (LA > 0) + (LA > 1);
+  constexpr int WAIT_ODD = 2 * LB + LA;
   auto step = [&](auto par_c, int ks) {
     constexpr int par = decltype(par_c)::value;
-    const uint32_t sbn = (sb + kColSlot) & (kRowRing - 1), sbp = (sb - kColSlot) & (kRowRing - 1);
-    const uint32_t san = par ? (sa + kRowStage == kLds ? kRowRing : sa + kRowStage) : sa;
-    const uint32_t sap = sa == kRowRing ? kLds - kRowStage : sa - kRowStage;
+    const uint32_t sbn = sb + R::ColSlot == R::RowRing ? 0 : sb + R::ColSlot, sbp = (sb == 0 ? R::RowRing : sb) - R::ColSlot;
+    const uint32_t san = par ? (sa + R::RowStage == R::End ? R::RowRing : sa + R::RowStage) : sa;
+    const uint32_t sap = (sa == R::RowRing ? R::End : sa) - R::RowStage;
     constexpr int NM1 = NM ? NM : 1;
     {  // first half: even: A(jd + 2) m = 1; odd: m = 3
-      constexpr int RD = RBW, AM = par ? 3 : 1, SD = RD + 1 + (AM < LA), SIDE = (SD + NM1 - 1) / NM1;
+      constexpr int RD = RBW, AM = par ? 3 : 1, SD = RD + LB - 1 + (AM < LA), SIDE = (SD + NM1 - 1) / NM1;
       const int ks_b = min(ks + 3, last);
 #pragma unroll
       for (int m = 0; m < NM1; m++) {
@@ -263,8 +288,8 @@ __device__ __forceinline__ void wave_tile(const Tile &t, uint32_t lds0) {
         for (int s = m * SIDE; s < (m + 1) * SIDE; s++) {
           if (s < RD) {
             read_a(sa, par, 1, s);
-          } else if (s == RD) {
-            issue_b(sbp, ks_b, 1);
+          } else if (s < RD + LB - 1) {
+            issue_b(sbp, ks_b, 1 + s - RD);
           } else if (s < SD) {
             issue_a(sap, AM);
           }
@@ -277,7 +302,7 @@ __device__ __forceinline__ void wave_tile(const Tile &t, uint32_t lds0) {
     if constexpr (par) WAIT_VMCNT(WAIT_ODD); else WAIT_VMCNT(WAIT_EVEN);
     lds_barrier();
     {  // second half: even: A(jd + 2) m = 2; odd: A(jd + 3) m = 0
-      constexpr int RD = RBW ? RBW + 4 : 0, AM = par ? 0 : 2, SD = RD + 1 + (AM < LA),
+      constexpr int RD = RBW ? RBW + NC : 0, AM = par ? 0 : 2, SD = RD + 1 + (AM < LA),
                     SIDE = (SD + NM1 - 1) / NM1;  // side items per MFMA
       const int ks_b = min(ks + 4, last);
 #pragma unroll
@@ -285,8 +310,8 @@ __device__ __forceinline__ void wave_tile(const Tile &t, uint32_t lds0) {
 #pragma unroll
         for (int s = m * SIDE; s < (m + 1) * SIDE; s++) {
           if (s < RD) {
-            if (s < 4) read_b(sbn, par ^ 1, s);
-            else read_a(san, par ^ 1, 0, s - 4);
+            if (s < NC) read_b(sbn, par ^ 1, s);
+            else read_a(san, par ^ 1, 0, s - NC);
           } else if (s == RD) {
             issue_b(sb, ks_b, 0);
           } else if (s < SD) {
@@ -305,37 +330,37 @@ __device__ __forceinline__ void wave_tile(const Tile &t, uint32_t lds0) {
     step(std::integral_constant<int, 1>{}, ks + 1);
   }
   if constexpr (RBW > 0) {
-    if (wn * NBW >= t.nb_valid) return;  // a wave without columns (last column tile only)
+    if (2 * wn >= t.nb_valid) return;  // a wave without columns (last column tile only)
     if constexpr (GATE_UP) {
       // bf16 fragments, as the down GEMM reads them: one exchange of 16-lane rows between the two
       // row groups of a block per dword gives every lane 8 consecutive columns of a row.
       u32x4 *act = reinterpret_cast<u32x4 *>(t.out);
       const int kb2_total = t.N / kFragK;
-      const int P0 = (t.nb0 >> 1) + wn;
 #pragma unroll
       for (int i = 0; i < RBW; i++) {
         const int blk = i * S + rg;
         if (S > 2 && blk >= t.rbt) break;
-        u32x4 *dst = act + ((size_t)(t.rb0 + blk) * kb2_total + 2 * P0) * 64 + lane;
+        u32x4 *dst = act + ((size_t)(t.rb0 + blk) * kb2_total + t.nb0) * 64 + lane;
 #pragma unroll
-        for (int c = 0; c < 2; c++) {
+        for (int j = 0; j < NU; j++) {
+          if (j > 1 && unit(j) >= t.nb_valid) break;
           uint32_t pk[2][2];
 #pragma unroll
           for (int h = 0; h < 2; h++)
 #pragma unroll
             for (int d = 0; d < 2; d++)
-              pk[h][d] = pack_bf16(swiglu_shifted(acc[2 * i + h][c][2 * d], acc[2 * i + h][c + 2][2 * d], t.limit),
-                                   swiglu_shifted(acc[2 * i + h][c][2 * d + 1], acc[2 * i + h][c + 2][2 * d + 1], t.limit));
+              pk[h][d] = pack_bf16(swiglu_shifted(acc[2 * i + h][j][2 * d], acc[2 * i + h][j + NU][2 * d], t.limit),
+                                   swiglu_shifted(acc[2 * i + h][j][2 * d + 1], acc[2 * i + h][j + NU][2 * d + 1], t.limit));
           const u32x2 s0 = __builtin_amdgcn_permlane16_swap(pk[0][0], pk[1][0], false, false);
           const u32x2 s1 = __builtin_amdgcn_permlane16_swap(pk[0][1], pk[1][1], false, false);
-          store_output<STREAM>(&dst[c * 64], u32x4{s0[0], s1[0], s0[1], s1[1]});
+          store_output<STREAM>(&dst[unit(j) * 64], u32x4{s0[0], s1[0], s0[1], s1[1]});
         }
       }
     } else {
       float *y = reinterpret_cast<float *>(t.out);
       // The same exchange between two groups of columns: a store then writes 128 bytes of two rows
       // (16 bytes per lane of 16 rows: 4.2 us per tile instead of 1.9).
-      const int col = kRowBlock * (t.nb0 + wn * NBW) + (lane & 31), row = 8 * (lane >> 5);
+      const int col = kRowBlock * t.nb0 + (lane & 31), row = 8 * (lane >> 5);
 #pragma unroll
       for (int i = 0; i < RBW; i++) {
         const int blk = i * S + rg;
@@ -345,15 +370,29 @@ __device__ __forceinline__ void wave_tile(const Tile &t, uint32_t lds0) {
 #pragma unroll
           for (int q = 0; q < 4; q++)
 #pragma unroll
-            for (int c = 0; c < 4; c += 2) {
-              const f32x4 u = acc[2 * i + h][c], v = acc[2 * i + h][c + 1];
+            for (int j = 0; j < NU; j++) {
+              if (j > 1 && unit(j) >= t.nb_valid) break;
+              const f32x4 u = acc[2 * i + h][2 * j], v = acc[2 * i + h][2 * j + 1];
               const u32x2 x = __builtin_amdgcn_permlane16_swap(__float_as_uint(u[q]), __float_as_uint(v[q]), false, false);
-              float *dst = y + ((size_t)(t.rb0 + blk) * kRowBlock + 16 * h + row + q) * t.N + col + 16 * c;
+              float *dst = y + ((size_t)(t.rb0 + blk) * kRowBlock + 16 * h + row + q) * t.N + col + kRowBlock * unit(j);
               store_output<STREAM>(dst, __uint_as_float(x[0]));
               store_output<STREAM>(dst + 4 * (size_t)t.N, __uint_as_float(x[1]));
             }
       }
     }
+  }
+}
+
+// A tile whose row blocks two waves split: rbw of them, MAX at most, are this one's.
+template <int MAX, int NU, int LB, typename R, bool GATE_UP, bool STREAM>
+__device__ __forceinline__ void split_rows(const Tile &t, uint32_t lds0, int rbw) {
+  switch (rbw) {
+    case 0: wave_tile<0, 0, 2, NU, LB, R, GATE_UP, STREAM>(t, lds0); break;
+    case 1: wave_tile<1, 1, 2, NU, LB, R, GATE_UP, STREAM>(t, lds0); break;
+    case 2: wave_tile<2, 2, 2, NU, LB, R, GATE_UP, STREAM>(t, lds0); break;
+    case MAX: wave_tile<MAX, MAX, 2, NU, LB, R, GATE_UP, STREAM>(t, lds0); break;
+    default:
+      if constexpr (MAX > 3) wave_tile<3, 3, 2, NU, LB, R, GATE_UP, STREAM>(t, lds0);
   }
 }
 
@@ -383,36 +422,42 @@ __global__ __launch_bounds__(kThreads, 2) void bf16_gemm_kernel(const char *__re
   t.N = N;
   t.rb0 = tc.rb0;
   t.rbt = tc.rbt;
-  t.nb0 = tc.nt * kGemmTileNb;
-  t.nb_valid = min(kGemmTileNb, nb_total - t.nb0);
+  t.nb0 = tc.nb0;
+  t.nb_valid = tc.nbt;
   t.limit = limit;
   const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-  if (t.nb_valid > 4) {
-    switch ((t.rbt + 1 - (w >> 2)) >> 1) {
-      case 0: wave_tile<0, 0, 2, GATE_UP, STREAM>(t, lds0); break;
-      case 1: wave_tile<1, 1, 2, GATE_UP, STREAM>(t, lds0); break;
-      case 2: wave_tile<2, 2, 2, GATE_UP, STREAM>(t, lds0); break;
-      case 3: wave_tile<3, 3, 2, GATE_UP, STREAM>(t, lds0); break;
-      default: wave_tile<4, 4, 2, GATE_UP, STREAM>(t, lds0); break;
+  const int rbw = (t.rbt + 1 - (w >> 2)) >> 1;  // the wave's row blocks where the waves split them in two
+  if constexpr (STREAM) {
+    if (t.nb_valid > kGemmTileNb) {  // plans for these loads only (bf16_wide_tiles)
+      switch (w >> 1) {
+        case 0: split_rows<3, 3, 3, Wide, GATE_UP, STREAM>(t, lds0, rbw); break;
+        case 1: split_rows<3, 2, 3, Wide, GATE_UP, STREAM>(t, lds0, rbw); break;
+        case 2: split_rows<3, 2, 2, Wide, GATE_UP, STREAM>(t, lds0, rbw); break;
+        default: split_rows<3, 3, 2, Wide, GATE_UP, STREAM>(t, lds0, rbw); break;
+      }
+      return;
     }
+  }
+  if (t.nb_valid > 4) {
+    split_rows<4, 2, 2, Square, GATE_UP, STREAM>(t, lds0, rbw);
   } else if (t.nb_valid > 2) {
-    if (t.rbt <= 4) wave_tile<1, 2, 4, GATE_UP, STREAM>(t, lds0);
-    else wave_tile<2, 4, 4, GATE_UP, STREAM>(t, lds0);
+    if (t.rbt <= 4) wave_tile<1, 2, 4, 2, 2, Square, GATE_UP, STREAM>(t, lds0);
+    else wave_tile<2, 4, 4, 2, 2, Square, GATE_UP, STREAM>(t, lds0);
   } else {
-    if (t.rbt <= 4) wave_tile<1, 2, 8, GATE_UP, STREAM>(t, lds0);
-    else wave_tile<1, 4, 8, GATE_UP, STREAM>(t, lds0);
+    if (t.rbt <= 4) wave_tile<1, 2, 8, 2, 2, Square, GATE_UP, STREAM>(t, lds0);
+    else wave_tile<1, 4, 8, 2, 2, Square, GATE_UP, STREAM>(t, lds0);
   }
 }
 
 template <bool GATE_UP>
 hipError_t launch(const void *a, const void *w, const float *ba, const float *bb, const DispatchBuffers &d, void *out,
-                  int K, int N, float limit, int T, int E, int tile_rows, bool stream, hipStream_t s) {
+                  int K, int N, float limit, int T, int E, int tile_rows, bool wide, bool stream, hipStream_t s) {
   const int nb_total = (GATE_UP ? 2 * N : N) / kRowBlock;
   const int n_ct = (nb_total + kGemmTileNb - 1) / kGemmTileNb;
   const int grid = kXcds * xcd_tile_cap(gemm_tile_cap(T, E, tile_rows) * n_ct);
   const TileDesc *tiles = GATE_UP ? d.tiles_gate_up : d.tiles_down;
   const char *ac = static_cast<const char *>(a), *wc = static_cast<const char *>(w);
-  if (stream)
+  if (stream || wide)
     bf16_gemm_kernel<GATE_UP, true><<<grid, kThreads, 0, s>>>(ac, wc, ba, bb, tiles, d.totals, d.rowmap, out, K, N, limit);
   else
     bf16_gemm_kernel<GATE_UP, false><<<grid, kThreads, 0, s>>>(ac, wc, ba, bb, tiles, d.totals, d.rowmap, out, K, N, limit);
@@ -423,13 +468,13 @@ hipError_t launch(const void *a, const void *w, const float *ba, const float *bb
 
 hipError_t launch_bf16_gate_up(const uint16_t *x, const void *w1, const float *b1g, const float *b1u,
                                const DispatchBuffers &d, uint16_t *act, int H, int IM, float limit, int T, int E,
-                               int tile_rows, bool stream, hipStream_t s) {
-  return launch<true>(x, w1, b1g, b1u, d, act, H, IM, limit, T, E, tile_rows, stream, s);
+                               int tile_rows, bool wide, bool stream, hipStream_t s) {
+  return launch<true>(x, w1, b1g, b1u, d, act, H, IM, limit, T, E, tile_rows, wide, stream, s);
 }
 
 hipError_t launch_bf16_down(const uint16_t *act, const void *w2, const float *b2, const DispatchBuffers &d, float *y,
-                            int H, int IM, int T, int E, int tile_rows, bool stream, hipStream_t s) {
-  return launch<false>(act, w2, b2, nullptr, d, y, IM, H, 0.f, T, E, tile_rows, stream, s);
+                            int H, int IM, int T, int E, int tile_rows, bool wide, bool stream, hipStream_t s) {
+  return launch<false>(act, w2, b2, nullptr, d, y, IM, H, 0.f, T, E, tile_rows, wide, stream, s);
 }
 
 }  // namespace moe

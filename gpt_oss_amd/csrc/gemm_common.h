@@ -51,7 +51,8 @@ __host__ __device__ inline int row_split_of(int nb_valid, int nw, int nbw) {
 
 // Maps the workgroup id to a tile (see "Tile order" above): two dependent
 // loads, the XCD's range and the tile's descriptor.  Returns false for the
-// surplus workgroups of the upper-bound grid.
+// surplus workgroups of the upper-bound grid.  A wide plan (tile_width; a handle with layers of both formats,
+// dispatched before the layer is named) has two workgroups to a tile, for its first column blocks and the rest.
 __device__ __forceinline__ bool locate_tile(const TileDesc *__restrict__ tiles,
                                             const int *__restrict__ bounds, TileDesc &d) {
   const int bid = blockIdx.x;
@@ -59,7 +60,10 @@ __device__ __forceinline__ bool locate_tile(const TileDesc *__restrict__ tiles,
   const int L = bounds[xcd] + (bid >> 3);
   if (L >= bounds[xcd + 1]) return false;
   d = tiles[L];
-  return true;
+  const int first = blockIdx.y * kGemmTileNb, nbt = min(d.nbt - first, kGemmTileNb);
+  d.nb0 += first;
+  d.nbt = (uint16_t)nbt;
+  return nbt > 0;
 }
 
 // ---- vector-memory instructions of the main loop ----

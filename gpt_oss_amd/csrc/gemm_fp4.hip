@@ -590,8 +590,7 @@ __global__ __launch_bounds__(C::THREADS, C::WGS) void fp4_gemm_kernel(
   const int nb_total = (GATE_UP ? 2 * N : N) / kRowBlock;  // weight row blocks per expert
   TileDesc tc;
   if (!locate_tile(tiles, totals + (GATE_UP ? kTotBoundsGateUp : kTotBoundsDown), tc)) return;
-  const int nb0 = tc.nt * C::TILE_NB;
-  const int nb_valid = min(C::TILE_NB, nb_total - nb0);
+  const int nb0 = tc.nb0, nb_valid = tc.nbt;
   // per expert (nb_total/2) * (KB/2) chunks of 1 KB
   const uint4 *b_frag = w_frag + (size_t)tc.e * nb_total * KB * 16;
   const uint16_t *b_scale = w_scale + (size_t)tc.e * nb_total * KB * 8;
@@ -633,11 +632,11 @@ static_assert(Cfg::RBT_MAX * kRowBlock == kHalfTileRows && Cfg::TILE_NB == kGemm
 
 template <bool GATE_UP>
 hipError_t launch(const void *a, const void *w, const uint16_t *w_scale, const float *ba, const float *bb,
-                  const DispatchBuffers &d, void *out, int K, int N, float limit, int T, int E, bool stream,
+                  const DispatchBuffers &d, void *out, int K, int N, float limit, int T, int E, bool wide, bool stream,
                   hipStream_t s) {
   const int nb_total = (GATE_UP ? 2 * N : N) / kRowBlock;
   const int n_ct = (nb_total + kGemmTileNb - 1) / kGemmTileNb;
-  const int grid = kXcds * xcd_tile_cap(gemm_tile_cap(T, E, kHalfTileRows) * n_ct);
+  const dim3 grid(kXcds * xcd_tile_cap(gemm_tile_cap(T, E, kHalfTileRows) * n_ct), wide ? 2 : 1);
   const TileDesc *tiles = GATE_UP ? d.tiles_gate_up : d.tiles_down;
   const uint4 *af = static_cast<const uint4 *>(a), *wf = static_cast<const uint4 *>(w);
   if (stream)
@@ -653,13 +652,14 @@ hipError_t launch(const void *a, const void *w, const uint16_t *w_scale, const f
 
 hipError_t launch_fp4_gate_up(const uint16_t *x, const void *w1, const uint16_t *w1_scale, const float *b1g,
                               const float *b1u, const DispatchBuffers &d, uint16_t *act, int H, int IM, float limit,
-                              int T, int E, bool stream, hipStream_t s) {
-  return launch<true>(x, w1, w1_scale, b1g, b1u, d, act, H, IM, limit, T, E, stream, s);
+                              int T, int E, bool wide, bool stream, hipStream_t s) {
+  return launch<true>(x, w1, w1_scale, b1g, b1u, d, act, H, IM, limit, T, E, wide, stream, s);
 }
 
 hipError_t launch_fp4_down(const uint16_t *act, const void *w2, const uint16_t *w2_scale, const float *b2,
-                           const DispatchBuffers &d, float *y, int H, int IM, int T, int E, bool stream, hipStream_t s) {
-  return launch<false>(act, w2, w2_scale, b2, nullptr, d, y, IM, H, 0.f, T, E, stream, s);
+                           const DispatchBuffers &d, float *y, int H, int IM, int T, int E, bool wide, bool stream,
+                           hipStream_t s) {
+  return launch<false>(act, w2, w2_scale, b2, nullptr, d, y, IM, H, 0.f, T, E, wide, stream, s);
 }
 
 }  // namespace moe

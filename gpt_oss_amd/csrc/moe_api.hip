@@ -67,6 +67,7 @@ struct moe_handle {
   int a_pad_cap = 0;  // max padded rows
   int n_blk_cap = 0;
   int plan_rows = kTileRows;  // tallest row tile of the last plan
+  bool plan_wide = false;     // ... and whether its tiles are of tile_width
   int disp_tokens = -1;  // batch of the last moe_dispatch (stage-level calls), -1: none
   bool gemms_done = false;  // moe_expert_gemms has run on that dispatch: y holds its rows
   bool distinct_ids = false;  // moe_set_distinct_ids: caller-supplied ids name an expert once per token
@@ -154,8 +155,11 @@ int run_dispatch(moe_handle *h, const int *topk_i, const int *pos, int T, bool m
   h->plan_rows = plan_tile_rows(T, E, h->Hp, h->IMp, mxfp4, h->expert_bytes <= kCachedWeightBytes);
   // the kernels of stream.hip go by row blocks and need no tile tables
   const bool tables = !stream_batch(T, E);
-  HIP_TRY(launch_dispatch(topk_i, pos, T, E, tables ? gate_up_col_tiles(h) : 0, tables ? down_col_tiles(h) : 0,
-                          h->plan_rows, h->disp, s));
+  h->plan_wide = tables && !mxfp4 &&
+                 bf16_wide_tiles(T, E, h->Hp, h->IMp,
+                                 gemm_streams_weights(T, E, false, h->plan_rows, h->expert_bytes <= kCachedWeightBytes));
+  HIP_TRY(launch_dispatch(topk_i, pos, T, E, tables ? 2 * h->IMp / kRowBlock : 0, tables ? h->Hp / kRowBlock : 0,
+                          h->plan_rows, h->plan_wide, h->disp, s));
   return MOE_OK;
 }
 
@@ -189,9 +193,9 @@ int run_gemms(moe_handle *h, int layer, const uint16_t *x, int T, const DirectId
     return MOE_OK;
   }
   HIP_TRY(launch_gate_up(x, w1, lw.w1s, lw.b1g, lw.b1u, h->disp, h->act, h->Hp, h->IMp, c.swiglu_limit, T,
-                         c.experts, h->plan_rows, cached, s));
+                         c.experts, h->plan_rows, h->plan_wide, cached, s));
   HIP_TRY(tm.mark(MOE_STAGE_DOWN));
-  HIP_TRY(launch_down(h->act, w2, lw.w2s, lw.b2, h->disp, h->y, h->Hp, h->IMp, T, c.experts, h->plan_rows, cached, s));
+  HIP_TRY(launch_down(h->act, w2, lw.w2s, lw.b2, h->disp, h->y, h->Hp, h->IMp, T, c.experts, h->plan_rows, h->plan_wide, cached, s));
   return MOE_OK;
 }
 

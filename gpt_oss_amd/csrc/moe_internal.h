@@ -40,7 +40,7 @@ constexpr float kAlpha = 1.702f;  // run.cpp:709
 // range of about an eighth of the estimated cost.  (Cutting the last tiles of a range into smaller pieces, so
 // that its CUs run dry together, was measured and does not pay: the pieces are
 // less efficient than what they save.)
-constexpr int kGemmTileNb = 8;  // column blocks (of 32) per tile of the grouped GEMMs
+constexpr int kGemmTileNb = 8;  // column blocks (of 32) per tile of the grouped GEMMs (tile_width: wider plans)
 constexpr int kRowTileGroup = 4;  // row tiles of one expert that run side by side (see write_expert_tiles)
 constexpr int kXcds = 8;
 // estimated cost of a tile: kCostPerTile + kCostPerRowBlock * row blocks.  The
@@ -67,7 +67,7 @@ struct ExpertInfo {
   int rb;         // row blocks of the expert's shorter tiles (0..8)
   int tile_base;  // number of row tiles of all lower experts
   int extra;      // its first `extra` tiles have rb + 1 row blocks
-  int pad_[2];
+  int tiles0[2];  // tiles of all lower experts in the sequences of gate_up and down
 };
 
 // One tile of a grouped GEMM, looked up by its number in the tile sequence.
@@ -77,9 +77,14 @@ struct ExpertInfo {
 struct TileDesc {
   int e;    // expert
   int rb0;  // first row block of the tile in the padded row space
-  int rbt;  // its row blocks (1..8)
-  int nt;   // column tile
+  uint16_t rbt, nbt;  // its row blocks (1..8) and column blocks (1..10)
+  int nb0;  // its first column block
 };
+// Column blocks of a tile of so many row blocks.  wide: see bf16_wide_tiles.
+constexpr int kWideTileRb = 6, kWideTileNb = 10;
+__host__ __device__ inline int tile_width(int height, bool wide) {
+  return wide && height <= kWideTileRb ? kWideTileNb : kGemmTileNb;
+}
 
 struct LayerWeights {
   uint16_t *wr = nullptr;  // router weight, bf16 in the operand order of v_mfma_f32_16x16x32_bf16
@@ -165,9 +170,10 @@ struct DispatchBuffers {
   TileDesc *tiles_down;     // [tile_cap_down]    ... of the down GEMM
   int tile_cap_gate_up, tile_cap_down;
 };
-// tile_rows: tallest row tile of the plan (kTileRows or kHalfTileRows)
-hipError_t launch_dispatch(const int *topk_i, const int *pos, int T, int E, int n_ct_gate_up,
-                           int n_ct_down, int tile_rows, const DispatchBuffers &d, hipStream_t s);
+// tile_rows: tallest row tile of the plan (kTileRows or kHalfTileRows); wide: tile_width; nb_*: column blocks of
+// an expert's matrices (0: no tile tables)
+hipError_t launch_dispatch(const int *topk_i, const int *pos, int T, int E, int nb_gate_up, int nb_down,
+                           int tile_rows, bool wide, const DispatchBuffers &d, hipStream_t s);
 
 // Batches of at most kDirectTokens tokens run without a dispatch pass: the 256
 // threads of a workgroup hold one assignment each, so every workgroup of the
@@ -291,6 +297,18 @@ inline bool gemm_streams_weights(int T, int E, bool mxfp4, int tile_rows, bool c
   if (cached || tile_rows != (mxfp4 ? kHalfTileRows : kTileRows)) return false;
   return T * kTopK <= (mxfp4 ? kStreamRowsFp4 : kStreamRowsBf16) * E;
 }
+// bf16 weights past the caches: whether tiles of up to 6 row blocks take 10 column blocks instead of 8 (the
+// registers and the LDS of a workgroup hold 60 as well as 64).  A tile streams its weights for its
+// whole life but for a fill and an epilogue, and reads its rows once per tile: fewer tiles, less of either.  But a
+// wider tile makes the CUs' last round of tiles longer, so there have to be rounds enough.  us per
+// layer call, 8 / 10 column blocks: 128 experts, 6144 tokens (9 rounds in gate_up, 4.5 in down) 1555 / 1457, 2000, Zipf's
+// routing, 1211 / 1205; 32 experts, 256 tokens (2.3, 1.1) 294 / 329, 672 of 896 315 / 354, 512, Zipf's, 346 /
+// 340, 1400 (exponent 0.6) 415 / 390; 8 experts, 250 135 / 152.
+inline bool bf16_wide_tiles(int T, int E, int H, int IM, bool past_caches) {
+  const int cols = (H < 2 * IM ? H : 2 * IM) / kRowBlock;
+  const int row_tiles = T * kTopK / kTileRows > E ? T * kTopK / kTileRows : E;
+  return past_caches && (long long)row_tiles * ((cols + kWideTileNb - 1) / kWideTileNb) >= 4 * kCus;
+}
 // Row tiles of a plan, and what runs on it.
 inline int plan_tile_rows(int T, int E, int H, int IM, bool mxfp4, bool cached) {
   return (mxfp4 ? half_tiles(T, E, 2 * IM) : bf16_half_tiles(T, E, H, IM, cached)) ? kHalfTileRows : kTileRows;
@@ -319,23 +337,24 @@ constexpr size_t kCachedWeightBytes = (size_t)256 << 20;
 // same file reads it: MFMA fragments (gemm.hip), quads or rows (stream.hip).
 hipError_t launch_gate_up(const uint16_t *x, const void *w1, const uint16_t *w1_scale, const float *b1g,
                           const float *b1u, const DispatchBuffers &d, uint16_t *act, int H, int IM,
-                          float limit, int T, int E, int tile_rows, bool cached, hipStream_t s);
+                          float limit, int T, int E, int tile_rows, bool wide, bool cached, hipStream_t s);
 hipError_t launch_down(const uint16_t *act, const void *w2, const uint16_t *w2_scale, const float *b2,
                        const DispatchBuffers &d, float *y, int H, int IM, int T, int E, int tile_rows,
-                       bool cached, hipStream_t s);
+                       bool wide, bool cached, hipStream_t s);
 // bf16 weights (gemm_bf16.hip; launch_gate_up and launch_down call them), a plan of either height.
 // stream: weights past the caches.
 hipError_t launch_bf16_gate_up(const uint16_t *x, const void *w1, const float *b1g, const float *b1u,
                                const DispatchBuffers &d, uint16_t *act, int H, int IM, float limit, int T, int E,
-                               int tile_rows, bool stream, hipStream_t s);
+                               int tile_rows, bool wide, bool stream, hipStream_t s);
 hipError_t launch_bf16_down(const uint16_t *act, const void *w2, const float *b2, const DispatchBuffers &d, float *y,
-                            int H, int IM, int T, int E, int tile_rows, bool stream, hipStream_t s);
+                            int H, int IM, int T, int E, int tile_rows, bool wide, bool stream, hipStream_t s);
 // MXFP4 weights with many rows per expert (gemm_fp4.hip; likewise), a plan of kHalfTileRows.
 hipError_t launch_fp4_gate_up(const uint16_t *x, const void *w1, const uint16_t *w1_scale, const float *b1g,
                               const float *b1u, const DispatchBuffers &d, uint16_t *act, int H, int IM, float limit,
-                              int T, int E, bool stream, hipStream_t s);
+                              int T, int E, bool wide, bool stream, hipStream_t s);
 hipError_t launch_fp4_down(const uint16_t *act, const void *w2, const uint16_t *w2_scale, const float *b2,
-                           const DispatchBuffers &d, float *y, int H, int IM, int T, int E, bool stream, hipStream_t s);
+                           const DispatchBuffers &d, float *y, int H, int IM, int T, int E, bool wide, bool stream,
+                           hipStream_t s);
 // tiles: row tiles, at most (stream_direct_tile_cap with ids.topk_i, otherwise stream_tile_cap).
 // T, E: tokens and experts of the batch, the same for both (the order of act between them follows from these).
 // cached: kCachedWeightBytes.

@@ -224,3 +224,69 @@ def test_sides_of_the_product_lines(n_experts, H, IM, T, fp4_route, bf16_rows):
     d = got[0][rows] - want
     assert np.abs(d).max() <= 2e-2 * max(1.0, float(np.abs(want).max()))
     assert np.linalg.norm(d) <= 1e-3 * np.linalg.norm(want)
+
+
+# H, IM of wide plans at 256 experts (tests/test_host_rules.py holds the rule to them): remainders of 2 column blocks
+# in both GEMMs, of 6 in gate_up and 4 in down, of none in gate_up and 8 in down
+WIDE = [(1024, 512), (1088, 576), (1216, 640)]
+
+
+@pytest.mark.parametrize("H,IM", WIDE)
+def test_wide_tiles(H, IM):
+    """Tiles of ten column blocks (up to 6 row blocks high, weights past the caches) beside
+    tiles of eight, every height, and their last column tiles: the bits of the MXFP4 kernels, whose tiles have
+    eight, stage by stage and with an MXFP4 layer under a wide plan as well, and the oracle."""
+    n, kinds = 256, 4  # experts of four kinds
+    rng = np.random.default_rng(H)
+    rows = [1, 31, 32, 33, 64, 65, 96, 97, 128, 129, 160, 161, 191, 192, 193, 224, 225, 256, 257, 321, 385]
+    rows = rng.permutation(rows + [2] * (n - len(rows)))
+    ids = np.repeat(np.arange(n), rows).astype(np.int32)
+    T = n * 4 + 4  # stream.hip has batches of up to 16 rows per expert on average
+    assert len(ids) <= 4 * T
+    ids = rng.permutation(np.concatenate([ids, np.full(4 * T - len(ids), -1, np.int32)])).reshape(T, 4)
+    tv = rng.random((T, 4)).astype(np.float32)
+    sh = synth.LayerShape("wide", T, H, IM, kinds)
+    x = synth.round_bf16(synth.make_activations(sh))
+    wr, br = (synth.round_bf16(a) for a in synth.make_router(synth.LayerShape("wide", T, H, IM, n)))
+    kind = synth.make_experts_mxfp4(sh)
+    b1k, s1, b1, b2k, s2, b2 = (np.tile(a, (n // kinds,) + (1,) * (a.ndim - 1)) for a in kind)
+    b1, b2 = synth.round_bf16(b1), synth.round_bf16(b2)
+    w1, w2 = ob.mxfp4_dequant(kind[0], kind[1]), ob.mxfp4_dequant(kind[3], kind[4])
+    dx, dti = abi.DevBuf.from_numpy(synth.to_bf16_bits(x)), abi.DevBuf.from_numpy(ids)
+    dtv, dout = abi.DevBuf.from_numpy(tv), abi.DevBuf(T * H * 4)
+    assert abi.batch_kernel(H, IM, n, T, False) == (BF16, 256, True)
+    got = []
+
+    def staged(m, layer):
+        dout.memset(0xFF)
+        m.dispatch(dti, None, T)
+        m.expert_gemms(layer, dx, T)
+        m.combine(dtv, None, T, dout)
+        abi.sync()
+        got.append(dout.download((T, H), np.float32))
+
+    m = abi.Moe(H, IM, n, max_tokens=T, swiglu_limit=sh.limit, layers=2)
+    m.upload_layer_mxfp4(1, wr, br, b1k, s1, b1, b2k, s2, b2)
+    staged(m, 1)  # no bf16 layer: not a wide plan
+    m.upload_layer(0, wr, br, np.tile(w1, (n // kinds, 1, 1)), b1, np.tile(w2, (n // kinds, 1, 1)), b2)
+    for _ in range(3):
+        dout.memset(0xFF)
+        m.experts(0, dx, None, dti, dtv, T, dout)
+        abi.sync()
+        got.append(dout.download((T, H), np.float32))
+    for layer in (0, 1):
+        staged(m, layer)
+    m.close()
+    for other in got[1:]:
+        assert np.array_equal(got[0], other)
+    experts = np.nonzero(np.asarray(rows) > 2)[0]
+    some = np.unique(np.concatenate([np.nonzero((ids == e).any(1))[0][[0, -1]] for e in experts]))
+    want = np.zeros((len(some), H), np.float32)
+    for i, t in enumerate(some):
+        for k, e in enumerate(ids[t]):
+            if e >= 0:
+                want[i] += tv[t, k] * ob.expert_token(x[t], w1[e % kinds], b1[e], w2[e % kinds], b2[e], sh.limit,
+                                                      mode=ob.ROUND_ACT_BF16)
+    d = got[0][some] - want
+    assert np.abs(d).max() <= 2e-2 * max(1.0, float(np.abs(want).max()))
+    assert np.linalg.norm(d) <= 1e-3 * np.linalg.norm(want)

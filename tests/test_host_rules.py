@@ -10,6 +10,7 @@ from gpt_oss_amd import build
 SOURCE = """
 #include "%s/moe_internal.h"
 extern "C" int split_router_tokens(int E_pad, int H) { return moe::split_router_tokens(E_pad, H); }
+extern "C" int bf16_wide_tiles(int T, int E, int H, int IM, int past) { return moe::bf16_wide_tiles(T, E, H, IM, past); }
 extern "C" int norm_wave_per_token(int T, int H) { return moe::norm_wave_per_token(T, H); }
 """ % build.CSRC
 
@@ -39,3 +40,12 @@ def test_router_splits_where_it_gains(rules, E_pad, H, tokens):
 def test_norm_of_short_rows_takes_a_wave(rules, T, H, wave):
     """A workgroup per token of short rows is mostly idle threads (times in norm.hip)."""
     assert rules.norm_wave_per_token(T, H) == wave
+
+
+@pytest.mark.parametrize("T,E,H,IM,past,wide", [
+    (6144, 128, 2880, 2880, 1, 1), (2000, 128, 2880, 2880, 1, 1), (6144, 128, 2880, 2880, 0, 0),
+    (256, 32, 2880, 2880, 1, 0), (1400, 32, 2880, 2880, 1, 0), (250, 8, 2880, 2880, 1, 0),
+    (1028, 256, 1024, 512, 1, 1), (1028, 256, 1088, 576, 1, 1), (1028, 256, 1216, 640, 1, 1), (1028, 256, 960, 512, 1, 0)])
+def test_wide_tiles_where_the_cus_take_many_rounds(rules, T, E, H, IM, past, wide):
+    """Tiles of ten column blocks gain with four rounds of tiles and lose with two (times in moe_internal.h)."""
+    assert rules.bf16_wide_tiles(T, E, H, IM, past) == wide
