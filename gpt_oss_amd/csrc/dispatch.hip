@@ -50,10 +50,11 @@ struct PlanOut {
   int tile_rb;  // row blocks of the tallest tile
   int nb[2];    // column blocks of an expert's matrices, gate_up and down (0: no tile tables)
   bool wide;    // tile_width
+  int tile_cost;  // fixed part of a tile's estimated cost
   // column tiles of GEMM g over an expert whose tallest tile has so many row blocks
   __device__ __forceinline__ int col_tiles(int g, int height) const {
-    const int width = tile_width(height, wide);
-    return (nb[g] + width - 1) / width;
+    return tile_width(height, wide) == kGemmTileNb ? (nb[g] + kGemmTileNb - 1) / kGemmTileNb
+                                                   : (nb[g] + kWideTileNb - 1) / kWideTileNb;
   }
 };
 
@@ -110,7 +111,7 @@ __device__ __forceinline__ void write_expert_tiles(int ee, int nmt, int rbe, int
 __device__ __forceinline__ int build_plan(int count, int E, const PlanOut &out, bool with_tiles, int *ex_count_out,
                                           int *tot_count_out = nullptr, bool write_global = true,
                                           ExpertInfo *info_out = nullptr) {
-  constexpr int kSums = 6;
+  constexpr int kSums = 6, kSumsPlan = 3;  // the last ones are of the tile tables
   __shared__ int sh_wave[4][kSums];  // [wave][quantity]: the waves' sums
   __shared__ int sh_nmt[256], sh_rb[256], sh_extra[256], sh_rowblk[256];
   __shared__ int sh_cost[257];      // exclusive prefix of the experts' cost
@@ -127,9 +128,10 @@ __device__ __forceinline__ int build_plan(int count, int E, const PlanOut &out, 
   const int rb = n_mt ? n_rb / n_mt : 0;
   const int extra = n_mt ? n_rb - rb * n_mt : 0;
   const int height = rb + (extra ? 1 : 0);
+  const bool tables = out.nb[0] > 0;
   const int n_up = n_mt * out.col_tiles(0, height), n_down = n_mt * out.col_tiles(1, height);
   // cost of kGemmTileNb column blocks' worth of the expert's row tiles: of tiles of any width, whose cost goes by it
-  const int cost = n_mt * (kCostPerTile + kCostPerRowBlock * rb) + kCostPerRowBlock * extra;
+  const int cost = n_mt * (out.tile_cost + kCostPerRowBlock * rb) + kCostPerRowBlock * extra;
   // Exclusive prefix sums over the experts of six quantities at once: rows,
   // padded rows, row tiles, cost, tiles of either GEMM.  In a wave by lane shifts, across the four
   // waves through LDS.
@@ -141,6 +143,7 @@ __device__ __forceinline__ int build_plan(int count, int E, const PlanOut &out, 
   for (int off = 1; off < 64; off <<= 1) {
 #pragma unroll
     for (int i = 0; i < kSums; i++) {
+      if (i >= kSumsPlan && !tables) break;
       const int up = __shfl_up(incl[i], off, 64);
       if (lane >= off) incl[i] += up;
     }
@@ -181,7 +184,6 @@ __device__ __forceinline__ int build_plan(int count, int E, const PlanOut &out, 
     }
     if (info_out) *info_out = inf;
   }
-  const bool tables = out.nb[0] > 0;
   if (write_global && !tables && e == 0) {
     offsets[E] = tot_count;
     totals[kTotTiles] = tot_mt;
@@ -275,7 +277,7 @@ __device__ __forceinline__ int build_plan(int count, int E, const PlanOut &out, 
 // the padded row space is its row blocks and no more, so an expert pads to at
 // most 31 rows.  The tile sequence of either GEMM (n_ct column tiles per row
 // tile) is cut into the 8 ranges of the XCDs by estimated cost: a tile of r row
-// blocks costs kCostPerTile + kCostPerRowBlock * r.
+// blocks costs tile_cost + kCostPerRowBlock * r.
 
 // Ranks inside one wave: for each of the lane's kTopK expert ids, how many of
 // the wave's assignments to the same expert come before it in (lane, slot)
@@ -548,7 +550,7 @@ __global__ __launch_bounds__(256) void combine_kernel(const float *__restrict__ 
 }
 
 hipError_t launch_dispatch(const int *topk_i, const int *pos, int T, int E, int nb_gate_up, int nb_down,
-                           int tile_rows, bool wide, const DispatchBuffers &d, hipStream_t s) {
+                           int tile_rows, bool wide, int tile_cost, const DispatchBuffers &d, hipStream_t s) {
   const int n_blk = (T + kDispThreads - 1) / kDispThreads;
   // Rows of the padded space this batch can reach: every expert rounds its
   // rows up to a multiple of 32.
@@ -567,6 +569,7 @@ hipError_t launch_dispatch(const int *topk_i, const int *pos, int T, int E, int 
   plan.nb[0] = nb_gate_up;
   plan.nb[1] = nb_down;
   plan.wide = wide;
+  plan.tile_cost = tile_cost;
   if (n_blk <= kSmallRounds) {
     // small batches: one workgroup does both passes, one launch fewer
     dispatch_small_kernel<<<1, kDispThreads, 0, s>>>(topk_i, pos, T, E, plan, d.perm,
@@ -681,7 +684,7 @@ extern "C" int moe_dispatch_static(const int *topk_i, const int *pos, int n_toke
   // no GEMM follows: with no column tiles the plan kernel writes no tile tables
   d.tiles_gate_up = d.tiles_down = nullptr;
   d.tile_cap_gate_up = d.tile_cap_down = 0;
-  const hipError_t el = launch_dispatch(topk_i, pos, n_tokens, n_experts, 0, 0, kTileRows, false, d, static_cast<hipStream_t>(stream));
+  const hipError_t el = launch_dispatch(topk_i, pos, n_tokens, n_experts, 0, 0, kTileRows, false, 0, d, static_cast<hipStream_t>(stream));
   if (el != hipSuccess)
     return set_error(MOE_ERR_HIP, "dispatch launch failed: %s", hipGetErrorString(el));
   return MOE_OK;

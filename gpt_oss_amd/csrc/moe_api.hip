@@ -159,7 +159,7 @@ int run_dispatch(moe_handle *h, const int *topk_i, const int *pos, int T, bool m
                  bf16_wide_tiles(T, E, h->Hp, h->IMp,
                                  gemm_streams_weights(T, E, false, h->plan_rows, h->expert_bytes <= kCachedWeightBytes));
   HIP_TRY(launch_dispatch(topk_i, pos, T, E, tables ? 2 * h->IMp / kRowBlock : 0, tables ? h->Hp / kRowBlock : 0,
-                          h->plan_rows, h->plan_wide, h->disp, s));
+                          h->plan_rows, h->plan_wide, plan_tile_cost(T, E, 2 * h->IMp, mxfp4), h->disp, s));
   return MOE_OK;
 }
 

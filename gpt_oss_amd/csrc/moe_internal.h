@@ -43,11 +43,7 @@ constexpr float kAlpha = 1.702f;  // run.cpp:709
 constexpr int kGemmTileNb = 8;  // column blocks (of 32) per tile of the grouped GEMMs (tile_width: wider plans)
 constexpr int kRowTileGroup = 4;  // row tiles of one expert that run side by side (see write_expert_tiles)
 constexpr int kXcds = 8;
-// estimated cost of a tile: kCostPerTile + kCostPerRowBlock * row blocks.  The
-// fixed part (4 row blocks' worth) was fitted on measured runs with even,
-// Zipf-skewed and 128-expert routing; it stands for the column operand, which
-// a tile streams in full however few rows it has.
-constexpr int kCostPerTile = 32;
+// Estimated cost of a tile: a fixed part (plan_tile_cost) + kCostPerRowBlock * row blocks.
 constexpr int kCostPerRowBlock = 8;
 // layout of DispatchBuffers::totals
 constexpr int kTotTiles = 0, kTotRows = 1, kTotAssign = 2;
@@ -170,10 +166,10 @@ struct DispatchBuffers {
   TileDesc *tiles_down;     // [tile_cap_down]    ... of the down GEMM
   int tile_cap_gate_up, tile_cap_down;
 };
-// tile_rows: tallest row tile of the plan (kTileRows or kHalfTileRows); wide: tile_width; nb_*: column blocks of
-// an expert's matrices (0: no tile tables)
+// tile_rows: tallest row tile of the plan (kTileRows or kHalfTileRows); wide: tile_width; tile_cost: fixed part of a
+// tile's estimated cost; nb_*: column blocks of an expert's matrices (0: no tile tables)
 hipError_t launch_dispatch(const int *topk_i, const int *pos, int T, int E, int nb_gate_up, int nb_down,
-                           int tile_rows, bool wide, const DispatchBuffers &d, hipStream_t s);
+                           int tile_rows, bool wide, int tile_cost, const DispatchBuffers &d, hipStream_t s);
 
 // Batches of at most kDirectTokens tokens run without a dispatch pass: the 256
 // threads of a workgroup hold one assignment each, so every workgroup of the
@@ -312,6 +308,19 @@ inline bool bf16_wide_tiles(int T, int E, int H, int IM, bool past_caches) {
 // Row tiles of a plan, and what runs on it.
 inline int plan_tile_rows(int T, int E, int H, int IM, bool mxfp4, bool cached) {
   return (mxfp4 ? half_tiles(T, E, 2 * IM) : bf16_half_tiles(T, E, H, IM, cached)) ? kHalfTileRows : kTileRows;
+}
+// Fixed part of a tile's estimated cost, by which the XCDs' ranges are cut.  It stands for the column
+// operand, which a tile streams in full however few rows it has: 8 row blocks' worth with bf16 weights, one
+// and a half with MXFP4, which are a quarter of the bytes, and four in the kernels of many rows.  us per layer call,
+// Zipf's routing of exponent 1.2 (* 0.6) at 2880 x 2880, fixed part 32 / 64 / 96 with bf16: 128 experts, 1000 tokens
+// 1012 / 984 / 989, 2000 1299 / 1215 / 1206, 4000* 1479 / 1416 / 1409, 6144 1995 / 1842 / 1856; 32 experts, 400 333 /
+// 340 / 339, 600* 337 / 346 / 345, 700 387 / 363 / 373, 1000 436 / 412 / 411, 1400* 429 / 410 / 414, 3000 683 / 663 /
+// 670, 7168 1306 / 1292 / 1297; 8 experts, 400 174 / 150 / 150; even routing at 4096 tokens 775 / 778 / 776.
+// 4 / 12 / 20 / 32 with MXFP4: gemm.hip, 128 experts, 1000 tokens 463 / 436 / 462 / 492, 2000 639 / 613 / 636 / 670, 32
+// experts, 300* 168 / 151 / 166 / 167; gemm_fp4.hip, 32 experts, 512 195 / 183 / 184 / 184, 2000* 400 / 390 / 389 /
+// 390, 7168 1168 / 1162 / 1156 / 1165; even routing, 724 194 with 12, 190 with 32, 1000 242 / 252 / 245 / 246.
+inline int plan_tile_cost(int T, int E, int w1_rows, bool mxfp4) {
+  return !mxfp4 ? 64 : (fp4_many_rows(T, E, w1_rows) ? 32 : 12);
 }
 enum TileKernel { kBf16Tiles /* gemm_bf16.hip */, kFp4Tiles /* gemm.hip */, kFp4ManyTiles /* gemm_fp4.hip */ };
 struct TileRoute {
