@@ -11,7 +11,7 @@ namespace moe {
 
 constexpr int kDispThreads = 256;  // tokens per workgroup in count / scatter
 
-// Pass 1: per-workgroup histogram of expert ids over active rows.  Also resets
+// Pass 1 of batches beyond kOnceTokens: per-workgroup histogram of expert ids over active rows.  Also resets
 // rowmap and perm to -1 (a fill kernel rather than a memset so that the call
 // sequence can be captured in a graph).
 __global__ __launch_bounds__(kDispThreads) void dispatch_count_kernel(
@@ -105,15 +105,13 @@ __device__ __forceinline__ void write_expert_tiles(int ee, int nmt, int rbe, int
   }
 }
 
+// Threads from 256 on, if there are any, only take part in the barriers.
 // write_global: this workgroup stores the plan (offsets, per-expert records,
 // totals, XCD bounds); the others only need the values returned to them.
-// with_tiles: this workgroup also writes the tile tables of all experts.
-__device__ __forceinline__ int build_plan(int count, int E, const PlanOut &out, bool with_tiles, int *ex_count_out,
-                                          int *tot_count_out = nullptr, bool write_global = true,
-                                          ExpertInfo *info_out = nullptr) {
+__device__ __forceinline__ int build_plan(int count, int E, const PlanOut &out, bool write_global, int *ex_count_out,
+                                          int *tot_count_out, ExpertInfo *info_out) {
   constexpr int kSums = 6, kSumsPlan = 3;  // the last ones are of the tile tables
   __shared__ int sh_wave[4][kSums];  // [wave][quantity]: the waves' sums
-  __shared__ int sh_nmt[256], sh_rb[256], sh_extra[256], sh_rowblk[256];
   __shared__ int sh_cost[257];      // exclusive prefix of the experts' cost
   __shared__ int sh_tiles[2][257];  // exclusive prefix of their tiles in either GEMM
   __shared__ int sh_bound[2][kXcds + 1];
@@ -148,7 +146,7 @@ __device__ __forceinline__ int build_plan(int count, int E, const PlanOut &out, 
       if (lane >= off) incl[i] += up;
     }
   }
-  if (lane == 63) {
+  if (lane == 63 && w < 4) {
 #pragma unroll
     for (int i = 0; i < kSums; i++) sh_wave[w][i] = incl[i];
   }
@@ -182,8 +180,10 @@ __device__ __forceinline__ int build_plan(int count, int E, const PlanOut &out, 
       offsets[e] = ex_count;
       info[e] = inf;
     }
-    if (info_out) *info_out = inf;
+    *info_out = inf;
   }
+  *ex_count_out = ex_count;
+  *tot_count_out = tot_count;
   if (write_global && !tables && e == 0) {
     offsets[E] = tot_count;
     totals[kTotTiles] = tot_mt;
@@ -194,17 +194,13 @@ __device__ __forceinline__ int build_plan(int count, int E, const PlanOut &out, 
   // divisions are left out (us per call, 128 experts, 200 tokens 313.8 / 310.0; 512 x 512, 32 experts, 128
   // tokens 35.7 / 33.8).
   if (!write_global || !tables) {  // (the same for the whole workgroup)
-    *ex_count_out = ex_count;
-    if (tot_count_out) *tot_count_out = tot_count;
     return ex_pad;
   }
-  sh_cost[e] = ex_cost;
-  sh_tiles[0][e] = ex[4];
-  sh_tiles[1][e] = ex[5];
-  sh_nmt[e] = n_mt;
-  sh_rb[e] = rb;
-  sh_extra[e] = extra;
-  sh_rowblk[e] = ex_pad / kRowBlock;
+  if (e < 256) {
+    sh_cost[e] = ex_cost;
+    sh_tiles[0][e] = ex[4];
+    sh_tiles[1][e] = ex[5];
+  }
   if (e == 0) {
     sh_cost[256] = tot_cost;
     sh_tiles[0][256] = tot[4];
@@ -236,18 +232,11 @@ __device__ __forceinline__ int build_plan(int count, int E, const PlanOut &out, 
       }
       const int c_e = sh_cost[lo + 1] - sh_cost[lo];  // > 0: the search stops on an expert with tiles
       const int n_e = sh_tiles[g][lo + 1] - sh_tiles[g][lo];
-      const long long rest = target - (long long)sh_cost[lo] * kXcds;
-      bound = sh_tiles[g][lo] + (c_e ? min((int)(rest * n_e / ((long long)c_e * kXcds)), n_e) : 0);
+      const long long rest = target - (long long)sh_cost[lo] * kXcds;  // of kXcds * c_e, the expert's share
+      bound = sh_tiles[g][lo] + (c_e ? min((int)((float)rest / ((float)c_e * kXcds) * (float)n_e), n_e) : 0);
       bound = min(bound, total_tiles);
     }
     sh_bound[g][x] = bound;
-  }
-  // The tile sequences (two-launch form: written by the scatter kernel's
-  // workgroups instead, which are many).  The waves take the experts in turn.
-  if (with_tiles) {
-    for (int ee = w; ee < E; ee += 4)
-      write_expert_tiles(ee, sh_nmt[ee], sh_rb[ee], sh_extra[ee], sh_rowblk[ee], sh_tiles[0][ee], sh_tiles[1][ee],
-                         lane, out);
   }
   __syncthreads();
   // keep every range within what the launch grid provides for (xcd_tile_cap)
@@ -255,10 +244,13 @@ __device__ __forceinline__ int build_plan(int count, int E, const PlanOut &out, 
     const int total_tiles = tot[4 + e];
     const int cap = xcd_tile_cap(total_tiles);
     int *bounds = totals + (e ? kTotBoundsDown : kTotBoundsGateUp);
-    int prev = 0;
+    int prev = 0, want[kXcds];
+#pragma unroll
+    for (int x = 1; x < kXcds; x++) want[x] = sh_bound[e][x];
     bounds[0] = 0;
+#pragma unroll
     for (int x = 1; x < kXcds; x++) {
-      int bnd = sh_bound[e][x];
+      int bnd = want[x];
       bnd = max(bnd, max(prev, total_tiles - (kXcds - x) * cap));
       bnd = min(bnd, prev + cap);
       bounds[x] = bnd;
@@ -266,8 +258,6 @@ __device__ __forceinline__ int build_plan(int count, int E, const PlanOut &out, 
     }
     bounds[kXcds] = total_tiles;
   }
-  *ex_count_out = ex_count;
-  if (tot_count_out) *tot_count_out = tot_count;
   return ex_pad;
 }
 
@@ -288,15 +278,27 @@ __device__ __forceinline__ int build_plan(int count, int E, const PlanOut &out, 
 // that slot.  The work no longer grows with the number of experts (4 x faster
 // at 128).  Ids < 0 match nothing; their results are not used.
 template <int NBITS>
-__device__ __forceinline__ void wave_ranks(const int (&id)[kTopK], int lane, int (&rank)[kTopK],
-                                           int (&total)[kTopK]) {
+struct IdPlanes {
   unsigned long long valid[kTopK], plane[kTopK][NBITS];
+  __device__ __forceinline__ explicit IdPlanes(const int (&id)[kTopK]) {
 #pragma unroll
-  for (int k = 0; k < kTopK; k++) {
-    valid[k] = __ballot(id[k] >= 0);
+    for (int k = 0; k < kTopK; k++) {
+      valid[k] = __ballot(id[k] >= 0);
 #pragma unroll
-    for (int b = 0; b < NBITS; b++) plane[k][b] = __ballot(id[k] >= 0 && ((id[k] >> b) & 1));
+      for (int b = 0; b < NBITS; b++) plane[k][b] = __ballot(id[k] >= 0 && ((id[k] >> b) & 1));
+    }
   }
+  // lanes that hold expert e in slot k
+  __device__ __forceinline__ unsigned long long holders(int k, int e) const {
+    unsigned long long m = valid[k];
+#pragma unroll
+    for (int b = 0; b < NBITS; b++) m &= ((e >> b) & 1) ? plane[k][b] : ~plane[k][b];
+    return m;
+  }
+};
+template <int NBITS>
+__device__ __forceinline__ void wave_ranks(const IdPlanes<NBITS> &p, const int (&id)[kTopK], int lane,
+                                           int (&rank)[kTopK], int (&total)[kTopK]) {
   const unsigned long long me = 1ull << lane;
   const unsigned long long lt = me - 1ull;
 #pragma unroll
@@ -304,9 +306,7 @@ __device__ __forceinline__ void wave_ranks(const int (&id)[kTopK], int lane, int
     int r = 0, n = 0;
 #pragma unroll
     for (int k2 = 0; k2 < kTopK; k2++) {
-      unsigned long long m = valid[k2];
-#pragma unroll
-      for (int b = 0; b < NBITS; b++) m &= ((id[k] >> b) & 1) ? plane[k2][b] : ~plane[k2][b];
+      const unsigned long long m = p.holders(k2, id[k]);
       n += __popcll(m);
       r += __popcll(m & lt);             // lower lanes, any slot
       if (k2 < k) r += (m & me) ? 1 : 0;  // this lane, lower slots
@@ -316,23 +316,16 @@ __device__ __forceinline__ void wave_ranks(const int (&id)[kTopK], int lane, int
   }
 }
 
-__device__ __forceinline__ void wave_ranks_for(int E, const int (&id)[kTopK], int lane, int (&rank)[kTopK],
-                                               int (&total)[kTopK]) {
-  if (E <= 32) wave_ranks<5>(id, lane, rank, total);
-  else if (E <= 128) wave_ranks<7>(id, lane, rank, total);
-  else wave_ranks<8>(id, lane, rank, total);
-}
-
-// Pass 2: the plan and the stable permutation in one launch.  Every workgroup
+// Pass 2 of batches beyond kOnceTokens: the plan and the stable permutation in one launch.  Every workgroup
 // adds up the per-workgroup counts of pass 1 itself (at most a few dozen loads
 // per expert): the experts' totals, from which it derives offsets and padded
-// first rows exactly as workgroup 0 does, and the counts of the workgroups
-// before it, its own base inside every expert.  Workgroup 0 also stores the
-// plan for the GEMMs; a one-workgroup kernel between the passes did that before
-// and cost a launch more than the repeated sums cost here.
+// first rows exactly as every other does, and the counts of the workgroups
+// before it, its own base inside every expert.  One more workgroup, the last, stores the
+// plan for the GEMMs, whose search for the XCDs' bounds the others need not wait for.
 // Rank of an assignment inside its expert = (assignments of lower workgroups)
 // + (lower waves of this workgroup) + (lower lanes of this wave) + (lower slots
 // of this token), all for the same expert.
+template <int NBITS>
 __global__ __launch_bounds__(kDispThreads) void dispatch_scatter_kernel(
     const int *__restrict__ topk_i, const int *__restrict__ pos, int T, int E,
     const int *__restrict__ blk_counts, int n_blk, int *__restrict__ perm, int *__restrict__ rowmap,
@@ -366,21 +359,21 @@ __global__ __launch_bounds__(kDispThreads) void dispatch_scatter_kernel(
       }
     }
   }
-  int ex_count;
+  int ex_count, tot_count;
   ExpertInfo inf;
-  const int row0 = build_plan(count, E, plan, /*with_tiles=*/false, &ex_count, nullptr,
-                              /*write_global=*/blockIdx.x == 0, &inf);
+  const int row0 = build_plan(count, E, plan, /*write_global=*/(int)blockIdx.x == n_blk, &ex_count, &tot_count, &inf);
+  if ((int)blockIdx.x == n_blk) return;
   sh_base[tid] = base;
   sh_off[tid] = ex_count;
   sh_row0[tid] = row0;
   sh_info[tid] = inf;
   for (int e = tid; e < (kDispThreads / 64) * 256; e += kDispThreads) (&wave_cnt[0][0])[e] = 0;
   int rank[kTopK], total[kTopK];
-  wave_ranks_for(E, id, lane, rank, total);
+  wave_ranks(IdPlanes<NBITS>(id), id, lane, rank, total);
   __syncthreads();
   // The tile sequences of the GEMMs: the waves of all workgroups take the
   // experts in turn.
-  for (int ee = blockIdx.x * (kDispThreads / 64) + w; ee < E; ee += gridDim.x * (kDispThreads / 64)) {
+  for (int ee = blockIdx.x * (kDispThreads / 64) + w; ee < E; ee += n_blk * (kDispThreads / 64)) {
     const ExpertInfo f = sh_info[ee];
     write_expert_tiles(ee, f.n_mt, f.rb, f.extra, f.row0 / kRowBlock, f.tiles0[0], f.tiles0[1], lane, plan);
   }
@@ -407,94 +400,109 @@ __global__ __launch_bounds__(kDispThreads) void dispatch_scatter_kernel(
       make_int4(out_inv[0], out_inv[1], out_inv[2], out_inv[3]);
 }
 
-// Both passes in one workgroup for batches of at most kSmallRounds x 256 tokens:
-// the rounds of 256 tokens play the part of the workgroups of the two-kernel
-// form (round r's assignments come after those of the rounds before it), so
-// the result is the same, bit for bit.
-constexpr int kSmallRounds = 1;
+// Both passes in one launch for batches of at most kOnceGroups x 64 tokens: every workgroup counts the whole
+// batch, 64 tokens to a wave (lane l counts experts l, l + 64, ...: the holders of each are a mask of
+// bits, see IdPlanes), so that it needs no launch in front, and scatters 256 tokens, one wave
+// to a SIMD.  One more workgroup, the last, stores the plan.  Same result as the two launches, bit for bit.
+// Bound by latency: a launch and a chain of LDS steps.  us of the stage in a call, two launches (one
+// workgroup up to 256 tokens) / this: 200 tokens 14.3 / 10.7, 512 15.5 / 9.8, 896 14.5 / 10.4, 1900 14.6 / 12.2; 128
+// experts, 1000 tokens 18.5 / 13.5.  Every further 1024 tokens are another round of counting, at 4096
+// tokens nothing is left of the gain (14.8 with two launches).
+constexpr int kOnceThreads = 1024, kOnceWaves = kOnceThreads / 64;
+constexpr int kOnceRounds = 2, kOnceGroups = kOnceRounds * kOnceWaves;
+constexpr int kOnceTokens = 64 * kOnceGroups;
 
-__global__ __launch_bounds__(kDispThreads) void dispatch_small_kernel(
-    const int *__restrict__ topk_i, const int *__restrict__ pos, int T, int E, PlanOut out, int *__restrict__ perm, int *__restrict__ rowmap,
-    int *__restrict__ inv, int *__restrict__ blk_expert) {
-  __shared__ int hist[kSmallRounds][256];  // per round and expert: count, then exclusive base
+template <int NBITS>
+__global__ __launch_bounds__(kOnceThreads) void dispatch_once_kernel(
+    const int *__restrict__ topk_i, const int *__restrict__ pos, int T, int E, PlanOut plan, int n_blk,
+    int *__restrict__ perm, int *__restrict__ rowmap, int *__restrict__ inv, int *__restrict__ blk_expert) {
+  __shared__ int cnt[kOnceGroups][256];  // per group of 64 tokens and expert: count, then the rows before the group's
   __shared__ int sh_off[256], sh_row0[256];
-  __shared__ int wave_cnt[kDispThreads / 64][256];
+  __shared__ ExpertInfo sh_info[256];
   const int tid = threadIdx.x;
   const int lane = tid & 63;
-  const int w = tid >> 6;
-  const int n_round = (T + kDispThreads - 1) / kDispThreads;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int groups = (T + 63) / 64;
+  int4 ids[kOnceRounds];
 #pragma unroll
-  for (int r = 0; r < kSmallRounds; r++) hist[r][tid] = 0;
-  __syncthreads();
-  int id[kSmallRounds][kTopK];
-#pragma unroll
-  for (int r = 0; r < kSmallRounds; r++) {
-    const int t = r * kDispThreads + tid;
-#pragma unroll
-    for (int k = 0; k < kTopK; k++) id[r][k] = -1;
-    if (r < n_round && t < T && !(pos && pos[t] < 0)) {
-      const int4 ids = *reinterpret_cast<const int4 *>(topk_i + (size_t)t * kTopK);
-      id[r][0] = ids.x; id[r][1] = ids.y; id[r][2] = ids.z; id[r][3] = ids.w;
-#pragma unroll
-      for (int k = 0; k < kTopK; k++) {
-        if (id[r][k] < 0 || id[r][k] >= E) id[r][k] = -1;
-        if (id[r][k] >= 0) atomicAdd(&hist[r][id[r][k]], 1);
-      }
-    }
+  for (int r = 0; r < kOnceRounds; r++) {
+    const int t = (w + r * kOnceWaves) * 64 + lane;
+    ids[r] = make_int4(-1, -1, -1, -1);
+    if (t < T && !(pos && pos[t] < 0)) ids[r] = *reinterpret_cast<const int4 *>(topk_i + (size_t)t * kTopK);
   }
-  __syncthreads();
-  // expert tid: counts of the rounds -> exclusive bases, total -> plan
-  int count = 0;
-#pragma unroll
-  for (int r = 0; r < kSmallRounds; r++) {
-    const int c = hist[r][tid];
-    hist[r][tid] = count;
-    count += c;
-  }
-  int ex_count, tot_count;
-  const int row0 = build_plan(tid < E ? count : 0, E, out, /*with_tiles=*/true, &ex_count, &tot_count);
-  sh_off[tid] = ex_count;
-  sh_row0[tid] = row0;
-  // -1 where the scatter below writes nothing: the padding rows of the experts
-  // and the tail of perm that inactive rows and invalid ids leave unused
-  if (tid < E) {
-    const int end = row0 + (count + kRowBlock - 1) / kRowBlock * kRowBlock;
-    for (int i = row0 + count; i < end; i++) rowmap[i] = -1;
-  }
-  for (int i = tot_count + tid; i < T * kTopK; i += kDispThreads) perm[i] = -1;
-  __syncthreads();
-  // stable ranks, as dispatch_scatter_kernel
-#pragma unroll
-  for (int r = 0; r < kSmallRounds; r++) {
-    if (r >= n_round) break;
-    for (int e = tid; e < (kDispThreads / 64) * 256; e += kDispThreads) (&wave_cnt[0][0])[e] = 0;
-    int rank[kTopK], total[kTopK];
-    wave_ranks_for(E, id[r], lane, rank, total);
-    __syncthreads();
+  int own[kTopK] = {-1, -1, -1, -1}, rank[kTopK], total[kTopK], own_group = -1;
+#pragma unroll 1
+  for (int r = 0; r < kOnceRounds; r++) {
+    const int g = w + r * kOnceWaves;
+    if (g >= groups) break;
+    const int4 v = r ? ids[1] : ids[0];
+    int id[kTopK] = {v.x, v.y, v.z, v.w};
 #pragma unroll
     for (int k = 0; k < kTopK; k++)
-      if (id[r][k] >= 0) wave_cnt[w][id[r][k]] = total[k];
-    __syncthreads();
-    const int t = r * kDispThreads + tid;
-    if (t < T) {
-      int out_inv[kTopK];
+      if (id[k] >= E) id[k] = -1;
+    const IdPlanes<NBITS> planes(id);
+    for (int e = lane; e < E; e += 64) {
+      int c = 0;
 #pragma unroll
-      for (int k = 0; k < kTopK; k++) {
-        const int e = id[r][k];
-        if (e < 0) { out_inv[k] = -1; continue; }
-        int rk = hist[r][e] + rank[k];
-        for (int ww = 0; ww < w; ww++) rk += wave_cnt[ww][e];
-        const int prow = sh_row0[e] + rk;
-        perm[sh_off[e] + rk] = t * kTopK + k;
-        rowmap[prow] = t * kTopK + k;
-        if (blk_expert && prow % kRowBlock == 0) blk_expert[prow / kRowBlock] = e;
-        out_inv[k] = prow;
-      }
-      *reinterpret_cast<int4 *>(inv + (size_t)t * kTopK) =
-          make_int4(out_inv[0], out_inv[1], out_inv[2], out_inv[3]);
+      for (int k = 0; k < kTopK; k++) c += __popcll(planes.holders(k, e));
+      cnt[g][e] = c;
     }
-    __syncthreads();  // wave_cnt is reused by the next round
+    if (g / (kDispThreads / 64) == (int)blockIdx.x) {
+      own_group = g;
+#pragma unroll
+      for (int k = 0; k < kTopK; k++) own[k] = id[k];
+      wave_ranks(planes, id, lane, rank, total);
+    }
   }
+  __syncthreads();
+  int count = 0;
+  if (tid < E) {
+    for (int g = 0; g < groups; g++) {
+      const int c = cnt[g][tid];
+      cnt[g][tid] = count;
+      count += c;
+    }
+  }
+  int ex_count, tot_count;
+  ExpertInfo inf;
+  const int row0 = build_plan(count, E, plan, /*write_global=*/(int)blockIdx.x == n_blk, &ex_count, &tot_count, &inf);
+  if ((int)blockIdx.x == n_blk) {
+    // -1 where the scatter below writes nothing: the padding rows of the experts
+    // and the tail of perm that inactive rows and invalid ids leave unused
+    if (tid < E) {
+      const int end = row0 + (count + kRowBlock - 1) / kRowBlock * kRowBlock;
+      for (int i = row0 + count; i < end; i++) rowmap[i] = -1;
+    }
+    for (int i = tot_count + tid; i < T * kTopK; i += kOnceThreads) perm[i] = -1;
+    return;
+  }
+  if (tid < E) {
+    sh_off[tid] = ex_count;
+    sh_row0[tid] = row0;
+    sh_info[tid] = inf;
+  }
+  __syncthreads();
+  if (plan.nb[0] > 0) {  // the tile sequences of the GEMMs: the waves of all workgroups take the experts in turn
+    for (int ee = blockIdx.x * kOnceWaves + w; ee < E; ee += n_blk * kOnceWaves) {
+      const ExpertInfo f = sh_info[ee];
+      write_expert_tiles(ee, f.n_mt, f.rb, f.extra, f.row0 / kRowBlock, f.tiles0[0], f.tiles0[1], lane, plan);
+    }
+  }
+  const int t = own_group * 64 + lane;
+  if (own_group < 0 || t >= T) return;
+  int out_inv[kTopK];
+#pragma unroll
+  for (int k = 0; k < kTopK; k++) {
+    const int e = own[k];
+    if (e < 0) { out_inv[k] = -1; continue; }
+    const int rk = cnt[own_group][e] + rank[k];
+    const int prow = sh_row0[e] + rk;
+    perm[sh_off[e] + rk] = t * kTopK + k;
+    rowmap[prow] = t * kTopK + k;
+    if (blk_expert && prow % kRowBlock == 0) blk_expert[prow / kRowBlock] = e;
+    out_inv[k] = prow;
+  }
+  *reinterpret_cast<int4 *>(inv + (size_t)t * kTopK) = make_int4(out_inv[0], out_inv[1], out_inv[2], out_inv[3]);
 }
 
 // out[t,:] (+)= sum_k topk_v[t,k] * y[inv[t,k],:], slots added in order 0..3
@@ -570,16 +578,29 @@ hipError_t launch_dispatch(const int *topk_i, const int *pos, int T, int E, int 
   plan.nb[1] = nb_down;
   plan.wide = wide;
   plan.tile_cost = tile_cost;
-  if (n_blk <= kSmallRounds) {
-    // small batches: one workgroup does both passes, one launch fewer
-    dispatch_small_kernel<<<1, kDispThreads, 0, s>>>(topk_i, pos, T, E, plan, d.perm,
-                                                     d.rowmap, d.inv, d.blk_expert);
+  // ids are compared in as many bits as the experts have
+#define MOE_BY_EXPERTS(LAUNCH)  \
+  do {                          \
+    if (E <= 32) LAUNCH(5);     \
+    else if (E <= 128) LAUNCH(7); \
+    else LAUNCH(8);             \
+  } while (0)
+  if (T <= kOnceTokens) {
+#define MOE_ONCE(BITS)                                                                                         \
+  dispatch_once_kernel<BITS><<<n_blk + 1, kOnceThreads, 0, s>>>(topk_i, pos, T, E, plan, n_blk, d.perm, d.rowmap, \
+                                                                d.inv, d.blk_expert)
+    MOE_BY_EXPERTS(MOE_ONCE);
+#undef MOE_ONCE
     return hipGetLastError();
   }
   dispatch_count_kernel<<<n_blk, kDispThreads, 0, s>>>(topk_i, pos, T, E, d.blk_counts, d.rowmap,
                                                        fill_rows, d.perm);
-  dispatch_scatter_kernel<<<n_blk, kDispThreads, 0, s>>>(topk_i, pos, T, E, d.blk_counts, n_blk, d.perm,
-                                                         d.rowmap, d.inv, d.blk_expert, plan);
+#define MOE_SCATTER(BITS)                                                                                         \
+  dispatch_scatter_kernel<BITS><<<n_blk + 1, kDispThreads, 0, s>>>(topk_i, pos, T, E, d.blk_counts, n_blk, d.perm, \
+                                                               d.rowmap, d.inv, d.blk_expert, plan)
+  MOE_BY_EXPERTS(MOE_SCATTER);
+#undef MOE_SCATTER
+#undef MOE_BY_EXPERTS
   return hipGetLastError();
 }
 

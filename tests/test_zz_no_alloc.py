@@ -21,6 +21,14 @@ def _routing(rng, T, E):
     return ti, pos
 
 
+def _stable(ti, pos, E):
+    """Ids outside [0, E), which the oracle does not take, are left out."""
+    ids = np.where((pos[:, None] >= 0) & (ti >= 0) & (ti < E), ti, E).reshape(-1)
+    order = np.argsort(ids, kind="stable")
+    off = np.searchsorted(ids[order], np.arange(E + 1)).astype(np.int32)
+    return off, order[:off[-1]].astype(np.int32)
+
+
 def _both(m, ti, pos, E):
     T = ti.shape[0]
     dti = abi.DevBuf.from_numpy(ti)
@@ -37,7 +45,7 @@ def _both(m, ti, pos, E):
     got_off, got_perm = off_b.download((E + 1,), np.int32), perm_b.download((T * 4,), np.int32)
     assert np.array_equal(got_off, want_off), "offsets differ from moe_dispatch"
     assert np.array_equal(got_perm, want_perm), "permutation differs from moe_dispatch"
-    o_off, o_perm, _ = ob.dispatch(ti, pos, E)
+    o_off, o_perm = _stable(ti, pos, E) if ((ti < 0) | (ti >= E)).any() else ob.dispatch(ti, pos, E)[:2]
     assert np.array_equal(got_off, o_off) and np.array_equal(got_perm[:o_off[-1]], o_perm)
     assert np.all(got_perm[o_off[-1]:] == -1)
 
@@ -52,6 +60,21 @@ def test_static_dispatch_matches_handle_dispatch(E):
         _both(m, ti, pos, E)
     ti, _ = _routing(rng, 300, E)
     _both(m, ti, None, E)
+
+
+@pytest.mark.parametrize("E", [4, 32, 33, 64, 65, 128, 129, 256])
+def test_dispatch_at_its_edges(E):
+    """Groups of 64 tokens and workgroups of 256 short, full and one over, and either side of the line between
+    one launch and two (2048 tokens); ids outside the experts, the same expert twice in a token."""
+    rng = np.random.default_rng(E)
+    m = abi.Moe(64, 64, E, max_tokens=2113)
+    for T in (1, 63, 64, 65, 255, 256, 257, 1023, 1024, 1025, 1984, 2047, 2048, 2049, 2113):
+        ti, pos = _routing(rng, T, E)
+        ti[rng.random((T, 4)) < 0.05] = -1
+        ti[rng.random((T, 4)) < 0.05] = E
+        ti[rng.random(T) < 0.05, 3] = 1
+        _both(m, ti, pos, E)
+    m.close()
 
 
 def test_static_dispatch_limits():
