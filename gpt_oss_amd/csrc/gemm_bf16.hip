@@ -275,7 +275,14 @@ __device__ __forceinline__ void wave_tile(const Tile &t, uint32_t lds0) {
   constexpr int WAIT_ODD = 2 * LB + LA;
   auto step = [&](auto par_c, int ks) {
     constexpr int par = decltype(par_c)::value;
-    const uint32_t sbn = sb + R::ColSlot == R::RowRing ? 0 : sb + R::ColSlot, sbp = (sb == 0 ? R::RowRing : sb) - R::ColSlot;
+    uint32_t sbn, sbp;  // next and last slot of columns
+    if constexpr ((R::RowRing & (R::RowRing - 1)) == 0) {
+      sbn = (sb + R::ColSlot) & (R::RowRing - 1);
+      sbp = (sb - R::ColSlot) & (R::RowRing - 1);
+    } else {
+      sbn = sb + R::ColSlot == R::RowRing ? 0 : sb + R::ColSlot;
+      sbp = (sb == 0 ? R::RowRing : sb) - R::ColSlot;
+    }
     const uint32_t san = par ? (sa + R::RowStage == R::End ? R::RowRing : sa + R::RowStage) : sa;
     const uint32_t sap = (sa == R::RowRing ? R::End : sa) - R::RowStage;
     constexpr int NM1 = NM ? NM : 1;
