@@ -10,6 +10,7 @@
 namespace moe {
 
 constexpr int kDispThreads = 256;  // tokens per workgroup in count / scatter
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 // Pass 1 of batches beyond kOnceTokens: per-workgroup histogram of expert ids over active rows.  Also resets
 // rowmap and perm to -1 (a fill kernel rather than a memset so that the call
@@ -517,7 +518,14 @@ __global__ __launch_bounds__(kOnceThreads) void dispatch_once_kernel(
 //
 // One workgroup per token; for few tokens gridDim.y workgroups share its columns
 // (a single token: 5.4 -> 2.7 us with that and inv in place of a ballot over the ids).
-template <bool RESID>
+//
+// PAST: y is read past the caches.  Bound by HBM with many tokens: the down GEMM's last rows of a large y are
+// all that the caches hold, and nothing reads a row again.  us of this kernel's stage, through / past: 4096
+// tokens 41.3 / 41.0 (MXFP4, residual stream, 43.3 / 40.7), 7168 80.1 / 71.1, 6144 at 128 experts, where
+// the rows that it leaves in the caches cost the next call as well, 73.1 / 66.5 (1442 / 1412 per call); 1500 (69 MB)
+// 19.8 / 20.4.
+constexpr size_t kCombinePastBytes = (size_t)128 << 20;
+template <bool RESID, bool PAST>
 __global__ __launch_bounds__(256) void combine_kernel(const float *__restrict__ y,
                                                      const int *__restrict__ inv,
                                                      const float *__restrict__ topk_v,
@@ -541,8 +549,9 @@ __global__ __launch_bounds__(256) void combine_kernel(const float *__restrict__ 
 #pragma unroll
     for (int k = 0; k < kTopK; k++) {
       if (p[k] >= 0) {
-        const float4 v = reinterpret_cast<const float4 *>(y + (size_t)p[k] * ldy)[c];
-        s.x += w[k] * v.x; s.y += w[k] * v.y; s.z += w[k] * v.z; s.w += w[k] * v.w;
+        const f32x4 *row = reinterpret_cast<const f32x4 *>(y + (size_t)p[k] * ldy);
+        const f32x4 v = PAST ? __builtin_nontemporal_load(row + c) : row[c];
+        s.x += w[k] * v[0]; s.y += w[k] * v[1]; s.z += w[k] * v[2]; s.w += w[k] * v[3];
       }
     }
     if (RESID) {
@@ -609,7 +618,10 @@ static hipError_t launch_combine_any(const float *y, int ldy, const int *inv, co
                                      void *out, int T, int H, int accumulate, hipStream_t s) {
   // workgroups of one token each fill the GPU from about four per CU on
   const dim3 grid(T, T < 4 * kCus ? (H / 4 + 255) / 256 : 1);
-  combine_kernel<RESID><<<grid, 256, 0, s>>>(y, inv, topk_v, pos, out, H, ldy, accumulate);
+  if ((size_t)T * kTopK * ldy * sizeof(float) > kCombinePastBytes)
+    combine_kernel<RESID, true><<<grid, 256, 0, s>>>(y, inv, topk_v, pos, out, H, ldy, accumulate);
+  else
+    combine_kernel<RESID, false><<<grid, 256, 0, s>>>(y, inv, topk_v, pos, out, H, ldy, accumulate);
   return hipGetLastError();
 }
 

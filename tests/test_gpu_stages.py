@@ -538,3 +538,41 @@ def test_yardstick_of_the_other_product_runs():
     tf, ghz = abi.yardstick_mfma(256, 2000, data=2, small=True)
     tf0, _ = abi.yardstick_mfma(256, 2000, data=0, small=True)
     assert 200 < tf < 2600 and 0.5 < ghz < 3.0 and tf0 > 0.9 * tf
+
+
+def test_combine_past_the_caches():
+    """Either side of the line from which the combine reads the down GEMM's rows past the caches (128 MiB of
+    them: 131072 tokens of 64 columns): a token's sums are the same bits, overwritten, added and in the residual
+    stream, and the oracle's."""
+    H, IM, E, T = 64, 32, 8, 131073
+    sh = synth.LayerShape("combine", T, H, IM, E)
+    x = synth.round_bf16(synth.make_activations(sh))
+    L = {k: (synth.round_bf16(v) if v.dtype == np.float32 else v)
+         for k, v in synth.make_layer(synth.LayerShape("combine", 64, H, IM, E), seed=3).items()}
+    w = [L[k] for k in ("w_router", "b_router", "w_mlp1", "b_mlp1", "w_mlp2", "b_mlp2")]
+    pos = np.zeros(T, np.int32)
+    pos[5::97] = -1
+    m = abi.Moe(H, IM, E, max_tokens=T, swiglu_limit=sh.limit)
+    m.upload_layer(0, *w)
+    m.upload_norm(0, np.ones(H, np.float32))
+    dx, dpos, dout = abi.DevBuf.from_numpy(synth.to_bf16_bits(x)), abi.DevBuf.from_numpy(pos), abi.DevBuf(T * H * 4)
+    got = []
+    for n in (T - 1, T):
+        for accumulate in (False, True):
+            dout.memset(0)
+            m.forward(0, dx, dpos, n, dout, accumulate=accumulate)
+            abi.sync()
+            got.append(dout.download((T, H), np.float32)[:T - 1])
+    for other in got[1:]:
+        assert np.array_equal(got[0], other)
+    streams = []
+    for n in (T - 1, T):
+        ds = abi.DevBuf.from_numpy(synth.to_bf16_bits(x))
+        m.block_forward(0, ds, dpos, n)
+        abi.sync()
+        streams.append(ds.download((T, H), np.uint16)[:T - 1])
+    assert np.array_equal(*streams)
+    m.close()
+    rows = np.arange(0, T - 1, 4001)
+    want = ob.moe_layer(np.ascontiguousarray(x[rows]), pos[rows], *w, 4, sh.limit, mode=ob.ROUND_ACT_BF16 | ob.PAR_TOKENS)
+    assert np.abs(got[0][rows] - want).max() <= 2e-2 and np.linalg.norm(got[0][rows] - want) <= 1e-3 * np.linalg.norm(want)
