@@ -78,18 +78,58 @@ __device__ __forceinline__ void select_top(const float (&v)[PER], int q, int E, 
   }
 }
 
-// run.cpp:336-354 with size = 4; v[0] is the maximum.
-__device__ __forceinline__ float4 softmax4(const float (&v)[kTopK]) {
-  const double mx = (double)v[0];
-  float ev[kTopK];
-  double sum = 0.0;
+// The largest of the wave's values, in every lane.
+__device__ __forceinline__ uint32_t wave_max(uint32_t x) {
+#define MOE_DPP_MAX(CTRL, ROWS) \
+  x = max(x, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, CTRL, ROWS, 0xf, false))
+  MOE_DPP_MAX(0x111, 0xf);  // row_shr 1, 2, 4, 8: lane 15 of a row of 16 has the row's
+  MOE_DPP_MAX(0x112, 0xf);
+  MOE_DPP_MAX(0x114, 0xf);
+  MOE_DPP_MAX(0x118, 0xf);
+  MOE_DPP_MAX(0x142, 0xa);  // row_bcast15 into rows 1 and 3, row_bcast31 into 2 and 3
+  MOE_DPP_MAX(0x143, 0xc);
+#undef MOE_DPP_MAX
+  return (uint32_t)__builtin_amdgcn_readlane((int)x, 63);
+}
+
+// select_top's rule for one token on a whole wave, lane q owning experts q*PER .. q*PER+PER-1 (more than 32
+// experts).  Logits become whole numbers of the same order (zeros of either sign the same one), places past the
+// experts and places taken 0, which is below all of them; a round is a maximum over the wave and the first lane
+// that holds it.  A row with a NaN goes through the comparisons.  Eight lanes per token with 16 experts
+// each took 5.5 us for the 16 tokens of a workgroup and 128 experts.
+template <int PER, int NSEL>
+__device__ __forceinline__ void wave_top(const float (&v)[PER], int lane, int E, float (&sel_v)[NSEL],
+                                         int (&sel_i)[NSEL]) {
+  bool nan = false;
+  uint32_t key[PER];
 #pragma unroll
-  for (int r = 0; r < kTopK; r++) {
-    ev[r] = expf((float)((double)v[r] - mx));
-    sum += (double)ev[r];
+  for (int j = 0; j < PER; j++) {
+    const bool is_expert = lane * PER + j < E;
+    nan |= is_expert && v[j] != v[j];
+    const uint32_t u = __float_as_uint(v[j] + 0.f);
+    key[j] = is_expert ? u ^ ((uint32_t)((int32_t)u >> 31) | 0x80000000u) : 0u;
   }
-  return make_float4((float)((double)ev[0] / sum), (float)((double)ev[1] / sum),
-                     (float)((double)ev[2] / sum), (float)((double)ev[3] / sum));
+  if (__ballot(nan) != 0ull) {
+    select_top<PER, 64, NSEL>(v, lane, E, sel_v, sel_i);
+    return;
+  }
+#pragma unroll
+  for (int r = 0; r < NSEL; r++) {
+    uint32_t own = key[0];
+#pragma unroll
+    for (int j = 1; j < PER; j++) own = max(own, key[j]);
+    const uint32_t best = wave_max(own);
+    const int l = __builtin_ctzll(__ballot(own == best));
+    int at = 0;
+#pragma unroll
+    for (int j = PER - 1; j >= 0; j--)
+      if (key[j] == best) at = j;
+    sel_v[r] = __uint_as_float(best ^ (~(uint32_t)((int32_t)best >> 31) | 0x80000000u));
+    sel_i[r] = l * PER + __builtin_amdgcn_readlane(at, l);
+#pragma unroll
+    for (int j = 0; j < PER; j++)
+      if (lane == l && at == j) key[j] = 0u;
+  }
 }
 
 // Top-NSEL of one token's logits for up to 32 experts, one lane per expert (the
@@ -176,13 +216,15 @@ __global__ __launch_bounds__(WPC * 64) void router_kernel(
     const float *__restrict__ first) {
   constexpr int E_pad = NT * 16;
   constexpr int TOK = MT * 16;
-  // selection: LPT lanes per token, each owning PER experts; SW waves take part.
-  // Up to 32 experts: one lane per expert, places found by counting (ranked_top).
+  // selection: LPT lanes per token, each owning PER experts.
+  // Up to 32 experts: one lane per expert, places found by counting (ranked_top), SW waves take part.
+  // More: the waves take the tokens in turn (wave_top).
   constexpr bool RANKED = E_pad <= 32;
-  constexpr int LPT = RANKED ? 32 : (E_pad <= 64 ? 4 : (E_pad == 128 ? 8 : 16));
+  constexpr int LPT = RANKED ? 32 : 64;
   constexpr int PER = RANKED ? 1 : E_pad / LPT;
   constexpr int SW = TOK * LPT / 64;
-  static_assert(SW >= 1 && SW <= WPC, "waves of the selection");
+  constexpr int TPV = RANKED ? 1 : TOK / WPC;  // tokens of a wave, one after the other
+  static_assert(RANKED ? SW <= WPC : TOK % WPC == 0, "waves of the selection");
   constexpr int LOG_LD = RANKED ? E_pad + 4 : E_pad + 1;  // RANKED reads rows of logits in 16-byte pieces
   // cross-wave sum: GB blocks of 16 x 16 outputs at a time through 32 KB
   constexpr int NBLK = MT * NT;
@@ -206,11 +248,14 @@ __global__ __launch_bounds__(WPC * 64) void router_kernel(
   const int kc_total = H / 32;
   if (tid == 0) n_tasks = 0;
   if (tid < E_pad) sh_br[tid] = br[tid];
-  // the selection's own inputs, loaded long before they are needed
-  const int tr = w * (64 / LPT) + lane / LPT;  // token within the workgroup (waves < SW only)
-  const int q = lane % LPT;
-  const int t = tok0 + tr;
-  const bool active = w < SW && t < T && !(pos && pos[min(t, T - 1)] < 0);
+  const int q = lane % LPT;  // place among the token's lanes
+  auto token_of = [&](int i) { return RANKED ? w * (64 / LPT) + lane / LPT : w + i * WPC; };  // within the workgroup
+  bool active[TPV];  // asked for long before it is needed
+#pragma unroll
+  for (int i = 0; i < TPV; i++) {
+    const int t = tok0 + token_of(i);
+    active[i] = (!RANKED || w < SW) && t < T && !(pos && pos[min(t, T - 1)] < 0);
+  }
   const float wn_max = rstat[0], bmax = rstat[1];
 
   if constexpr (SPLIT) {
@@ -333,58 +378,60 @@ __global__ __launch_bounds__(WPC * 64) void router_kernel(
   }
   }
 
-  // Pass 2, selection: LPT lanes per token.
-  bool undecided = false;
-  if (w < SW) {
-    float v[PER];
-    float s_v[kTopK + 1];
-    int s_i[kTopK + 1];
-    if constexpr (RANKED) {
-      v[0] = q < E_pad ? logits[tr][q] : -__builtin_inff();
-      ranked_top<E_pad, kTopK + 1>(reinterpret_cast<const float4 *>(&logits[tr][0]), v[0], q, E, posted[tr],
-                                   s_v, s_i);
-    } else {
+  // Pass 2, selection.
+  unsigned undecided = 0;  // bit i: the wave's (RANKED: the half wave's) token i
+  if (!RANKED || w < SW) {
+#pragma unroll 1
+    for (int i = 0; i < TPV; i++) {
+      const int tr = token_of(i), t = tok0 + tr;
+      float v[PER];
+      float s_v[kTopK + 1];
+      int s_i[kTopK + 1];
+      if constexpr (RANKED) {
+        v[0] = q < E_pad ? logits[tr][q] : -__builtin_inff();
+        ranked_top<E_pad, kTopK + 1>(reinterpret_cast<const float4 *>(&logits[tr][0]), v[0], q, E, posted[tr],
+                                     s_v, s_i);
+      } else {
 #pragma unroll
-      for (int j = 0; j < PER; j++) v[j] = logits[tr][q * PER + j];
-      select_top<PER, LPT, kTopK + 1>(v, q, E, s_v, s_i);
-    }
-    if (active) {
-      float ss = 0.f;
+        for (int j = 0; j < PER; j++) v[j] = logits[tr][q * PER + j];
+        wave_top<PER, kTopK + 1>(v, q, E, s_v, s_i);
+      }
+      bool is_active = active[0];
 #pragma unroll
-      for (int ww = 0; ww < SQ; ww++) ss += sumsq[ww][tr];
-      // bound on |first-pass logit - exact logit|: the accumulation error plus
-      // the two float roundings (sum -> float, + bias) of either arithmetic
-      const float err0 = router_gamma(FLUSH) * sqrtf(ss * 1.002f) * wn_max;
-      auto up = [&](float a) { return a + (4.76837158e-7f * (fabsf(a) + bmax) + err0); };
-      auto lo = [&](float a) { return a - (4.76837158e-7f * (fabsf(a) + bmax) + err0); };
-      const bool decided = lo(s_v[0]) > up(s_v[1]) && lo(s_v[1]) > up(s_v[2]) && lo(s_v[2]) > up(s_v[3]) &&
-                           (s_i[4] == kNone || lo(s_v[3]) > up(s_v[4]));
-      if (decided) {
-        if constexpr (RANKED) {
+      for (int k = 1; k < TPV; k++)
+        if (k == i) is_active = active[k];
+      if (is_active) {
+        float ss = 0.f;
+#pragma unroll
+        for (int ww = 0; ww < SQ; ww++) ss += sumsq[ww][tr];
+        // bound on |first-pass logit - exact logit|: the accumulation error plus
+        // the two float roundings (sum -> float, + bias) of either arithmetic
+        const float err0 = router_gamma(FLUSH) * sqrtf(ss * 1.002f) * wn_max;
+        auto up = [&](float a) { return a + (4.76837158e-7f * (fabsf(a) + bmax) + err0); };
+        auto lo = [&](float a) { return a - (4.76837158e-7f * (fabsf(a) + bmax) + err0); };
+        const bool decided = lo(s_v[0]) > up(s_v[1]) && lo(s_v[1]) > up(s_v[2]) && lo(s_v[2]) > up(s_v[3]) &&
+                             (s_i[4] == kNone || lo(s_v[3]) > up(s_v[4]));
+        if (decided) {
           // (tokens of one wave can differ in `decided`: the shuffles inside are
           // among the lanes of one token, which agree)
           const float sv[kTopK] = {s_v[0], s_v[1], s_v[2], s_v[3]};
           const int si[kTopK] = {s_i[0], s_i[1], s_i[2], s_i[3]};
           store_topk_spread(sv, si, q, lane - q, topk_i + (size_t)t * kTopK, topk_v + (size_t)t * kTopK);
-        } else if (q == 0) {
-          const float sv[kTopK] = {s_v[0], s_v[1], s_v[2], s_v[3]};
-          *reinterpret_cast<int4 *>(topk_i + (size_t)t * kTopK) = make_int4(s_i[0], s_i[1], s_i[2], s_i[3]);
-          *reinterpret_cast<float4 *>(topk_v + (size_t)t * kTopK) = softmax4(sv);
-        }
-      } else {
-        undecided = true;
-        // contenders: everything not provably below the fourth best (a NaN
-        // anywhere makes the comparison fail, and the expert a contender)
-        const float floor4 = lo(s_v[3]);
+        } else {
+          undecided |= 1u << i;
+          // contenders: everything not provably below the fourth best (a NaN
+          // anywhere makes the comparison fail, and the expert a contender)
+          const float floor4 = lo(s_v[3]);
 #pragma unroll
-        for (int j = 0; j < PER; j++) {
-          const int e = q * PER + j;
-          if (e < E && !(up(v[j]) < floor4)) tasks[atomicAdd(&n_tasks, 1)] = (unsigned short)(tr * E_pad + e);
+          for (int j = 0; j < PER; j++) {
+            const int e = q * PER + j;
+            if (e < E && !(up(v[j]) < floor4)) tasks[atomicAdd(&n_tasks, 1)] = (unsigned short)(tr * E_pad + e);
+          }
         }
+      } else if (t < T && q == 0) {
+        *reinterpret_cast<int4 *>(topk_i + (size_t)t * kTopK) = make_int4(-1, -1, -1, -1);
+        *reinterpret_cast<float4 *>(topk_v + (size_t)t * kTopK) = make_float4(0.f, 0.f, 0.f, 0.f);
       }
-    } else if (t < T && q == 0) {
-      *reinterpret_cast<int4 *>(topk_i + (size_t)t * kTopK) = make_int4(-1, -1, -1, -1);
-      *reinterpret_cast<float4 *>(topk_v + (size_t)t * kTopK) = make_float4(0.f, 0.f, 0.f, 0.f);
     }
   }
   __syncthreads();
@@ -449,23 +496,25 @@ __global__ __launch_bounds__(WPC * 64) void router_kernel(
   __syncthreads();
 
   if constexpr (RANKED) {
-    if (w < SW && __ballot(undecided) != 0ull) {  // per wave: ranked_top is a wave's work
+    if (w < SW && __ballot(undecided != 0u) != 0ull) {  // per wave: ranked_top is a wave's work
+      const int tr = token_of(0), t = tok0 + tr;
       const float v = q < E_pad ? logits[tr][q] : -__builtin_inff();
       float s_v[kTopK];
       int s_i[kTopK];
       ranked_top<E_pad, kTopK>(reinterpret_cast<const float4 *>(&logits[tr][0]), v, q, E, posted[tr], s_v, s_i);
       if (undecided) store_topk_spread(s_v, s_i, q, lane - q, topk_i + (size_t)t * kTopK, topk_v + (size_t)t * kTopK);
     }
-  } else if (undecided) {  // waves < SW only
-    float v[PER];
+  } else {
+    while (undecided) {  // the same in all lanes
+      const int tr = token_of(__builtin_ctz(undecided)), t = tok0 + tr;
+      undecided &= undecided - 1u;
+      float v[PER];
 #pragma unroll
-    for (int j = 0; j < PER; j++) v[j] = logits[tr][q * PER + j];
-    float s_v[kTopK];
-    int s_i[kTopK];
-    select_top<PER, LPT, kTopK>(v, q, E, s_v, s_i);
-    if (q == 0) {
-      *reinterpret_cast<int4 *>(topk_i + (size_t)t * kTopK) = make_int4(s_i[0], s_i[1], s_i[2], s_i[3]);
-      *reinterpret_cast<float4 *>(topk_v + (size_t)t * kTopK) = softmax4(s_v);
+      for (int j = 0; j < PER; j++) v[j] = logits[tr][q * PER + j];
+      float s_v[kTopK];
+      int s_i[kTopK];
+      wave_top<PER, kTopK>(v, q, E, s_v, s_i);
+      store_topk_spread(s_v, s_i, q, 0, topk_i + (size_t)t * kTopK, topk_v + (size_t)t * kTopK);
     }
   }
   if (score) {
@@ -482,8 +531,9 @@ __global__ __launch_bounds__(WPC * 64) void router_kernel(
 // matrix (0.74 MB at 128 experts and 2880 columns, 12 us and more), and a small batch has few
 // of them.  The same chunks to the same four waves and the same order of the sums: the same
 // bits.  Written to `first` (see SPLIT), which a second launch reads.  us at 128 experts and
-// 2880 columns, one kernel / both launches: 6 tokens 16.7 / 5.0 + 6.3, 200 tokens 32.5 / 7.7 + 17.2 (the
-// rest is the second pass of a few undecided tokens).
+// 2880 columns, one kernel / both launches, with the selection by eight lanes per token: 6 tokens 16.7 / 5.0
+// + 6.3, 200 tokens 32.5 / 7.7 + 17.2; with wave_top the second launch takes 4.1 and 12.9 (of which the
+// second pass of a few undecided tokens).
 template <int D>
 __global__ __launch_bounds__(kSplitWaves * 64) void router_logits_kernel(
     const uint16_t *__restrict__ x, const uint16_t *__restrict__ wr, const float *__restrict__ br, int T, int H,

@@ -273,6 +273,39 @@ def test_router_near_ties(E, T):
         assert list(r).index(1) < list(r).index(5)  # exact tie: the lower id first
 
 
+@pytest.mark.parametrize("E", [33, 63, 64, 65, 127, 128, 129, 200, 256])
+def test_router_selection_of_many_experts(E):
+    """Ranks over a whole wave, and its fall back to comparisons: plateaus of equal logits at the first and the
+    last experts, zeros of either sign, experts at minus infinity, one NaN among the logits, rows of NaN; in
+    moe_router's one launch and in the two of a whole layer (768 columns, from 65 experts on)."""
+    H, T = 768, 40
+    sh = synth.LayerShape("many", T, H, 64, E)
+    L = bf16_layer(sh, seed=E)
+    wr, br, x = L["w_router"].copy(), np.zeros(E, np.float32), L["x"].copy()
+    x[3] = 0.0               # its logits are the biases
+    x[::9] = 0.0
+    wr[[0, 1, E - 2, E - 1]] = wr[7]
+    wr[E // 2] = 0.0
+    br[::3] = -0.0           # equal to 0, whatever the sign
+    br[[4, E - 3]] = -np.inf
+    x[20] = np.nan
+    for bias in (br, np.full(E, -np.inf, np.float32), np.arange(E, dtype=np.float32) // 5):
+        L["w_router"], L["b_router"], L["x"] = wr, synth.round_bf16(bias), x
+        m = make_moe(sh, L, T)
+        R = abi.run_layer(m, 0, x, None)
+        _, ti, tv = ob.router(x, None, wr, L["b_router"], 4)
+        assert np.array_equal(R["topk_i"], ti)
+        np.testing.assert_allclose(R["topk_v"], tv, rtol=0, atol=2e-6)
+        want = ob.moe_layer(x, None, wr, L["b_router"], L["w_mlp1"], L["b_mlp1"], L["w_mlp2"], L["b_mlp2"], 4, sh.limit,
+                            mode=ob.ROUND_ACT_BF16 | ob.PAR_TOKENS)
+        assert np.array_equal(np.isnan(R["out"]), np.isnan(want))
+        fine = ~np.isnan(want).any(1)
+        if fine.any():
+            assert np.abs(R["out"][fine] - want[fine]).max() <= 2e-2
+            assert np.linalg.norm(R["out"][fine] - want[fine]) <= 1e-3 * np.linalg.norm(want[fine])
+        m.close()
+
+
 def test_router_first_pass_error_bound():
     """The first pass decides a token only when its logits are further apart
     than twice kGamma * |x| * max|w_e|; the scores it reports for experts it did
