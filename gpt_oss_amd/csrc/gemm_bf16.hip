@@ -200,11 +200,18 @@ __device__ __forceinline__ void wave_tile(const Tile &t, uint32_t lds0) {
   const uint32_t dst_x = lds0 + 8 * kColBlockBytes + w * 1024;
 
   auto issue_a = [&](uint32_t stage, int m) { dma_lanes(dst_a + stage + m * 2 * kRowBlockBytes, a_src[m]); };
-  auto issue_b = [&](uint32_t slot, int ks, int n) {
+  auto issue_b = [&](uint32_t slot, int ks, int n, uint32_t off) {
     const size_t at = (size_t)ks * kColBlockBytes;
-    if (n == 0) dma_wave<0, STREAM>(dst_b + slot, b_src + at, lane16);
-    else if (n == 1) dma_wave<kFragBytes, STREAM>(dst_b + slot, b_src + at, lane16);
-    else dma_wave<0, STREAM>(dst_x + slot, x_src + at, lane16);
+    if (n == 0) dma_wave<0, STREAM>(dst_b + slot, b_src + at, off);
+    else if (n == 1) dma_wave<kFragBytes, STREAM>(dst_b + slot, b_src + at, off);
+    else dma_wave<0, STREAM>(dst_x + slot, x_src + at, off);
+  };
+  // Lanes' offsets of a load of step ks.  Past the tile's end, where nothing reads what is loaded: the same 16 bytes
+  // in every lane with weights past the caches, whose loads would come from HBM once more (672 of 896 tokens 313.3
+  // / 312.1 us per call, on another box 318.8 / 314.3, 1400 364.1 / 362.3, 6144 at 128 experts 1440 / 1434).
+  auto lanes_of = [&](int ks) -> uint32_t {
+    if constexpr (STREAM) return ks > last ? 0u : lane16;
+    return lane16;
   };
   auto adv_a = [&](int jd_next) {
     const int d = jd_next <= last_d ? A_STEP : 0;
@@ -238,14 +245,14 @@ __device__ __forceinline__ void wave_tile(const Tile &t, uint32_t lds0) {
   };
   auto fill_b = [&](int ks) {
 #pragma unroll
-    for (int n = 0; n < LB; n++) issue_b(ks * R::ColSlot, min(ks, last), n);
+    for (int n = 0; n < LB; n++) issue_b(ks * R::ColSlot, min(ks, last), n, lane16);
   };
   fill_a(0);
   fill_b(0);
   fill_b(1);
   fill_a(1);
   fill_b(2);
-  issue_b(3 * R::ColSlot, min(3, last), 0);
+  issue_b(3 * R::ColSlot, min(3, last), 0, lane16);
   if (LA > 0) issue_a(R::RowRing + 2 * R::RowStage, 0);
   WAIT_VMCNT(LA + (LA > 0) + 2 * LB + 1);  // A(0), B(0)
   lds_barrier();
@@ -269,8 +276,8 @@ __device__ __forceinline__ void wave_tile(const Tile &t, uint32_t lds0) {
   // halves that follow.  At the barrier of step ks B(ks + 1) has to have landed, and at an odd one
   // A(jd + 1).  Behind B(ks + 1) an even step has issued twice B, m = 1, 2, 3 of A(jd + 1) and m =
   // 0, 1 of A(jd + 2); behind A(jd + 1) an odd one twice B and A(jd + 2).  Every step
-  // is the same code with the same counts: past the tile's end the refills load its last step again,
-  // hits that nobody reads.  The wave ends with those in flight; s_endpgm waits for them.
+  // is the same code with the same counts: past the tile's end the refills load its last step again
+  // (lanes_of), which nobody reads.  The wave ends with those in flight; s_endpgm waits for them.
   constexpr int WAIT_EVEN = 2 * LB + (LA > 1) + (LA > 2) + (LA > 3) + (LA > 0) + (LA > 1);
   constexpr int WAIT_ODD = 2 * LB + LA;
   auto step = [&](auto par_c, int ks) {
@@ -296,7 +303,7 @@ __device__ __forceinline__ void wave_tile(const Tile &t, uint32_t lds0) {
           if (s < RD) {
             read_a(sa, par, 1, s);
           } else if (s < RD + LB - 1) {
-            issue_b(sbp, ks_b, 1 + s - RD);
+            issue_b(sbp, ks_b, 1 + s - RD, lanes_of(ks + 3));
           } else if (s < SD) {
             issue_a(sap, AM);
           }
@@ -320,7 +327,7 @@ __device__ __forceinline__ void wave_tile(const Tile &t, uint32_t lds0) {
             if (s < NC) read_b(sbn, par ^ 1, s);
             else read_a(san, par ^ 1, 0, s - NC);
           } else if (s == RD) {
-            issue_b(sb, ks_b, 0);
+            issue_b(sb, ks_b, 0, lanes_of(ks + 4));
           } else if (s < SD) {
             if constexpr (par) issue_a(sa, AM); else issue_a(sap, AM);
           }
