@@ -39,9 +39,7 @@ __global__ __launch_bounds__(kDispThreads) void dispatch_count_kernel(
     perm[i] = -1;
 }
 
-// The plan of one batch from the experts' row counts (thread e holds expert e's
-// count; all 256 threads of the workgroup call this together).  Returns the
-// expert's first row in the padded row space.
+// Where the plan of a batch goes, and what it is of.
 struct PlanOut {
   int *offsets;
   ExpertInfo *info;
@@ -106,7 +104,9 @@ __device__ __forceinline__ void write_expert_tiles(int ee, int nmt, int rbe, int
   }
 }
 
-// Threads from 256 on, if there are any, only take part in the barriers.
+// The plan of one batch from the experts' row counts (thread e < 256 holds expert e's count; all threads of the
+// workgroup call this together, those from 256 on only take part in the barriers).  Returns the
+// expert's first row in the padded row space.
 // write_global: this workgroup stores the plan (offsets, per-expert records,
 // totals, XCD bounds); the others only need the values returned to them.
 __device__ __forceinline__ int build_plan(int count, int E, const PlanOut &out, bool write_global, int *ex_count_out,

@@ -249,12 +249,13 @@ __global__ __launch_bounds__(WPC * 64) void router_kernel(
   if (tid == 0) n_tasks = 0;
   if (tid < E_pad) sh_br[tid] = br[tid];
   const int q = lane % LPT;  // place among the token's lanes
-  auto token_of = [&](int i) { return RANKED ? w * (64 / LPT) + lane / LPT : w + i * WPC; };  // within the workgroup
+  const int tr = RANKED ? w * (64 / LPT) + lane / LPT : w;  // (first) token within the workgroup
+  const int t = tok0 + tr;
   bool active[TPV];  // asked for long before it is needed
 #pragma unroll
   for (int i = 0; i < TPV; i++) {
-    const int t = tok0 + token_of(i);
-    active[i] = (!RANKED || w < SW) && t < T && !(pos && pos[min(t, T - 1)] < 0);
+    const int ti = t + i * WPC;
+    active[i] = (!RANKED || w < SW) && ti < T && !(pos && pos[min(ti, T - 1)] < 0);
   }
   const float wn_max = rstat[0], bmax = rstat[1];
 
@@ -378,60 +379,66 @@ __global__ __launch_bounds__(WPC * 64) void router_kernel(
   }
   }
 
-  // Pass 2, selection.
-  unsigned undecided = 0;  // bit i: the wave's (RANKED: the half wave's) token i
-  if (!RANKED || w < SW) {
+  // Pass 2, selection: whether token tr of the workgroup, t of the batch, is left undecided.
+  auto select = [&](int tr, int t, bool is_active) {
+    float v[PER];
+    float s_v[kTopK + 1];
+    int s_i[kTopK + 1];
+    if constexpr (RANKED) {
+      v[0] = q < E_pad ? logits[tr][q] : -__builtin_inff();
+      ranked_top<E_pad, kTopK + 1>(reinterpret_cast<const float4 *>(&logits[tr][0]), v[0], q, E, posted[tr],
+                                   s_v, s_i);
+    } else {
+#pragma unroll
+      for (int j = 0; j < PER; j++) v[j] = logits[tr][q * PER + j];
+      wave_top<PER, kTopK + 1>(v, q, E, s_v, s_i);
+    }
+    if (is_active) {
+      float ss = 0.f;
+#pragma unroll
+      for (int ww = 0; ww < SQ; ww++) ss += sumsq[ww][tr];
+      // bound on |first-pass logit - exact logit|: the accumulation error plus
+      // the two float roundings (sum -> float, + bias) of either arithmetic
+      const float err0 = router_gamma(FLUSH) * sqrtf(ss * 1.002f) * wn_max;
+      auto up = [&](float a) { return a + (4.76837158e-7f * (fabsf(a) + bmax) + err0); };
+      auto lo = [&](float a) { return a - (4.76837158e-7f * (fabsf(a) + bmax) + err0); };
+      const bool decided = lo(s_v[0]) > up(s_v[1]) && lo(s_v[1]) > up(s_v[2]) && lo(s_v[2]) > up(s_v[3]) &&
+                           (s_i[4] == kNone || lo(s_v[3]) > up(s_v[4]));
+      if (decided) {
+        // (tokens of one wave can differ in `decided`: the shuffles inside are
+        // among the lanes of one token, which agree)
+        const float sv[kTopK] = {s_v[0], s_v[1], s_v[2], s_v[3]};
+        const int si[kTopK] = {s_i[0], s_i[1], s_i[2], s_i[3]};
+        store_topk_spread(sv, si, q, lane - q, topk_i + (size_t)t * kTopK, topk_v + (size_t)t * kTopK);
+      } else {
+        // contenders: everything not provably below the fourth best (a NaN
+        // anywhere makes the comparison fail, and the expert a contender)
+        const float floor4 = lo(s_v[3]);
+#pragma unroll
+        for (int j = 0; j < PER; j++) {
+          const int e = q * PER + j;
+          if (e < E && !(up(v[j]) < floor4)) tasks[atomicAdd(&n_tasks, 1)] = (unsigned short)(tr * E_pad + e);
+        }
+        return true;
+      }
+    } else if (t < T && q == 0) {
+      *reinterpret_cast<int4 *>(topk_i + (size_t)t * kTopK) = make_int4(-1, -1, -1, -1);
+      *reinterpret_cast<float4 *>(topk_v + (size_t)t * kTopK) = make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+    return false;
+  };
+  bool undecided = false;    // RANKED: the half wave's token
+  unsigned undecided_of = 0;  // otherwise bit i: the wave's token i
+  if constexpr (RANKED) {
+    if (w < SW) undecided = select(tr, t, active[0]);
+  } else {
 #pragma unroll 1
     for (int i = 0; i < TPV; i++) {
-      const int tr = token_of(i), t = tok0 + tr;
-      float v[PER];
-      float s_v[kTopK + 1];
-      int s_i[kTopK + 1];
-      if constexpr (RANKED) {
-        v[0] = q < E_pad ? logits[tr][q] : -__builtin_inff();
-        ranked_top<E_pad, kTopK + 1>(reinterpret_cast<const float4 *>(&logits[tr][0]), v[0], q, E, posted[tr],
-                                     s_v, s_i);
-      } else {
-#pragma unroll
-        for (int j = 0; j < PER; j++) v[j] = logits[tr][q * PER + j];
-        wave_top<PER, kTopK + 1>(v, q, E, s_v, s_i);
-      }
       bool is_active = active[0];
 #pragma unroll
       for (int k = 1; k < TPV; k++)
         if (k == i) is_active = active[k];
-      if (is_active) {
-        float ss = 0.f;
-#pragma unroll
-        for (int ww = 0; ww < SQ; ww++) ss += sumsq[ww][tr];
-        // bound on |first-pass logit - exact logit|: the accumulation error plus
-        // the two float roundings (sum -> float, + bias) of either arithmetic
-        const float err0 = router_gamma(FLUSH) * sqrtf(ss * 1.002f) * wn_max;
-        auto up = [&](float a) { return a + (4.76837158e-7f * (fabsf(a) + bmax) + err0); };
-        auto lo = [&](float a) { return a - (4.76837158e-7f * (fabsf(a) + bmax) + err0); };
-        const bool decided = lo(s_v[0]) > up(s_v[1]) && lo(s_v[1]) > up(s_v[2]) && lo(s_v[2]) > up(s_v[3]) &&
-                             (s_i[4] == kNone || lo(s_v[3]) > up(s_v[4]));
-        if (decided) {
-          // (tokens of one wave can differ in `decided`: the shuffles inside are
-          // among the lanes of one token, which agree)
-          const float sv[kTopK] = {s_v[0], s_v[1], s_v[2], s_v[3]};
-          const int si[kTopK] = {s_i[0], s_i[1], s_i[2], s_i[3]};
-          store_topk_spread(sv, si, q, lane - q, topk_i + (size_t)t * kTopK, topk_v + (size_t)t * kTopK);
-        } else {
-          undecided |= 1u << i;
-          // contenders: everything not provably below the fourth best (a NaN
-          // anywhere makes the comparison fail, and the expert a contender)
-          const float floor4 = lo(s_v[3]);
-#pragma unroll
-          for (int j = 0; j < PER; j++) {
-            const int e = q * PER + j;
-            if (e < E && !(up(v[j]) < floor4)) tasks[atomicAdd(&n_tasks, 1)] = (unsigned short)(tr * E_pad + e);
-          }
-        }
-      } else if (t < T && q == 0) {
-        *reinterpret_cast<int4 *>(topk_i + (size_t)t * kTopK) = make_int4(-1, -1, -1, -1);
-        *reinterpret_cast<float4 *>(topk_v + (size_t)t * kTopK) = make_float4(0.f, 0.f, 0.f, 0.f);
-      }
+      if (select(tr + i * WPC, t + i * WPC, is_active)) undecided_of |= 1u << i;
     }
   }
   __syncthreads();
@@ -496,8 +503,7 @@ __global__ __launch_bounds__(WPC * 64) void router_kernel(
   __syncthreads();
 
   if constexpr (RANKED) {
-    if (w < SW && __ballot(undecided != 0u) != 0ull) {  // per wave: ranked_top is a wave's work
-      const int tr = token_of(0), t = tok0 + tr;
+    if (w < SW && __ballot(undecided) != 0ull) {  // per wave: ranked_top is a wave's work
       const float v = q < E_pad ? logits[tr][q] : -__builtin_inff();
       float s_v[kTopK];
       int s_i[kTopK];
@@ -505,16 +511,15 @@ __global__ __launch_bounds__(WPC * 64) void router_kernel(
       if (undecided) store_topk_spread(s_v, s_i, q, lane - q, topk_i + (size_t)t * kTopK, topk_v + (size_t)t * kTopK);
     }
   } else {
-    while (undecided) {  // the same in all lanes
-      const int tr = token_of(__builtin_ctz(undecided)), t = tok0 + tr;
-      undecided &= undecided - 1u;
+    for (; undecided_of; undecided_of &= undecided_of - 1u) {  // the same in all lanes
+      const int d = __builtin_ctz(undecided_of) * WPC;
       float v[PER];
 #pragma unroll
-      for (int j = 0; j < PER; j++) v[j] = logits[tr][q * PER + j];
+      for (int j = 0; j < PER; j++) v[j] = logits[tr + d][q * PER + j];
       float s_v[kTopK];
       int s_i[kTopK];
       wave_top<PER, kTopK>(v, q, E, s_v, s_i);
-      store_topk_spread(s_v, s_i, q, 0, topk_i + (size_t)t * kTopK, topk_v + (size_t)t * kTopK);
+      store_topk_spread(s_v, s_i, q, 0, topk_i + (size_t)(t + d) * kTopK, topk_v + (size_t)(t + d) * kTopK);
     }
   }
   if (score) {

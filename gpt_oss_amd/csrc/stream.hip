@@ -19,9 +19,9 @@
 // step's four: that is the order in which one v_permlane16_swap turns a pair of
 // 32-row weight fragments (pack.hip) into two 16-row ones.
 //
-// Bound by HBM with bf16 weights; with MXFP4 weights the conversions, the rows'
-// loads through L1 and the few microseconds in which a launch fills and drains
-// show as well.  Measured at 2880 x 2880 and 32 experts, against the kernels this
+// Bound by HBM with bf16 weights; with MXFP4 weights the rows' loads through L1 (64 tokens, 32 experts: 92 us
+// per call, 87 without them), the scales' (88) and the few microseconds in which a launch fills and drains
+// show as well; the conversions do not (91.6).  Measured at 2880 x 2880 and 32 experts, against the kernels this
 // replaced (us, gate_up + down): 24 tokens bf16, 30 experts named, 147 + 79 (6.8 and
 // 6.3 TB/s of weights; were 194 + 102), 64 tokens MXFP4 52 + 28 (were 59 + 39), 1
 // token MXFP4 10 + 6 (were 23 + 14).  What that rests on, by leaving it out, measured on a
