@@ -193,6 +193,22 @@ __device__ __forceinline__ void store_topk_spread(const float (&v)[kTopK], const
   }
 }
 
+// Bound on |first-pass logit - exact logit| of one token: the accumulation error plus the two float roundings
+// (sum -> float, + bias) of either arithmetic.
+struct LogitBound {
+  float err0, bmax;
+  __device__ __forceinline__ float up(float a) const { return a + (4.76837158e-7f * (fabsf(a) + bmax) + err0); }
+  __device__ __forceinline__ float lo(float a) const { return a - (4.76837158e-7f * (fabsf(a) + bmax) + err0); }
+  // whether the exact logits have the same best four in the same order
+  __device__ __forceinline__ bool decides(const float (&s_v)[kTopK + 1], const int (&s_i)[kTopK + 1]) const {
+    return lo(s_v[0]) > up(s_v[1]) && lo(s_v[1]) > up(s_v[2]) && lo(s_v[2]) > up(s_v[3]) &&
+           (s_i[4] == kNone || lo(s_v[3]) > up(s_v[4]));
+  }
+  // everything not provably below the fourth best (a NaN anywhere makes the
+  // comparison fail, and the expert a contender)
+  __device__ __forceinline__ bool contends(float a, float fourth) const { return !(up(a) < lo(fourth)); }
+};
+
 __device__ __forceinline__ void unpack8(const uint4 v, float (&f)[8]) {
   f[0] = __uint_as_float(v.x << 16); f[1] = __uint_as_float(v.x & 0xffff0000u);
   f[2] = __uint_as_float(v.y << 16); f[3] = __uint_as_float(v.y & 0xffff0000u);
@@ -379,66 +395,74 @@ __global__ __launch_bounds__(WPC * 64) void router_kernel(
   }
   }
 
-  // Pass 2, selection: whether token tr of the workgroup, t of the batch, is left undecided.
-  auto select = [&](int tr, int t, bool is_active) {
-    float v[PER];
-    float s_v[kTopK + 1];
-    int s_i[kTopK + 1];
-    if constexpr (RANKED) {
-      v[0] = q < E_pad ? logits[tr][q] : -__builtin_inff();
-      ranked_top<E_pad, kTopK + 1>(reinterpret_cast<const float4 *>(&logits[tr][0]), v[0], q, E, posted[tr],
-                                   s_v, s_i);
-    } else {
-#pragma unroll
-      for (int j = 0; j < PER; j++) v[j] = logits[tr][q * PER + j];
-      wave_top<PER, kTopK + 1>(v, q, E, s_v, s_i);
-    }
-    if (is_active) {
-      float ss = 0.f;
-#pragma unroll
-      for (int ww = 0; ww < SQ; ww++) ss += sumsq[ww][tr];
-      // bound on |first-pass logit - exact logit|: the accumulation error plus
-      // the two float roundings (sum -> float, + bias) of either arithmetic
-      const float err0 = router_gamma(FLUSH) * sqrtf(ss * 1.002f) * wn_max;
-      auto up = [&](float a) { return a + (4.76837158e-7f * (fabsf(a) + bmax) + err0); };
-      auto lo = [&](float a) { return a - (4.76837158e-7f * (fabsf(a) + bmax) + err0); };
-      const bool decided = lo(s_v[0]) > up(s_v[1]) && lo(s_v[1]) > up(s_v[2]) && lo(s_v[2]) > up(s_v[3]) &&
-                           (s_i[4] == kNone || lo(s_v[3]) > up(s_v[4]));
-      if (decided) {
-        // (tokens of one wave can differ in `decided`: the shuffles inside are
-        // among the lanes of one token, which agree)
-        const float sv[kTopK] = {s_v[0], s_v[1], s_v[2], s_v[3]};
-        const int si[kTopK] = {s_i[0], s_i[1], s_i[2], s_i[3]};
-        store_topk_spread(sv, si, q, lane - q, topk_i + (size_t)t * kTopK, topk_v + (size_t)t * kTopK);
-      } else {
-        // contenders: everything not provably below the fourth best (a NaN
-        // anywhere makes the comparison fail, and the expert a contender)
-        const float floor4 = lo(s_v[3]);
-#pragma unroll
-        for (int j = 0; j < PER; j++) {
-          const int e = q * PER + j;
-          if (e < E && !(up(v[j]) < floor4)) tasks[atomicAdd(&n_tasks, 1)] = (unsigned short)(tr * E_pad + e);
-        }
-        return true;
-      }
-    } else if (t < T && q == 0) {
-      *reinterpret_cast<int4 *>(topk_i + (size_t)t * kTopK) = make_int4(-1, -1, -1, -1);
-      *reinterpret_cast<float4 *>(topk_v + (size_t)t * kTopK) = make_float4(0.f, 0.f, 0.f, 0.f);
-    }
-    return false;
-  };
+  // Pass 2, selection.
   bool undecided = false;    // RANKED: the half wave's token
   unsigned undecided_of = 0;  // otherwise bit i: the wave's token i
+  auto bound = [&](int tr) {
+    float ss = 0.f;
+#pragma unroll
+    for (int ww = 0; ww < SQ; ww++) ss += sumsq[ww][tr];
+    return LogitBound{router_gamma(FLUSH) * sqrtf(ss * 1.002f) * wn_max, bmax};
+  };
+  auto store_inactive = [&](int t) {
+    *reinterpret_cast<int4 *>(topk_i + (size_t)t * kTopK) = make_int4(-1, -1, -1, -1);
+    *reinterpret_cast<float4 *>(topk_v + (size_t)t * kTopK) = make_float4(0.f, 0.f, 0.f, 0.f);
+  };
+  // Written out for either form: as one function of a token, or one loop over a wave's, it cost batches of up to 64 tokens
+  // 0.1 to 0.2 us where RANKED (one token, MXFP4, 24.62 / 24.75 us per call).
   if constexpr (RANKED) {
-    if (w < SW) undecided = select(tr, t, active[0]);
+    if (w < SW) {
+      const float v = q < E_pad ? logits[tr][q] : -__builtin_inff();
+      float s_v[kTopK + 1];
+      int s_i[kTopK + 1];
+      ranked_top<E_pad, kTopK + 1>(reinterpret_cast<const float4 *>(&logits[tr][0]), v, q, E, posted[tr], s_v, s_i);
+      if (active[0]) {
+        const LogitBound lb = bound(tr);
+        if (lb.decides(s_v, s_i)) {
+          // (tokens of one wave can differ here: the shuffles inside are among the
+          // lanes of one token, which agree)
+          const float sv[kTopK] = {s_v[0], s_v[1], s_v[2], s_v[3]};
+          const int si[kTopK] = {s_i[0], s_i[1], s_i[2], s_i[3]};
+          store_topk_spread(sv, si, q, lane - q, topk_i + (size_t)t * kTopK, topk_v + (size_t)t * kTopK);
+        } else {
+          undecided = true;
+          if (q < E && lb.contends(v, s_v[3])) tasks[atomicAdd(&n_tasks, 1)] = (unsigned short)(tr * E_pad + q);
+        }
+      } else if (t < T && q == 0) {
+        store_inactive(t);
+      }
+    }
   } else {
 #pragma unroll 1
     for (int i = 0; i < TPV; i++) {
+      const int tri = tr + i * WPC, ti = t + i * WPC;
       bool is_active = active[0];
 #pragma unroll
       for (int k = 1; k < TPV; k++)
         if (k == i) is_active = active[k];
-      if (select(tr + i * WPC, t + i * WPC, is_active)) undecided_of |= 1u << i;
+      float v[PER];
+#pragma unroll
+      for (int j = 0; j < PER; j++) v[j] = logits[tri][q * PER + j];
+      float s_v[kTopK + 1];
+      int s_i[kTopK + 1];
+      wave_top<PER, kTopK + 1>(v, q, E, s_v, s_i);
+      if (is_active) {
+        const LogitBound lb = bound(tri);
+        if (lb.decides(s_v, s_i)) {
+          const float sv[kTopK] = {s_v[0], s_v[1], s_v[2], s_v[3]};
+          const int si[kTopK] = {s_i[0], s_i[1], s_i[2], s_i[3]};
+          store_topk_spread(sv, si, q, lane - q, topk_i + (size_t)ti * kTopK, topk_v + (size_t)ti * kTopK);
+        } else {
+          undecided_of |= 1u << i;
+#pragma unroll
+          for (int j = 0; j < PER; j++) {
+            const int e = q * PER + j;
+            if (e < E && lb.contends(v[j], s_v[3])) tasks[atomicAdd(&n_tasks, 1)] = (unsigned short)(tri * E_pad + e);
+          }
+        }
+      } else if (ti < T && q == 0) {
+        store_inactive(ti);
+      }
     }
   }
   __syncthreads();
