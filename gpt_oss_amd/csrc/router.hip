@@ -43,43 +43,27 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 __host__ __device__ constexpr float router_gamma(int flush) { return 2.0f * 33.0f * flush * 1.1920929e-7f; }
 constexpr int kNone = 0x7fffffff;
 
-// Top-NSEL of a token's logits held by LPT neighbouring lanes (lane q of them
-// owns experts q*PER .. q*PER+PER-1), by the rule of the reference's CPU top-k under a stable
-// sort: value descending, index ascending; a candidate replaces the incumbent
-// (the one with the lower index) only if it compares strictly greater, so a
-// NaN neither wins nor loses a comparison and a row of NaNs selects 0, 1, 2, 3.
-// Experts >= E are never selected.  All LPT lanes end with the same result.
-template <int PER, int LPT, int NSEL>
-__device__ __forceinline__ void select_top(const float (&v)[PER], int q, int E, float (&sel_v)[NSEL],
-                                           int (&sel_i)[NSEL]) {
-  static_assert(PER <= 32, "one bit per owned expert");
-  unsigned taken = 0;
-#pragma unroll
-  for (int r = 0; r < NSEL; r++) {
-    float best = 0.f;
-    int bi = kNone;
-#pragma unroll
-    for (int j = 0; j < PER; j++) {
-      const int e = q * PER + j;
-      const bool ok = e < E && !((taken >> j) & 1u);
-      if (ok && (bi == kNone || v[j] > best)) { best = v[j]; bi = e; }
-    }
-#pragma unroll
-    for (int off = 1; off < LPT; off <<= 1) {
-      const float ov = __shfl_xor(best, off, 64);
-      const int oi = __shfl_xor(bi, off, 64);
-      // the lower index is the incumbent; kNone is above every index
-      const bool take = oi < bi ? !(bi != kNone && best > ov) : (oi != kNone && oi != bi && ov > best);
-      if (take) { best = ov; bi = oi; }
-    }
-    sel_v[r] = best;
-    sel_i[r] = bi;
-    if (bi != kNone && bi / PER == q) taken |= 1u << (bi % PER);
-  }
+// The selection's rule is that of the reference's CPU top-k under a stable sort: value descending, index
+// ascending, where a candidate replaces the incumbent (the one with the lower index) only if it compares strictly
+// greater.  Beside a NaN that does not order the logits, and comparisons of parts of them do not give
+// what one walk over all gives: that is the greatest number left, but a NaN while it is the first
+// expert left (a row of NaNs selects 0, 1, 2, 3).
+//
+// A logit as a whole number of the same order, zeros of either sign the same one.
+constexpr uint32_t kTakenKey = 0u, kNanKey = 1u;  // below every number's, minus infinity's too
+__device__ __forceinline__ uint32_t order_key(float v) {
+  const uint32_t u = __float_as_uint(v + 0.f);
+  return v != v ? kNanKey : u ^ ((uint32_t)((int32_t)u >> 31) | 0x80000000u);
+}
+__device__ __forceinline__ float key_value(uint32_t key) {  // kNanKey: a NaN
+  return __uint_as_float(key ^ (~(uint32_t)((int32_t)key >> 31) | 0x80000000u));
 }
 
-// The largest of the wave's values, in every lane.
-__device__ __forceinline__ uint32_t wave_max(uint32_t x) {
+// Among the LPT lanes of a token (a wave, or either half of one): the largest value, in every lane, and the first
+// lane that has something, which one of them does.
+template <int LPT>
+__device__ __forceinline__ uint32_t lanes_max(uint32_t x) {
+  static_assert(LPT == 32 || LPT == 64, "a token has a wave or half of one");
 #define MOE_DPP_MAX(CTRL, ROWS) \
   x = max(x, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, CTRL, ROWS, 0xf, false))
   MOE_DPP_MAX(0x111, 0xf);  // row_shr 1, 2, 4, 8: lane 15 of a row of 16 has the row's
@@ -87,15 +71,55 @@ __device__ __forceinline__ uint32_t wave_max(uint32_t x) {
   MOE_DPP_MAX(0x114, 0xf);
   MOE_DPP_MAX(0x118, 0xf);
   MOE_DPP_MAX(0x142, 0xa);  // row_bcast15 into rows 1 and 3, row_bcast31 into 2 and 3
-  MOE_DPP_MAX(0x143, 0xc);
+  if (LPT == 64) MOE_DPP_MAX(0x143, 0xc);
 #undef MOE_DPP_MAX
-  return (uint32_t)__builtin_amdgcn_readlane((int)x, 63);
+  const uint32_t high = (uint32_t)__builtin_amdgcn_readlane((int)x, 63);
+  return LPT == 64 || (threadIdx.x & 32) ? high : (uint32_t)__builtin_amdgcn_readlane((int)x, 31);
+}
+template <int LPT>
+__device__ __forceinline__ int first_lane(bool has) {
+  const unsigned long long m = __ballot(has);
+  return LPT == 64 ? __builtin_ctzll(m) : __builtin_ctz((uint32_t)(m >> (threadIdx.x & 32)));
 }
 
-// select_top's rule for one token on a whole wave, lane q owning experts q*PER .. q*PER+PER-1 (more than 32
-// experts).  Logits become whole numbers of the same order (zeros of either sign the same one), places past the
-// experts and places taken 0, which is below all of them; a round is a maximum over the wave and the first lane
-// that holds it.  A row with a NaN goes through the comparisons.  Eight lanes per token with 16 experts
+// Top-NSEL of a token's keys, lane q of its LPT owning those of experts q*PER .. q*PER+PER-1; places past the
+// experts hold kTakenKey.  A round is a maximum over the lanes and the first one that holds it.  NANS: there may be
+// NaNs.  All lanes end with the same result, kNone where no expert is left (a whole wave has more than 32).
+template <int PER, int LPT, int NSEL, bool NANS>
+__device__ __forceinline__ void top_keys(uint32_t (&key)[PER], int q, float (&sel_v)[NSEL], int (&sel_i)[NSEL]) {
+  static_assert(LPT == 64 || PER == 1, "a lane of half a wave has one expert");
+#pragma unroll
+  for (int r = 0; r < NSEL; r++) {
+    uint32_t own = key[0];
+#pragma unroll
+    for (int j = 1; j < PER; j++) own = max(own, key[j]);
+    uint32_t best = lanes_max<LPT>(own);
+    int l = first_lane<LPT>(own == best);
+    if constexpr (NANS) {
+      uint32_t first = kTakenKey;  // the lane's first key that is left
+#pragma unroll
+      for (int j = PER - 1; j >= 0; j--)
+        if (key[j] != kTakenKey) first = key[j];
+      const int lf = first_lane<LPT>(first != kTakenKey || best == kTakenKey);
+      if (__shfl((int)first, lf, LPT) == (int)kNanKey) {
+        best = kNanKey;
+        l = lf;
+      }
+    }
+    int at = 0;
+#pragma unroll
+    for (int j = PER - 1; j >= 0; j--)
+      if (key[j] == best) at = j;
+    sel_v[r] = key_value(best);
+    if constexpr (LPT == 64) sel_i[r] = l * PER + __builtin_amdgcn_readlane(at, l);
+    else sel_i[r] = best == kTakenKey ? kNone : l;
+#pragma unroll
+    for (int j = 0; j < PER; j++)
+      if (q == l && at == j) key[j] = kTakenKey;
+  }
+}
+
+// One token on a whole wave (more than 32 experts).  Eight lanes per token with 16 experts
 // each took 5.5 us for the 16 tokens of a workgroup and 128 experts.
 template <int PER, int NSEL>
 __device__ __forceinline__ void wave_top(const float (&v)[PER], int lane, int E, float (&sel_v)[NSEL],
@@ -104,46 +128,25 @@ __device__ __forceinline__ void wave_top(const float (&v)[PER], int lane, int E,
   uint32_t key[PER];
 #pragma unroll
   for (int j = 0; j < PER; j++) {
-    const bool is_expert = lane * PER + j < E;
-    nan |= is_expert && v[j] != v[j];
-    const uint32_t u = __float_as_uint(v[j] + 0.f);
-    key[j] = is_expert ? u ^ ((uint32_t)((int32_t)u >> 31) | 0x80000000u) : 0u;
+    key[j] = lane * PER + j < E ? order_key(v[j]) : kTakenKey;
+    nan |= key[j] == kNanKey;
   }
-  if (__ballot(nan) != 0ull) {
-    select_top<PER, 64, NSEL>(v, lane, E, sel_v, sel_i);
-    return;
-  }
-#pragma unroll
-  for (int r = 0; r < NSEL; r++) {
-    uint32_t own = key[0];
-#pragma unroll
-    for (int j = 1; j < PER; j++) own = max(own, key[j]);
-    const uint32_t best = wave_max(own);
-    const int l = __builtin_ctzll(__ballot(own == best));
-    int at = 0;
-#pragma unroll
-    for (int j = PER - 1; j >= 0; j--)
-      if (key[j] == best) at = j;
-    sel_v[r] = __uint_as_float(best ^ (~(uint32_t)((int32_t)best >> 31) | 0x80000000u));
-    sel_i[r] = l * PER + __builtin_amdgcn_readlane(at, l);
-#pragma unroll
-    for (int j = 0; j < PER; j++)
-      if (lane == l && at == j) key[j] = 0u;
-  }
+  if (__ballot(nan) != 0ull) top_keys<PER, 64, NSEL, true>(key, lane, sel_v, sel_i);
+  else top_keys<PER, 64, NSEL, false>(key, lane, sel_v, sel_i);
 }
 
 // Top-NSEL of one token's logits for up to 32 experts, one lane per expert (the
 // 32 lanes of a half wave; lane e owns expert e, v = its logit, -inf for a lane
 // without an expert).  row4 points at the token's E_pad logits in LDS, 16-byte
-// aligned.  Same rule as select_top, found by counting instead of five rounds
-// of comparisons: an expert's place is the number of experts with a greater
+// aligned.  The same rule, found by counting instead of five rounds
+// of maxima: an expert's place is the number of experts with a greater
 // value; the lanes at places 0 .. NSEL-1 post themselves to `post` (LDS, NSEL
 // floats then NSEL ints, owned by this token) and every lane reads the list
 // back.  Of experts with equal values the lowest index takes the place (an
 // atomic minimum) and the place behind it stays empty: an empty place among the
 // first NSEL, like a NaN among the logits (which no count orders), sends the
-// wave -- the branch is per wave -- through select_top's comparison-by-
-// comparison rule instead.  Places past the number of experts hold kNone.
+// wave -- the branch is per wave -- through top_keys instead.  Places past the
+// number of experts hold kNone.
 template <int E_pad, int NSEL>
 __device__ __forceinline__ void ranked_top(const float4 *row4, float v, int e, int E, float *post,
                                            float (&sel_v)[NSEL], int (&sel_i)[NSEL]) {
@@ -169,8 +172,8 @@ __device__ __forceinline__ void ranked_top(const float4 *row4, float v, int e, i
     redo |= r < E && sel_i[r] == kNone;
   }
   if (__ballot(redo) != 0ull) {
-    const float own[1] = {v};
-    select_top<1, 32, NSEL>(own, e, E, sel_v, sel_i);
+    uint32_t key[1] = {e < E ? order_key(v) : kTakenKey};
+    top_keys<1, 32, NSEL, true>(key, e, sel_v, sel_i);
   }
 }
 

@@ -275,8 +275,8 @@ def test_router_near_ties(E, T):
 
 @pytest.mark.parametrize("E", [33, 63, 64, 65, 127, 128, 129, 200, 256])
 def test_router_selection_of_many_experts(E):
-    """Ranks over a whole wave, and its fall back to comparisons: plateaus of equal logits at the first and the
-    last experts, zeros of either sign, experts at minus infinity, one NaN among the logits, rows of NaN; in
+    """Ranks over a whole wave: plateaus of equal logits at the first and the
+    last experts, zeros of either sign, experts at minus infinity, rows of NaN (some NaNs: the next test); in
     moe_router's one launch and in the two of a whole layer (768 columns, from 65 experts on)."""
     H, T = 768, 40
     sh = synth.LayerShape("many", T, H, 64, E)
@@ -304,6 +304,46 @@ def test_router_selection_of_many_experts(E):
             assert np.abs(R["out"][fine] - want[fine]).max() <= 2e-2
             assert np.linalg.norm(R["out"][fine] - want[fine]) <= 1e-3 * np.linalg.norm(want[fine])
         m.close()
+
+
+@pytest.mark.parametrize("E", [4, 5, 8, 16, 17, 31, 32, 33, 63, 64, 65, 127, 128, 129, 200, 256])
+def test_router_selection_beside_nans(E):
+    """Some NaNs among a token's logits: one is chosen when every expert before it has been, and at no other time.
+    From NaN biases, at the ends, in the middle, at even and odd places, next to experts that every token
+    names, and at random; in tokens with an infinity also where its weight is zero.  The ids of moe_router and those
+    that a whole layer ran on."""
+    H, T = 768, 64
+    rng = np.random.default_rng(E)
+    sh = synth.LayerShape("nans", T, H, 64, E)
+    L = bf16_layer(sh, seed=E)
+    x, wr, br = L["x"].copy(), L["w_router"].copy(), L["b_router"]
+    wr[::3, 5] = 0.0
+    wr[1::3, 6] = 0.0
+    x[::11, 5], x[1::11, 6], x[2::11, [5, 6]] = np.inf, -np.inf, np.inf
+    sets = [[0], [1], [2], [3], [E - 1], [E // 2], [E // 2 + 1], [E // 3], [0, 1], [0, E - 1], range(0, E, 2), range(1, E, 2),
+            range(3, E), range(E - 3), *(np.nonzero(rng.random(E) < p)[0] for p in (0.05, 0.05, 0.2, 0.5, 0.8))]
+    L["x"], L["w_router"] = x, wr
+    m = abi.Moe(H, 64, E, max_tokens=T, swiglu_limit=sh.limit)
+    doff, dperm, dout = abi.DevBuf((E + 1) * 4), abi.DevBuf(T * 16), abi.DevBuf(T * H * 4)
+    dx = abi.DevBuf.from_numpy(synth.to_bf16_bits(x))
+    chosen = False
+    for lift in (0.0, 64.0):  # 64: the first experts lead every token, in their order
+        for nans in sets:
+            L["b_router"] = br.copy()
+            L["b_router"][:3] += lift * np.arange(3, 0, -1)
+            L["b_router"][list(nans)] = np.nan
+            L["b_router"] = synth.round_bf16(L["b_router"])
+            m.upload_layer(0, *[L[k] for k in W])
+            _, score, ti = _check_ids(m, L, x, None, E)
+            chosen |= bool(np.isnan(np.take_along_axis(score, ti, 1)[:, 1:]).any())
+            m.forward(0, dx, None, T, dout)
+            m.get_dispatch(doff, dperm, T)
+            abi.sync()
+            off, perm, _ = ob.dispatch(ti, None, E)
+            assert np.array_equal(doff.download((E + 1,), np.int32), off), (lift, list(nans))
+            assert np.array_equal(dperm.download((T * 4,), np.int32), perm), (lift, list(nans))
+    m.close()
+    assert chosen
 
 
 def test_router_first_pass_error_bound():
