@@ -709,7 +709,7 @@ hipError_t launch_gate_up(const uint16_t *x, const void *w1, const uint16_t *w1_
   if (r.kernel == kBf16Tiles)
     return launch_bf16_gate_up(x, w1, b1g, b1u, d, act, H, IM, limit, T, E, tile_rows, wide, r.past_caches, s);
   if (r.kernel == kFp4ManyTiles)
-    return launch_fp4_gate_up(x, w1, w1_scale, b1g, b1u, d, act, H, IM, limit, T, E, wide, r.past_caches, s);
+    return launch_fp4_gate_up(x, w1, w1_scale, b1g, b1u, d, act, H, IM, limit, T, E, r.past_caches, s);
   return launch_gemm<true>(x, w1, w1_scale, b1g, b1u, d, act, H, IM, limit, T, E, tile_rows, wide, r.past_caches, s);
 }
 
@@ -719,7 +719,7 @@ hipError_t launch_down(const uint16_t *act, const void *w2, const uint16_t *w2_s
   if (H % 64 || IM % 64) return hipErrorInvalidValue;  // the kernels take steps of 32 in pairs
   const TileRoute r = tile_route(T, E, 2 * IM, w2_scale != nullptr, tile_rows, cached);
   if (r.kernel == kBf16Tiles) return launch_bf16_down(act, w2, b2, d, y, H, IM, T, E, tile_rows, wide, r.past_caches, s);
-  if (r.kernel == kFp4ManyTiles) return launch_fp4_down(act, w2, w2_scale, b2, d, y, H, IM, T, E, wide, r.past_caches, s);
+  if (r.kernel == kFp4ManyTiles) return launch_fp4_down(act, w2, w2_scale, b2, d, y, H, IM, T, E, r.past_caches, s);
   return launch_gemm<false>(act, w2, w2_scale, b2, nullptr, d, y, IM, H, 0.f, T, E, tile_rows, wide, r.past_caches, s);
 }
 

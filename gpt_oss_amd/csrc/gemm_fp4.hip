@@ -632,11 +632,11 @@ static_assert(Cfg::RBT_MAX * kRowBlock == kHalfTileRows && Cfg::TILE_NB == kGemm
 
 template <bool GATE_UP>
 hipError_t launch(const void *a, const void *w, const uint16_t *w_scale, const float *ba, const float *bb,
-                  const DispatchBuffers &d, void *out, int K, int N, float limit, int T, int E, bool wide, bool stream,
+                  const DispatchBuffers &d, void *out, int K, int N, float limit, int T, int E, bool stream,
                   hipStream_t s) {
   const int nb_total = (GATE_UP ? 2 * N : N) / kRowBlock;
   const int n_ct = (nb_total + kGemmTileNb - 1) / kGemmTileNb;
-  const dim3 grid(kXcds * xcd_tile_cap(gemm_tile_cap(T, E, kHalfTileRows) * n_ct), wide ? 2 : 1);
+  const int grid = kXcds * xcd_tile_cap(gemm_tile_cap(T, E, kHalfTileRows) * n_ct);
   const TileDesc *tiles = GATE_UP ? d.tiles_gate_up : d.tiles_down;
   const uint4 *af = static_cast<const uint4 *>(a), *wf = static_cast<const uint4 *>(w);
   if (stream)
@@ -652,14 +652,13 @@ hipError_t launch(const void *a, const void *w, const uint16_t *w_scale, const f
 
 hipError_t launch_fp4_gate_up(const uint16_t *x, const void *w1, const uint16_t *w1_scale, const float *b1g,
                               const float *b1u, const DispatchBuffers &d, uint16_t *act, int H, int IM, float limit,
-                              int T, int E, bool wide, bool stream, hipStream_t s) {
-  return launch<true>(x, w1, w1_scale, b1g, b1u, d, act, H, IM, limit, T, E, wide, stream, s);
+                              int T, int E, bool stream, hipStream_t s) {
+  return launch<true>(x, w1, w1_scale, b1g, b1u, d, act, H, IM, limit, T, E, stream, s);
 }
 
 hipError_t launch_fp4_down(const uint16_t *act, const void *w2, const uint16_t *w2_scale, const float *b2,
-                           const DispatchBuffers &d, float *y, int H, int IM, int T, int E, bool wide, bool stream,
-                           hipStream_t s) {
-  return launch<false>(act, w2, w2_scale, b2, nullptr, d, y, IM, H, 0.f, T, E, wide, stream, s);
+                           const DispatchBuffers &d, float *y, int H, int IM, int T, int E, bool stream, hipStream_t s) {
+  return launch<false>(act, w2, w2_scale, b2, nullptr, d, y, IM, H, 0.f, T, E, stream, s);
 }
 
 }  // namespace moe

@@ -357,13 +357,12 @@ hipError_t launch_bf16_gate_up(const uint16_t *x, const void *w1, const float *b
                                int tile_rows, bool wide, bool stream, hipStream_t s);
 hipError_t launch_bf16_down(const uint16_t *act, const void *w2, const float *b2, const DispatchBuffers &d, float *y,
                             int H, int IM, int T, int E, int tile_rows, bool wide, bool stream, hipStream_t s);
-// MXFP4 weights with many rows per expert (gemm_fp4.hip; likewise), a plan of kHalfTileRows.
+// MXFP4 weights with many rows per expert (gemm_fp4.hip; likewise), a plan of kHalfTileRows, which is never a wide one.
 hipError_t launch_fp4_gate_up(const uint16_t *x, const void *w1, const uint16_t *w1_scale, const float *b1g,
                               const float *b1u, const DispatchBuffers &d, uint16_t *act, int H, int IM, float limit,
-                              int T, int E, bool wide, bool stream, hipStream_t s);
+                              int T, int E, bool stream, hipStream_t s);
 hipError_t launch_fp4_down(const uint16_t *act, const void *w2, const uint16_t *w2_scale, const float *b2,
-                           const DispatchBuffers &d, float *y, int H, int IM, int T, int E, bool wide, bool stream,
-                           hipStream_t s);
+                           const DispatchBuffers &d, float *y, int H, int IM, int T, int E, bool stream, hipStream_t s);
 // tiles: row tiles, at most (stream_direct_tile_cap with ids.topk_i, otherwise stream_tile_cap).
 // T, E: tokens and experts of the batch, the same for both (the order of act between them follows from these).
 // cached: kCachedWeightBytes.
