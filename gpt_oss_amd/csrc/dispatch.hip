@@ -39,10 +39,18 @@ __global__ __launch_bounds__(kDispThreads) void dispatch_count_kernel(
     perm[i] = -1;
 }
 
+// An expert's part of the plan, held in LDS for the workgroup's own use.
+struct ExpertPlan {
+  int row0;       // first padded row of the expert's segment (multiple of 32)
+  int n_mt;       // number of row tiles
+  int rb;         // row blocks of the expert's shorter tiles (0..8)
+  int extra;      // its first `extra` tiles have rb + 1 row blocks
+  int tiles0[2];  // tiles of all lower experts in the sequences of gate_up and down
+};
+
 // Where the plan of a batch goes, and what it is of.
 struct PlanOut {
   int *offsets;
-  ExpertInfo *info;
   int *totals;
   TileDesc *tiles_gate_up, *tiles_down;
   int tile_cap_gate_up, tile_cap_down;
@@ -68,8 +76,8 @@ struct PlanOut {
 // down GEMM's 1.75 -> 1.51 GB, durations unchanged; experts with up to
 // kRowTileGroup row tiles (even routing at 4096 tokens) are laid out as before.
 // One wave; its lanes run over the expert's tiles of both GEMMs in one sweep.
-__device__ __forceinline__ void write_expert_tiles(int ee, int nmt, int rbe, int exe, int rowblk, int first_up,
-                                                   int first_down, int lane, const PlanOut &out) {
+__device__ __forceinline__ void write_expert_tiles(int ee, const ExpertPlan p, int lane, const PlanOut &out) {
+  const int nmt = p.n_mt, rbe = p.rb, exe = p.extra, rowblk = p.row0 / kRowBlock;
   if (nmt == 0) return;
   const int height = rbe + (exe ? 1 : 0), width = tile_width(height, out.wide);
   const int n_ct_up = out.col_tiles(0, height), n_ct_down = out.col_tiles(1, height);
@@ -77,7 +85,7 @@ __device__ __forceinline__ void write_expert_tiles(int ee, int nmt, int rbe, int
   for (int ii = lane; ii < n; ii += 64) {
     const bool g = ii >= n_up;
     const int i = g ? ii - n_up : ii;
-    const int L = (g ? first_down : first_up) + i;
+    const int L = (g ? p.tiles0[1] : p.tiles0[0]) + i;
     const int n_ct = g ? n_ct_down : n_ct_up;
     const int n_grp = (nmt + kRowTileGroup - 1) / kRowTileGroup;
     const int gs = nmt / n_grp, gx = nmt - gs * n_grp;  // the first gx groups hold gs + 1 row tiles
@@ -106,12 +114,12 @@ __device__ __forceinline__ void write_expert_tiles(int ee, int nmt, int rbe, int
 
 // The plan of one batch from the experts' row counts (thread e < 256 holds expert e's count; all threads of the
 // workgroup call this together, those from 256 on only take part in the barriers).  Returns the
-// expert's first row in the padded row space.
-// write_global: this workgroup stores the plan (offsets, per-expert records,
-// totals, XCD bounds); the others only need the values returned to them.
-__device__ __forceinline__ int build_plan(int count, int E, const PlanOut &out, bool write_global, int *ex_count_out,
-                                          int *tot_count_out, ExpertInfo *info_out) {
-  constexpr int kSums = 6, kSumsPlan = 3;  // the last ones are of the tile tables
+// expert's part; the rows of all lower experts and of all experts go where the pointers say.
+// write_global: this workgroup stores the plan (offsets, padded rows,
+// XCD bounds); the others only need the values returned to them.
+__device__ __forceinline__ ExpertPlan build_plan(int count, int E, const PlanOut &out, bool write_global,
+                                                 int *ex_count_out, int *tot_count_out) {
+  constexpr int kSums = 5, kSumsPlan = 2;  // the last ones are of the tile tables
   __shared__ int sh_wave[4][kSums];  // [wave][quantity]: the waves' sums
   __shared__ int sh_cost[257];      // exclusive prefix of the experts' cost
   __shared__ int sh_tiles[2][257];  // exclusive prefix of their tiles in either GEMM
@@ -120,7 +128,6 @@ __device__ __forceinline__ int build_plan(int count, int E, const PlanOut &out, 
   const int lane = e & 63;
   const int w = e >> 6;
   int *offsets = out.offsets;
-  ExpertInfo *info = out.info;
   int *totals = out.totals;
   const int n_rb = (count + kRowBlock - 1) / kRowBlock;
   const int n_mt = (n_rb + out.tile_rb - 1) / out.tile_rb;
@@ -131,10 +138,10 @@ __device__ __forceinline__ int build_plan(int count, int E, const PlanOut &out, 
   const int n_up = n_mt * out.col_tiles(0, height), n_down = n_mt * out.col_tiles(1, height);
   // cost of kGemmTileNb column blocks' worth of the expert's row tiles: of tiles of any width, whose cost goes by it
   const int cost = n_mt * (out.tile_cost + kCostPerRowBlock * rb) + kCostPerRowBlock * extra;
-  // Exclusive prefix sums over the experts of six quantities at once: rows,
-  // padded rows, row tiles, cost, tiles of either GEMM.  In a wave by lane shifts, across the four
+  // Exclusive prefix sums over the experts of five quantities at once: rows,
+  // padded rows, cost, tiles of either GEMM.  In a wave by lane shifts, across the four
   // waves through LDS.
-  const int own[kSums] = {count, n_rb * kRowBlock, n_mt, cost, n_up, n_down};
+  const int own[kSums] = {count, n_rb * kRowBlock, cost, n_up, n_down};
   int incl[kSums];
 #pragma unroll
   for (int i = 0; i < kSums; i++) incl[i] = own[i];
@@ -165,59 +172,38 @@ __device__ __forceinline__ int build_plan(int count, int E, const PlanOut &out, 
     ex[i] = below + incl[i] - own[i];
     tot[i] = all;
   }
-  const int ex_count = ex[0], ex_pad = ex[1], ex_mt = ex[2], ex_cost = ex[3];
-  const int tot_count = tot[0], tot_pad = tot[1], tot_mt = tot[2], tot_cost = tot[3];
-  {
-    ExpertInfo inf;
-    inf.row0 = ex_pad;
-    inf.rows = count;
-    inf.n_mt = n_mt;
-    inf.rb = rb;
-    inf.tile_base = ex_mt;
-    inf.extra = extra;
-    inf.tiles0[0] = ex[4];
-    inf.tiles0[1] = ex[5];
-    if (e < E && write_global) {
-      offsets[e] = ex_count;
-      info[e] = inf;
-    }
-    *info_out = inf;
-  }
+  const int ex_count = ex[0], ex_pad = ex[1], ex_cost = ex[2];
+  const int tot_count = tot[0], tot_pad = tot[1], tot_cost = tot[2];
+  const ExpertPlan mine = {ex_pad, n_mt, rb, extra, {ex[3], ex[4]}};
   *ex_count_out = ex_count;
   *tot_count_out = tot_count;
-  if (write_global && !tables && e == 0) {
-    offsets[E] = tot_count;
-    totals[kTotTiles] = tot_mt;
-    totals[kTotRows] = tot_pad;
-    totals[kTotAssign] = tot_count;
+  if (write_global) {
+    if (e < E) offsets[e] = ex_count;
+    if (e == 0) {
+      offsets[E] = tot_count;
+      totals[kTotRows] = tot_pad;
+    }
   }
   // Without column tiles (stream.hip) the XCDs' ranges are of no tiles: their search and its
   // divisions are left out (us per call, 128 experts, 200 tokens 313.8 / 310.0; 512 x 512, 32 experts, 128
   // tokens 35.7 / 33.8).
-  if (!write_global || !tables) {  // (the same for the whole workgroup)
-    return ex_pad;
-  }
+  if (!write_global || !tables) return mine;  // (the same for the whole workgroup)
   if (e < 256) {
     sh_cost[e] = ex_cost;
-    sh_tiles[0][e] = ex[4];
-    sh_tiles[1][e] = ex[5];
+    sh_tiles[0][e] = ex[3];
+    sh_tiles[1][e] = ex[4];
   }
   if (e == 0) {
     sh_cost[256] = tot_cost;
-    sh_tiles[0][256] = tot[4];
-    sh_tiles[1][256] = tot[5];
-    offsets[E] = tot_count;
-    totals[kTotTiles] = tot_mt;
-    totals[kTotRows] = tot_pad;
-    totals[kTotAssign] = tot_count;
-    totals[3] = 0;
+    sh_tiles[0][256] = tot[3];
+    sh_tiles[1][256] = tot[4];
   }
   __syncthreads();
   // Thread (g, x): boundary x of GEMM g = first tile at which the cost so far
   // reaches x/8 of the total (an expert's tiles taken as equally dear: their heights differ by one block at most).
   if (e < 2 * (kXcds + 1)) {
     const int g = e / (kXcds + 1), x = e % (kXcds + 1);
-    const int total_tiles = tot[4 + g];
+    const int total_tiles = tot[3 + g];
     int bound;
     if (x == 0) {
       bound = 0;
@@ -242,7 +228,7 @@ __device__ __forceinline__ int build_plan(int count, int E, const PlanOut &out, 
   __syncthreads();
   // keep every range within what the launch grid provides for (xcd_tile_cap)
   if (e < 2) {
-    const int total_tiles = tot[4 + e];
+    const int total_tiles = tot[3 + e];
     const int cap = xcd_tile_cap(total_tiles);
     int *bounds = totals + (e ? kTotBoundsDown : kTotBoundsGateUp);
     int prev = 0, want[kXcds];
@@ -259,7 +245,7 @@ __device__ __forceinline__ int build_plan(int count, int E, const PlanOut &out, 
     }
     bounds[kXcds] = total_tiles;
   }
-  return ex_pad;
+  return mine;
 }
 
 // The row-tile plan (see build_plan): an expert with M rows has ceil(M / 32) row
@@ -332,8 +318,8 @@ __global__ __launch_bounds__(kDispThreads) void dispatch_scatter_kernel(
     const int *__restrict__ blk_counts, int n_blk, int *__restrict__ perm, int *__restrict__ rowmap,
     int *__restrict__ inv, int *__restrict__ blk_expert, PlanOut plan) {
   __shared__ int wave_cnt[kDispThreads / 64][256];
-  __shared__ int sh_base[256], sh_off[256], sh_row0[256];
-  __shared__ ExpertInfo sh_info[256];
+  __shared__ int sh_base[256], sh_off[256];
+  __shared__ ExpertPlan sh_plan[256];
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int w = tid >> 6;
@@ -361,13 +347,11 @@ __global__ __launch_bounds__(kDispThreads) void dispatch_scatter_kernel(
     }
   }
   int ex_count, tot_count;
-  ExpertInfo inf;
-  const int row0 = build_plan(count, E, plan, /*write_global=*/(int)blockIdx.x == n_blk, &ex_count, &tot_count, &inf);
+  const ExpertPlan mine = build_plan(count, E, plan, /*write_global=*/(int)blockIdx.x == n_blk, &ex_count, &tot_count);
   if ((int)blockIdx.x == n_blk) return;
   sh_base[tid] = base;
   sh_off[tid] = ex_count;
-  sh_row0[tid] = row0;
-  sh_info[tid] = inf;
+  sh_plan[tid] = mine;
   for (int e = tid; e < (kDispThreads / 64) * 256; e += kDispThreads) (&wave_cnt[0][0])[e] = 0;
   int rank[kTopK], total[kTopK];
   wave_ranks(IdPlanes<NBITS>(id), id, lane, rank, total);
@@ -375,8 +359,7 @@ __global__ __launch_bounds__(kDispThreads) void dispatch_scatter_kernel(
   // The tile sequences of the GEMMs: the waves of all workgroups take the
   // experts in turn.
   for (int ee = blockIdx.x * (kDispThreads / 64) + w; ee < E; ee += n_blk * (kDispThreads / 64)) {
-    const ExpertInfo f = sh_info[ee];
-    write_expert_tiles(ee, f.n_mt, f.rb, f.extra, f.row0 / kRowBlock, f.tiles0[0], f.tiles0[1], lane, plan);
+    write_expert_tiles(ee, sh_plan[ee], lane, plan);
   }
 #pragma unroll
   for (int k = 0; k < kTopK; k++)
@@ -391,7 +374,7 @@ __global__ __launch_bounds__(kDispThreads) void dispatch_scatter_kernel(
     if (e < 0) { out_inv[k] = -1; continue; }
     int r = sh_base[e] + rank[k];
     for (int ww = 0; ww < w; ww++) r += wave_cnt[ww][e];
-    const int prow = sh_row0[e] + r;
+    const int prow = sh_plan[e].row0 + r;
     perm[sh_off[e] + r] = a;
     rowmap[prow] = a;
     if (blk_expert && prow % kRowBlock == 0) blk_expert[prow / kRowBlock] = e;
@@ -418,8 +401,8 @@ __global__ __launch_bounds__(kOnceThreads) void dispatch_once_kernel(
     const int *__restrict__ topk_i, const int *__restrict__ pos, int T, int E, PlanOut plan, int n_blk,
     int *__restrict__ perm, int *__restrict__ rowmap, int *__restrict__ inv, int *__restrict__ blk_expert) {
   __shared__ int cnt[kOnceGroups][256];  // per group of 64 tokens and expert: count, then the rows before the group's
-  __shared__ int sh_off[256], sh_row0[256];
-  __shared__ ExpertInfo sh_info[256];
+  __shared__ int sh_off[256];
+  __shared__ ExpertPlan sh_plan[256];
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -465,29 +448,25 @@ __global__ __launch_bounds__(kOnceThreads) void dispatch_once_kernel(
     }
   }
   int ex_count, tot_count;
-  ExpertInfo inf;
-  const int row0 = build_plan(count, E, plan, /*write_global=*/(int)blockIdx.x == n_blk, &ex_count, &tot_count, &inf);
+  const ExpertPlan mine = build_plan(count, E, plan, /*write_global=*/(int)blockIdx.x == n_blk, &ex_count, &tot_count);
   if ((int)blockIdx.x == n_blk) {
     // -1 where the scatter below writes nothing: the padding rows of the experts
     // and the tail of perm that inactive rows and invalid ids leave unused
     if (tid < E) {
-      const int end = row0 + (count + kRowBlock - 1) / kRowBlock * kRowBlock;
-      for (int i = row0 + count; i < end; i++) rowmap[i] = -1;
+      const int end = mine.row0 + (count + kRowBlock - 1) / kRowBlock * kRowBlock;
+      for (int i = mine.row0 + count; i < end; i++) rowmap[i] = -1;
     }
     for (int i = tot_count + tid; i < T * kTopK; i += kOnceThreads) perm[i] = -1;
     return;
   }
   if (tid < E) {
     sh_off[tid] = ex_count;
-    sh_row0[tid] = row0;
-    sh_info[tid] = inf;
+    sh_plan[tid] = mine;
   }
   __syncthreads();
   if (plan.nb[0] > 0) {  // the tile sequences of the GEMMs: the waves of all workgroups take the experts in turn
-    for (int ee = blockIdx.x * kOnceWaves + w; ee < E; ee += n_blk * kOnceWaves) {
-      const ExpertInfo f = sh_info[ee];
-      write_expert_tiles(ee, f.n_mt, f.rb, f.extra, f.row0 / kRowBlock, f.tiles0[0], f.tiles0[1], lane, plan);
-    }
+    for (int ee = blockIdx.x * kOnceWaves + w; ee < E; ee += n_blk * kOnceWaves)
+      write_expert_tiles(ee, sh_plan[ee], lane, plan);
   }
   const int t = own_group * 64 + lane;
   if (own_group < 0 || t >= T) return;
@@ -497,7 +476,7 @@ __global__ __launch_bounds__(kOnceThreads) void dispatch_once_kernel(
     const int e = own[k];
     if (e < 0) { out_inv[k] = -1; continue; }
     const int rk = cnt[own_group][e] + rank[k];
-    const int prow = sh_row0[e] + rk;
+    const int prow = sh_plan[e].row0 + rk;
     perm[sh_off[e] + rk] = t * kTopK + k;
     rowmap[prow] = t * kTopK + k;
     if (blk_expert && prow % kRowBlock == 0) blk_expert[prow / kRowBlock] = e;
@@ -576,7 +555,6 @@ hipError_t launch_dispatch(const int *topk_i, const int *pos, int T, int E, int 
   const int fill_rows = (int)(reach < d.a_pad_cap ? reach : d.a_pad_cap);
   PlanOut plan;
   plan.offsets = d.offsets;
-  plan.info = d.info;
   plan.totals = d.totals;
   plan.tiles_gate_up = d.tiles_gate_up;
   plan.tiles_down = d.tiles_down;
@@ -642,7 +620,7 @@ hipError_t launch_combine_residual(const float *y, int ldy, const int *inv, cons
 // moe_dispatch_static runs the same kernels as moe_dispatch, but needs no
 // handle and calls no allocating routine: the buffers the kernels use beyond
 // the caller's inputs and outputs (per-workgroup counts, the padded row map,
-// the inverse map, the per-expert records and the plan's totals) live in one
+// the inverse map and the plan's totals) live in one
 // file-scope device array.  Every GPU the library runs on holds that array
 // until the process ends; every call on a GPU shares it, so calls that overlap
 // on one GPU (two streams, two threads) race.  The kernels rewrite everything
@@ -658,8 +636,7 @@ constexpr size_t kStaticRowmap =
     kStaticBlkCounts + align256(sizeof(int) * ((kStaticMaxTokens + kDispThreads - 1) / kDispThreads) * kStaticMaxExperts);
 constexpr int kStaticPadRows = kStaticMaxTokens * kTopK + kTileGran * kStaticMaxExperts;
 constexpr size_t kStaticInv = kStaticRowmap + align256(sizeof(int) * kStaticPadRows);
-constexpr size_t kStaticInfo = kStaticInv + align256(sizeof(int) * kStaticMaxTokens * kTopK);
-constexpr size_t kStaticTotals = kStaticInfo + align256(sizeof(ExpertInfo) * kStaticMaxExperts);
+constexpr size_t kStaticTotals = kStaticInv + align256(sizeof(int) * kStaticMaxTokens * kTopK);
 constexpr size_t kStaticBytes = kStaticTotals + align256(sizeof(int) * kTotInts);
 
 static __device__ __align__(256) unsigned char scratch[kStaticBytes];
@@ -709,7 +686,6 @@ extern "C" int moe_dispatch_static(const int *topk_i, const int *pos, int n_toke
   d.blk_counts = reinterpret_cast<int *>(base + kStaticBlkCounts);
   d.rowmap = reinterpret_cast<int *>(base + kStaticRowmap);
   d.inv = reinterpret_cast<int *>(base + kStaticInv);
-  d.info = reinterpret_cast<ExpertInfo *>(base + kStaticInfo);
   d.totals = reinterpret_cast<int *>(base + kStaticTotals);
   d.offsets = offsets;
   d.perm = perm;

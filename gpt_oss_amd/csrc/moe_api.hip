@@ -287,7 +287,6 @@ int moe_create(const moe_config *cfg, moe_handle **out) {
   ALLOC(h->disp.rowmap, (size_t)h->a_pad_cap);
   ALLOC(h->disp.inv, (size_t)h->a_cap);
   ALLOC(h->disp.blk_expert, (size_t)h->a_pad_cap / kRowBlock);
-  ALLOC(h->disp.info, (size_t)E);
   ALLOC(h->disp.totals, (size_t)kTotInts);
   {
     const int mt_cap = gemm_tile_cap(T, E, kHalfTileRows);  // row tiles at max_tokens, at most
@@ -321,7 +320,7 @@ int moe_destroy(moe_handle *h) {
   }
   (void)hipFree(h->topk_i); (void)hipFree(h->topk_v);
   (void)hipFree(h->disp.blk_counts); (void)hipFree(h->disp.offsets); (void)hipFree(h->disp.perm);
-  (void)hipFree(h->disp.rowmap); (void)hipFree(h->disp.inv); (void)hipFree(h->disp.info); (void)hipFree(h->disp.blk_expert); (void)hipFree(h->disp.totals);
+  (void)hipFree(h->disp.rowmap); (void)hipFree(h->disp.inv); (void)hipFree(h->disp.blk_expert); (void)hipFree(h->disp.totals);
   (void)hipFree(h->disp.tiles_gate_up); (void)hipFree(h->disp.tiles_down);
   (void)hipFree(h->act); (void)hipFree(h->y); (void)hipFree(h->t_norm); (void)hipFree(h->x_pad);
   for (hipEvent_t ev : h->events) (void)hipEventDestroy(ev);

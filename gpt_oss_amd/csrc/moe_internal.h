@@ -46,25 +46,14 @@ constexpr int kXcds = 8;
 // Estimated cost of a tile: a fixed part (plan_tile_cost) + kCostPerRowBlock * row blocks.
 constexpr int kCostPerRowBlock = 8;
 // layout of DispatchBuffers::totals
-constexpr int kTotTiles = 0, kTotRows = 1, kTotAssign = 2;
-constexpr int kTotBoundsGateUp = 4;            // 9 ints
-constexpr int kTotBoundsDown = 4 + kXcds + 1;  // 9 ints
-constexpr int kTotInts = 4 + 2 * (kXcds + 1);
+constexpr int kTotRows = 0;                                  // padded rows
+constexpr int kTotBoundsGateUp = 1;                          // 9 ints
+constexpr int kTotBoundsDown = kTotBoundsGateUp + kXcds + 1;  // 9 ints
+constexpr int kTotInts = kTotBoundsDown + kXcds + 1;
 
 // Most tiles one XCD can be given out of `total`: the balancing never moves a
 // boundary further than this, so that the launch grid can be sized on the host.
 __host__ __device__ inline int xcd_tile_cap(int total) { return (total + 7) / 8 + (total + 15) / 16 + 1; }
-
-// Per-expert record written by the scan kernel and read by the GEMMs.
-struct ExpertInfo {
-  int row0;       // first padded row of the expert's segment (multiple of 32)
-  int rows;       // valid rows (assignments) of the expert
-  int n_mt;       // number of row tiles
-  int rb;         // row blocks of the expert's shorter tiles (0..8)
-  int tile_base;  // number of row tiles of all lower experts
-  int extra;      // its first `extra` tiles have rb + 1 row blocks
-  int tiles0[2];  // tiles of all lower experts in the sequences of gate_up and down
-};
 
 // One tile of a grouped GEMM, looked up by its number in the tile sequence.
 // Written by the scan kernel for both GEMMs, so that a GEMM workgroup finds its
@@ -159,8 +148,7 @@ struct DispatchBuffers {
   int *rowmap;        // [A_pad] padded position -> assignment id, -1 = padding
   int *inv;           // [A]     assignment id -> padded position, -1 = inactive
   int *blk_expert;    // [A_pad / 32] row block of the padded rows -> expert (nullptr: not wanted)
-  ExpertInfo *info;   // [E]
-  int *totals;        // [kTotInts]: total row tiles, padded rows, assignments; XCD bounds of both GEMMs
+  int *totals;        // [kTotInts]: padded rows; XCD bounds of both GEMMs
   int a_pad_cap;      // capacity of rowmap in rows
   TileDesc *tiles_gate_up;  // [tile_cap_gate_up] tile sequence of the gate_up GEMM
   TileDesc *tiles_down;     // [tile_cap_down]    ... of the down GEMM
