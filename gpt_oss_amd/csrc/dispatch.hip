@@ -419,6 +419,7 @@ __global__ __launch_bounds__(kOnceThreads) void dispatch_once_kernel(
   for (int r = 0; r < kOnceRounds; r++) {
     const int g = w + r * kOnceWaves;
     if (g >= groups) break;
+    static_assert(kOnceRounds == 2, "which round's ids");
     const int4 v = r ? ids[1] : ids[0];
     int id[kTopK] = {v.x, v.y, v.z, v.w};
 #pragma unroll
