@@ -22,7 +22,7 @@ SYMBOLS = [
     "moe_create", "moe_destroy", "moe_upload_layer", "moe_upload_layer_mxfp4", "moe_upload_norm",
     "moe_forward", "moe_block_forward",
     "moe_router",
-    "moe_dispatch", "moe_get_dispatch", "moe_experts", "moe_expert_gemms", "moe_combine",
+    "moe_dispatch", "moe_get_dispatch", "moe_get_tile_ranges", "moe_experts", "moe_expert_gemms", "moe_combine",
     "moe_dispatch_static", "moe_set_distinct_ids", "moe_profile_enable",
     "moe_profile_read", "moe_weight_bytes", "moe_workspace_bytes", "moe_last_error",
     "moe_version", "moe_dev_alloc", "moe_dev_free", "moe_dev_upload", "moe_dev_download",
@@ -65,6 +65,7 @@ def lib() -> C.CDLL:
         L.moe_router.argtypes = [vp, ci, vp, vp, ci, vp, vp, vp, vp]
         L.moe_dispatch.argtypes = [vp, vp, vp, ci, vp]
         L.moe_get_dispatch.argtypes = [vp, vp, vp, ci, vp]
+        L.moe_get_tile_ranges.argtypes = [vp, vp, vp]
         L.moe_experts.argtypes = [vp, ci, vp, vp, vp, vp, ci, vp, ci, vp]
         L.moe_expert_gemms.argtypes = [vp, ci, vp, ci, vp]
         L.moe_combine.argtypes = [vp, vp, vp, ci, vp, ci, vp]
@@ -239,6 +240,13 @@ class Moe:
 
     def get_dispatch(self, offsets, perm, n_tokens, stream=None):
         check(lib().moe_get_dispatch(self.h, _p(offsets), _p(perm), n_tokens, stream))
+
+    def tile_ranges(self):
+        """[2, 9]: first tiles of the XCDs and number of tiles, gate_up and down, of the last dispatch."""
+        b = DevBuf(18 * 4)
+        check(lib().moe_get_tile_ranges(self.h, _p(b), None))
+        sync()
+        return b.download((2, 9), np.int32)
 
     def experts(self, layer, x, pos, topk_i, topk_v, n_tokens, out, accumulate=False, stream=None):
         check(lib().moe_experts(self.h, layer, _p(x), _p(pos), _p(topk_i), _p(topk_v), n_tokens,

@@ -68,6 +68,7 @@ struct moe_handle {
   int n_blk_cap = 0;
   int plan_rows = kTileRows;  // tallest row tile of the last plan
   bool plan_wide = false;     // ... and whether its tiles are of tile_width
+  bool plan_tiles = false;    // whether the last call has a plan with tiles
   int disp_tokens = -1;  // batch of the last moe_dispatch (stage-level calls), -1: none
   bool gemms_done = false;  // moe_expert_gemms has run on that dispatch: y holds its rows
   bool distinct_ids = false;  // moe_set_distinct_ids: caller-supplied ids name an expert once per token
@@ -155,6 +156,7 @@ int run_dispatch(moe_handle *h, const int *topk_i, const int *pos, int T, bool m
   h->plan_rows = plan_tile_rows(T, E, h->Hp, h->IMp, mxfp4, h->expert_bytes <= kCachedWeightBytes);
   // the kernels of stream.hip go by row blocks and need no tile tables
   const bool tables = !stream_batch(T, E);
+  h->plan_tiles = tables;
   h->plan_wide = tables && !mxfp4 &&
                  bf16_wide_tiles(T, E, h->Hp, h->IMp,
                                  gemm_streams_weights(T, E, false, h->plan_rows, h->expert_bytes <= kCachedWeightBytes));
@@ -225,6 +227,7 @@ int run_experts(moe_handle *h, int layer, const uint16_t *x, const int *pos, con
   const DirectIds direct{direct_plan ? topk_i : nullptr, pos, T, c.experts};
   int rc = direct_plan ? MOE_OK : run_dispatch(h, topk_i, pos, T, h->layers[layer].w1q != nullptr, s);
   if (rc != MOE_OK) return rc;
+  if (direct_plan) h->plan_tiles = false;
   h->unplanned = direct;
   h->disp_tokens = -1;  // the plan now belongs to this call, not to a moe_dispatch
   h->gemms_done = false;
@@ -525,6 +528,14 @@ int moe_get_dispatch(moe_handle *h, int *offsets, int *perm, int n_tokens, void 
   if (perm && n_tokens > 0)
     HIP_TRY(hipMemcpyAsync(perm, h->disp.perm, (size_t)n_tokens * kTopK * sizeof(int),
                            hipMemcpyDeviceToDevice, s));
+  return MOE_OK;
+}
+
+int moe_get_tile_ranges(moe_handle *h, int *ranges, void *stream) {
+  if (!h || !ranges) return fail(MOE_ERR_BAD_ARG, "null argument");
+  if (!h->plan_tiles) return fail(MOE_ERR_STATE, "moe_get_tile_ranges: the last call planned no tiles");
+  HIP_TRY(hipMemcpyAsync(ranges, h->disp.totals + kTotBoundsGateUp, 2 * (kXcds + 1) * sizeof(int),
+                         hipMemcpyDeviceToDevice, static_cast<hipStream_t>(stream)));
   return MOE_OK;
 }
 

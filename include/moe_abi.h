@@ -179,6 +179,13 @@ int moe_dispatch(moe_handle *h, const int *topk_i, const int *pos, int n_tokens,
 int moe_get_dispatch(moe_handle *h, int *offsets, int *perm, int n_tokens,
                      void *stream);
 
+/* For tests: the tiles of the last dispatch.  ranges int [2][9] (device): in the
+ * tile sequence of the gate_up, then of the down GEMM, the first tile of each of
+ * the 8 XCDs, then the number of tiles.  MOE_ERR_STATE where the last call
+ * planned no tiles (the batches of stream_gemm_kernel, see moe_batch_kernel).
+ * Has no counterpart in the reference. */
+int moe_get_tile_ranges(moe_handle *h, int *ranges, void *stream);
+
 /* Everything after the router (dispatch, both GEMMs, combine) from
  * caller-supplied routing: the body of gpu_forward_device_batch_ep
  * (expert.cpp:1366), which reads d_t, d_topk_i, d_topk_v, d_pos and adds into

@@ -60,6 +60,7 @@ def test_null_arguments_are_errors_not_crashes():
     assert L.moe_forward(None, 0, None, None, 1, None, 0, None) == -1
     assert L.moe_router(None, 0, None, None, 1, None, None, None, None) == -1
     assert L.moe_dispatch(None, None, None, 1, None) == -1
+    assert L.moe_get_tile_ranges(None, None, None) == -1
     assert L.moe_experts(None, 0, None, None, None, None, 1, None, 0, None) == -1
     assert L.moe_upload_layer(None, 0, None, None, None, None, None, None) == -1
     assert L.moe_profile_enable(None, 1) == -1

@@ -233,7 +233,7 @@ WIDE = [(1024, 512), (1088, 576), (1216, 640)]
 
 @pytest.mark.parametrize("H,IM", WIDE)
 def test_wide_tiles(H, IM):
-    """Tiles of ten column blocks (up to 6 row blocks high, weights past the caches) beside
+    """Tiles of ten column blocks (up to 6 row blocks high, weights past the caches; the plan's tiles are counted) beside
     tiles of eight, every height, and their last column tiles: the bits of the MXFP4 kernels, whose tiles have
     eight, stage by stage and with an MXFP4 layer under a wide plan as well, and the oracle."""
     n, kinds = 256, 4  # experts of four kinds
@@ -257,9 +257,23 @@ def test_wide_tiles(H, IM):
     assert abi.batch_kernel(H, IM, n, T, False) == (BF16, 256, True)
     got = []
 
-    def staged(m, layer):
+    def tiles(tallest, narrow_only=False):
+        """of both GEMMs; 10 column blocks where they are up to 6 row blocks high, 8 elsewhere"""
+        counts = []
+        for nb in (2 * IM // 32, H // 32):
+            counts.append(0)
+            for b in (-(-r // 32) for r in rows):
+                n_mt = -(-b // tallest)
+                counts[-1] += n_mt * -(-nb // (8 if narrow_only or -(-b // n_mt) > 6 else 10))
+        return counts
+
+    wide = tiles(8)
+    assert (wide == tiles(8, narrow_only=True)) == (H == 1024)  # there 10 + 10 + 10 + 2 column blocks for four times 8
+
+    def staged(m, layer, planned):
         dout.memset(0xFF)
         m.dispatch(dti, None, T)
+        assert list(m.tile_ranges()[:, 8]) == planned
         m.expert_gemms(layer, dx, T)
         m.combine(dtv, None, T, dout)
         abi.sync()
@@ -267,15 +281,22 @@ def test_wide_tiles(H, IM):
 
     m = abi.Moe(H, IM, n, max_tokens=T, swiglu_limit=sh.limit, layers=2)
     m.upload_layer_mxfp4(1, wr, br, b1k, s1, b1, b2k, s2, b2)
-    staged(m, 1)  # no bf16 layer: not a wide plan
+    assert abi.batch_kernel(H, IM, n, T, True)[1] == 128
+    staged(m, 1, tiles(4, narrow_only=True))  # no bf16 layer: not a wide plan
     m.upload_layer(0, wr, br, np.tile(w1, (n // kinds, 1, 1)), b1, np.tile(w2, (n // kinds, 1, 1)), b2)
     for _ in range(3):
         dout.memset(0xFF)
         m.experts(0, dx, None, dti, dtv, T, dout)
         abi.sync()
         got.append(dout.download((T, H), np.float32))
+        assert list(m.tile_ranges()[:, 8]) == wide
     for layer in (0, 1):
-        staged(m, layer)
+        staged(m, layer, wide)
+    few = 4 * n  # 16 rows per expert: no tiles
+    m.experts(0, dx, None, dti, dtv, few, dout)
+    with pytest.raises(abi.MoeError) as e:
+        m.tile_ranges()
+    assert e.value.code == -5
     m.close()
     for other in got[1:]:
         assert np.array_equal(got[0], other)
