@@ -57,7 +57,7 @@ struct PlanOut {
   int tile_rb;  // row blocks of the tallest tile
   int nb[2];    // column blocks of an expert's matrices, gate_up and down (0: no tile tables)
   bool wide;    // tile_width
-  int tile_cost;  // fixed part of a tile's estimated cost
+  int tile_cost, tile_cost_few;  // TileCost
   // column tiles of GEMM g over an expert whose tallest tile has so many row blocks
   __device__ __forceinline__ int col_tiles(int g, int height) const {
     return tile_width(height, wide) == kGemmTileNb ? (nb[g] + kGemmTileNb - 1) / kGemmTileNb
@@ -121,8 +121,8 @@ __device__ __forceinline__ ExpertPlan build_plan(int count, int E, const PlanOut
                                                  int *ex_count_out, int *tot_count_out) {
   constexpr int kSums = 5, kSumsPlan = 2;  // the last ones are of the tile tables
   __shared__ int sh_wave[4][kSums];  // [wave][quantity]: the waves' sums
-  __shared__ int sh_cost[257];      // exclusive prefix of the experts' cost
-  __shared__ int sh_tiles[2][257];  // exclusive prefix of their tiles in either GEMM
+  __shared__ int sh_mt[257], sh_rb[257];  // exclusive prefixes of the experts' row tiles and row blocks
+  __shared__ int sh_tiles[2][257];        // ... and tiles in either GEMM
   __shared__ int sh_bound[2][kXcds + 1];
   const int e = threadIdx.x;
   const int lane = e & 63;
@@ -136,12 +136,10 @@ __device__ __forceinline__ ExpertPlan build_plan(int count, int E, const PlanOut
   const int height = rb + (extra ? 1 : 0);
   const bool tables = out.nb[0] > 0;
   const int n_up = n_mt * out.col_tiles(0, height), n_down = n_mt * out.col_tiles(1, height);
-  // cost of kGemmTileNb column blocks' worth of the expert's row tiles: of tiles of any width, whose cost goes by it
-  const int cost = n_mt * (out.tile_cost + kCostPerRowBlock * rb) + kCostPerRowBlock * extra;
   // Exclusive prefix sums over the experts of five quantities at once: rows,
-  // padded rows, cost, tiles of either GEMM.  In a wave by lane shifts, across the four
+  // padded rows, row tiles, tiles of either GEMM.  In a wave by lane shifts, across the four
   // waves through LDS.
-  const int own[kSums] = {count, n_rb * kRowBlock, cost, n_up, n_down};
+  const int own[kSums] = {count, n_rb * kRowBlock, n_mt, n_up, n_down};
   int incl[kSums];
 #pragma unroll
   for (int i = 0; i < kSums; i++) incl[i] = own[i];
@@ -172,8 +170,8 @@ __device__ __forceinline__ ExpertPlan build_plan(int count, int E, const PlanOut
     ex[i] = below + incl[i] - own[i];
     tot[i] = all;
   }
-  const int ex_count = ex[0], ex_pad = ex[1], ex_cost = ex[2];
-  const int tot_count = tot[0], tot_pad = tot[1], tot_cost = tot[2];
+  const int ex_count = ex[0], ex_pad = ex[1], ex_mt = ex[2];
+  const int tot_count = tot[0], tot_pad = tot[1], tot_mt = tot[2];
   const ExpertPlan mine = {ex_pad, n_mt, rb, extra, {ex[3], ex[4]}};
   *ex_count_out = ex_count;
   *tot_count_out = tot_count;
@@ -189,41 +187,58 @@ __device__ __forceinline__ ExpertPlan build_plan(int count, int E, const PlanOut
   // tokens 35.7 / 33.8).
   if (!write_global || !tables) return mine;  // (the same for the whole workgroup)
   if (e < 256) {
-    sh_cost[e] = ex_cost;
+    sh_mt[e] = ex_mt;
+    sh_rb[e] = ex_pad / kRowBlock;
     sh_tiles[0][e] = ex[3];
     sh_tiles[1][e] = ex[4];
   }
   if (e == 0) {
-    sh_cost[256] = tot_cost;
+    sh_mt[256] = tot_mt;
+    sh_rb[256] = tot_pad / kRowBlock;
     sh_tiles[0][256] = tot[3];
     sh_tiles[1][256] = tot[4];
   }
   __syncthreads();
-  // Thread (g, x): boundary x of GEMM g = first tile at which the cost so far
-  // reaches x/8 of the total (an expert's tiles taken as equally dear: their heights differ by one block at most).
-  if (e < 2 * (kXcds + 1)) {
-    const int g = e / (kXcds + 1), x = e % (kXcds + 1);
-    const int total_tiles = tot[3 + g];
-    int bound;
-    if (x == 0) {
-      bound = 0;
-    } else if (x == kXcds) {
-      bound = total_tiles;
-    } else {
-      const long long target = (long long)tot_cost * x;  // kXcds times the cost in front of the boundary
-      // last expert whose first tile starts at or before the target
-      int lo = 0, hi = 255;
-      while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if ((long long)sh_cost[mid] * kXcds <= target) lo = mid; else hi = mid - 1;
-      }
-      const int c_e = sh_cost[lo + 1] - sh_cost[lo];  // > 0: the search stops on an expert with tiles
-      const int n_e = sh_tiles[g][lo + 1] - sh_tiles[g][lo];
-      const long long rest = target - (long long)sh_cost[lo] * kXcds;  // of kXcds * c_e, the expert's share
-      bound = sh_tiles[g][lo] + (c_e ? min((int)((float)rest / ((float)c_e * kXcds) * (float)n_e), n_e) : 0);
-      bound = min(bound, total_tiles);
+  // Lane (c, g, x) of the first wave: boundary x of GEMM g = first tile at which the cost so far reaches x/8 of the
+  // total (an expert's tiles taken as equally dear: their heights differ by one block at most), with candidate c
+  // for the fixed part of a tile's cost.
+  if (w == 0) {
+    const int c = e >> 5, g = (e >> 4) & 1, x = min(e & 15, kXcds);
+    const int fixed = c ? out.tile_cost_few : out.tile_cost;
+    // cost of kGemmTileNb column blocks' worth of the row tiles of all lower experts: of tiles of any width, whose
+    // cost goes by it
+    auto cost_of = [&](int part, int i) { return part * sh_mt[i] + kCostPerRowBlock * sh_rb[i]; };
+    const int total_tiles = tot[3 + g], tot_cost = cost_of(fixed, 256);
+    const long long target = (long long)tot_cost * x;  // kXcds times the cost in front of the boundary
+    // last expert whose first tile starts at or before the target
+    int lo = 0, hi = 255;
+    while (lo < hi) {
+      const int mid = (lo + hi + 1) >> 1;
+      if ((long long)cost_of(fixed, mid) * kXcds <= target) lo = mid; else hi = mid - 1;
     }
-    sh_bound[g][x] = bound;
+    const int c_e = cost_of(fixed, lo + 1) - cost_of(fixed, lo);  // > 0 in front of the end: an expert with tiles
+    const int n_e = sh_tiles[g][lo + 1] - sh_tiles[g][lo];
+    const long long rest = target - (long long)cost_of(fixed, lo) * kXcds;  // of kXcds * c_e, the expert's share
+    int k = c_e ? min((int)((float)rest / ((float)c_e * kXcds) * (float)n_e), n_e) : 0;  // its tiles in front
+    int bound = sh_tiles[g][lo] + k;
+    if (x == kXcds) bound = total_tiles;
+    // Few rounds (see TileCost): the slowest XCD's time, as its rounds of tiles of its mean cost, decides.
+    bool few = false;
+    if (out.tile_cost_few && total_tiles <= kFewRounds * kCus) {
+      const float before = x == kXcds ? (float)cost_of(kFewRoundsCost, 256)
+                                      : (float)cost_of(kFewRoundsCost, lo) +
+                                            (n_e ? (float)k * (float)(cost_of(kFewRoundsCost, lo + 1) -
+                                                                      cost_of(kFewRoundsCost, lo)) / (float)n_e : 0.f);
+      const int n = __shfl_down(bound, 1, 16) - bound;
+      const float sum = __shfl_down(before, 1, 16) - before;
+      constexpr int kCusPerXcd = kCus / kXcds;
+      float time = (e & 15) < kXcds && n > 0 ? (float)((n + kCusPerXcd - 1) / kCusPerXcd) * sum / (float)n : 0.f;
+#pragma unroll
+      for (int off = 1; off < 16; off <<= 1) time = fmaxf(time, __shfl_xor(time, off, 16));
+      const float other = __shfl_xor(time, 32, 64);
+      few = (c ? time : other) < kFewRoundsGain * (c ? other : time);
+    }
+    if (c == (few ? 1 : 0) && (e & 15) <= kXcds) sh_bound[g][x] = bound;
   }
   __syncthreads();
   // keep every range within what the launch grid provides for (xcd_tile_cap)
@@ -254,7 +269,7 @@ __device__ __forceinline__ ExpertPlan build_plan(int count, int E, const PlanOut
 // the padded row space is its row blocks and no more, so an expert pads to at
 // most 31 rows.  The tile sequence of either GEMM (n_ct column tiles per row
 // tile) is cut into the 8 ranges of the XCDs by estimated cost: a tile of r row
-// blocks costs tile_cost + kCostPerRowBlock * r.
+// blocks costs tile_cost (or tile_cost_few) + kCostPerRowBlock * r.
 
 // Ranks inside one wave: for each of the lane's kTopK expert ids, how many of
 // the wave's assignments to the same expert come before it in (lane, slot)
@@ -547,7 +562,7 @@ __global__ __launch_bounds__(256) void combine_kernel(const float *__restrict__ 
 }
 
 hipError_t launch_dispatch(const int *topk_i, const int *pos, int T, int E, int nb_gate_up, int nb_down,
-                           int tile_rows, bool wide, int tile_cost, const DispatchBuffers &d, hipStream_t s) {
+                           int tile_rows, bool wide, TileCost tile_cost, const DispatchBuffers &d, hipStream_t s) {
   const int n_blk = (T + kDispThreads - 1) / kDispThreads;
   // Rows of the padded space this batch can reach: every expert rounds its
   // rows up to a multiple of 32.
@@ -565,7 +580,8 @@ hipError_t launch_dispatch(const int *topk_i, const int *pos, int T, int E, int 
   plan.nb[0] = nb_gate_up;
   plan.nb[1] = nb_down;
   plan.wide = wide;
-  plan.tile_cost = tile_cost;
+  plan.tile_cost = tile_cost.fixed;
+  plan.tile_cost_few = tile_cost.few;
   // ids are compared in as many bits as the experts have
 #define MOE_BY_EXPERTS(LAUNCH)  \
   do {                          \
@@ -694,7 +710,8 @@ extern "C" int moe_dispatch_static(const int *topk_i, const int *pos, int n_toke
   // no GEMM follows: with no column tiles the plan kernel writes no tile tables
   d.tiles_gate_up = d.tiles_down = nullptr;
   d.tile_cap_gate_up = d.tile_cap_down = 0;
-  const hipError_t el = launch_dispatch(topk_i, pos, n_tokens, n_experts, 0, 0, kTileRows, false, 0, d, static_cast<hipStream_t>(stream));
+  const hipError_t el = launch_dispatch(topk_i, pos, n_tokens, n_experts, 0, 0, kTileRows, false, TileCost{0, 0}, d,
+                                       static_cast<hipStream_t>(stream));
   if (el != hipSuccess)
     return set_error(MOE_ERR_HIP, "dispatch launch failed: %s", hipGetErrorString(el));
   return MOE_OK;

@@ -157,11 +157,10 @@ int run_dispatch(moe_handle *h, const int *topk_i, const int *pos, int T, bool m
   // the kernels of stream.hip go by row blocks and need no tile tables
   const bool tables = !stream_batch(T, E);
   h->plan_tiles = tables;
-  h->plan_wide = tables && !mxfp4 &&
-                 bf16_wide_tiles(T, E, h->Hp, h->IMp,
-                                 gemm_streams_weights(T, E, false, h->plan_rows, h->expert_bytes <= kCachedWeightBytes));
+  const bool past_caches = gemm_streams_weights(T, E, mxfp4, h->plan_rows, h->expert_bytes <= kCachedWeightBytes);
+  h->plan_wide = tables && !mxfp4 && bf16_wide_tiles(T, E, h->Hp, h->IMp, past_caches);
   HIP_TRY(launch_dispatch(topk_i, pos, T, E, tables ? 2 * h->IMp / kRowBlock : 0, tables ? h->Hp / kRowBlock : 0,
-                          h->plan_rows, h->plan_wide, plan_tile_cost(T, E, 2 * h->IMp, mxfp4), h->disp, s));
+                          h->plan_rows, h->plan_wide, plan_tile_cost(T, E, 2 * h->IMp, mxfp4, past_caches), h->disp, s));
   return MOE_OK;
 }
 

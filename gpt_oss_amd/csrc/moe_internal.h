@@ -154,10 +154,15 @@ struct DispatchBuffers {
   TileDesc *tiles_down;     // [tile_cap_down]    ... of the down GEMM
   int tile_cap_gate_up, tile_cap_down;
 };
-// tile_rows: tallest row tile of the plan (kTileRows or kHalfTileRows); wide: tile_width; tile_cost: fixed part of a
-// tile's estimated cost; nb_*: column blocks of an expert's matrices (0: no tile tables)
+// Fixed part of a tile's estimated cost (plan_tile_cost), and another (0: none) that a GEMM of few rounds of tiles may
+// be cut by instead.
+struct TileCost {
+  int fixed, few;
+};
+// tile_rows: tallest row tile of the plan (kTileRows or kHalfTileRows); wide: tile_width; nb_*: column blocks of an
+// expert's matrices (0: no tile tables)
 hipError_t launch_dispatch(const int *topk_i, const int *pos, int T, int E, int nb_gate_up, int nb_down,
-                           int tile_rows, bool wide, int tile_cost, const DispatchBuffers &d, hipStream_t s);
+                           int tile_rows, bool wide, TileCost tile_cost, const DispatchBuffers &d, hipStream_t s);
 
 // Batches of at most kDirectTokens tokens run without a dispatch pass: the 256
 // threads of a workgroup hold one assignment each, so every workgroup of the
@@ -299,16 +304,31 @@ inline int plan_tile_rows(int T, int E, int H, int IM, bool mxfp4, bool cached) 
 }
 // Fixed part of a tile's estimated cost, by which the XCDs' ranges are cut.  It stands for the column
 // operand, which a tile streams in full however few rows it has: 8 row blocks' worth with bf16 weights, one
-// and a half with MXFP4, which are a quarter of the bytes, and four in the kernels of many rows.  us per layer call,
-// Zipf's routing of exponent 1.2 (* 0.6) at 2880 x 2880, fixed part 32 / 64 / 96 with bf16: 128 experts, 1000 tokens
-// 1012 / 984 / 989, 2000 1299 / 1215 / 1206, 4000* 1479 / 1416 / 1409, 6144 1995 / 1842 / 1856; 32 experts, 400 333 /
-// 340 / 339, 600* 337 / 346 / 345, 700 387 / 363 / 373, 1000 436 / 412 / 411, 1400* 429 / 410 / 414, 3000 683 / 663 /
-// 670, 7168 1306 / 1292 / 1297; 8 experts, 400 174 / 150 / 150; even routing at 4096 tokens 775 / 778 / 776.
-// 4 / 12 / 20 / 32 with MXFP4: gemm.hip, 128 experts, 1000 tokens 463 / 436 / 462 / 492, 2000 639 / 613 / 636 / 670, 32
-// experts, 300* 168 / 151 / 166 / 167; gemm_fp4.hip, 32 experts, 512 195 / 183 / 184 / 184, 2000* 400 / 390 / 389 /
-// 390, 7168 1168 / 1162 / 1156 / 1165; even routing, 724 194 with 12, 190 with 32, 1000 242 / 252 / 245 / 246.
-inline int plan_tile_cost(int T, int E, int w1_rows, bool mxfp4) {
-  return !mxfp4 ? 64 : (fp4_many_rows(T, E, w1_rows) ? 32 : 12);
+// and a half with MXFP4, which are a quarter of the bytes, and four in the kernels of many rows.  us per moe_experts
+// call, means of two to four routings, even or Zipf's (exponent in brackets), 2880 x 2880 unless stated.  bf16, 32 / 64:
+// 128 experts, 600 tokens (1.2) 895 / 842, 1000 (0.6) 1075 / 1053, 2000 (1.2) 1270 / 1188, 4000 (1.2) 1598 / 1500, even
+// 1164 / 1164; 32 experts, 200 (0.6) 297 / 276, 600 (1.2) 362 / 339, 1000 412 / 394, 1400 457 / 431, even, 256 289 /
+// 277, 1000 321 / 313; 8 experts, 400 (1.2) 161 / 153.  Matrices that the caches hold: 512 x 512, 32 experts, 1000
+// (1.2; tiles of 128 rows) 34.8 / 33.8, 3000, even, 55.5 / 52.6, (1.2) 54.9 / 55.8; 1024 x 1024, 3000, even, 124 / 119;
+// 4 experts, 600 (128 rows) 134 / 134.  MXFP4, 12 / 32: tiles of 256 rows, 8 experts, 128 (1.2) 68.3 / 69.1, 250 104.4 /
+// 104.6, even 81.3 / 81.6; gemm.hip with 128, 32 experts, 200 (1.2) 128 / 147, 300 (0.6) 124 / 147, even 124.8 / 125.5;
+// 128 experts, 1000 (1.2) 411 / 462, 2000 575 / 629, even, 600 326 / 324, 1000 383 / 378, 2000 491 / 497.
+// gemm_fp4.hip, 12 / 20 / 32: 32 experts, 512 (1.2) 183 / 184 / 184, 2000 (0.6) 390 / 389 / 390, 7168 (1.2) 1162 /
+// 1156 / 1165, even, 1000 252 / 245 / 246.
+//
+// Few rounds, bf16 past the caches: an XCD that gets one tile more than its CUs take at a time begins another
+// round, which a cut by cost does not see.  With 64 an XCD of tall tiles had 35 to 40 of the down GEMM's at 32 experts,
+// 350 to 500 tokens (1.2), with 32 no more than its 32, and the others 60 of low ones.  So a GEMM of up to two rounds of
+// tiles is cut by 32 where the slowest XCD's time (its rounds times its tiles' mean cost, with a fixed part of 96: 64 to
+// 128 predict the measured times best) is estimated 2 % lower.  us per call, 64 throughout / this: 32 experts, 256
+// (1.2) 307 / 298, 350 317 / 305, 400 325 / 311, 450 337 / 315, 480 338 / 319, 560 (0.6) 326 / 318; 16 experts, 200 (1.2)
+// 175 / 167; 32 experts of 2048 x 1440, 400 (1.2) 143 / 136.  Over 396 batches of 8 to 128 experts, 100 to 7000 tokens, no
+// GEMM that this cuts by 32 was slower by more than 1 %; without the 2 % or with more rounds some were, by 2 to 10.
+constexpr int kFewRounds = 2, kFewRoundsCost = 96;
+constexpr float kFewRoundsGain = 0.98f;
+inline TileCost plan_tile_cost(int T, int E, int w1_rows, bool mxfp4, bool past_caches) {
+  if (mxfp4) return {fp4_many_rows(T, E, w1_rows) ? 32 : 12, 0};
+  return {64, past_caches ? 32 : 0};
 }
 enum TileKernel { kBf16Tiles /* gemm_bf16.hip */, kFp4Tiles /* gemm.hip */, kFp4ManyTiles /* gemm_fp4.hip */ };
 struct TileRoute {

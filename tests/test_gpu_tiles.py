@@ -311,3 +311,60 @@ def test_wide_tiles(H, IM):
     d = got[0][some] - want
     assert np.abs(d).max() <= 2e-2 * max(1.0, float(np.abs(want).max()))
     assert np.linalg.norm(d) <= 1e-3 * np.linalg.norm(want)
+
+
+def _cut(rows, tile_rb, nb, fixed):
+    """First tiles of the XCDs' ranges, and the estimated time of the slowest, in fp32 as the plan kernel works it out."""
+    f = np.float32
+    n_rb = (rows + 31) // 32
+    n_mt = -(-n_rb // tile_rb)
+    mt, rb, tiles = (np.concatenate([[0], np.cumsum(a)]) for a in (n_mt, n_rb, n_mt * -(-nb // 8)))
+    cost, slow = fixed * mt + 8 * rb, 96 * mt + 8 * rb
+    bounds, before = [], []
+    for x in range(8):
+        lo = int(np.nonzero(cost[:-1] * 8 <= cost[-1] * x)[0][-1])
+        c, n = cost[lo + 1] - cost[lo], tiles[lo + 1] - tiles[lo]
+        k = min(int(f(cost[-1] * x - cost[lo] * 8) / (f(c) * f(8)) * f(n)), n) if c else 0
+        bounds.append(int(tiles[lo] + k))
+        before.append(f(slow[lo]) + (f(k) * f(slow[lo + 1] - slow[lo]) / f(n) if n else f(0)))
+    bounds.append(int(tiles[-1]))
+    before.append(f(slow[-1]))
+    time = max([f(-(-n // 32)) * (b - a) / f(n) for n, a, b in zip(np.diff(bounds), before, before[1:]) if n > 0], default=f(0))
+    cap = (bounds[8] + 7) // 8 + (bounds[8] + 15) // 16 + 1
+    for x in range(1, 8):
+        bounds[x] = min(max(bounds[x], bounds[x - 1], bounds[8] - (8 - x) * cap), bounds[x - 1] + cap)
+    return bounds, time
+
+
+@pytest.mark.parametrize("H,IM,past", [(2880, 512, True), (2880, 384, False), (1984, 768, True)])
+def test_ranges_of_the_xcds(H, IM, past):
+    """The cut of either GEMM's tiles into the XCDs' ranges against the rule in numpy: by cost, and with few
+    rounds of tiles and weights past the caches by the one of two costs whose slowest XCD is expected to be
+    quicker by 2 %; popularities even and uneven, experts without rows, one expert alone."""
+    E, top = 32, 700
+    m = abi.Moe(H, IM, E, max_tokens=top)
+    z = np.zeros
+    m.upload_layer(0, z((E, H)), z(E), z((E, 2 * IM, H), np.float32), z((E, 2 * IM)), z((E, H, IM), np.float32), z((E, H)))
+    rng = np.random.default_rng(H + IM)
+    chosen = [0, 0]
+    for T in (129, 150, 200, 256, 300, 350, 400, 450, 480, 512, 600, 700):
+        kernel, tile_rows, streams = abi.batch_kernel(H, IM, E, T, False)
+        assert kernel == BF16 and streams == past
+        for exponent in (0.0, 0.6, 1.2, 1.2, 2.0, None):
+            if exponent is None:
+                ids = np.full((T, 4), 7, np.int32)
+                ids[:, 1:] = -1
+            else:
+                keys = rng.gumbel(size=(T, E)) + 0.65 / 0.78 * np.log(synth.zipf_popularity(E, exponent))
+                ids = np.argsort(-keys, axis=1)[:, :4].astype(np.int32)
+            rows = np.bincount(ids[ids >= 0], minlength=E)
+            m.dispatch(abi.DevBuf.from_numpy(ids), None, T)
+            got = m.tile_ranges()
+            for g, nb in enumerate((2 * IM // 32, H // 32)):
+                (by_64, slow_64), (by_32, slow_32) = (_cut(rows, tile_rows // 32, nb, fixed) for fixed in (64, 32))
+                few = past and by_64[8] <= 512 and slow_32 < np.float32(0.98) * slow_64
+                if abs(slow_32 - np.float32(0.98) * slow_64) > 1e-5 * slow_64:
+                    assert list(got[g]) == (by_32 if few else by_64), (T, exponent, g)
+                    chosen[int(few)] += 1
+    m.close()
+    assert chosen[0] and bool(chosen[1]) == past
