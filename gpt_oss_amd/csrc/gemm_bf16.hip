@@ -119,7 +119,7 @@ struct Tile {
 // it and is not stored) times NU units of columns.  A unit is what ends as 32 columns of down (a column
 // block) or 16 of the activation (half a pair of gate and up blocks): units 2 wn and 2 wn + 1, and with
 // NU = 3 unit 8 + wx.  LA: its loads of rows per double step, LB: of columns per step.
-template <int RBW, int LA, int S, int NU, int LB, typename R, bool GATE_UP, bool STREAM>
+template <int RBW, int LA, int S, int NU, int LB, typename R, bool GATE_UP, bool STREAM, bool PAST>
 __device__ __forceinline__ void wave_tile(const Tile &t, uint32_t lds0) {
   constexpr int NC = 2 * NU;  // groups of 16 columns: gate_up: the units' gates, then their ups; down: the units' halves
   const int tid = threadIdx.x, lane = tid & 63;
@@ -367,7 +367,7 @@ __device__ __forceinline__ void wave_tile(const Tile &t, uint32_t lds0) {
                                    swiglu_shifted(acc[2 * i + h][j][2 * d + 1], acc[2 * i + h][j + NU][2 * d + 1], t.limit));
           const u32x2 s0 = __builtin_amdgcn_permlane16_swap(pk[0][0], pk[1][0], false, false);
           const u32x2 s1 = __builtin_amdgcn_permlane16_swap(pk[0][1], pk[1][1], false, false);
-          store_output<STREAM>(&dst[unit(j) * 64], u32x4{s0[0], s1[0], s0[1], s1[1]});
+          store_output<PAST>(&dst[unit(j) * 64], u32x4{s0[0], s1[0], s0[1], s1[1]});
         }
       }
     } else {
@@ -389,8 +389,8 @@ __device__ __forceinline__ void wave_tile(const Tile &t, uint32_t lds0) {
               const f32x4 u = acc[2 * i + h][2 * j], v = acc[2 * i + h][2 * j + 1];
               const u32x2 x = __builtin_amdgcn_permlane16_swap(__float_as_uint(u[q]), __float_as_uint(v[q]), false, false);
               float *dst = y + ((size_t)(t.rb0 + blk) * kRowBlock + 16 * h + row + q) * t.N + col + kRowBlock * unit(j);
-              store_output<STREAM>(dst, __uint_as_float(x[0]));
-              store_output<STREAM>(dst + 4 * (size_t)t.N, __uint_as_float(x[1]));
+              store_output<PAST>(dst, __uint_as_float(x[0]));
+              store_output<PAST>(dst + 4 * (size_t)t.N, __uint_as_float(x[1]));
             }
       }
     }
@@ -398,19 +398,19 @@ __device__ __forceinline__ void wave_tile(const Tile &t, uint32_t lds0) {
 }
 
 // A tile whose row blocks two waves split: rbw of them, MAX at most, are this one's.
-template <int MAX, int NU, int LB, typename R, bool GATE_UP, bool STREAM>
+template <int MAX, int NU, int LB, typename R, bool GATE_UP, bool STREAM, bool PAST>
 __device__ __forceinline__ void split_rows(const Tile &t, uint32_t lds0, int rbw) {
   switch (rbw) {
-    case 0: wave_tile<0, 0, 2, NU, LB, R, GATE_UP, STREAM>(t, lds0); break;
-    case 1: wave_tile<1, 1, 2, NU, LB, R, GATE_UP, STREAM>(t, lds0); break;
-    case 2: wave_tile<2, 2, 2, NU, LB, R, GATE_UP, STREAM>(t, lds0); break;
-    case MAX: wave_tile<MAX, MAX, 2, NU, LB, R, GATE_UP, STREAM>(t, lds0); break;
+    case 0: wave_tile<0, 0, 2, NU, LB, R, GATE_UP, STREAM, PAST>(t, lds0); break;
+    case 1: wave_tile<1, 1, 2, NU, LB, R, GATE_UP, STREAM, PAST>(t, lds0); break;
+    case 2: wave_tile<2, 2, 2, NU, LB, R, GATE_UP, STREAM, PAST>(t, lds0); break;
+    case MAX: wave_tile<MAX, MAX, 2, NU, LB, R, GATE_UP, STREAM, PAST>(t, lds0); break;
     default:
-      if constexpr (MAX > 3) wave_tile<3, 3, 2, NU, LB, R, GATE_UP, STREAM>(t, lds0);
+      if constexpr (MAX > 3) wave_tile<3, 3, 2, NU, LB, R, GATE_UP, STREAM, PAST>(t, lds0);
   }
 }
 
-template <bool GATE_UP, bool STREAM>
+template <bool GATE_UP, bool STREAM, bool PAST>
 __global__ __launch_bounds__(kThreads, 2) void bf16_gemm_kernel(const char *__restrict__ a, const char *__restrict__ wt,
                                                            const float *__restrict__ ba, const float *__restrict__ bb,
                                                            const TileDesc *__restrict__ tiles,
@@ -441,25 +441,25 @@ __global__ __launch_bounds__(kThreads, 2) void bf16_gemm_kernel(const char *__re
   t.limit = limit;
   const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int rbw = (t.rbt + 1 - (w >> 2)) >> 1;  // the wave's row blocks where the waves split them in two
-  if constexpr (STREAM) {
-    if (t.nb_valid > kGemmTileNb) {  // plans for these loads only (bf16_wide_tiles)
+  if constexpr (STREAM && PAST) {
+    if (t.nb_valid > kGemmTileNb) {  // plans for these loads and stores only (bf16_wide_tiles)
       switch (w >> 1) {
-        case 0: split_rows<3, 3, 3, Wide, GATE_UP, STREAM>(t, lds0, rbw); break;
-        case 1: split_rows<3, 2, 3, Wide, GATE_UP, STREAM>(t, lds0, rbw); break;
-        case 2: split_rows<3, 2, 2, Wide, GATE_UP, STREAM>(t, lds0, rbw); break;
-        default: split_rows<3, 3, 2, Wide, GATE_UP, STREAM>(t, lds0, rbw); break;
+        case 0: split_rows<3, 3, 3, Wide, GATE_UP, STREAM, PAST>(t, lds0, rbw); break;
+        case 1: split_rows<3, 2, 3, Wide, GATE_UP, STREAM, PAST>(t, lds0, rbw); break;
+        case 2: split_rows<3, 2, 2, Wide, GATE_UP, STREAM, PAST>(t, lds0, rbw); break;
+        default: split_rows<3, 3, 2, Wide, GATE_UP, STREAM, PAST>(t, lds0, rbw); break;
       }
       return;
     }
   }
   if (t.nb_valid > 4) {
-    split_rows<4, 2, 2, Square, GATE_UP, STREAM>(t, lds0, rbw);
+    split_rows<4, 2, 2, Square, GATE_UP, STREAM, PAST>(t, lds0, rbw);
   } else if (t.nb_valid > 2) {
-    if (t.rbt <= 4) wave_tile<1, 2, 4, 2, 2, Square, GATE_UP, STREAM>(t, lds0);
-    else wave_tile<2, 4, 4, 2, 2, Square, GATE_UP, STREAM>(t, lds0);
+    if (t.rbt <= 4) wave_tile<1, 2, 4, 2, 2, Square, GATE_UP, STREAM, PAST>(t, lds0);
+    else wave_tile<2, 4, 4, 2, 2, Square, GATE_UP, STREAM, PAST>(t, lds0);
   } else {
-    if (t.rbt <= 4) wave_tile<1, 2, 8, 2, 2, Square, GATE_UP, STREAM>(t, lds0);
-    else wave_tile<1, 4, 8, 2, 2, Square, GATE_UP, STREAM>(t, lds0);
+    if (t.rbt <= 4) wave_tile<1, 2, 8, 2, 2, Square, GATE_UP, STREAM, PAST>(t, lds0);
+    else wave_tile<1, 4, 8, 2, 2, Square, GATE_UP, STREAM, PAST>(t, lds0);
   }
 }
 
@@ -471,10 +471,13 @@ hipError_t launch(const void *a, const void *w, const float *ba, const float *bb
   const int grid = kXcds * xcd_tile_cap(gemm_tile_cap(T, E, tile_rows) * n_ct);
   const TileDesc *tiles = GATE_UP ? d.tiles_gate_up : d.tiles_down;
   const char *ac = static_cast<const char *>(a), *wc = static_cast<const char *>(w);
-  if (stream || wide)
-    bf16_gemm_kernel<GATE_UP, true><<<grid, kThreads, 0, s>>>(ac, wc, ba, bb, tiles, d.totals, d.rowmap, out, K, N, limit);
-  else
-    bf16_gemm_kernel<GATE_UP, false><<<grid, kThreads, 0, s>>>(ac, wc, ba, bb, tiles, d.totals, d.rowmap, out, K, N, limit);
+#define MOE_GEMM(STREAM, PAST)                                                                                   \
+  bf16_gemm_kernel<GATE_UP, STREAM, PAST><<<grid, kThreads, 0, s>>>(ac, wc, ba, bb, tiles, d.totals, d.rowmap, out, K, \
+                                                                    N, limit)
+  if (wide || (stream && bf16_stores_past(GATE_UP, E * n_ct, T, E))) MOE_GEMM(true, true);
+  else if (stream) MOE_GEMM(true, false);
+  else MOE_GEMM(false, false);
+#undef MOE_GEMM
   return hipGetLastError();
 }
 

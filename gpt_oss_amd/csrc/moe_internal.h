@@ -298,6 +298,17 @@ inline bool bf16_wide_tiles(int T, int E, int H, int IM, bool past_caches) {
   const int row_tiles = T * kTopK / kTileRows > E ? T * kTopK / kTileRows : E;
   return past_caches && (long long)row_tiles * ((cols + kWideTileNb - 1) / kWideTileNb) >= 4 * kCus;
 }
+// bf16 weights past the caches: whether the rows that a GEMM stores go past them as well (store_output has what that
+// gains).  Not where few rows are stored and the GEMM is over after a round or two: its end then waits for them and the
+// kernel behind would have found them in the caches.  us per moe_experts call, even routing, past / through, gate_up: 16
+// experts, 2880 x 2880 (368 tiles), 100 tokens (25 rows) 148.5 / 145.1, 150 155.4 / 153.0, 200 155.0 / 154.2, 300 (75)
+// 162 / 171; 20 experts (460 tiles), 90 (18) 164 / 162, 150 (30) 168.9 / 167.6, 200 (40) 169.8 / 172.1; 32 experts, 2048 x 1440 (384 tiles), 150 (19) 111.7 / 108.7, 300 (37) 130.2 / 128.4, 500 (62) 135 / 138; 2880 x
+// 2880 (736 tiles), 150 265.5 / 266.3, 400 273 / 293; 8 experts (184 tiles), 70 to 500 within 0.5 %.  Down: 16 experts
+// (192 tiles), 150 155.4 / 151.6, 200 155.0 / 152.0, 600 188.0 / 188.0; 32 experts of 2048 x 1440 (256 tiles), 300
+// 130.2 / 128.7, 500 135.0 / 135.6; 2880 x 2880 (384 tiles), 150 265.5 / 267.8, 400 273 / 278.
+inline bool bf16_stores_past(bool gate_up, int tiles, int T, int E) {
+  return gate_up ? tiles >= 2 * kCus || T * kTopK > 36 * E : tiles > kCus || T * kTopK > 64 * E;
+}
 // Row tiles of a plan, and what runs on it.
 inline int plan_tile_rows(int T, int E, int H, int IM, bool mxfp4, bool cached) {
   return (mxfp4 ? half_tiles(T, E, 2 * IM) : bf16_half_tiles(T, E, H, IM, cached)) ? kHalfTileRows : kTileRows;

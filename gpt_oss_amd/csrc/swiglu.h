@@ -24,17 +24,17 @@ __device__ __forceinline__ uint32_t pack_bf16(float a, float b) {
   return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2));
 }
 
-// A store of a GEMM's output.  STREAM: past the caches, where the weights are read past them
-// (gemm_streams_weights).  Written through L2 the output pushes out the rows that the tiles beside this one read,
+// A store of a GEMM's output.  PAST: past the caches, where the weights are read past them
+// (gemm_streams_weights; bf16_stores_past has where not).  Written through L2 the output pushes out the rows that the tiles beside this one read,
 // and its eviction gets in the way of the weights' stream.  us per GEMM (gate_up + down), plain stores / these:
 // gemm_bf16.hip, 2880 x 2880, 896 tokens (672 active) at 32 experts 198 + 118 / 174 + 110, 6144 tokens at
 // 128 experts 979 + 562 / 918 + 520 (the combine, which then reads from HBM, 66 / 72); gemm.hip, MXFP4, 800
 // tokens at 128 experts 228 + 138 / 205 + 126, 256 at 32 experts 67 + 45 / 65 + 42.  Where the matrix cores are the time
 // they gain nothing and the combine loses (4096 tokens at 32 experts 797 / 802 us per call), nor do
 // they gain in gemm_fp4.hip (3000 tokens at 128 experts 615 / 620) and in stream.hip (64 tokens, MXFP4, 91 / 94).
-template <bool STREAM, typename V>
+template <bool PAST, typename V>
 __device__ __forceinline__ void store_output(V *p, V v) {
-  if constexpr (STREAM) __builtin_nontemporal_store(v, p);
+  if constexpr (PAST) __builtin_nontemporal_store(v, p);
   else *p = v;
 }
 

@@ -17,15 +17,28 @@ pytestmark = pytest.mark.gpu
 E = 32
 FEW = (1, 31, 32, 33, 63, 64, 65, 95, 96, 97, 127, 128, 129, 160, 161, 256, 257)  # 1795 rows: 56 per expert
 MANY = FEW + (255, 288, 383, 384, 385, 512, 513, 640, 800, 1024)  # 6979 rows: 218 per expert
+LOW = (1, 31, 32, 33, 65, 97, 129, 161, 193, 256)  # 998 rows: 31 per expert
 BF16, FP4, FP4_MANY = "bf16_gemm_kernel", "grouped_gemm_kernel", "fp4_gemm_kernel"
 # kernel, rows of a tile, past the caches: MXFP4 and bf16 weights that the caches hold, then that they do not
 ROUTES = {FEW: [(FP4, 128, False), (BF16, 256, False), (FP4, 128, True), (BF16, 256, True)],
+          LOW: [(FP4, 256, False), (BF16, 256, False), (FP4, 256, False), (BF16, 256, True)],
           MANY: [(FP4_MANY, 128, False), (BF16, 128, False), (FP4_MANY, 128, False), (BF16, 256, True)]}
 
 
 @pytest.mark.parametrize("rows", [FEW, MANY], ids=["few", "many"])
 @pytest.mark.parametrize("H,IM", [(64, 2048), (128, 2112), (192, 2080)])
 def test_row_tiles(rows, H, IM):
+    check_row_tiles(rows, H, IM)
+
+
+@pytest.mark.parametrize("H,IM", [(64, 1024), (128, 1088), (192, 992)])
+def test_row_tiles_of_few_rounds(H, IM):
+    """Few rows per expert and less than two rounds of tiles: bf16 weights past the caches, the rows
+    that the GEMMs store through them (bf16_stores_past)."""
+    check_row_tiles(LOW, H, IM)
+
+
+def check_row_tiles(rows, H, IM):
     rng = np.random.default_rng(H + len(rows))
     experts = rng.permutation(E)[:len(rows)]
     ids = np.repeat(experts, rows).astype(np.int32)

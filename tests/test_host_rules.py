@@ -11,6 +11,7 @@ SOURCE = """
 #include "%s/moe_internal.h"
 extern "C" int split_router_tokens(int E_pad, int H) { return moe::split_router_tokens(E_pad, H); }
 extern "C" int bf16_wide_tiles(int T, int E, int H, int IM, int past) { return moe::bf16_wide_tiles(T, E, H, IM, past); }
+extern "C" int bf16_stores_past(int gate_up, int tiles, int T, int E) { return moe::bf16_stores_past(gate_up, tiles, T, E); }
 extern "C" int norm_wave_per_token(int T, int H) { return moe::norm_wave_per_token(T, H); }
 """ % build.CSRC
 
@@ -49,3 +50,11 @@ def test_norm_of_short_rows_takes_a_wave(rules, T, H, wave):
 def test_wide_tiles_where_the_cus_take_many_rounds(rules, T, E, H, IM, past, wide):
     """Tiles of ten column blocks gain with four rounds of tiles and lose with two (times in moe_internal.h)."""
     assert rules.bf16_wide_tiles(T, E, H, IM, past) == wide
+
+
+@pytest.mark.parametrize("gate_up,tiles,T,E,past", [
+    (1, 368, 144, 16, 0), (1, 368, 145, 16, 1), (1, 512, 144, 16, 1), (1, 736, 150, 32, 1), (1, 256, 250, 32, 0), (1, 460, 200, 20, 1),
+    (0, 192, 256, 16, 0), (0, 192, 257, 16, 1), (0, 256, 300, 32, 0), (0, 257, 300, 32, 1), (0, 384, 150, 32, 1), (0, 32, 449, 32, 0)])
+def test_stores_past_the_caches_where_they_gain(rules, gate_up, tiles, T, E, past):
+    """Few rows of a GEMM of a round or two are found in the caches by the next kernel (times in moe_internal.h)."""
+    assert rules.bf16_stores_past(gate_up, tiles, T, E) == past
