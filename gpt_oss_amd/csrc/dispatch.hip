@@ -57,7 +57,7 @@ struct PlanOut {
   int tile_rb;  // row blocks of the tallest tile
   int nb[2];    // column blocks of an expert's matrices, gate_up and down (0: no tile tables)
   bool wide;    // tile_width
-  int tile_cost, tile_cost_few;  // TileCost
+  TileCost cost;
   // column tiles of GEMM g over an expert whose tallest tile has so many row blocks
   __device__ __forceinline__ int col_tiles(int g, int height) const {
     return tile_width(height, wide) == kGemmTileNb ? (nb[g] + kGemmTileNb - 1) / kGemmTileNb
@@ -204,7 +204,7 @@ __device__ __forceinline__ ExpertPlan build_plan(int count, int E, const PlanOut
   // for the fixed part of a tile's cost.
   if (w == 0) {
     const int c = e >> 5, g = (e >> 4) & 1, x = min(e & 15, kXcds);
-    const int fixed = c ? out.tile_cost_few : out.tile_cost;
+    const int fixed = c ? out.cost.few : out.cost.fixed;
     // cost of kGemmTileNb column blocks' worth of the row tiles of all lower experts: of tiles of any width, whose
     // cost goes by it
     auto cost_of = [&](int part, int i) { return part * sh_mt[i] + kCostPerRowBlock * sh_rb[i]; };
@@ -224,11 +224,12 @@ __device__ __forceinline__ ExpertPlan build_plan(int count, int E, const PlanOut
     if (x == kXcds) bound = total_tiles;
     // Few rounds (see TileCost): the slowest XCD's time, as its rounds of tiles of its mean cost, decides.
     bool few = false;
-    if (out.tile_cost_few && total_tiles <= kFewRounds * kCus) {
-      const float before = x == kXcds ? (float)cost_of(kFewRoundsCost, 256)
-                                      : (float)cost_of(kFewRoundsCost, lo) +
-                                            (n_e ? (float)k * (float)(cost_of(kFewRoundsCost, lo + 1) -
-                                                                      cost_of(kFewRoundsCost, lo)) / (float)n_e : 0.f);
+    if (out.cost.few && total_tiles <= out.cost.rounds * kCus) {
+      const int slow = out.cost.slow;
+      const float before = x == kXcds ? (float)cost_of(slow, 256)
+                                      : (float)cost_of(slow, lo) +
+                                            (n_e ? (float)k * (float)(cost_of(slow, lo + 1) - cost_of(slow, lo)) / (float)n_e
+                                                 : 0.f);
       const int n = __shfl_down(bound, 1, 16) - bound;
       const float sum = __shfl_down(before, 1, 16) - before;
       constexpr int kCusPerXcd = kCus / kXcds;
@@ -236,7 +237,7 @@ __device__ __forceinline__ ExpertPlan build_plan(int count, int E, const PlanOut
 #pragma unroll
       for (int off = 1; off < 16; off <<= 1) time = fmaxf(time, __shfl_xor(time, off, 16));
       const float other = __shfl_xor(time, 32, 64);
-      few = (c ? time : other) < kFewRoundsGain * (c ? other : time);
+      few = (c ? time : other) < out.cost.gain * (c ? other : time);
     }
     if (c == (few ? 1 : 0) && (e & 15) <= kXcds) sh_bound[g][x] = bound;
   }
@@ -269,7 +270,7 @@ __device__ __forceinline__ ExpertPlan build_plan(int count, int E, const PlanOut
 // the padded row space is its row blocks and no more, so an expert pads to at
 // most 31 rows.  The tile sequence of either GEMM (n_ct column tiles per row
 // tile) is cut into the 8 ranges of the XCDs by estimated cost: a tile of r row
-// blocks costs tile_cost (or tile_cost_few) + kCostPerRowBlock * r.
+// blocks costs TileCost's fixed part + kCostPerRowBlock * r.
 
 // Ranks inside one wave: for each of the lane's kTopK expert ids, how many of
 // the wave's assignments to the same expert come before it in (lane, slot)
@@ -580,8 +581,7 @@ hipError_t launch_dispatch(const int *topk_i, const int *pos, int T, int E, int 
   plan.nb[0] = nb_gate_up;
   plan.nb[1] = nb_down;
   plan.wide = wide;
-  plan.tile_cost = tile_cost.fixed;
-  plan.tile_cost_few = tile_cost.few;
+  plan.cost = tile_cost;
   // ids are compared in as many bits as the experts have
 #define MOE_BY_EXPERTS(LAUNCH)  \
   do {                          \
@@ -710,7 +710,7 @@ extern "C" int moe_dispatch_static(const int *topk_i, const int *pos, int n_toke
   // no GEMM follows: with no column tiles the plan kernel writes no tile tables
   d.tiles_gate_up = d.tiles_down = nullptr;
   d.tile_cap_gate_up = d.tile_cap_down = 0;
-  const hipError_t el = launch_dispatch(topk_i, pos, n_tokens, n_experts, 0, 0, kTileRows, false, TileCost{0, 0}, d,
+  const hipError_t el = launch_dispatch(topk_i, pos, n_tokens, n_experts, 0, 0, kTileRows, false, TileCost{}, d,
                                        static_cast<hipStream_t>(stream));
   if (el != hipSuccess)
     return set_error(MOE_ERR_HIP, "dispatch launch failed: %s", hipGetErrorString(el));

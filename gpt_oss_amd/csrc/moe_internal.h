@@ -154,10 +154,12 @@ struct DispatchBuffers {
   TileDesc *tiles_down;     // [tile_cap_down]    ... of the down GEMM
   int tile_cap_gate_up, tile_cap_down;
 };
-// Fixed part of a tile's estimated cost (plan_tile_cost), and another (0: none) that a GEMM of few rounds of tiles may
-// be cut by instead.
+// How the XCDs' ranges of tiles are cut (plan_tile_cost): the fixed part of a tile's estimated cost, and another
+// (0: none) that a GEMM of up to `rounds` rounds of tiles on the CUs is cut by instead, where with it the slowest XCD's
+// time, estimated with fixed part `slow`, is below `gain` of what it is otherwise.
 struct TileCost {
-  int fixed, few;
+  int fixed, few, rounds, slow;
+  float gain;
 };
 // tile_rows: tallest row tile of the plan (kTileRows or kHalfTileRows); wide: tile_width; nb_*: column blocks of an
 // expert's matrices (0: no tile tables)
@@ -327,19 +329,22 @@ inline int plan_tile_rows(int T, int E, int H, int IM, bool mxfp4, bool cached) 
 // gemm_fp4.hip, 12 / 20 / 32: 32 experts, 512 (1.2) 183 / 184 / 184, 2000 (0.6) 390 / 389 / 390, 7168 (1.2) 1162 /
 // 1156 / 1165, even, 1000 252 / 245 / 246.
 //
-// Few rounds, bf16 past the caches: an XCD that gets one tile more than its CUs take at a time begins another
+// Few rounds, bf16: an XCD that gets one tile more than its CUs take at a time begins another
 // round, which a cut by cost does not see.  With 64 an XCD of tall tiles had 35 to 40 of the down GEMM's at 32 experts,
-// 350 to 500 tokens (1.2), with 32 no more than its 32, and the others 60 of low ones.  So a GEMM of up to two rounds of
-// tiles is cut by 32 where the slowest XCD's time (its rounds times its tiles' mean cost, with a fixed part of 96: 64 to
-// 128 predict the measured times best) is estimated 2 % lower.  us per call, 64 throughout / this: 32 experts, 256
-// (1.2) 307 / 298, 350 317 / 305, 400 325 / 311, 450 337 / 315, 480 338 / 319, 560 (0.6) 326 / 318; 16 experts, 200 (1.2)
-// 175 / 167; 32 experts of 2048 x 1440, 400 (1.2) 143 / 136.  Over 396 batches of 8 to 128 experts, 100 to 7000 tokens, no
-// GEMM that this cuts by 32 was slower by more than 1 %; without the 2 % or with more rounds some were, by 2 to 10.
-constexpr int kFewRounds = 2, kFewRoundsCost = 96;
-constexpr float kFewRoundsGain = 0.98f;
+// 350 to 500 tokens (1.2), with 32 no more than its 32, and the others 60 of low ones.  So a GEMM of few rounds of
+// tiles is cut by 32 where the slowest XCD's time (its rounds times its tiles' mean cost) is expected to be lower.
+// Past the caches, up to two rounds, a fixed part of 96 and 2 % predict the measured times best: us per call, 64
+// throughout / this: 32 experts, 256 (1.2) 307 / 298, 350 317 / 305, 400 325 / 311, 450 337 / 315, 480 338 / 319, 560 (0.6)
+// 326 / 318; 16 experts, 200 (1.2) 175 / 167; 32 experts of 2048 x 1440, 400 (1.2) 143 / 136; over 396 batches of 8 to 128
+// experts, 100 to 7000 tokens, no GEMM that this cuts by 32 was slower by more than 1 %; without the 2 % or with more
+// rounds some were, by 2 to 10.  Through the caches, where a tile's columns cost it less, up to three rounds, 64 and
+// 5 %: 128 experts of 512 x 512, 4000 tokens (1.2) 93.8 / 89.7, 4500 102.6 / 96.2, 5000 107.4 / 100.8, of 800 x 320, 1500,
+// even, 67.5 / 62.7; 32 experts of 1024 x 1024, 1000 (0.6) 70.5 / 67.2; over 1356 batches 0.874 to 1.031 of the time with
+// 64 throughout.  (32 throughout is as quick on average there, 0.82 to 1.18 from batch to batch: what the last rounds do
+// beyond their number is not foreseen.)
 inline TileCost plan_tile_cost(int T, int E, int w1_rows, bool mxfp4, bool past_caches) {
-  if (mxfp4) return {fp4_many_rows(T, E, w1_rows) ? 32 : 12, 0};
-  return {64, past_caches ? 32 : 0};
+  if (mxfp4) return {fp4_many_rows(T, E, w1_rows) ? 32 : 12, 0, 0, 0, 0.f};
+  return past_caches ? TileCost{64, 32, 2, 96, 0.98f} : TileCost{64, 32, 3, 64, 0.95f};
 }
 enum TileKernel { kBf16Tiles /* gemm_bf16.hip */, kFp4Tiles /* gemm.hip */, kFp4ManyTiles /* gemm_fp4.hip */ };
 struct TileRoute {
