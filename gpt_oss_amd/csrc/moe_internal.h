@@ -291,10 +291,13 @@ inline bool gemm_streams_weights(int T, int E, bool mxfp4, int tile_rows, bool c
 // bf16 weights past the caches: whether tiles of up to 6 row blocks take 10 column blocks instead of 8 (the
 // registers and the LDS of a workgroup hold 60 as well as 64).  A tile streams its weights for its
 // whole life but for a fill and an epilogue, and reads its rows once per tile: fewer tiles, less of either.  But a
-// wider tile makes the CUs' last round of tiles longer, so there have to be rounds enough.  us per
-// layer call, 8 / 10 column blocks: 128 experts, 6144 tokens (9 rounds in gate_up, 4.5 in down) 1555 / 1457, 2000, Zipf's
-// routing, 1211 / 1205; 32 experts, 256 tokens (2.3, 1.1) 294 / 329, 672 of 896 315 / 354, 512, Zipf's, 346 /
-// 340, 1400 (exponent 0.6) 415 / 390; 8 experts, 250 135 / 152.
+// wider tile makes the CUs' last round of tiles longer, so there have to be rounds enough that it is small beside the
+// others whatever the routing, which the host does not know.  us per moe_experts call, 8 / 10 column blocks, means of two
+// to four routings, even or Zipf's (exponent in brackets): 128 experts (9 rounds in gate_up, 4.5 in down at 6144 tokens),
+// 6144, even, 1555 / 1457 per layer call, 4000 1206 / 1164, (0.6) 1393 / 1360, (1.2) 1530 / 1500, 2000, even, 1102 / 1095,
+// (1.2) 1185 / 1188, 600, even, 1000 / 1012, (1.2) 861 / 842.  32 experts (2.3 rounds, 1.1), where either may win: even, 256
+// 277 / 308, 512 281 / 320, 1000 313 / 351, 1400 350 / 387, but (1.2) 450 337 / 310, 512 331 / 322, 600 339 / 345, (0.6) 1400
+// 417 / 403; 1800 405 / 399, (0.6) 460 / 441.  8 experts, 250, even, 116 / 130, 500 167 / 143.
 inline bool bf16_wide_tiles(int T, int E, int H, int IM, bool past_caches) {
   const int cols = (H < 2 * IM ? H : 2 * IM) / kRowBlock;
   const int row_tiles = T * kTopK / kTileRows > E ? T * kTopK / kTileRows : E;

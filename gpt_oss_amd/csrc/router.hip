@@ -43,11 +43,10 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 __host__ __device__ constexpr float router_gamma(int flush) { return 2.0f * 33.0f * flush * 1.1920929e-7f; }
 constexpr int kNone = 0x7fffffff;
 
-// The selection's rule is that of the reference's CPU top-k under a stable sort: value descending, index
-// ascending, where a candidate replaces the incumbent (the one with the lower index) only if it compares strictly
-// greater.  Beside a NaN that does not order the logits, and comparisons of parts of them do not give
-// what one walk over all gives: that is the greatest number left, but a NaN while it is the first
-// expert left (a row of NaNs selects 0, 1, 2, 3).
+// The selection's rule is that of the reference's CPU top-k under a stable sort (run.cpp:388-421): value descending,
+// index ascending.  Beside NaNs, which no sort orders, it is that of one walk over the experts left, from the first on,
+// where a candidate replaces the incumbent only if it compares strictly greater: the greatest number
+// left, but a NaN while it is the first expert left (a row of NaNs selects 0, 1, 2, 3).
 //
 // A logit as a whole number of the same order, zeros of either sign the same one.
 constexpr uint32_t kTakenKey = 0u, kNanKey = 1u;  // below every number's, minus infinity's too
