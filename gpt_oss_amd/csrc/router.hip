@@ -58,22 +58,26 @@ __device__ __forceinline__ float key_value(uint32_t key) {  // kNanKey: a NaN
   return __uint_as_float(key ^ (~(uint32_t)((int32_t)key >> 31) | 0x80000000u));
 }
 
-// Among the LPT lanes of a token (a wave, or either half of one): the largest value, in every lane, and the first
-// lane that has something, which one of them does.
-template <int LPT>
-__device__ __forceinline__ uint32_t lanes_max(uint32_t x) {
+// Among the LPT lanes of a token (a wave, or either half of one): the largest value of each of N tokens, in every lane, and
+// the first lane that has something, which one of them does.
+template <int LPT, int N>
+__device__ __forceinline__ void lanes_max(uint32_t (&x)[N]) {
   static_assert(LPT == 32 || LPT == 64, "a token has a wave or half of one");
-#define MOE_DPP_MAX(CTRL, ROWS) \
-  x = max(x, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, CTRL, ROWS, 0xf, false))
+#define MOE_DPP_MAX(CTRL, ROWS)                                                                              \
+  _Pragma("unroll") for (int n = 0; n < N; n++)                                                               \
+    x[n] = max(x[n], (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x[n], CTRL, ROWS, 0xf, false))
   MOE_DPP_MAX(0x111, 0xf);  // row_shr 1, 2, 4, 8: lane 15 of a row of 16 has the row's
   MOE_DPP_MAX(0x112, 0xf);
   MOE_DPP_MAX(0x114, 0xf);
   MOE_DPP_MAX(0x118, 0xf);
   MOE_DPP_MAX(0x142, 0xa);  // row_bcast15 into rows 1 and 3, row_bcast31 into 2 and 3
-  if (LPT == 64) MOE_DPP_MAX(0x143, 0xc);
+  if constexpr (LPT == 64) MOE_DPP_MAX(0x143, 0xc);
 #undef MOE_DPP_MAX
-  const uint32_t high = (uint32_t)__builtin_amdgcn_readlane((int)x, 63);
-  return LPT == 64 || (threadIdx.x & 32) ? high : (uint32_t)__builtin_amdgcn_readlane((int)x, 31);
+#pragma unroll
+  for (int n = 0; n < N; n++) {
+    const uint32_t high = (uint32_t)__builtin_amdgcn_readlane((int)x[n], 63);
+    x[n] = LPT == 64 || (threadIdx.x & 32) ? high : (uint32_t)__builtin_amdgcn_readlane((int)x[n], 31);
+  }
 }
 template <int LPT>
 __device__ __forceinline__ int first_lane(bool has) {
@@ -81,57 +85,70 @@ __device__ __forceinline__ int first_lane(bool has) {
   return LPT == 64 ? __builtin_ctzll(m) : __builtin_ctz((uint32_t)(m >> (threadIdx.x & 32)));
 }
 
-// Top-NSEL of a token's keys, lane q of its LPT owning those of experts q*PER .. q*PER+PER-1; places past the
-// experts hold kTakenKey.  A round is a maximum over the lanes and the first one that holds it.  NANS: there may be
-// NaNs.  All lanes end with the same result, kNone where no expert is left (a whole wave has more than 32).
-template <int PER, int LPT, int NSEL, bool NANS>
-__device__ __forceinline__ void top_keys(uint32_t (&key)[PER], int q, float (&sel_v)[NSEL], int (&sel_i)[NSEL]) {
+// Top-NSEL of the keys of N tokens side by side, lane q of a token's LPT owning those of experts q*PER .. q*PER+PER-1;
+// places past the experts hold kTakenKey.  A round is a maximum over the lanes and the first one that holds it.  NANS:
+// there may be NaNs.  All lanes end with the same result, kNone where no expert is left (a whole wave has more than 32).
+template <int PER, int LPT, int N, int NSEL, bool NANS>
+__device__ __forceinline__ void top_keys(uint32_t (&key)[N][PER], int q, float (&sel_v)[N][NSEL],
+                                         int (&sel_i)[N][NSEL]) {
   static_assert(LPT == 64 || PER == 1, "a lane of half a wave has one expert");
 #pragma unroll
   for (int r = 0; r < NSEL; r++) {
-    uint32_t own = key[0];
+    uint32_t own[N], best[N];
 #pragma unroll
-    for (int j = 1; j < PER; j++) own = max(own, key[j]);
-    uint32_t best = lanes_max<LPT>(own);
-    int l = first_lane<LPT>(own == best);
-    if constexpr (NANS) {
-      uint32_t first = kTakenKey;  // the lane's first key that is left
+    for (int n = 0; n < N; n++) {
+      own[n] = key[n][0];
+#pragma unroll
+      for (int j = 1; j < PER; j++) own[n] = max(own[n], key[n][j]);
+      best[n] = own[n];
+    }
+    lanes_max<LPT, N>(best);
+#pragma unroll
+    for (int n = 0; n < N; n++) {
+      int l = first_lane<LPT>(own[n] == best[n]);
+      if constexpr (NANS) {
+        uint32_t first = kTakenKey;  // the lane's first key that is left
+#pragma unroll
+        for (int j = PER - 1; j >= 0; j--)
+          if (key[n][j] != kTakenKey) first = key[n][j];
+        const int lf = first_lane<LPT>(first != kTakenKey || best[n] == kTakenKey);
+        if (__shfl((int)first, lf, LPT) == (int)kNanKey) {
+          best[n] = kNanKey;
+          l = lf;
+        }
+      }
+      int at = 0;
 #pragma unroll
       for (int j = PER - 1; j >= 0; j--)
-        if (key[j] != kTakenKey) first = key[j];
-      const int lf = first_lane<LPT>(first != kTakenKey || best == kTakenKey);
-      if (__shfl((int)first, lf, LPT) == (int)kNanKey) {
-        best = kNanKey;
-        l = lf;
-      }
+        if (key[n][j] == best[n]) at = j;
+      sel_v[n][r] = key_value(best[n]);
+      if constexpr (LPT == 64) sel_i[n][r] = l * PER + __builtin_amdgcn_readlane(at, l);
+      else sel_i[n][r] = best[n] == kTakenKey ? kNone : l;
+#pragma unroll
+      for (int j = 0; j < PER; j++)
+        if (q == l && at == j) key[n][j] = kTakenKey;
     }
-    int at = 0;
-#pragma unroll
-    for (int j = PER - 1; j >= 0; j--)
-      if (key[j] == best) at = j;
-    sel_v[r] = key_value(best);
-    if constexpr (LPT == 64) sel_i[r] = l * PER + __builtin_amdgcn_readlane(at, l);
-    else sel_i[r] = best == kTakenKey ? kNone : l;
-#pragma unroll
-    for (int j = 0; j < PER; j++)
-      if (q == l && at == j) key[j] = kTakenKey;
   }
 }
 
-// One token on a whole wave (more than 32 experts).  Eight lanes per token with 16 experts
-// each took 5.5 us for the 16 tokens of a workgroup and 128 experts.
-template <int PER, int NSEL>
-__device__ __forceinline__ void wave_top(const float (&v)[PER], int lane, int E, float (&sel_v)[NSEL],
-                                         int (&sel_i)[NSEL]) {
+// N tokens on a whole wave (more than 32 experts).  A chain of latencies, so two tokens go side by side, and their
+// softmax and stores, too, on lanes of their own.  us of moe_router, with eight or sixteen lanes per token and
+// comparisons / a wave for one token after the other / this: 128 experts of 2880, 24 tokens 16.4 / 16.9 / 14.7, 200 26.4 /
+// 23.3 / 21.2, 7168 37.8 / 40.3 / 35.6; of 512, 64 9.6 / 10.3 / 7.7, 7168 21.2 / 22.4 / 17.9; 64 of 512, 64 8.5 / 6.8 / 6.1.
+template <int PER, int N, int NSEL>
+__device__ __forceinline__ void wave_top(const float (&v)[N][PER], int lane, int E, float (&sel_v)[N][NSEL],
+                                         int (&sel_i)[N][NSEL]) {
   bool nan = false;
-  uint32_t key[PER];
+  uint32_t key[N][PER];
 #pragma unroll
-  for (int j = 0; j < PER; j++) {
-    key[j] = lane * PER + j < E ? order_key(v[j]) : kTakenKey;
-    nan |= key[j] == kNanKey;
-  }
-  if (__ballot(nan) != 0ull) top_keys<PER, 64, NSEL, true>(key, lane, sel_v, sel_i);
-  else top_keys<PER, 64, NSEL, false>(key, lane, sel_v, sel_i);
+  for (int n = 0; n < N; n++)
+#pragma unroll
+    for (int j = 0; j < PER; j++) {
+      key[n][j] = lane * PER + j < E ? order_key(v[n][j]) : kTakenKey;
+      nan |= key[n][j] == kNanKey;
+    }
+  if (__ballot(nan) != 0ull) top_keys<PER, 64, N, NSEL, true>(key, lane, sel_v, sel_i);
+  else top_keys<PER, 64, N, NSEL, false>(key, lane, sel_v, sel_i);
 }
 
 // Top-NSEL of one token's logits for up to 32 experts, one lane per expert (the
@@ -171,8 +188,15 @@ __device__ __forceinline__ void ranked_top(const float4 *row4, float v, int e, i
     redo |= r < E && sel_i[r] == kNone;
   }
   if (__ballot(redo) != 0ull) {
-    uint32_t key[1] = {e < E ? order_key(v) : kTakenKey};
-    top_keys<1, 32, NSEL, true>(key, e, sel_v, sel_i);
+    uint32_t key[1][1] = {{e < E ? order_key(v) : kTakenKey}};
+    float best_v[1][NSEL];
+    int best_i[1][NSEL];
+    top_keys<1, 32, 1, NSEL, true>(key, e, best_v, best_i);
+#pragma unroll
+    for (int r = 0; r < NSEL; r++) {
+      sel_v[r] = best_v[0][r];
+      sel_i[r] = best_i[0][r];
+    }
   }
 }
 
@@ -236,13 +260,13 @@ __global__ __launch_bounds__(WPC * 64) void router_kernel(
   constexpr int TOK = MT * 16;
   // selection: LPT lanes per token, each owning PER experts.
   // Up to 32 experts: one lane per expert, places found by counting (ranked_top), SW waves take part.
-  // More: the waves take the tokens in turn (wave_top).
+  // More: the waves take the tokens in turn, two at a time (wave_top), and then a wave's tokens have OWN lanes each.
   constexpr bool RANKED = E_pad <= 32;
   constexpr int LPT = RANKED ? 32 : 64;
   constexpr int PER = RANKED ? 1 : E_pad / LPT;
   constexpr int SW = TOK * LPT / 64;
-  constexpr int TPV = RANKED ? 1 : TOK / WPC;  // tokens of a wave, one after the other
-  static_assert(RANKED ? SW <= WPC : TOK % WPC == 0, "waves of the selection");
+  constexpr int TPV = RANKED ? 2 : TOK / WPC, OWN = 64 / TPV;  // tokens of a wave
+  static_assert(RANKED ? SW <= WPC : TOK % WPC == 0 && TPV % 2 == 0 && OWN >= 2 * kTopK, "waves of the selection");
   constexpr int LOG_LD = RANKED ? E_pad + 4 : E_pad + 1;  // RANKED reads rows of logits in 16-byte pieces
   // cross-wave sum: GB blocks of 16 x 16 outputs at a time through 32 KB
   constexpr int NBLK = MT * NT;
@@ -266,15 +290,10 @@ __global__ __launch_bounds__(WPC * 64) void router_kernel(
   const int kc_total = H / 32;
   if (tid == 0) n_tasks = 0;
   if (tid < E_pad) sh_br[tid] = br[tid];
-  const int q = lane % LPT;  // place among the token's lanes
-  const int tr = RANKED ? w * (64 / LPT) + lane / LPT : w;  // (first) token within the workgroup
-  const int t = tok0 + tr;
-  bool active[TPV];  // asked for long before it is needed
-#pragma unroll
-  for (int i = 0; i < TPV; i++) {
-    const int ti = t + i * WPC;
-    active[i] = (!RANKED || w < SW) && ti < T && !(pos && pos[min(ti, T - 1)] < 0);
-  }
+  const int q = lane % OWN;  // place among the token's lanes
+  auto token_of = [&](int i) { return RANKED ? w * TPV + i : w + i * WPC; };  // a wave's token i within the workgroup
+  const int tr = token_of(lane / OWN), t = tok0 + tr;
+  const bool active = (!RANKED || w < SW) && t < T && !(pos && pos[min(t, T - 1)] < 0);  // asked for long before it is needed
   const float wn_max = rstat[0], bmax = rstat[1];
 
   if constexpr (SPLIT) {
@@ -398,8 +417,7 @@ __global__ __launch_bounds__(WPC * 64) void router_kernel(
   }
 
   // Pass 2, selection.
-  bool undecided = false;    // RANKED: the half wave's token
-  unsigned undecided_of = 0;  // otherwise bit i: the wave's token i
+  bool undecided = false;  // the lane's token
   auto bound = [&](int tr) {
     float ss = 0.f;
 #pragma unroll
@@ -410,7 +428,7 @@ __global__ __launch_bounds__(WPC * 64) void router_kernel(
     *reinterpret_cast<int4 *>(topk_i + (size_t)t * kTopK) = make_int4(-1, -1, -1, -1);
     *reinterpret_cast<float4 *>(topk_v + (size_t)t * kTopK) = make_float4(0.f, 0.f, 0.f, 0.f);
   };
-  // Written out for either form: as one function of a token, or one loop over a wave's, it cost batches of up to 64 tokens
+  // Written out for either form: as one function of a token it cost batches of up to 64 tokens
   // 0.1 to 0.2 us where RANKED (one token, MXFP4, 24.62 / 24.75 us per call).
   if constexpr (RANKED) {
     if (w < SW) {
@@ -418,7 +436,7 @@ __global__ __launch_bounds__(WPC * 64) void router_kernel(
       float s_v[kTopK + 1];
       int s_i[kTopK + 1];
       ranked_top<E_pad, kTopK + 1>(reinterpret_cast<const float4 *>(&logits[tr][0]), v, q, E, posted[tr], s_v, s_i);
-      if (active[0]) {
+      if (active) {
         const LogitBound lb = bound(tr);
         if (lb.decides(s_v, s_i)) {
           // (tokens of one wave can differ here: the shuffles inside are among the
@@ -435,35 +453,45 @@ __global__ __launch_bounds__(WPC * 64) void router_kernel(
       }
     }
   } else {
+    float s_v[kTopK + 1] = {};  // of the lane's token
+    int s_i[kTopK + 1] = {};
 #pragma unroll 1
-    for (int i = 0; i < TPV; i++) {
-      const int tri = tr + i * WPC, ti = t + i * WPC;
-      bool is_active = active[0];
+    for (int i = 0; i < TPV; i += 2) {
+      float v[2][PER], two_v[2][kTopK + 1];
+      int two_i[2][kTopK + 1];
 #pragma unroll
-      for (int k = 1; k < TPV; k++)
-        if (k == i) is_active = active[k];
-      float v[PER];
+      for (int n = 0; n < 2; n++)
 #pragma unroll
-      for (int j = 0; j < PER; j++) v[j] = logits[tri][q * PER + j];
-      float s_v[kTopK + 1];
-      int s_i[kTopK + 1];
-      wave_top<PER, kTopK + 1>(v, q, E, s_v, s_i);
-      if (is_active) {
-        const LogitBound lb = bound(tri);
-        if (lb.decides(s_v, s_i)) {
-          const float sv[kTopK] = {s_v[0], s_v[1], s_v[2], s_v[3]};
-          const int si[kTopK] = {s_i[0], s_i[1], s_i[2], s_i[3]};
-          store_topk_spread(sv, si, q, lane - q, topk_i + (size_t)ti * kTopK, topk_v + (size_t)ti * kTopK);
-        } else {
-          undecided_of |= 1u << i;
+        for (int j = 0; j < PER; j++) v[n][j] = logits[token_of(i + n)][lane * PER + j];
+      wave_top<PER, 2, kTopK + 1>(v, lane, E, two_v, two_i);
 #pragma unroll
-          for (int j = 0; j < PER; j++) {
-            const int e = q * PER + j;
-            if (e < E && lb.contends(v[j], s_v[3])) tasks[atomicAdd(&n_tasks, 1)] = (unsigned short)(tri * E_pad + e);
+      for (int n = 0; n < 2; n++)
+#pragma unroll
+        for (int r = 0; r <= kTopK; r++)
+          if (lane / OWN == i + n) {
+            s_v[r] = two_v[n][r];
+            s_i[r] = two_i[n][r];
           }
-        }
-      } else if (ti < T && q == 0) {
-        store_inactive(ti);
+    }
+    if (active) {
+      if (bound(tr).decides(s_v, s_i)) {
+        const float sv[kTopK] = {s_v[0], s_v[1], s_v[2], s_v[3]};
+        const int si[kTopK] = {s_i[0], s_i[1], s_i[2], s_i[3]};
+        store_topk_spread(sv, si, q, lane - q, topk_i + (size_t)t * kTopK, topk_v + (size_t)t * kTopK);
+      } else {
+        undecided = true;
+      }
+    } else if (t < T && q == 0) {
+      store_inactive(t);
+    }
+    for (unsigned long long left = __ballot(undecided && q == 0); left; left &= left - 1) {
+      const int l = __builtin_ctzll(left), tri = token_of(l / OWN);
+      const LogitBound lb = bound(tri);
+      const float fourth = __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(s_v[3]), l));
+#pragma unroll
+      for (int j = 0; j < PER; j++) {
+        const int e = lane * PER + j;
+        if (e < E && lb.contends(logits[tri][e], fourth)) tasks[atomicAdd(&n_tasks, 1)] = (unsigned short)(tri * E_pad + e);
       }
     }
   }
@@ -537,15 +565,14 @@ __global__ __launch_bounds__(WPC * 64) void router_kernel(
       if (undecided) store_topk_spread(s_v, s_i, q, lane - q, topk_i + (size_t)t * kTopK, topk_v + (size_t)t * kTopK);
     }
   } else {
-    for (; undecided_of; undecided_of &= undecided_of - 1u) {  // the same in all lanes
-      const int d = __builtin_ctz(undecided_of) * WPC;
-      float v[PER];
+    for (unsigned long long left = __ballot(undecided && q == 0); left; left &= left - 1) {
+      const int tri = token_of(__builtin_ctzll(left) / OWN);
+      float v[1][PER], s_v[1][kTopK];
+      int s_i[1][kTopK];
 #pragma unroll
-      for (int j = 0; j < PER; j++) v[j] = logits[tr + d][q * PER + j];
-      float s_v[kTopK];
-      int s_i[kTopK];
-      wave_top<PER, kTopK>(v, q, E, s_v, s_i);
-      store_topk_spread(s_v, s_i, q, 0, topk_i + (size_t)(t + d) * kTopK, topk_v + (size_t)(t + d) * kTopK);
+      for (int j = 0; j < PER; j++) v[0][j] = logits[tri][lane * PER + j];
+      wave_top<PER, 1, kTopK>(v, lane, E, s_v, s_i);
+      store_topk_spread(s_v[0], s_i[0], lane, 0, topk_i + (size_t)(tok0 + tri) * kTopK, topk_v + (size_t)(tok0 + tri) * kTopK);
     }
   }
   if (score) {
@@ -563,8 +590,8 @@ __global__ __launch_bounds__(WPC * 64) void router_kernel(
 // of them.  The same chunks to the same four waves and the same order of the sums: the same
 // bits.  Written to `first` (see SPLIT), which a second launch reads.  us at 128 experts and
 // 2880 columns, one kernel / both launches, with the selection by eight lanes per token: 6 tokens 16.7 / 5.0
-// + 6.3, 200 tokens 32.5 / 7.7 + 17.2; with wave_top the second launch takes 4.1 and 12.9 (of which the
-// second pass of a few undecided tokens).
+// + 6.3, 200 tokens 32.5 / 7.7 + 17.2; with wave_top the second launch takes 4.3 and, by the tokens
+// that take the second pass, 9 to 13.
 template <int D>
 __global__ __launch_bounds__(kSplitWaves * 64) void router_logits_kernel(
     const uint16_t *__restrict__ x, const uint16_t *__restrict__ wr, const float *__restrict__ br, int T, int H,
