@@ -240,7 +240,7 @@ def _check_ids(m, L, x, pos, E):
     return R, score, ti
 
 
-@pytest.mark.parametrize("E,T", [(32, 2048), (128, 1000), (256, 300)])
+@pytest.mark.parametrize("E,T", [(32, 2048), (128, 1000), (128, 4111), (256, 300)])
 def test_router_near_ties(E, T):
     """Logits one bf16 step of one weight apart, and exactly
     equal ones, at the top of every token's ranking: the first pass of the
